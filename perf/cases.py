@@ -252,3 +252,119 @@ def tolerance(case):
     if case["kind"] in ("linear", "mixed"):
         return {"rel": 4e-4}
     return {"rel": 1.4e-3}
+
+
+# What run() returns, in 64 bits from plain torch.  The decoded weights are part of the path's definition (every step of a
+# type's decode rounds to fp16, the result to bf16), so the decode below keeps those steps; the sums, the norm and the
+# gated product behind it are in 64 bits throughout.
+def _fp16(blocks, at):
+    return blocks[:, at:at + 2].contiguous().view(torch.float16)
+
+
+def _bits(b, shifts, mask):
+    """Bytes [n, groups, width] -> [n, groups * shifts, width]: the fields at each shift, lowest first."""
+    s = torch.tensor(shifts, dtype=torch.uint8, device=b.device).reshape(1, 1, -1, 1)
+    return ((b.unsqueeze(2) >> s) & mask).reshape(b.shape[0], -1, b.shape[2])
+
+
+def _six_bit_pairs(s):
+    low, high, top = s[:, 0:4], s[:, 4:8], s[:, 8:12]
+    return (torch.cat([low & 63, (top & 15) | ((low >> 2) & 48)], 1), torch.cat([high & 63, (top >> 4) | ((high >> 2) & 48)], 1))
+
+
+def _decoded(qtype, packed):
+    """Packed rows -> the fp16 weights [n, k] (bf16 weights: as they are)."""
+    if qtype == "bf16":
+        return packed.view(torch.bfloat16)
+    n = packed.shape[0]
+    b = packed.reshape(-1, GGML_QUANT_SIZES[TYPES[qtype]][1])
+    if qtype == "q8_0":
+        w = _fp16(b, 0) * b[:, 2:].contiguous().view(torch.int8)
+    elif qtype in ("q4_0", "q4_1", "q5_0", "q5_1"):
+        at = 4 if qtype[-1] == "1" else 2
+        fifth = qtype[1] == "5"
+        q = _bits(b[:, at + (4 if fifth else 0):].unsqueeze(1), [0, 4], 15).reshape(-1, 32)
+        if fifth:
+            q = q | (_bits(b[:, at:at + 4].unsqueeze(1), range(8), 1).transpose(1, 2).reshape(-1, 32) << 4)
+        w = _fp16(b, 0) * q + _fp16(b, 2) if qtype[-1] == "1" else _fp16(b, 0) * (q.to(torch.int8) - (16 if fifth else 8))
+    elif qtype == "q2_k":
+        q = _bits(b[:, 16:80].reshape(-1, 2, 32), [0, 2, 4, 6], 3).reshape(-1, 16, 16)
+        w = (_fp16(b, 80) * (b[:, :16] & 15)).unsqueeze(2) * q - (_fp16(b, 82) * (b[:, :16] >> 4)).unsqueeze(2)
+    elif qtype == "q3_k":
+        q = _bits(b[:, 32:96].reshape(-1, 2, 32), [0, 2, 4, 6], 3).reshape(-1, 16, 16).to(torch.int8)
+        low = _bits(b[:, :32].unsqueeze(1), range(8), 1).reshape(-1, 16, 16).to(torch.int8)
+        s = _bits(b[:, 96:104].unsqueeze(1), [0, 4], 15).reshape(-1, 16) | (_bits(b[:, 104:108].unsqueeze(1), [0, 2, 4, 6], 3).reshape(-1, 16) << 4)
+        w = (_fp16(b, 108) * (s.to(torch.int8) - 32)).unsqueeze(2) * (q - 4 * (1 - low))
+    elif qtype in ("q4_k", "q5_k"):
+        scale, low = _six_bit_pairs(b[:, 4:16])
+        q = _bits(b[:, -128:].reshape(-1, 4, 32), [0, 4], 15)
+        if qtype == "q5_k":
+            q = q | (_bits(b[:, 16:48].unsqueeze(1), range(8), 1) << 4)
+        w = (_fp16(b, 0) * scale).unsqueeze(2) * q - (_fp16(b, 2) * low).unsqueeze(2)
+    else:
+        q = _bits(b[:, :128].reshape(-1, 2, 64), [0, 4], 15).reshape(-1, 16, 16)
+        q = q | (_bits(b[:, 128:192].reshape(-1, 2, 32), [0, 2, 4, 6], 3).reshape(-1, 16, 16) << 4)
+        w = (_fp16(b, 208) * b[:, 192:208].contiguous().view(torch.int8)).unsqueeze(2) * (q.to(torch.int8) - 32)
+    return w.reshape(n, -1)
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    seed = seed * 7919 + 17
+
+    def packed(qtype, n, k, s):
+        return synthetic.make_packed(TYPES[qtype], n, k, seed=s, device="cuda")
+
+    def weights(qtype, n, k, s):
+        return _decoded(qtype, packed(qtype, n, k, s)).to(torch.bfloat16).double()
+
+    def activations(rows, k, s):
+        return synthetic.make_activations(rows, k, seed=s, device="cuda").double()
+
+    if kind == "greedy":
+        return None
+    if kind == "dequantize":
+        return [_decoded(case["type"], packed(case["type"], case["n"], case["k"], seed + i)).double() for i in range(case["count"])]
+    rows = case["rows"]
+    if kind == "linear":
+        y = activations(rows, case["k"], seed + 2) @ weights(case["type"], case["n"], case["k"], seed).T
+        return y + activations(1, case["n"], seed + 1)[0] if case["bias"] else y
+    hidden = case["hidden"]
+    x, context = activations(rows, hidden, seed + 2), activations(rows, hidden, seed + 3)
+    shapes = _layer_shapes(case)
+
+    def weight(i, name):
+        qtype = case["down_type"] if name == "mlp.down_proj" else case["type"]
+        return weights(qtype, *shapes[name], seed * 1000 + i * 10 + list(shapes).index(name)).T
+
+    def mlp(i, rows):
+        return (torch.nn.functional.silu(rows @ weight(i, "mlp.gate_proj")) * (rows @ weight(i, "mlp.up_proj"))) @ weight(i, "mlp.down_proj")
+
+    out = []
+    if kind == "mixed":
+        image = torch.arange(rows, device="cuda") >= case["text"]
+        if case["scattered"]:
+            image = image[torch.randperm(rows, generator=torch.Generator().manual_seed(seed)).to("cuda")]
+        wide = activations(rows, case["inter"], seed + 4)
+        for name in shapes:
+            a = wide if name == "mlp.down_proj" else context if name == "o_proj" else x
+            y = torch.empty(rows, shapes[name][0], dtype=torch.float64, device="cuda")
+            y[~image] = a[~image] @ weight(0, name)
+            y[image] = a[image] @ weight(1, name)
+            out.append(y)
+        return out
+    if kind == "folded":
+        gammas = (synthetic.make_activations(2, hidden, seed=seed + 4, device="cuda") * 0.1 + 1.0).double()
+
+        def norm(rows, gamma):
+            return rows * torch.rsqrt(rows.square().mean(1, keepdim=True) + EPS) * gamma
+    for i in range(case["layers"]):
+        a = norm(x, gammas[0]) if kind == "folded" else x
+        out += [a @ weight(i, name) for name in ("q_proj", "k_proj", "v_proj")]
+        h = context @ weight(i, "o_proj")
+        if kind == "folded":
+            h = h + x
+            out += [h, h + mlp(i, norm(h, gammas[1]))]
+        else:
+            out += [h, mlp(i, x)]
+    return out
