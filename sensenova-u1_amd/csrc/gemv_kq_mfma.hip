@@ -663,12 +663,15 @@ int launch_r(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64
     const int nsb = (int)(K >> 8);
     const int mt = (M + 15) / 16;
     // wavefronts per row group: enough that the launch fills the chip (about 12 per compute unit),
-    // at least one super-block each, at most 8 per workgroup
-    const int64_t per_group = gated ? 2 : 1;
-    int64_t w = (256 * 12 + groups * per_group - 1) / (groups * per_group);
+    // at least one super-block each, at most 8 per workgroup.  Beyond 16 rows they are counted per 16 weight rows whatever
+    // R is, so that a row's K is cut into the same pieces (and its partial sums are added in the same order) for both.
+    const int64_t per_group = gated ? 2 : 1, counted = mt > 1 ? (N + 15) / 16 : groups;
+    int64_t w = (256 * 12 + counted * per_group - 1) / (counted * per_group);
     if (w < 1) w = 1;
     if (w > nsb) w = nsb;
-    const int64_t cap = gated ? 4 : 8;
+    // long rows beyond 16 activation rows, every compute unit with a workgroup: four wavefronts with twice the run of K
+    // each (4096 x 12288, 40 rows: Q8_0 35.9 against 38.2 us, Q6_K 37.2 against 38.9)
+    const int64_t cap = gated || (mt > 1 && nsb >= 32 && groups >= 256) ? 4 : 8;
     if (w > cap) w = cap;
     const int waves = (int)(gated ? 2 * w : w);
     const size_t slab = (size_t)waves * 16 * R * Slab<QT>::stride;
@@ -711,15 +714,21 @@ int launch_r(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64
 #define SNGGUF_LAUNCH(G, WM, MT_) \
     gemv_kq_mfma_kernel<QT, NUM, R, G, WM, MT_><<<grid, block, lds_bytes, stream>>>(x, M, qa, qb, N, K, bias, residual, y, nullptr, 0.f, amax)
     if (mt > 1) {
-        // more than 16 activation rows: plain projections with one row group per wavefront only
-        if constexpr (R == 1) {
-            if (gated || mt > 4) return SNGGUF_E_BADSHAPE;
-            if (mt == 2) SNGGUF_LAUNCH(false, 8, 2);
-            else if (mt == 3) SNGGUF_LAUNCH(false, 8, 3);
-            else SNGGUF_LAUNCH(false, 8, 4);
-        } else {
-            return SNGGUF_E_BADSHAPE;
-        }
+        // more than 16 activation rows: plain projections only.  The slabs of two row groups on eight wavefronts can pass
+        // the default dynamic-LDS limit: raised once per kernel instance
+        if (gated || mt > 4) return SNGGUF_E_BADSHAPE;
+#define SNGGUF_LAUNCH_MT(MT_)                                                                                          \
+    do {                                                                                                               \
+        static const hipError_t attr = hipFuncSetAttribute(                                                            \
+            reinterpret_cast<const void*>(&gemv_kq_mfma_kernel<QT, NUM, R, false, 8, MT_>),                            \
+            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                                                    \
+        if (attr != hipSuccess) return SNGGUF_E_LAUNCH;                                                                 \
+        SNGGUF_LAUNCH(false, 8, MT_);                                                                                   \
+    } while (0)
+        if (mt == 2) SNGGUF_LAUNCH_MT(2);
+        else if (mt == 3) SNGGUF_LAUNCH_MT(3);
+        else SNGGUF_LAUNCH_MT(4);
+#undef SNGGUF_LAUNCH_MT
     } else if (gated) {
         if (waves <= 4) SNGGUF_LAUNCH(true, 4, 1);
         else SNGGUF_LAUNCH(true, 8, 1);
@@ -731,15 +740,20 @@ int launch_r(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64
     return hipGetLastError() == hipSuccess ? SNGGUF_OK : SNGGUF_E_LAUNCH;
 }
 
-// Row groups per wavefront (see launch_qt) as a function, so that the arg-max caller can size its slot array.
-inline int rows_per_workgroup(int64_t M, int64_t N) { return (N >= 32768 && M <= 16) ? 32 : 16; }
+// Weight rows per workgroup (see launch_qt) as a function, so that the arg-max caller can size its slot array.
+inline int rows_per_workgroup(int64_t M, int64_t N) { return (M <= 16 ? N >= 32768 : N > 4096) ? 32 : 16; }
 
 template <int QT, int NUM>
 int launch_qt(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64_t N, int64_t K, const bf16_t* bias,
               const bf16_t* residual, bf16_t* y, bool gated, const bf16_t* gamma, float eps, hipStream_t stream, uint64_t* amax) {
-    // Two row groups per wavefront only when one per wavefront would already give far more
-    // wavefronts than the chip holds (a vocabulary-sized projection): otherwise more, smaller
-    // workgroups spread more evenly over the 256 compute units.
+    // Up to 16 activation rows, two row groups per wavefront only when one per wavefront would already give far more
+    // wavefronts than the chip holds (a vocabulary-sized projection): otherwise more, smaller workgroups spread more
+    // evenly over the 256 compute units.  Beyond 16 rows what bounds the launch is the activation traffic - every
+    // workgroup reads all of x, 16 rows a fragment - and two or more operands take so many registers that a compute unit
+    // holds one workgroup of eight wavefronts: as soon as 16-row groups need a second round of workgroups (more than 256
+    // of them), 32 rows per workgroup halve both.  40 rows, Q8_0 / Q4_K: 6144 x 4096 28.9 -> 20.3 / 26.7 -> 19.1 us,
+    // 12288 x 4096 36.2 -> 31.9 / 34.2 -> 29.0 us; at 64 rows 39.8 -> 29.7 and 50.4 -> 47.3 us (Q8_0); where 16-row
+    // groups fit one round it loses (4096 x 4096, 40 rows: 15.2 -> 18.9 us).
     if (rows_per_workgroup(M, N) == 32) return launch_r<QT, NUM, 2>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax);
     return launch_r<QT, NUM, 1>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax);
 }
