@@ -35,6 +35,8 @@ int launch_gemm_dense(const void* x, int64_t M, const void* w, int64_t N, int64_
                       hipStream_t stream);
 int launch_dequantize_interleaved(const void* q, int qtype, int64_t rows, int64_t cols, void* out, int second, int numerics,
                                   hipStream_t stream);
+int launch_gemm_splitk_gated(const void* x, int64_t M, const void* q_gate, const void* q_up, int qtype, int64_t N, int64_t K, void* h,
+                             float* partial, int slices, int numerics, hipStream_t stream);
 int launch_gemm_dense_gated(const void* x, int64_t M, const void* w2, int64_t cols, int64_t K, void* h, hipStream_t stream);
 int launch_gemm(const void* x, int64_t M, const void* q, int qtype, int64_t N, int64_t K, const void* bias,
                 const void* residual, void* y,
@@ -242,6 +244,22 @@ int64_t pick_k_slices(int64_t M, int64_t N, int64_t tiles, int64_t ksteps, int64
     return best;
 }
 
+// The same for a gate / up pair in one launch (`tiles` of both): any number of rounds, since a pair's tiles come closer to
+// whole ones.  A round takes its K steps and about 5 us for the first loads and the partial sums' stores.  0 if there is
+// no room for one fp32 copy of each output.
+int64_t pick_pair_slices(int64_t M, int64_t N, int64_t tiles, int64_t ksteps, int64_t room) {
+    int64_t smax = room < ksteps / 2 ? room : ksteps / 2;   // at least two K steps per workgroup
+    if (smax > 64) smax = 64;
+    int64_t best = 0;
+    double best_t = 1e30;
+    for (int64_t sl = 1; sl <= smax; sl++) {
+        const double rounds = (double)((tiles * sl + 255) / 256);
+        const double t = rounds * ((double)((ksteps + sl - 1) / sl) * 1.9 + 5.0) + (double)sl * 16.0 * (double)M * (double)N / 5e6;   // us
+        if (t < best_t) { best_t = t; best = sl; }
+    }
+    return best;
+}
+
 bool dense_route_fits(int64_t M, int64_t N, int64_t K) {
     (void)N;
     return M >= 65 && K % 64 == 0 && M * K < ((int64_t)1 << 31);
@@ -350,6 +368,18 @@ int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const v
     if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return qtype == SNGGUF_TYPE_BF16 ? SNGGUF_E_BADTYPE : SNGGUF_E_BADSHAPE;
     if (workspace_bytes < sngguf_gate_up_silu_workspace_bytes(N, K)) return SNGGUF_E_BADSHAPE;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // Few output tiles: the gated launch has no K split and would leave much of the chip idle (below 512 rows, or tiles that
+    // fill less than 0.7 of their rounds), so both matrices run as one launch with K split over workgroups, and the
+    // reduction ends in the gated product.  Types the large-tile kernel decodes itself; the whole workspace is free for the
+    // partial sums.
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), gated_tiles = ((M + 255) / 256) * ((N + 127) / 128);
+    const bool fills = M >= 512 && 10 * gated_tiles >= 7 * 256 * ((gated_tiles + 255) / 256);
+    if ((qtype == SNGGUF_TYPE_Q8_0 || qtype == SNGGUF_TYPE_Q4_K) && M >= 65 && M < 4096 && tiles <= 128 && !fills) {
+        const int64_t slices = pick_pair_slices(M, N, 2 * tiles, K / 64, workspace_bytes / (8 * M * N));
+        if (slices >= 1)
+            return sngguf::launch_gemm_splitk_gated(x, M, q_gate, q_up, qtype, N, K, h, static_cast<float*>(workspace), (int)slices,
+                                                    numerics, s);
+    }
     int rd = sngguf::launch_dequantize_interleaved(q_gate, qtype, N, K, workspace, 0, numerics, s);
     if (rd != SNGGUF_OK) return rd;
     rd = sngguf::launch_dequantize_interleaved(q_up, qtype, N, K, workspace, 1, numerics, s);

@@ -303,6 +303,28 @@ int launch_gemm_splitk(const void* x, int64_t M, const void* q, int qtype, int64
     return launch_splitk_reduce(a, nullptr, M, stream);
 }
 
+int launch_splitk_reduce_gated(const float* gate, const float* up, int slices, int64_t M, int64_t N, bf16_t* h, hipStream_t stream);
+
+// h = silu(x Wg^T) * (x Wu^T): both matrices in one launch of the large-tile kernel, K split over `slices` >= 1 workgroups
+// per tile, and one reduction that ends in the gated product; `partial` holds 2 * slices * M * N floats.  qtype: Q8_0
+// (K % 64 == 0) or Q4_K, slices <= K / 64, N % 4 == 0, M K < 2^31 (checked by the caller).
+int launch_gemm_splitk_gated(const void* x, int64_t M, const void* q_gate, const void* q_up, int qtype, int64_t N, int64_t K, void* h,
+                             float* partial, int slices, int numerics, hipStream_t stream) {
+    GemmArgs a{};
+    a.x = static_cast<const bf16_t*>(x);
+    a.M = M; a.N = N; a.K = K;
+    a.n0 = M;
+    a.q[0] = static_cast<const uint8_t*>(q_gate);
+    a.q[1] = static_cast<const uint8_t*>(q_up);
+    a.group_mask = 1;
+    a.partial = partial;
+    a.ksplit = slices;
+    a.pair = true;
+    const int rc = launch_gemm_tiles(a, qtype, numerics, stream);
+    if (rc != SNGGUF_OK) return rc;
+    return launch_splitk_reduce_gated(partial, partial + (int64_t)slices * M * N, slices, M, N, static_cast<bf16_t*>(h), stream);
+}
+
 int64_t grouped_workspace_bytes(int64_t M) { return 16 + 4 * (M > 0 ? M : 0); }
 
 int launch_grouped_gemm(const void* x, int64_t M, const uint8_t* indicator, int64_t n_text, const void* q_und,

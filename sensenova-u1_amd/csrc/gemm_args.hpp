@@ -24,6 +24,9 @@ struct GemmArgs {
     // (no bias, no residual, nothing written to y); a second kernel adds the slices up.
     float* partial;
     int ksplit;
+    // Two matrices of one shape in one launch (large-tile kernel on packed weights, with `partial`, one row group): the column
+    // tiles of q[0] are followed by those of q[1], whose partial sums lie max(ksplit, 1) * M * N floats behind.
+    bool pair;
     // Gated pair (four-wavefront dense kernel only): the N weight rows are blocks of 128 gate rows, each followed by the
     // 128 up rows of the same output columns, and y is [M][gated_cols]: silu(gate) * up, rounded as the decode kernels'
     // gated pair rounds (no bias, no residual, no K split).  0 = a plain projection.

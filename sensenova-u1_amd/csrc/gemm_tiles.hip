@@ -116,7 +116,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(GemmArgs a) {
     const int64_t n0 = a.n0_dev ? (int64_t)*a.n0_dev : a.n0;
     const int64_t t0 = (a.group_mask & 1) ? (n0 + TM - 1) / TM : 0;            // row tiles of group 0
     const int64_t t1 = (a.group_mask & 2) ? (a.M - n0 + TM - 1) / TM : 0;      // row tiles of group 1
-    const int64_t ntn = (a.N + TN - 1) / TN;
+    const int64_t ntn = (a.N + TN - 1) / TN * (a.pair ? 2 : 1);                // column tiles (of both matrices of a pair)
     const int S = a.ksplit > 1 ? a.ksplit : 1;                                 // workgroups per output tile (K slices)
     const int64_t total = (t0 + t1) * ntn * S;
     const int64_t pid = blockIdx.x;
@@ -140,6 +140,8 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(GemmArgs a) {
         ty = tile / ntn;
         tn = tile - ty * ntn;
     }
+    const int second = a.pair && tn >= ntn / 2;   // matrix of a pair
+    if (second) tn -= ntn / 2;
     int g;
     int64_t row_begin, row_end;
     if (ty < t0) {
@@ -148,7 +150,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(GemmArgs a) {
         g = 1; row_begin = n0 + (ty - t0) * TM; row_end = a.M;
     }
     if (row_end > row_begin + TM) row_end = row_begin + TM;
-    const uint8_t* __restrict__ q = a.q[g];
+    const uint8_t* __restrict__ q = a.q[a.pair ? second : g];
     const bf16_t* __restrict__ bias = a.bias[g];
     const int64_t nb0 = tn * TN;
     const int64_t row_bytes = kDense ? 2 * a.K : kQ4K ? (a.K >> 8) * 144 : (a.K >> 5) * 34;
@@ -482,7 +484,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(GemmArgs a) {
     // lane: j = lane % 32; register v: i = 8 * (v / 4) + 4 * (lane / 32) + v % 4
     if (a.partial) {
         // K split over workgroups: this slice's sums go out as fp32, to be added up by splitk_reduce_kernel
-        float* part = a.partial + (int64_t)slice * a.M * a.N;
+        float* part = a.partial + ((int64_t)second * S + slice) * a.M * a.N;
         const bool vec = (a.N & 3) == 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -597,7 +599,7 @@ int launch_tiles(const GemmArgs& a, hipStream_t stream) {
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (attr != hipSuccess) return SNGGUF_E_LAUNCH;
     const int64_t row_tiles = (a.M + TM - 1) / TM + 1;  // a split adds at most one partial tile
-    const int64_t ntn = (a.N + TN - 1) / TN;
+    const int64_t ntn = (a.N + TN - 1) / TN * (a.pair ? 2 : 1);
     const int64_t slices = a.ksplit > 1 ? a.ksplit : 1;
     gemm_tile_kernel<QT, NUM><<<dim3((unsigned)(row_tiles * ntn * slices)), dim3(512), kLdsBytes, stream>>>(a);
     return hipGetLastError() == hipSuccess ? SNGGUF_OK : SNGGUF_E_LAUNCH;
@@ -639,6 +641,30 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     }
 }
 
+// The gated form for a gate / up pair whose K was split: h = silu(g) * u with g, u the two projections' sums rounded to
+// bf16 as their own reductions would write them, silu rounded to bf16, the product rounded to bf16.  Bound by reading the
+// 2 x slices fp32 copies once; as two reductions, silu and a product on tensors the four launches also write and read g, u
+// and silu(g).  N % 4 == 0; one thread per four outputs.
+__global__ __launch_bounds__(256) void splitk_reduce_gated_kernel(const float* __restrict__ gate, const float* __restrict__ up, int slices,
+                                                                  int64_t total, bf16_t* __restrict__ h) {
+    const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i0 >= total) return;
+    f32x4_t g = *reinterpret_cast<const f32x4_t*>(gate + i0), u = *reinterpret_cast<const f32x4_t*>(up + i0);
+    for (int k = 1; k < slices; k++) {
+        const f32x4_t tg = *reinterpret_cast<const f32x4_t*>(gate + (int64_t)k * total + i0);
+        const f32x4_t tu = *reinterpret_cast<const f32x4_t*>(up + (int64_t)k * total + i0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) { g[e] += tg[e]; u[e] += tu[e]; }
+    }
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float gt = bf16_to_f32(f32_to_bf16(g[e])), ut = bf16_to_f32(f32_to_bf16(u[e]));
+        o[e] = bf16_to_f32(f32_to_bf16(gt / (1.0f + expf(-gt)))) * ut;
+    }
+    *reinterpret_cast<u32x2_t*>(h + i0) = u32x2_t{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
+}
+
 }  // namespace
 
 int launch_gemm_dense4(const GemmArgs& a, hipStream_t stream);
@@ -668,6 +694,13 @@ int launch_splitk_reduce(const GemmArgs& a, const uint8_t* indicator, int64_t n_
     const int64_t quads = (a.M * a.N + 3) / 4;
     splitk_reduce_kernel<<<dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream>>>(a.partial, a.ksplit, a.M, a.N, indicator, n_text,
                                                                                           a.bias[0], a.bias[1], a.y);
+    return hipGetLastError() == hipSuccess ? SNGGUF_OK : SNGGUF_E_LAUNCH;
+}
+
+// As launch_splitk_reduce for a gate / up pair: h = silu(sum of `gate`) * (sum of `up`), N % 4 == 0, no bias.
+int launch_splitk_reduce_gated(const float* gate, const float* up, int slices, int64_t M, int64_t N, bf16_t* h, hipStream_t stream) {
+    const int64_t quads = M * N / 4;
+    splitk_reduce_gated_kernel<<<dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream>>>(gate, up, slices, M * N, h);
     return hipGetLastError() == hipSuccess ? SNGGUF_OK : SNGGUF_E_LAUNCH;
 }
 

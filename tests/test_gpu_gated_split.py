@@ -1,0 +1,69 @@
+"""GPU: the SiLU-gated pair over a few hundred rows - both matrices in one launch with K split over workgroups, the
+reduction ending in the gated product - against the oracle (rel-L2 <= 1e-3: bf16 outputs, decoded weights the same bits)
+and against the two projections and the product as bf16 tensors.  Sizes around the 256 x 256 tile, one and several K
+slices, and a workspace too small for any (the dense gated launch)."""
+import pytest
+import torch
+
+from oracle import gguf_oracle as go
+from sensenova_u1_amd import GGUFLinear, GGUFParameter, ops, synthetic
+from sensenova_u1_amd.modality import gated_mlp
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(dev, qt, m, n, k, num=1, x=None, gate=None, ws_bytes=None):
+    gate = synthetic.make_packed(qt, n, k, seed=n + k) if gate is None else gate
+    up = synthetic.make_packed(qt, n, k, seed=n + k + 1)
+    x = synthetic.make_activations(m, k, seed=m) if x is None else x
+    ws = torch.empty(ws_bytes or ops.gate_up_silu_workspace_bytes(n, k), dtype=torch.uint8, device=dev)
+    h = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=dev)
+    ops.gate_up_silu_ws_into(x.to(dev), gate.to(dev), up.to(dev), qt, h, ws, num)
+    return h.cpu(), go.gguf_linear_forward(x, gate, qt, numerics=num), go.gguf_linear_forward(x, up, qt, numerics=num)
+
+
+@pytest.mark.parametrize("qt", [go.Q8_0, go.Q4_K])
+@pytest.mark.parametrize("num", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(65, 8, 1024), (256, 264, 512), (257, 248, 1280), (511, 520, 1024), (100, 2056, 2048)])
+def test_pair_with_split_k(dev, c_oracle, qt, num, m, n, k):
+    print(f"case gated split qt={qt} num={num} {m}x{n}x{k}", flush=True)
+    h, g, u = _run(dev, qt, m, n, k, num, ws_bytes=16 * 8 * m * n + ops.gate_up_silu_workspace_bytes(n, k))
+    assert go.rel_l2(h, c_oracle.silu_mul(g, u)) <= 1e-3
+
+
+def test_infinite_and_huge_gates(dev, c_oracle):
+    """silu(+inf) = +inf, silu(-inf) = NaN, silu(-1e30) = -0, as on bf16 tensors."""
+    qt, m, n, k = go.Q8_0, 130, 256, 256
+    gate = synthetic.make_packed(qt, n, k, seed=71)
+    gate[:64, 0:2] = torch.tensor([100.0], dtype=torch.float16).view(torch.uint8)
+    x = synthetic.make_activations(m, k, seed=5)
+    x[:3] = 0
+    x[0, 0], x[1, 0], x[2, 0] = 1e38, -1e38, 1e30
+    h, g, u = _run(dev, qt, m, n, k, x=x, gate=gate, ws_bytes=64 << 20)
+    want = c_oracle.silu_mul(g, u)
+    assert bool(torch.isnan(want.float()).any()) and bool(torch.isinf(want.float()).any())
+    assert torch.equal(torch.isnan(h.float()), torch.isnan(want.float()))
+    inf = torch.isinf(want.float())
+    assert torch.equal(torch.isinf(h.float()), inf) and torch.equal(h[inf], want[inf])
+    fin = torch.isfinite(want.float())
+    assert torch.equal(torch.signbit(h[:3][fin[:3]].float()), torch.signbit(want[:3][fin[:3]].float()))
+    assert go.rel_l2(torch.where(fin, h.float(), 0.0), torch.where(fin, want.float(), 0.0)) <= 1e-3
+
+
+@pytest.mark.parametrize("qt,m", [(go.Q4_K, 65), (go.Q8_0, 203), (go.Q8_0, 511)])
+def test_gated_mlp_takes_it(dev, monkeypatch, qt, m):
+    n, k = 1024, 2048
+    mods = []
+    for j, (o, i) in enumerate(((n, k), (n, k), (k, n))):
+        lin = GGUFLinear(i, o, bias=False, compute_dtype=torch.bfloat16, device="meta")
+        lin.weight = GGUFParameter(synthetic.make_packed(qt, o, i, seed=40 + j, device=dev), quant_type=qt)
+        mods.append(lin)
+    gate, up, down = mods
+    x = synthetic.make_activations(m, k, seed=m, device=dev)
+    calls = []
+    real = ops.gate_up_silu_ws_into
+    monkeypatch.setattr(ops, "gate_up_silu_ws_into", lambda *a, **kw: (calls.append(a[0].shape[0]), real(*a, **kw))[1])
+    got = gated_mlp(x, gate, up, down)
+    assert calls == [m]
+    # (another order of the fp32 sums: one bf16 step of a gated value now and then)
+    assert go.rel_l2(got.cpu(), down(torch.nn.functional.silu(gate(x)) * up(x)).cpu()) <= 5e-4
