@@ -142,24 +142,33 @@ class FusedProjections(nn.Module):
 ONE_LAUNCH_MLP = True
 
 
-def _one_launch_mlp(x, rows, gate_proj, up_proj, down_proj, norm_weight, residual) -> bool:
+def _one_launch_mlp(x, rows, gate_proj, up_proj, down_proj, norm_weight, residual):
+    """The plain packed tensors and quant types ``(gate, up, down, qt_gate_up, qt_down)`` if the whole MLP runs as one
+    launch, else ``None``.  (The call is as long on the host as on the device: every parameter is looked up and stripped of
+    its tag once.)"""
     if not (ONE_LAUNCH_MLP and 0 < rows <= 2 and x.is_cuda and x.dtype == torch.bfloat16):
-        return False
-    mods = (gate_proj, up_proj, down_proj)
-    if any(m.bias is not None or m.decode_layout != "native" or m.numerics != gate_proj.numerics or not m.weight.is_cuda
-           or (m.compute_dtype or x.dtype) != torch.bfloat16 for m in mods):
-        return False
+        return None
+    packed, types = [], []
+    for m in (gate_proj, up_proj, down_proj):
+        w = m.weight
+        plain = ops._plain(w)
+        if m.bias is not None or m.decode_layout != "native" or m.numerics != gate_proj.numerics or not plain.is_cuda \
+                or (m.compute_dtype or x.dtype) != torch.bfloat16:
+            return None
+        packed.append(plain)
+        types.append(m._weight_type())
     if norm_weight is not None and (norm_weight.dtype != torch.bfloat16 or norm_weight.numel() != gate_proj.in_features):
-        return False
+        return None
     if residual is not None and (residual.dtype != torch.bfloat16 or tuple(residual.shape) != (*x.shape[:-1], down_proj.out_features)):
-        return False
-    if int(gate_proj.weight.quant_type) != int(up_proj.weight.quant_type):
-        return False
+        return None
+    if types[0] != types[1]:
+        return None
     if (up_proj.in_features, up_proj.out_features) != (gate_proj.in_features, gate_proj.out_features) \
             or (down_proj.in_features, down_proj.out_features) != (gate_proj.out_features, gate_proj.in_features):
-        return False
-    return ops.mlp_decode_fits(int(gate_proj.weight.quant_type), int(down_proj.weight.quant_type), rows, gate_proj.in_features,
-                               gate_proj.out_features)
+        return None
+    if not ops.mlp_decode_fits(types[0], types[2], rows, gate_proj.in_features, gate_proj.out_features):
+        return None
+    return (*packed, types[0], types[2])
 
 
 def gated_mlp(x: torch.Tensor, gate_proj: GGUFLinear, up_proj: GGUFLinear, down_proj: GGUFLinear,
@@ -176,19 +185,21 @@ def gated_mlp(x: torch.Tensor, gate_proj: GGUFLinear, up_proj: GGUFLinear, down_
     down projection's partial sums are added.  Beyond 64 rows, where ``_gated_tile_route`` says so, gate / up / SiLU run as
     ``sngguf_gate_up_silu_ws``."""
     rows = x.numel() // x.shape[-1] if x.numel() else 0
-    if _one_launch_mlp(x, rows, gate_proj, up_proj, down_proj, norm_weight, residual):
-        x2d = gate_proj._checked_rows(x, norm_weight, residual)
-        up_proj._checked_rows(x)
-        # (the down projection's input never exists as a tensor here: its packed weight is checked by itself)
-        ops._require_device(x, down_proj.weight)
-        _, dn, dk = ops._packed_2d(down_proj.weight, down_proj._weight_type())
-        if (dn, dk) != (down_proj.out_features, down_proj.in_features) or not down_proj.weight.is_contiguous():
-            raise ops.SnGgufError("gated_mlp: the down projection's packed weight does not match the module")
+    one = _one_launch_mlp(x, rows, gate_proj, up_proj, down_proj, norm_weight, residual)
+    if one is not None:
+        gate, up, down, qt, qt_down = one
+        ops._require_device(x, gate, up, down, norm_weight, residual)
+        for mod, w, t in ((gate_proj, gate, qt), (up_proj, up, qt), (down_proj, down, qt_down)):
+            _, n, k = ops._packed_2d(w, t)
+            if (n, k) != (mod.out_features, mod.in_features):
+                raise ops.SnGgufError(f"gated_mlp: packed weight decodes to {(n, k)}, the module is {(mod.out_features, mod.in_features)}")
+            if not w.is_contiguous():
+                raise ops.SnGgufError("gated_mlp: the packed weights must be contiguous")
+        x2d = ops._as_bf16_rows(x, gate_proj.in_features, "gated_mlp")
         out = torch.empty((*x.shape[:-1], down_proj.out_features), dtype=torch.bfloat16, device=x.device)
         res2d = residual.reshape(-1, down_proj.out_features).contiguous() if residual is not None else None
         ws = ops.mlp_decode_workspace(x.device, rows, gate_proj.in_features, gate_proj.out_features)
-        ops.mlp_decode_into(x2d, norm_weight.contiguous() if norm_weight is not None else None, eps, gate_proj.weight, up_proj.weight,
-                            int(gate_proj.weight.quant_type), down_proj.weight, int(down_proj.weight.quant_type), res2d,
+        ops.mlp_decode_into(x2d, norm_weight.contiguous() if norm_weight is not None else None, eps, gate, up, qt, down, qt_down, res2d,
                             out.view(-1, down_proj.out_features), ws, gate_proj.numerics)
         return out
     if residual is not None:
@@ -214,7 +225,7 @@ def _gated_activations(x, rows, gate_proj, up_proj, norm_weight, eps) -> torch.T
                 ops.rmsnorm_gate_up_silu_tiled_into(x2d, norm_weight.contiguous(), eps, tg, tu,
                                                     h.view(-1, gate_proj.out_features), gate_proj.numerics)
             else:
-                ops.rmsnorm_gate_up_silu_into(x2d, norm_weight.contiguous(), eps, gate_proj.weight, up_proj.weight,
+                ops.rmsnorm_gate_up_silu_into(x2d, norm_weight.contiguous(), eps, ops._plain(gate_proj.weight), ops._plain(up_proj.weight),
                                               int(gate_proj.weight.quant_type), h.view(-1, gate_proj.out_features),
                                               gate_proj.numerics)
             return h
@@ -238,7 +249,7 @@ def _gated_activations(x, rows, gate_proj, up_proj, norm_weight, eps) -> torch.T
         n, k = gate_proj.out_features, gate_proj.in_features
         h = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=x.device)
         ws = ops.pooled_workspace(x.device, ops.gate_up_silu_workspace_bytes(n, k))
-        ops.gate_up_silu_ws_into(x2d, gate_proj.weight, up_proj.weight, int(gate_proj.weight.quant_type), h.view(-1, n), ws,
+        ops.gate_up_silu_ws_into(x2d, ops._plain(gate_proj.weight), ops._plain(up_proj.weight), int(gate_proj.weight.quant_type), h.view(-1, n), ws,
                                  gate_proj.numerics)
     else:
         h = torch.nn.functional.silu(gate_proj(x)) * up_proj(x)
@@ -396,13 +407,21 @@ class SharedInputStack:
         if self.stacked is None:
             return False
         base = self.stacked.data_ptr()
+        device = self.stacked.device
         first = self.members[0]
-        for mod, off in zip(self.members, self.offsets):
-            w = mod.weight
-            if (w.data_ptr() != base + off * self.row_bytes or w.device != self.stacked.device or mod.decode_layout != "native"
-                    or mod.numerics != first.numerics or int(w.quant_type) != int(first.weight.quant_type) or mod.bias is not None):
-                self.release_if_moved()
-                return False
+        quant_type = int(first.weight.quant_type)
+        moved = False
+        # (reads of the tagged parameters' attributes go through Python unless the subclass hook is off: 3 us each)
+        with torch._C.DisableTorchFunctionSubclass():
+            for mod, off in zip(self.members, self.offsets):
+                w = mod.weight
+                if (w.data_ptr() != base + off * self.row_bytes or w.device != device or mod.decode_layout != "native"
+                        or mod.numerics != first.numerics or int(w.quant_type) != quant_type or mod.bias is not None):
+                    moved = True
+                    break
+        if moved:
+            self.release_if_moved()
+            return False
         return True
 
     def release_if_moved(self) -> bool:

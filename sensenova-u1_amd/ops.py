@@ -267,7 +267,7 @@ def pooled_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
     handed out instead (it then belongs to the graph's own memory pool)."""
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), torch.cuda.current_stream(dev).cuda_stream)
+    key = (dev.index if dev.index is not None else torch.cuda.current_device(), _stream(dev))
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)

@@ -215,11 +215,12 @@ class GGUFLinear(nn.Linear):
         ops make: every tensor (inputs, weight, bias, ``others``) on one HIP device, the packed weight a whole
         number of blocks of shape ``[out_features, in_features]``, the input's last dim ``in_features``.  Raises
         ``SnGgufError`` before anything is launched - a host pointer handed to a kernel is a GPU memory fault."""
-        ops._require_device(inputs, self.weight, self.bias, *others)
-        _, n, k = ops._packed_2d(self.weight, self._weight_type())
+        weight = ops._plain(self.weight)   # every attribute read of the tagged parameter itself goes through Python
+        ops._require_device(inputs, weight, self.bias, *others)
+        _, n, k = ops._packed_2d(weight, self._weight_type())
         if (n, k) != (self.out_features, self.in_features):
             raise ops.SnGgufError(f"GGUFLinear: packed weight decodes to {(n, k)}, the module is {(self.out_features, self.in_features)}")
-        if not self.weight.is_contiguous():
+        if not weight.is_contiguous():
             raise ops.SnGgufError("GGUFLinear: the packed weight must be contiguous")
         return ops._as_bf16_rows(inputs, self.in_features, "GGUFLinear")
 
@@ -280,7 +281,7 @@ class GGUFLinear(nn.Linear):
                 # pooled workspace + the dense tile kernel (sngguf_linear_ws picks)
                 workspace = ops.pooled_workspace(inputs.device, self._workspace_bytes(rows))
                 bias = self.bias.detach().to(torch.bfloat16).contiguous() if self.bias is not None else None
-                ops.linear_ws_into(x2d, self.weight, qtype, bias, out.view(-1, self.out_features), workspace, self.numerics)
+                ops.linear_ws_into(x2d, ops._plain(self.weight), qtype, bias, out.view(-1, self.out_features), workspace, self.numerics)
             else:
                 self.two_pass_into(x2d, out.view(-1, self.out_features))
             return out
@@ -310,7 +311,7 @@ class GGUFLinear(nn.Linear):
             ops.rmsnorm_linear_tiled_into(x2d, norm_weight.contiguous(), eps, tiled, bias, out.view(-1, self.out_features),
                                           self.numerics)
         else:
-            ops.rmsnorm_linear_into(x2d, norm_weight.contiguous(), eps, self.weight, self._weight_type(), bias,
+            ops.rmsnorm_linear_into(x2d, norm_weight.contiguous(), eps, ops._plain(self.weight), self._weight_type(), bias,
                                     out.view(-1, self.out_features), self.numerics)
         return out
 
