@@ -253,7 +253,12 @@ int sngguf_gate_up_silu(const void* x, int64_t M, const void* q_gate, const void
  *              16-byte aligned; nothing in it outlives the call
  *  M <= 16 runs sngguf_gate_up_silu (the workspace is not touched).  Otherwise the shape must satisfy
  *  sngguf_gate_up_silu_ws_fits(qtype, M, N, K) (M >= 17, K % 128 == 0, N % 8 == 0, M K < 2^31, a packed block
- *  format), else SNGGUF_E_BADSHAPE / SNGGUF_E_BADTYPE and the caller runs the two projections separately.  It
+ *  format), else SNGGUF_E_BADSHAPE / SNGGUF_E_BADTYPE and the caller runs the two projections separately.  Two other
+ *  forms with the same roundings take over where the dense launch does not pay: up to 64 rows with K % 256 == 0 the
+ *  gate projection on the decode kernel, then the up projection with silu and the product in its epilogue; and Q8_0 /
+ *  Q4_K from 65 rows on with at most 128 tiles of 256 x 256 (below 512 rows, or where the dense launch's tiles fill less
+ *  than 0.7 of their rounds) both matrices in one launch with K split over workgroups, fp32 partial sums in the
+ *  workspace, and a reduction that ends in the gated product.  The dense form
  *  pays from about 512 rows on when the launch's ceil(M / 256) x ceil(N / 128) tiles come close to whole rounds of
  *  the 256 compute units (there is no K split; 12288 x 4096 at
  *  4096 rows: 628 us against 695 us for two sngguf_linear_ws launches and the product, at 2048 rows 354 against 451).

@@ -15,7 +15,7 @@ int launch_gemv_q8_mfma(const void* x, int64_t M, const void* qa, const void* qb
                         float eps, uint64_t* amax = nullptr);
 int launch_gemv_kq_mfma(const void* x, int64_t M, const void* qa, const void* qb, int qtype, int64_t N, int64_t K,
                         const void* bias, const void* residual, void* y, int numerics, bool gated, hipStream_t stream,
-                        const void* gamma, float eps, uint64_t* amax = nullptr);
+                        const void* gamma, float eps, uint64_t* amax = nullptr, const void* gate = nullptr);
 int64_t gemv_argmax_slots(int qtype, int64_t M, int64_t N);
 int launch_argmax_reduce(const uint64_t* keys, int64_t M, int64_t slots, int64_t* out_index, hipStream_t stream);
 int launch_dequantize_bf16(const void* q, int64_t rows, int64_t cols, void* out, int out_dtype, hipStream_t stream);
@@ -368,6 +368,14 @@ int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const v
     if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return qtype == SNGGUF_TYPE_BF16 ? SNGGUF_E_BADTYPE : SNGGUF_E_BADSHAPE;
     if (workspace_bytes < sngguf_gate_up_silu_workspace_bytes(N, K)) return SNGGUF_E_BADSHAPE;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // 17 .. 64 rows of whole 256-element runs belong to the decode kernels: the gate projection into the workspace, then the
+    // up projection with silu and the product in its epilogue (a weight pass and the dense launch take three times as long)
+    if (M <= 64 && K % 256 == 0) {
+        const int rg = sngguf::launch_gemv(x, M, q_gate, nullptr, qtype, N, K, nullptr, nullptr, workspace, numerics, false, s);
+        if (rg != SNGGUF_OK) return rg;
+        return sngguf::launch_gemv_kq_mfma(x, M, q_up, nullptr, qtype, N, K, nullptr, nullptr, h, numerics, false, s, nullptr, 0.f, nullptr,
+                                           workspace);
+    }
     // Few output tiles: the gated launch has no K split and would leave much of the chip idle (below 512 rows, or tiles that
     // fill less than 0.7 of their rounds), so both matrices run as one launch with K split over workgroups, and the
     // reduction ends in the gated product.  Types the large-tile kernel decodes itself; the whole workspace is free for the

@@ -182,7 +182,7 @@ def gated_mlp(x: torch.Tensor, gate_proj: GGUFLinear, up_proj: GGUFLinear, down_
     is part of that same launch.  With ``residual`` the result is ``residual + mlp`` (modeling_qwen3.py:940-941), added
     in the down projection's epilogue.  One or two rows of the 8B model's shape in Q8_0 run as ONE launch
     (``sngguf_mlp_decode``; see ``ONE_LAUNCH_MLP``): same values as the separate launches up to the order in which the
-    down projection's partial sums are added.  Beyond 64 rows, where ``_gated_tile_route`` says so, gate / up / SiLU run as
+    down projection's partial sums are added.  Beyond 16 rows, where ``_gated_tile_route`` says so, gate / up / SiLU run as
     ``sngguf_gate_up_silu_ws``."""
     rows = x.numel() // x.shape[-1] if x.numel() else 0
     one = _one_launch_mlp(x, rows, gate_proj, up_proj, down_proj, norm_weight, residual)
@@ -270,11 +270,16 @@ def gated_tile_fill(rows: int, n: int) -> float:
     return tiles / (256 * -(-tiles // 256))
 
 
+def _called_as_modules(mod) -> bool:
+    """Whether calling ``mod`` does more than ``GGUFLinear.forward``: hooks, or a forward of its own."""
+    return bool(mod._forward_hooks or mod._forward_pre_hooks or "forward" in mod.__dict__ or type(mod).forward is not GGUFLinear.forward)
+
+
 def _gated_tile_route(x, rows, same, gate_proj, up_proj) -> bool:
     """Whether ``gated_mlp`` hands gate / up / SiLU to ``sngguf_gate_up_silu_ws``: both weights of one packed type and
-    shape, no bias, default GEMM policy, and either enough rows and tiles to fill the chip with the gated dense launch, or
-    a shape for which the library splits K of both matrices and ends the reduction in the gated product."""
-    if not (rows > 64 and same and x.is_cuda and x.dtype == torch.bfloat16):
+    shape, no bias, default GEMM policy, and enough rows and tiles to fill the chip with the gated dense launch, or a shape
+    for which the library splits K of both matrices and ends the reduction in the gated product, or at most 64 rows."""
+    if not (rows > 16 and same and x.is_cuda and x.dtype == torch.bfloat16):
         return False
     if gate_proj.bias is not None or up_proj.bias is not None:
         return False
@@ -284,8 +289,17 @@ def _gated_tile_route(x, rows, same, gate_proj, up_proj) -> bool:
         return False
     if gate_proj.numerics != up_proj.numerics:
         return False
+    if rows < GATED_TILE_MIN_ROWS and (_called_as_modules(gate_proj) or _called_as_modules(up_proj)):
+        return False
     n, k, qt = gate_proj.out_features, gate_proj.in_features, int(gate_proj.weight.quant_type)
-    if rows < GATED_TILE_MIN_ROWS or gated_tile_fill(rows, n) < GATED_TILE_MIN_FILL:
+    if rows <= 64:
+        # the decode kernels: the gate projection, then the up projection with silu and the product in its epilogue.
+        # 40 rows, whole layers of the 8B model in
+        # Q8_0: 130 us per layer against 142 with two projections, silu and the product
+        # (not while something traces or intercepts: the modules' own calls are registered ops at these sizes)
+        if k % 256 != 0 or not ops._eager(x):
+            return False
+    elif rows < GATED_TILE_MIN_ROWS or gated_tile_fill(rows, n) < GATED_TILE_MIN_FILL:
         # room for two fp32 copies of both outputs in the 4 n k bytes of workspace.  Against two projections, two
         # reductions, silu and the product (12288 x 4096 pair, whole layers of the 8B model, us): 203 rows Q4_K / Q6_K
         # 231 / 253 per layer, 509 rows Q8_0 333 / 374
@@ -317,7 +331,7 @@ def fuse_gated_mlps(model: nn.Module) -> int:
     ``mlp_mot_gen`` is the same class): children ``gate_proj``, ``up_proj``, ``down_proj`` that are all ``GGUFLinear``,
     an ``act_fn`` that computes SiLU, and a forward of one argument.  Its forward then is
     ``down_proj(silu(gate_proj(x)) * up_proj(x))`` with the gate / up pair and the SiLU product in one launch at decode
-    row counts, every rounding of the three-launch form kept, ``sngguf_gate_up_silu_ws`` beyond 64 rows where it is the
+    row counts, every rounding of the three-launch form kept, ``sngguf_gate_up_silu_ws`` beyond 16 rows where it is the
     faster form, and the unchanged three module calls elsewhere.  The
     original forward is kept and ``unfuse_gated_mlps`` puts it back."""
     import inspect

@@ -67,3 +67,47 @@ def test_gated_mlp_takes_it(dev, monkeypatch, qt, m):
     assert calls == [m]
     # (another order of the fp32 sums: one bf16 step of a gated value now and then)
     assert go.rel_l2(got.cpu(), down(torch.nn.functional.silu(gate(x)) * up(x)).cpu()) <= 5e-4
+
+
+@pytest.mark.parametrize("qt", [go.Q8_0, go.Q4_1, go.Q3_K, go.Q4_K, go.Q6_K])
+@pytest.mark.parametrize("m,n,k", [(17, 8, 256), (33, 136, 512), (40, 4104, 1024), (64, 264, 768)])
+def test_pair_of_17_to_64_rows(dev, c_oracle, qt, m, n, k):
+    """silu and the product in the up projection's epilogue: the outputs of the two projections and of silu are rounded as
+    the tensors of the separate calls are, so only the last place of exp() can differ from those."""
+    print(f"case gated 17..64 rows qt={qt} {m}x{n}x{k}", flush=True)
+    h, g, u = _run(dev, qt, m, n, k)
+    assert go.rel_l2(h, c_oracle.silu_mul(g, u)) <= 1e-3
+    x = synthetic.make_activations(m, k, seed=m).to(dev)
+    gt, ut = (ops.linear(x, synthetic.make_packed(qt, n, k, seed=n + k + j).to(dev), qt) for j in (0, 1))
+    assert go.rel_l2(h, (torch.nn.functional.silu(gt) * ut).cpu()) <= 1e-4
+
+
+def test_infinite_gates_at_40_rows(dev, c_oracle):
+    qt, m, n, k = go.Q8_0, 40, 256, 256
+    gate = synthetic.make_packed(qt, n, k, seed=71)
+    gate[:64, 0:2] = torch.tensor([100.0], dtype=torch.float16).view(torch.uint8)
+    x = synthetic.make_activations(m, k, seed=5)
+    x[:3] = 0
+    x[0, 0], x[1, 0], x[2, 0] = 1e38, -1e38, 1e30
+    h, g, u = _run(dev, qt, m, n, k, x=x, gate=gate)
+    want = c_oracle.silu_mul(g, u)
+    assert torch.equal(torch.isnan(h.float()), torch.isnan(want.float()))
+    inf = torch.isinf(want.float())
+    assert torch.equal(torch.isinf(h.float()), inf) and torch.equal(h[inf], want[inf])
+
+
+def test_hooked_projections_are_called(dev):
+    """A forward hook on a projection keeps the module calls."""
+    n, k, m = 512, 1024, 40
+    mods = []
+    for j, (o, i) in enumerate(((n, k), (n, k), (k, n))):
+        lin = GGUFLinear(i, o, bias=False, compute_dtype=torch.bfloat16, device="meta")
+        lin.weight = GGUFParameter(synthetic.make_packed(go.Q8_0, o, i, seed=60 + j, device=dev), quant_type=go.Q8_0)
+        mods.append(lin)
+    x = synthetic.make_activations(m, k, seed=m, device=dev)
+    want = gated_mlp(x, *mods)
+    seen = []
+    handle = mods[1].register_forward_hook(lambda mod, args, out: seen.append(out.shape))
+    got = gated_mlp(x, *mods)
+    handle.remove()
+    assert seen == [(m, n)] and go.rel_l2(got.cpu(), want.cpu()) <= 1e-4
