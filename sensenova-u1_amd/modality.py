@@ -271,8 +271,14 @@ def gated_tile_fill(rows: int, n: int) -> float:
 
 
 def _called_as_modules(mod) -> bool:
-    """Whether calling ``mod`` does more than ``GGUFLinear.forward``: hooks, or a forward of its own."""
-    return bool(mod._forward_hooks or mod._forward_pre_hooks or "forward" in mod.__dict__ or type(mod).forward is not GGUFLinear.forward)
+    """Whether calling ``mod`` does more than ``GGUFLinear.forward``: a forward or call of its own (a subclass, an attribute,
+    ``compile()``), or hooks of any kind, registered on it or on all modules."""
+    every = torch.nn.modules.module
+    return bool("forward" in mod.__dict__ or type(mod).forward is not GGUFLinear.forward or type(mod).__call__ is not nn.Module.__call__
+                or mod._compiled_call_impl is not None
+                or mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
+                or every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks
+                or every._global_backward_pre_hooks)
 
 
 def _gated_tile_route(x, rows, same, gate_proj, up_proj) -> bool:
@@ -289,7 +295,9 @@ def _gated_tile_route(x, rows, same, gate_proj, up_proj) -> bool:
         return False
     if gate_proj.numerics != up_proj.numerics:
         return False
-    if rows < GATED_TILE_MIN_ROWS and (_called_as_modules(gate_proj) or _called_as_modules(up_proj)):
+    filled = rows >= GATED_TILE_MIN_ROWS and gated_tile_fill(rows, gate_proj.out_features) >= GATED_TILE_MIN_FILL
+    # where gate_proj(x) and up_proj(x) would be the modules' own calls, whatever hangs on those calls keeps them
+    if not filled and (_called_as_modules(gate_proj) or _called_as_modules(up_proj)):
         return False
     n, k, qt = gate_proj.out_features, gate_proj.in_features, int(gate_proj.weight.quant_type)
     if rows <= 64:
@@ -299,7 +307,7 @@ def _gated_tile_route(x, rows, same, gate_proj, up_proj) -> bool:
         # (not while something traces or intercepts: the modules' own calls are registered ops at these sizes)
         if k % 256 != 0 or not ops._eager(x):
             return False
-    elif rows < GATED_TILE_MIN_ROWS or gated_tile_fill(rows, n) < GATED_TILE_MIN_FILL:
+    elif not filled:
         # room for two fp32 copies of both outputs in the 4 n k bytes of workspace.  Against two projections, two
         # reductions, silu and the product (12288 x 4096 pair, whole layers of the 8B model, us): 203 rows Q4_K / Q6_K
         # 231 / 253 per layer, 509 rows Q8_0 333 / 374

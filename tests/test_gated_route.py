@@ -1,0 +1,60 @@
+"""Which gate / up pairs beyond 16 rows ``gated_mlp`` hands to one library call: the rule needs no device, only sizes, types
+and what is registered on the two projections."""
+import types
+
+import pytest
+import torch
+
+from sensenova_u1_amd import GGUFLinear, GGUFParameter, modality, ops
+
+SPLIT_PAIRS = [(ops.Q8_0, 6144, 2048, 203), (ops.Q4_K, 9728, 2560, 511), (ops.Q8_0, 6144, 2048, 512), (ops.Q4_K, 9728, 2560, 512),
+               (ops.Q8_0, 4096, 4096, 768), (ops.Q8_0, 8960, 3584, 512)]
+FILLED = (ops.Q8_0, 12288, 4096, 4096)   # the dense gated launch, whose tiles fill the chip
+
+
+class Adapted(GGUFLinear):
+    def forward(self, inputs):
+        return super().forward(inputs) + 1
+
+
+def _linear(qt, n, k, cls=GGUFLinear, compute_dtype=torch.bfloat16):
+    bs, ts = ops.GGML_QUANT_SIZES[qt]
+    lin = cls(k, n, bias=False, compute_dtype=compute_dtype, device="meta")
+    lin.weight = GGUFParameter(torch.empty((n, k // bs * ts), dtype=torch.uint8, device="meta"), quant_type=qt)
+    return lin
+
+
+def _route(rows, gate, up):
+    x = types.SimpleNamespace(is_cuda=True, dtype=torch.bfloat16)   # (what the rule reads of its input beyond 64 rows)
+    return modality._gated_tile_route(x, rows, True, gate, up)
+
+
+@pytest.mark.parametrize("qt,n,k,rows", SPLIT_PAIRS)
+def test_a_forward_of_its_own_is_called(qt, n, k, rows):
+    plain = _linear(qt, n, k)
+    assert _route(rows, plain, _linear(qt, n, k))
+    assert not _route(rows, plain, _linear(qt, n, k, cls=Adapted)) and not _route(rows, _linear(qt, n, k, cls=Adapted), plain)
+    patched = _linear(qt, n, k)
+    patched.forward = lambda inputs: inputs
+    assert not _route(rows, patched, plain)
+
+
+@pytest.mark.parametrize("qt,n,k,rows", SPLIT_PAIRS)
+def test_hooks_keep_the_module_calls(qt, n, k, rows):
+    gate, up = _linear(qt, n, k), _linear(qt, n, k)
+    every = torch.nn.modules.module
+    hook = lambda *args: None
+    for register in (up.register_forward_hook, gate.register_forward_pre_hook, up.register_full_backward_hook,
+                     gate.register_full_backward_pre_hook, every.register_module_forward_hook, every.register_module_forward_pre_hook,
+                     every.register_module_full_backward_hook, every.register_module_full_backward_pre_hook):
+        handle = register(hook)
+        try:
+            assert not _route(rows, gate, up), register
+        finally:
+            handle.remove()
+    assert _route(rows, gate, up)
+
+
+def test_the_filled_dense_launch_stays_what_it_was():
+    qt, n, k, rows = FILLED
+    assert _route(rows, _linear(qt, n, k), _linear(qt, n, k, cls=Adapted))

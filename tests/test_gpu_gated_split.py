@@ -111,3 +111,27 @@ def test_hooked_projections_are_called(dev):
     got = gated_mlp(x, *mods)
     handle.remove()
     assert seen == [(m, n)] and go.rel_l2(got.cpu(), want.cpu()) <= 1e-4
+
+
+class _Adapted(GGUFLinear):
+    def forward(self, inputs):
+        return super().forward(inputs) * 2
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 512, 1024), (203, 1024, 2048), (512, 6144, 2048)])
+def test_projections_with_their_own_forward_are_called(dev, m, n, k):
+    """An overriding subclass and a hook that replaces the output, at sizes of each form that was module calls."""
+    print(f"case own forward {m}x{n}x{k}", flush=True)
+    mods = []
+    for j, (o, i, cls) in enumerate(((n, k, GGUFLinear), (n, k, _Adapted), (k, n, GGUFLinear))):
+        lin = cls(i, o, bias=False, compute_dtype=torch.bfloat16, device="meta")
+        lin.weight = GGUFParameter(synthetic.make_packed(go.Q8_0, o, i, seed=80 + j, device=dev), quant_type=go.Q8_0)
+        mods.append(lin)
+    gate, up, down = mods
+    x = synthetic.make_activations(m, k, seed=m, device=dev)
+    assert torch.equal(gated_mlp(x, gate, up, down), down(torch.nn.functional.silu(gate(x)) * up(x)))
+    plain = GGUFLinear(k, n, bias=False, compute_dtype=torch.bfloat16, device="meta")
+    plain.weight = up.weight
+    handle = plain.register_forward_hook(lambda mod, args, out: out * 2)
+    assert torch.equal(gated_mlp(x, gate, plain, down), gated_mlp(x, gate, up, down))
+    handle.remove()
