@@ -296,8 +296,9 @@ def _gated_tile_route(x, rows, same, gate_proj, up_proj) -> bool:
     if gate_proj.numerics != up_proj.numerics:
         return False
     filled = rows >= GATED_TILE_MIN_ROWS and gated_tile_fill(rows, gate_proj.out_features) >= GATED_TILE_MIN_FILL
-    # where gate_proj(x) and up_proj(x) would be the modules' own calls, whatever hangs on those calls keeps them
-    if not filled and (_called_as_modules(gate_proj) or _called_as_modules(up_proj)):
+    # where gate_proj(x) and up_proj(x) would be the modules' own calls, whatever hangs on those calls keeps them, the refusal
+    # of an input that is not in a module's compute dtype included
+    if not filled and any(_called_as_modules(m) or (m.compute_dtype or x.dtype) != torch.bfloat16 for m in (gate_proj, up_proj)):
         return False
     n, k, qt = gate_proj.out_features, gate_proj.in_features, int(gate_proj.weight.quant_type)
     if rows <= 64:

@@ -55,6 +55,15 @@ def test_hooks_keep_the_module_calls(qt, n, k, rows):
     assert _route(rows, gate, up)
 
 
+@pytest.mark.parametrize("qt,n,k,rows", SPLIT_PAIRS)
+def test_another_compute_dtype_is_left_to_the_modules(qt, n, k, rows):
+    """(a bf16 input to an fp16 or fp32 module: its forward raises)"""
+    for other in (torch.float16, torch.float32):
+        assert not _route(rows, _linear(qt, n, k), _linear(qt, n, k, compute_dtype=other))
+        assert not _route(rows, _linear(qt, n, k, compute_dtype=other), _linear(qt, n, k))
+    assert _route(rows, _linear(qt, n, k, compute_dtype=None), _linear(qt, n, k))
+
+
 def test_the_filled_dense_launch_stays_what_it_was():
     qt, n, k, rows = FILLED
     assert _route(rows, _linear(qt, n, k), _linear(qt, n, k, cls=Adapted))

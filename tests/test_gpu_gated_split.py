@@ -135,3 +135,14 @@ def test_projections_with_their_own_forward_are_called(dev, m, n, k):
     handle = plain.register_forward_hook(lambda mod, args, out: out * 2)
     assert torch.equal(gated_mlp(x, gate, plain, down), gated_mlp(x, gate, up, down))
     handle.remove()
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 512, 1024), (203, 1024, 2048), (512, 6144, 2048)])
+def test_bf16_input_to_an_fp16_projection_is_refused(dev, m, n, k):
+    mods = []
+    for j, (o, i, dtype) in enumerate(((n, k, torch.bfloat16), (n, k, torch.float16), (k, n, torch.bfloat16))):
+        lin = GGUFLinear(i, o, bias=False, compute_dtype=dtype, device="meta")
+        lin.weight = GGUFParameter(synthetic.make_packed(go.Q8_0, o, i, seed=20 + j, device=dev), quant_type=go.Q8_0)
+        mods.append(lin)
+    with pytest.raises(RuntimeError, match="compute dtype"):
+        gated_mlp(synthetic.make_activations(m, k, seed=m, device=dev), *mods)
