@@ -249,8 +249,10 @@ int sngguf_gate_up_silu(const void* x, int64_t M, const void* q_gate, const void
  * bf16, applies silu and multiplies, with the roundings above.  The two [M][N] projection outputs are never written
  * and no elementwise pass reads them back.  Same values as sngguf_linear_ws on each matrix followed by
  * silu(gate) * up on bf16 tensors (up to the last place of exp()).
- *  workspace   device scratch of at least sngguf_gate_up_silu_workspace_bytes(N, K) = 512 ceil(N / 128) K bytes,
- *              16-byte aligned; nothing in it outlives the call
+ *  workspace   device scratch, 16-byte aligned; nothing in it outlives the call, and no other call may use it between this
+ *              call's launches (threads that share a stream take one each).  sngguf_gate_up_silu_workspace_bytes(N, K) =
+ *              512 ceil(N / 128) K bytes are enough at any M; sngguf_gate_up_silu_ws_bytes(qtype, M, N, K) is what the form
+ *              that this shape takes needs (0 for shapes that do not fit and for M <= 16)
  *  M <= 16 runs sngguf_gate_up_silu (the workspace is not touched).  Otherwise the shape must satisfy
  *  sngguf_gate_up_silu_ws_fits(qtype, M, N, K) (M >= 17, K % 128 == 0, N % 8 == 0, M K < 2^31, a packed block
  *  format), else SNGGUF_E_BADSHAPE / SNGGUF_E_BADTYPE and the caller runs the two projections separately.  Two other
@@ -265,6 +267,7 @@ int sngguf_gate_up_silu(const void* x, int64_t M, const void* q_gate, const void
  */
 int64_t sngguf_gate_up_silu_workspace_bytes(int64_t N, int64_t K);
 int sngguf_gate_up_silu_ws_fits(int qtype, int64_t M, int64_t N, int64_t K);
+int64_t sngguf_gate_up_silu_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K);
 int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const void* q_up, int qtype,
                            int64_t N, int64_t K, void* h, void* workspace, int64_t workspace_bytes,
                            int numerics, void* stream);

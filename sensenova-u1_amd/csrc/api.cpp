@@ -358,6 +358,45 @@ int sngguf_gate_up_silu_ws_fits(int qtype, int64_t M, int64_t N, int64_t K) {
            K < kMaxDim && K % 128 == 0 && K % sngguf_block_size(qtype) == 0 && N % 8 == 0 && M * K < ((int64_t)1 << 31);
 }
 
+namespace {
+// How a pair beyond 16 rows runs; the shape is one that sngguf_gate_up_silu_ws_fits takes.
+enum PairForm {
+    // 17 .. 64 rows of whole 256-element runs belong to the decode kernels: the gate projection into the workspace, then the
+    // up projection with silu and the product in its epilogue (a weight pass and the dense launch take three times as long)
+    kPairDecode,
+    // Few output tiles: the gated launch has no K split and would leave much of the chip idle (below 512 rows, or tiles that
+    // fill less than 0.7 of their rounds), so both matrices run as one launch with K split over workgroups, and the
+    // reduction ends in the gated product.  Types the large-tile kernel decodes itself; the whole workspace is free for the
+    // partial sums.
+    kPairSplit,
+    kPairDense,   // two weight passes, one dense launch with the gated epilogue
+};
+
+PairForm pair_form(int qtype, int64_t M, int64_t N, int64_t K) {
+    if (M <= 64 && K % 256 == 0) return kPairDecode;
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), gated_tiles = ((M + 255) / 256) * ((N + 127) / 128);
+    const bool fills = M >= 512 && 10 * gated_tiles >= 7 * 256 * ((gated_tiles + 255) / 256);
+    if ((qtype == SNGGUF_TYPE_Q8_0 || qtype == SNGGUF_TYPE_Q4_K) && M >= 65 && M < 4096 && tiles <= 128 && !fills) return kPairSplit;
+    return kPairDense;
+}
+
+// K slices of the split form with `workspace_bytes` for the partial sums; 0 = not even one copy of each output fits (the
+// dense form then).
+int64_t pair_slices(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    return pick_pair_slices(M, N, 2 * tiles, K / 64, workspace_bytes / (8 * M * N));
+}
+}  // namespace
+
+int64_t sngguf_gate_up_silu_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
+    if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return 0;
+    const PairForm form = pair_form(qtype, M, N, K);
+    if (form == kPairDecode) return 2 * M * N;
+    const int64_t dense = sngguf_gate_up_silu_workspace_bytes(N, K);
+    const int64_t slices = form == kPairSplit ? pair_slices(M, N, K, dense) : 0;
+    return slices >= 1 ? slices * 8 * M * N : dense;
+}
+
 int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const void* q_up, int qtype, int64_t N, int64_t K,
                            void* h, void* workspace, int64_t workspace_bytes, int numerics, void* stream) {
     if (M >= 0 && M <= 16) return sngguf_gate_up_silu(x, M, q_gate, q_up, qtype, N, K, h, numerics, stream);
@@ -366,28 +405,22 @@ int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const v
     if (!q_up || !workspace) return SNGGUF_E_NULLPTR;
     if (!aligned(q_up, 16) || !aligned(workspace, 16)) return SNGGUF_E_ALIGN;
     if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return qtype == SNGGUF_TYPE_BF16 ? SNGGUF_E_BADTYPE : SNGGUF_E_BADSHAPE;
-    if (workspace_bytes < sngguf_gate_up_silu_workspace_bytes(N, K)) return SNGGUF_E_BADSHAPE;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // 17 .. 64 rows of whole 256-element runs belong to the decode kernels: the gate projection into the workspace, then the
-    // up projection with silu and the product in its epilogue (a weight pass and the dense launch take three times as long)
-    if (M <= 64 && K % 256 == 0) {
+    const PairForm form = pair_form(qtype, M, N, K);
+    if (form == kPairDecode) {
+        if (workspace_bytes < 2 * M * N) return SNGGUF_E_BADSHAPE;
         const int rg = sngguf::launch_gemv(x, M, q_gate, nullptr, qtype, N, K, nullptr, nullptr, workspace, numerics, false, s);
         if (rg != SNGGUF_OK) return rg;
         return sngguf::launch_gemv_kq_mfma(x, M, q_up, nullptr, qtype, N, K, nullptr, nullptr, h, numerics, false, s, nullptr, 0.f, nullptr,
                                            workspace);
     }
-    // Few output tiles: the gated launch has no K split and would leave much of the chip idle (below 512 rows, or tiles that
-    // fill less than 0.7 of their rounds), so both matrices run as one launch with K split over workgroups, and the
-    // reduction ends in the gated product.  Types the large-tile kernel decodes itself; the whole workspace is free for the
-    // partial sums.
-    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), gated_tiles = ((M + 255) / 256) * ((N + 127) / 128);
-    const bool fills = M >= 512 && 10 * gated_tiles >= 7 * 256 * ((gated_tiles + 255) / 256);
-    if ((qtype == SNGGUF_TYPE_Q8_0 || qtype == SNGGUF_TYPE_Q4_K) && M >= 65 && M < 4096 && tiles <= 128 && !fills) {
-        const int64_t slices = pick_pair_slices(M, N, 2 * tiles, K / 64, workspace_bytes / (8 * M * N));
+    if (form == kPairSplit) {
+        const int64_t slices = workspace_bytes > 0 ? pair_slices(M, N, K, workspace_bytes) : 0;
         if (slices >= 1)
             return sngguf::launch_gemm_splitk_gated(x, M, q_gate, q_up, qtype, N, K, h, static_cast<float*>(workspace), (int)slices,
                                                     numerics, s);
     }
+    if (workspace_bytes < sngguf_gate_up_silu_workspace_bytes(N, K)) return SNGGUF_E_BADSHAPE;
     int rd = sngguf::launch_dequantize_interleaved(q_gate, qtype, N, K, workspace, 0, numerics, s);
     if (rd != SNGGUF_OK) return rd;
     rd = sngguf::launch_dequantize_interleaved(q_up, qtype, N, K, workspace, 1, numerics, s);

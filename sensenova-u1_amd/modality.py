@@ -242,15 +242,14 @@ def _gated_activations(x, rows, gate_proj, up_proj, norm_weight, eps) -> torch.T
     elif decode and gate_proj.in_features % 64 == 0:
         h = ops.gate_up_silu(x, gate_proj.weight, up_proj.weight, int(gate_proj.weight.quant_type), gate_proj.numerics)
     elif _gated_tile_route(x, rows, same, gate_proj, up_proj):
-        # thousands of rows (the generation tower's image tokens): both weight passes into one interleaved workspace,
-        # then one dense GEMM launch whose epilogue applies silu and the product
         x2d = gate_proj._checked_rows(x)
         up_proj._checked_rows(x)
-        n, k = gate_proj.out_features, gate_proj.in_features
+        n, qt = gate_proj.out_features, int(gate_proj.weight.quant_type)
         h = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=x.device)
-        ws = ops.pooled_workspace(x.device, ops.gate_up_silu_workspace_bytes(n, k))
-        ops.gate_up_silu_ws_into(x2d, ops._plain(gate_proj.weight), ops._plain(up_proj.weight), int(gate_proj.weight.quant_type), h.view(-1, n), ws,
-                                 gate_proj.numerics)
+        nbytes = ops.gate_up_silu_ws_bytes(qt, rows, n, gate_proj.in_features)
+        ws = ops.pooled_workspace(x.device, nbytes)
+        ops.gate_up_silu_ws_into(x2d, ops._plain(gate_proj.weight), ops._plain(up_proj.weight), qt, h.view(-1, n), ws, gate_proj.numerics,
+                                 nbytes)
     else:
         h = torch.nn.functional.silu(gate_proj(x)) * up_proj(x)
     return h

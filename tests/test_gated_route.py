@@ -67,3 +67,17 @@ def test_another_compute_dtype_is_left_to_the_modules(qt, n, k, rows):
 def test_the_filled_dense_launch_stays_what_it_was():
     qt, n, k, rows = FILLED
     assert _route(rows, _linear(qt, n, k), _linear(qt, n, k, cls=Adapted))
+
+
+def test_workspace_is_what_the_form_needs():
+    """2 M N bytes for the gate outputs up to 64 rows; whole fp32 copies of both outputs for a K split, within what the dense
+    form would take; the interleaved weights for the dense form; never more than the size that is enough at any M."""
+    for qt, m, n, k in ((ops.Q8_0, 17, 12288, 4096), (ops.Q6_K, 64, 9728, 2560), (ops.Q2_K, 33, 8, 256)):
+        assert ops.gate_up_silu_ws_bytes(qt, m, n, k) == 2 * m * n
+    for qt, m, n, k in ((ops.Q8_0, 65, 12288, 4096), (ops.Q4_K, 203, 12288, 4096), (ops.Q8_0, 509, 12288, 4096), (ops.Q4_K, 512, 9728, 2560)):
+        nbytes = ops.gate_up_silu_ws_bytes(qt, m, n, k)
+        assert 0 < nbytes <= ops.gate_up_silu_workspace_bytes(n, k) and nbytes % (8 * m * n) == 0
+    for qt, m, n, k in ((ops.Q8_0, 40, 512, 384), (ops.Q6_K, 203, 12288, 4096), FILLED[:1] + FILLED[3:] + FILLED[1:3], (ops.Q8_0, 300, 512, 256)):
+        assert ops.gate_up_silu_ws_bytes(qt, m, n, k) == ops.gate_up_silu_workspace_bytes(n, k)
+    for qt, m, n, k in ((ops.Q8_0, 16, 512, 256), (ops.Q8_0, 300, 516, 256), (ops.Q8_0, 300, 512, 192), (ops.BF16, 300, 512, 256)):
+        assert ops.gate_up_silu_ws_bytes(qt, m, n, k) == 0

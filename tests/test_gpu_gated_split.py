@@ -146,3 +146,34 @@ def test_bf16_input_to_an_fp16_projection_is_refused(dev, m, n, k):
         mods.append(lin)
     with pytest.raises(RuntimeError, match="compute dtype"):
         gated_mlp(synthetic.make_activations(m, k, seed=m, device=dev), *mods)
+
+
+@pytest.mark.parametrize("qt,m,n,k", [(go.Q8_0, 40, 264, 512), (go.Q6_K, 17, 8, 256), (go.Q4_K, 64, 4104, 256), (go.Q8_0, 257, 264, 2048),
+                                      (go.Q4_K, 203, 1024, 2048), (go.Q6_K, 130, 264, 512)])
+def test_workspace_of_exactly_the_form_s_size(dev, c_oracle, qt, m, n, k):
+    """As many bytes as the form asks for, the 64 behind them untouched; 16 bytes less are refused where no smaller form exists."""
+    print(f"case exact workspace qt={qt} {m}x{n}x{k}", flush=True)
+    nbytes = ops.gate_up_silu_ws_bytes(qt, m, n, k)
+    gate, up = (synthetic.make_packed(qt, n, k, seed=n + j, device=dev) for j in (0, 1))
+    x = synthetic.make_activations(m, k, seed=m, device=dev)
+    ws = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device=dev)
+    h = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=dev)
+    ops.gate_up_silu_ws_into(x, gate, up, qt, h, ws, 1, nbytes)
+    g, u = (go.gguf_linear_forward(x.cpu(), w.cpu(), qt, numerics=1) for w in (gate, up))
+    assert go.rel_l2(h.cpu(), c_oracle.silu_mul(g, u)) <= 1e-3
+    assert bool((ws[nbytes:] == 0xA5).all())
+    if m <= 64 or qt == go.Q6_K:
+        with pytest.raises(ops.SnGgufError):
+            ops.gate_up_silu_ws_into(x, gate, up, qt, h, ws, 1, nbytes - 16)
+
+
+def test_forty_rows_leave_no_weight_sized_workspace(dev):
+    n, k, m = 2048, 1024, 40
+    mods = []
+    for j, (o, i) in enumerate(((n, k), (n, k), (k, n))):
+        lin = GGUFLinear(i, o, bias=False, compute_dtype=torch.bfloat16, device="meta")
+        lin.weight = GGUFParameter(synthetic.make_packed(go.Q8_0, o, i, seed=30 + j, device=dev), quant_type=go.Q8_0)
+        mods.append(lin)
+    ops.release_workspaces()
+    gated_mlp(synthetic.make_activations(m, k, seed=m, device=dev), *mods)
+    assert sum(ws.numel() for ws in ops._workspaces.values()) <= 2 * m * n
