@@ -2,6 +2,8 @@
 reduction ending in the gated product - against the oracle (rel-L2 <= 1e-3: bf16 outputs, decoded weights the same bits)
 and against the two projections and the product as bf16 tensors.  Sizes around the 256 x 256 tile, one and several K
 slices, and a workspace too small for any (the dense gated launch)."""
+import threading
+
 import pytest
 import torch
 
@@ -177,3 +179,30 @@ def test_forty_rows_leave_no_weight_sized_workspace(dev):
     ops.release_workspaces()
     gated_mlp(synthetic.make_activations(m, k, seed=m, device=dev), *mods)
     assert sum(ws.numel() for ws in ops._workspaces.values()) <= 2 * m * n
+
+
+@pytest.mark.parametrize("m", [17, 40, 64])
+def test_threads_on_one_stream(dev, m):
+    """Four host threads, each with rows of its own, through one MLP on the default stream."""
+    print(f"case threads on one stream m={m}", flush=True)
+    n, k = 1024, 2048
+    mods = []
+    for j, (o, i) in enumerate(((n, k), (n, k), (k, n))):
+        lin = GGUFLinear(i, o, bias=False, compute_dtype=torch.bfloat16, device="meta")
+        lin.weight = GGUFParameter(synthetic.make_packed(go.Q8_0, o, i, seed=50 + j, device=dev), quant_type=go.Q8_0)
+        mods.append(lin)
+    xs = [synthetic.make_activations(m, k, seed=100 + t, device=dev) for t in range(4)]
+    want = [gated_mlp(x, *mods) for x in xs]
+    got = [[] for _ in xs]
+
+    def body(t):
+        for _ in range(16):
+            got[t].append(gated_mlp(xs[t], *mods))
+    threads = [threading.Thread(target=body, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for w, outs in zip(want, got):
+        assert len(outs) == 16 and all(torch.equal(o, w) for o in outs)
