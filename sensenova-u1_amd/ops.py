@@ -17,6 +17,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import os
+import threading
 from typing import Optional
 
 import torch
@@ -260,12 +261,22 @@ def grouped_workspace_bytes(m: int) -> int:
 
 
 _workspaces: dict = {}
+_enqueue_locks: dict = {}
+
+
+def _whole_call(dev: torch.device):
+    """The lock under which a call with a caller's workspace is enqueued on the current stream of ``dev``.  Host threads that
+    share a stream get one pooled workspace, a call fills it with one launch and reads it with the next, and the foreign call
+    lets go of the interpreter lock: without this another thread's launches could come between them."""
+    key = (dev.index, _stream(dev))
+    lock = _enqueue_locks.get(key)
+    return lock if lock is not None else _enqueue_locks.setdefault(key, threading.Lock())
 
 
 def pooled_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
     """A device scratch tensor of at least ``nbytes`` bytes for the workspace entry points, kept per (device, stream)
-    and grown on demand, so that a forward pass over many modules allocates once.  Calls on one stream are ordered, and
-    nothing in a workspace outlives the call that filled it.  While a HIP graph is being captured a fresh tensor is
+    and grown on demand, so that a forward pass over many modules allocates once.  Calls on one stream are ordered (whole
+    calls, also of several host threads: ``_whole_call``), and nothing in a workspace outlives the call that filled it.  While a HIP graph is being captured a fresh tensor is
     handed out instead (it then belongs to the graph's own memory pool)."""
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
@@ -348,7 +359,7 @@ def linear_ws_into(x2d: torch.Tensor, packed: torch.Tensor, quant_type: int, bia
     dev = x2d.device
     n, k = y2d.shape[1], x2d.shape[1]
     ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
-    with _on(dev):
+    with _on(dev), _whole_call(dev):
         rc = load_library().sngguf_linear_ws(_ptr(x2d), x2d.shape[0], _ptr(packed), quant_type, n, k, _ptr(bias),
                                              _ptr(y2d), _ptr(workspace), ws_bytes, numerics, _stream(dev))
     _check(rc, "sngguf_linear_ws")
@@ -415,7 +426,7 @@ def gate_up_silu_ws_into(x2d: torch.Tensor, gate: torch.Tensor, up: torch.Tensor
     dev = x2d.device
     if workspace_bytes is None:
         workspace_bytes = workspace.numel() * workspace.element_size()
-    with _on(dev):
+    with _on(dev), _whole_call(dev):
         rc = load_library().sngguf_gate_up_silu_ws(_ptr(x2d), x2d.shape[0], _ptr(gate), _ptr(up), quant_type, h2d.shape[1],
                                                    x2d.shape[1], _ptr(h2d), _ptr(workspace), workspace_bytes, numerics, _stream(dev))
     _check(rc, "sngguf_gate_up_silu_ws")
@@ -534,7 +545,7 @@ def grouped_linear_ws_into(x2d, indicator, n_text, packed_und, qt_und, packed_ge
     bytes large problems decode both weight sets once and run one dense tile-GEMM launch over both row groups."""
     dev = x2d.device
     dw_bytes = dense_workspace.numel() * dense_workspace.element_size() if dense_workspace is not None else 0
-    with _on(dev):
+    with _on(dev), _whole_call(dev):
         rc = load_library().sngguf_grouped_linear_ws(
             _ptr(x2d), x2d.shape[0], _ptr(indicator), n_text, _ptr(packed_und), qt_und, _ptr(packed_gen), qt_gen,
             y2d.shape[1], x2d.shape[1], _ptr(bias_und), _ptr(bias_gen), _ptr(y2d), _ptr(workspace), _ptr(dense_workspace),

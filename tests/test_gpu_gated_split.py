@@ -181,9 +181,10 @@ def test_forty_rows_leave_no_weight_sized_workspace(dev):
     assert sum(ws.numel() for ws in ops._workspaces.values()) <= 2 * m * n
 
 
-@pytest.mark.parametrize("m", [17, 40, 64])
+@pytest.mark.parametrize("m", [17, 40, 64, 203])
 def test_threads_on_one_stream(dev, m):
-    """Four host threads, each with rows of its own, through one MLP on the default stream."""
+    """Four host threads, each with rows of its own, through one MLP on the default stream: scratch of the call (up to 64
+    rows) and of the pool (beyond)."""
     print(f"case threads on one stream m={m}", flush=True)
     n, k = 1024, 2048
     mods = []

@@ -59,3 +59,34 @@ def test_a_short_prompt_s_gate_outputs_are_the_call_s_own(host_scratch, monkeypa
         x = torch.full((m, k), float(i + 1), dtype=torch.bfloat16)
         assert torch.equal(modality._gated_activations(x, m, *mods, None, 1e-6), x[:, :n])
     _in_threads(4, one)
+
+
+@pytest.mark.parametrize("entry", ["linear_ws", "gate_up_silu_ws", "grouped_linear_ws"])
+def test_calls_that_share_a_pooled_workspace_do_not_interleave(host_scratch, monkeypatch, entry):
+    """The pool hands the threads of one stream the same memory; one call's launches are then enqueued as one run."""
+    import contextlib
+    import types
+    scratch, seen = [None], []
+
+    def launches(*args):
+        me = threading.get_ident()
+        scratch[0] = me                     # the first launch fills the workspace
+        time.sleep(0.01)                    # (a foreign call: the interpreter lock is free)
+        seen.append(scratch[0] == me)       # the second launch reads it
+        return 0
+
+    monkeypatch.setattr(ops, "_on", lambda dev: contextlib.nullcontext())
+    monkeypatch.setattr(ops, "load_library", lambda: types.SimpleNamespace(**{f"sngguf_{entry}": launches}))
+    x, y, w = torch.zeros((80, 64), dtype=torch.bfloat16), torch.zeros((80, 32), dtype=torch.bfloat16), torch.zeros((32, 68), dtype=torch.uint8)
+
+    def one(i):
+        for _ in range(5):
+            ws = ops.pooled_workspace(x.device, 4096 * (i + 1))
+            if entry == "linear_ws":
+                ops.linear_ws_into(x, w, ops.Q8_0, None, y, ws, 1)
+            elif entry == "gate_up_silu_ws":
+                ops.gate_up_silu_ws_into(x, w, w, ops.Q8_0, y, ws, 1)
+            else:
+                ops.grouped_linear_ws_into(x, None, 40, w, ops.Q8_0, w, ops.Q8_0, None, None, y, None, ws, 1)
+    _in_threads(4, one)
+    assert len(seen) == 20 and all(seen)
