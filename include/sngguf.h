@@ -146,6 +146,10 @@ int sngguf_linear_residual(const void* x, int64_t M, const void* q, int qtype, i
  * be ordered on one stream.  Never allocates.
  */
 int64_t sngguf_linear_workspace_bytes(int64_t N, int64_t K);
+/* The workspace with which M rows of this shape take their fastest form: the decoded weights where they go through memory,
+ * and the partial sums of as many K slices as pay.  More room changes nothing (the same launches, the same sums); 0 where no
+ * workspace is used (M < 65 among them). */
+int64_t sngguf_linear_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K);
 int sngguf_linear_ws(const void* x, int64_t M, const void* q, int qtype, int64_t N, int64_t K,
                      const void* bias, void* y, void* workspace, int64_t workspace_bytes, int numerics,
                      void* stream);

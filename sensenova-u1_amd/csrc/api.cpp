@@ -272,6 +272,43 @@ bool grouped_dense_route_fits(int64_t M, int64_t N, int64_t K) {
 int64_t sngguf_linear_workspace_bytes(int64_t N, int64_t K) { return N > 0 && K > 0 && N < kMaxDim && K < kMaxDim ? 2 * N * K : 0; }
 
 namespace {
+// How sngguf_linear_ws runs a shape of dense_route_fits when it is given `workspace_bytes`: the K slices of a split (1 = no
+// split), and what lies in front of their partial sums.
+struct LinearSplit {
+    bool tile_type;        // the large-tile kernel reads the packed rows itself: no weight pass in front of a split
+    int64_t dense_bytes;   // the decoded weights where it does not
+    int64_t slices;
+};
+
+LinearSplit linear_split(int qtype, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
+    const bool plain = qtype == SNGGUF_TYPE_BF16;   // rows that are bf16 already: no weight pass, the dense kernel reads them
+    // Few output tiles (a few hundred rows, or a narrow matrix): a 256 x 256 tile takes as long per K step whether
+    // or not the other compute units have work, so K is split over enough workgroups to occupy them, with the fp32
+    // partial sums in the workspace.  The formats the large-tile kernel decodes itself need no weight pass then and
+    // the whole workspace is free for the sums; the others put them behind the decoded weights if the caller's
+    // workspace is that large.
+    // (from 4096 rows on the weight pass pays for itself even here: a K step of the dense kernel takes 1.4 us against 2.0 us
+    // with the decode in the loop, and sixteen row tiles share one pass - 4096 x 1024 <- 4096: 56 against 61 us, 2048 wide
+    // 80 against 92 us; at 512 rows the pass costs more than it saves, 48 against 44 us on 4096 x 4096)
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    LinearSplit f{plain || ((qtype == SNGGUF_TYPE_Q8_0 || qtype == SNGGUF_TYPE_Q4_K) && M < 4096), 0, 1};
+    f.dense_bytes = f.tile_type ? 0 : 2 * N * K;
+    if (tiles <= 128 && workspace_bytes > f.dense_bytes)
+        f.slices = pick_k_slices(M, N, tiles, K / 64, (workspace_bytes - f.dense_bytes) / (4 * M * N), f.tile_type && !plain);
+    return f;
+}
+}  // namespace
+
+int64_t sngguf_linear_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
+    if (!known_type(qtype) || M <= 0 || N <= 0 || K <= 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || K % sngguf_block_size(qtype) != 0
+        || !dense_route_fits(M, N, K))
+        return 0;
+    const LinearSplit f = linear_split(qtype, M, N, K, INT64_MAX);
+    if (f.slices >= 2) return f.dense_bytes + f.slices * 4 * M * N;
+    return qtype == SNGGUF_TYPE_BF16 || row_chunks_win(M, N, K, qtype) ? 0 : 2 * N * K;
+}
+
+namespace {
 int linear_ws_impl(const void* x, int64_t M, const void* q, int qtype, int64_t N, int64_t K, const void* bias, void* y,
                    void* workspace, int64_t workspace_bytes, int numerics, void* stream) {
     const int rc = check_matmul(x, M, q, qtype, N, K, y, numerics);
@@ -282,29 +319,14 @@ int linear_ws_impl(const void* x, int64_t M, const void* q, int qtype, int64_t N
     const bool plain = qtype == SNGGUF_TYPE_BF16;   // rows that are bf16 already: no weight pass, the dense kernel reads them
     const bool fits = workspace && dense_route_fits(M, N, K);
     if (!fits) return linear_impl(x, M, q, qtype, N, K, bias, nullptr, y, numerics, stream);
-    // Few output tiles (a few hundred rows, or a narrow matrix): a 256 x 256 tile takes as long per K step whether
-    // or not the other compute units have work, so K is split over enough workgroups to occupy them, with the fp32
-    // partial sums in the workspace.  The formats the large-tile kernel decodes itself need no weight pass then and
-    // the whole workspace is free for the sums; the others put them behind the decoded weights if the caller's
-    // workspace is that large.
-    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-    const int64_t ksteps = K / 64;
-    // (from 4096 rows on the weight pass pays for itself even here: a K step of the dense kernel takes 1.4 us against 2.0 us
-    // with the decode in the loop, and sixteen row tiles share one pass - 4096 x 1024 <- 4096: 56 against 61 us, 2048 wide
-    // 80 against 92 us; at 512 rows the pass costs more than it saves, 48 against 44 us on 4096 x 4096)
-    const bool tile_type = plain || ((qtype == SNGGUF_TYPE_Q8_0 || qtype == SNGGUF_TYPE_Q4_K) && M < 4096);
-    const int64_t dense_bytes = tile_type ? 0 : 2 * N * K;
-    if (tiles <= 128 && workspace_bytes > dense_bytes) {
-        const int64_t room = (workspace_bytes - dense_bytes) / (4 * M * N);
-        const int64_t slices = pick_k_slices(M, N, tiles, ksteps, room, tile_type && !plain);
-        if (slices >= 2) {
-            float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + dense_bytes);
-            if (tile_type)
-                return sngguf::launch_gemm_splitk(x, M, q, plain ? 30 : qtype, N, K, bias, y, partial, (int)slices, numerics, s);
-            const int rd = sngguf::launch_dequantize(q, qtype, N, K, workspace, SNGGUF_OUT_BF16, numerics, s);
-            if (rd != SNGGUF_OK) return rd;
-            return sngguf::launch_gemm_splitk(x, M, workspace, 30, N, K, bias, y, partial, (int)slices, numerics, s);
-        }
+    const LinearSplit f = linear_split(qtype, M, N, K, workspace_bytes);
+    if (f.slices >= 2) {
+        float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + f.dense_bytes);
+        if (f.tile_type)
+            return sngguf::launch_gemm_splitk(x, M, q, plain ? 30 : qtype, N, K, bias, y, partial, (int)f.slices, numerics, s);
+        const int rd = sngguf::launch_dequantize(q, qtype, N, K, workspace, SNGGUF_OUT_BF16, numerics, s);
+        if (rd != SNGGUF_OK) return rd;
+        return sngguf::launch_gemm_splitk(x, M, workspace, 30, N, K, bias, y, partial, (int)f.slices, numerics, s);
     }
     if (plain) return linear_impl(x, M, q, qtype, N, K, bias, nullptr, y, numerics, stream);
     // no room for a K split: row chunks through the decode kernel where they beat the few tiles of the dense kernel too

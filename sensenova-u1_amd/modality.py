@@ -55,11 +55,15 @@ def grouped_linear(hidden_states: torch.Tensor, image_gen_indicators: Optional[t
                 # the library's workspace route: each group takes the kernels its own row count calls for
                 x2d = proj._checked_rows(hidden_states)
                 proj_mot_gen._checked_rows(hidden_states)
-                ws = ops.pooled_workspace(x2d.device, max(proj._workspace_bytes(split), proj._workspace_bytes(x2d.shape[0] - split)))
+                nbytes = max(proj._workspace_bytes(split), proj_mot_gen._workspace_bytes(x2d.shape[0] - split))
+                if split * proj.out_features % 8:
+                    # image rows that would not start at a 16-byte boundary: one launch over both groups, both weights decoded
+                    nbytes = max(nbytes, 2 * ops.linear_workspace_bytes(proj.out_features, proj.in_features))
+                ws = ops.pooled_workspace(x2d.device, nbytes)
                 bu = proj.bias.detach().to(torch.bfloat16).contiguous() if proj.bias is not None else None
                 bg = proj_mot_gen.bias.detach().to(torch.bfloat16).contiguous() if proj_mot_gen.bias is not None else None
                 ops.grouped_linear_ws_into(x2d, None, split, proj.weight, int(proj.weight.quant_type), proj_mot_gen.weight,
-                                           int(proj_mot_gen.weight.quant_type), bu, bg, out, None, ws, proj.numerics)
+                                           int(proj_mot_gen.weight.quant_type), bu, bg, out, None, ws, proj.numerics, nbytes)
                 return out.reshape(*hidden_states.shape[:-1], proj.out_features)
             for mod, lo, hi in ((proj, 0, split), (proj_mot_gen, split, x2d.shape[0])):
                 if hi - lo > 64:
@@ -489,10 +493,8 @@ class SharedInputStack:
                 y = ops.linear(x, self.stacked, qt, None, first.numerics)
             elif first.gemm_policy == "auto" and x.is_contiguous():
                 # the workspace route of a single module (quantized_linear.GGUFLinear.forward), on the stacked rows
-                n, k = self.stacked.shape[0], first.in_features
-                nbytes = ops.linear_workspace_bytes(n, k)
-                if -(-rows // 256) * -(-n // 256) <= 128:
-                    nbytes += 16 * rows * n
+                n = self.stacked.shape[0]
+                nbytes = ops.linear_ws_bytes(qt, rows, n, first.in_features)
                 x2d = first._checked_rows(x)
                 y = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=x.device)
                 ops.linear_ws_into(x2d, self.stacked, qt, None, y.view(-1, n), ops.pooled_workspace(x.device, nbytes), first.numerics)

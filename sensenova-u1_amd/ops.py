@@ -35,7 +35,7 @@ _OUT_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 EXPORTED_SYMBOLS = (
     "sngguf_version", "sngguf_strerror", "sngguf_type_size", "sngguf_block_size", "sngguf_dequantize",
-    "sngguf_linear", "sngguf_linear_residual", "sngguf_linear_workspace_bytes", "sngguf_linear_ws", "sngguf_linear_static_max_outputs", "sngguf_linear_static", "sngguf_gate_up_silu", "sngguf_gate_up_silu_workspace_bytes", "sngguf_gate_up_silu_ws_fits", "sngguf_gate_up_silu_ws_bytes", "sngguf_gate_up_silu_ws", "sngguf_lm_head_argmax_workspace_bytes", "sngguf_lm_head_argmax", "sngguf_grouped_workspace_bytes", "sngguf_grouped_linear",
+    "sngguf_linear", "sngguf_linear_residual", "sngguf_linear_workspace_bytes", "sngguf_linear_ws_bytes", "sngguf_linear_ws", "sngguf_linear_static_max_outputs", "sngguf_linear_static", "sngguf_gate_up_silu", "sngguf_gate_up_silu_workspace_bytes", "sngguf_gate_up_silu_ws_fits", "sngguf_gate_up_silu_ws_bytes", "sngguf_gate_up_silu_ws", "sngguf_lm_head_argmax_workspace_bytes", "sngguf_lm_head_argmax", "sngguf_grouped_workspace_bytes", "sngguf_grouped_linear",
     "sngguf_grouped_linear_ws", "sngguf_q8_0_tiled_bytes", "sngguf_q8_0_tile", "sngguf_linear_tiled", "sngguf_gate_up_silu_tiled",
     "sngguf_rmsnorm_fits", "sngguf_rmsnorm", "sngguf_rmsnorm_linear", "sngguf_rmsnorm_gate_up_silu",
     "sngguf_rmsnorm_linear_tiled", "sngguf_rmsnorm_gate_up_silu_tiled",
@@ -92,6 +92,8 @@ def load_library() -> ctypes.CDLL:
     lib.sngguf_gate_up_silu_workspace_bytes.restype = i64
     lib.sngguf_gate_up_silu_ws_fits.argtypes = [ci, i64, i64, i64]
     lib.sngguf_gate_up_silu_ws_fits.restype = ci
+    lib.sngguf_linear_ws_bytes.argtypes = [ci, i64, i64, i64]
+    lib.sngguf_linear_ws_bytes.restype = i64
     lib.sngguf_gate_up_silu_ws_bytes.argtypes = [ci, i64, i64, i64]
     lib.sngguf_gate_up_silu_ws_bytes.restype = i64
     lib.sngguf_gate_up_silu_ws.argtypes = [vp, i64, vp, vp, ci, i64, i64, vp, vp, i64, ci, vp]
@@ -352,6 +354,11 @@ def linear_workspace_bytes(n: int, k: int) -> int:
     return int(load_library().sngguf_linear_workspace_bytes(n, k))
 
 
+def linear_ws_bytes(quant_type: int, m: int, n: int, k: int) -> int:
+    """Bytes of workspace with which ``m`` rows take their fastest form in ``linear_ws_into``; more changes nothing."""
+    return int(load_library().sngguf_linear_ws_bytes(quant_type, m, n, k))
+
+
 def linear_ws_into(x2d: torch.Tensor, packed: torch.Tensor, quant_type: int, bias: Optional[torch.Tensor],
                    y2d: torch.Tensor, workspace: Optional[torch.Tensor], numerics: int) -> None:
     """As ``linear_into``; with a device ``workspace`` of at least ``linear_workspace_bytes(N, K)`` bytes large
@@ -540,11 +547,14 @@ def grouped_linear_into(x2d, indicator, n_text, packed_und, qt_und, packed_gen, 
 
 
 def grouped_linear_ws_into(x2d, indicator, n_text, packed_und, qt_und, packed_gen, qt_gen, bias_und, bias_gen, y2d,
-                           workspace, dense_workspace, numerics) -> None:
+                           workspace, dense_workspace, numerics, dense_workspace_bytes: Optional[int] = None) -> None:
     """As ``grouped_linear_into``; with a device ``dense_workspace`` of at least ``2 * linear_workspace_bytes(N, K)``
-    bytes large problems decode both weight sets once and run one dense tile-GEMM launch over both row groups."""
+    bytes large problems decode both weight sets once and run one dense tile-GEMM launch over both row groups.
+    ``dense_workspace_bytes``: how much of it to use (default all of it)."""
     dev = x2d.device
-    dw_bytes = dense_workspace.numel() * dense_workspace.element_size() if dense_workspace is not None else 0
+    dw_bytes = dense_workspace_bytes
+    if dw_bytes is None:
+        dw_bytes = dense_workspace.numel() * dense_workspace.element_size() if dense_workspace is not None else 0
     with _on(dev), _whole_call(dev):
         rc = load_library().sngguf_grouped_linear_ws(
             _ptr(x2d), x2d.shape[0], _ptr(indicator), n_text, _ptr(packed_und), qt_und, _ptr(packed_gen), qt_gen,

@@ -167,9 +167,9 @@ class GGUFLinear(nn.Linear):
     when ``in_features`` is a multiple of 256 - it is one fused dequant-GEMV launch that streams and
     decodes the weights once.  With more rows ``gemm_policy`` decides:
 
-    * ``"auto"`` (default): the library's own kernels through ``sngguf_linear_ws`` with a pooled workspace of
-      2 * N * K bytes, plus room for four fp32 copies of the output when the shape has few output tiles
-      (``ops.pooled_workspace``, one per device and stream, reused by every module): problems with few
+    * ``"auto"`` (default): the library's own kernels through ``sngguf_linear_ws`` with a pooled workspace
+      (``ops.pooled_workspace``, one per device and stream, reused by every module; each call asks for what its shape
+      can use, so the sums do not depend on how large the pool has grown): problems with few
       output tiles run the large-tile kernel with K split over workgroups, the rest one weight pass into the
       workspace (bf16, the same rounding chain) followed by the library's dense bf16 tile kernel.
     * ``"two_pass"`` (opt-in): one HIP dequantize launch writes a transient bf16 weight and the device library's
@@ -339,13 +339,7 @@ class GGUFLinear(nn.Linear):
         return residual + self(inputs)
 
     def _workspace_bytes(self, rows: int) -> int:
-        """What the workspace route is given for ``rows`` rows: the decoded weight, and for shapes with few 256 x 256
-        output tiles room for four fp32 copies of the output behind it (the library then splits K over workgroups)."""
-        n, k = self.out_features, self.in_features
-        nbytes = ops.linear_workspace_bytes(n, k)
-        if -(-rows // 256) * -(-n // 256) <= 128:
-            nbytes += 16 * rows * n
-        return nbytes
+        return ops.linear_ws_bytes(self._weight_type(), rows, self.out_features, self.in_features)
 
     def two_pass_into(self, x2d: torch.Tensor, out2d: torch.Tensor) -> None:
         """``out2d[M, N] = x2d[M, K] @ W^T (+ bias)`` for bf16 rows: one dequantize launch to a transient
@@ -357,9 +351,8 @@ class GGUFLinear(nn.Linear):
             if self._dense_cache is None or self._dense_cache[0] != key:
                 self._dense_cache = (key, ops.dequantize(self.weight, self._weight_type(), torch.bfloat16, self.numerics))
             weight = self._dense_cache[1]
-            rows, n = x2d.shape[0], self.out_features
-            few = -(-rows // 256) * -(-n // 256) <= 128
-            workspace = ops.pooled_workspace(x2d.device, 16 * rows * n) if few else None
+            nbytes = ops.linear_ws_bytes(ops.BF16, x2d.shape[0], self.out_features, self.in_features)
+            workspace = ops.pooled_workspace(x2d.device, nbytes) if nbytes else None
             bias = self.bias.detach().to(torch.bfloat16).contiguous() if self.bias is not None else None
             ops.linear_ws_into(x2d, weight.view(torch.uint8), ops.BF16, bias, out2d, workspace, self.numerics)
             return
