@@ -605,8 +605,8 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_kq_mfma_kernel(const bf16_t* _
     __syncthreads();
     if constexpr (MT > 1) {
         // R * MT groups of sums: one wavefront each (one wavefront alone would walk through all of them, 8 R MT reads, while
-        // the rest of the workgroup has left: with the gated
-        // epilogue below, 40 rows of an 8B layer in Q8_0 130 against 142 us).  Layout of a group as below, sums added in the same order.
+        // the rest of the workgroup has left: with the gated epilogue below, 40 rows of an 8B layer in Q8_0 130 against
+        // 142 us).  Layout of a group as below, sums added in the same order.
         for (int i = wave; i < R * MT; i += waves) {
             const int rg = i / MT, t = i - rg * MT, m = 16 * t + r;
             const int64_t n = n0 + 16 * rg + 4 * g, yi = (int64_t)m * N + n;
@@ -702,18 +702,25 @@ int launch_r(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64
     const int nsb = (int)(K >> 8);
     const int mt = (M + 15) / 16;
     // wavefronts per row group: enough that the launch fills the chip (about 12 per compute unit),
-    // at least one super-block each, at most 8 per workgroup.  Beyond 16 rows they are counted per 16 weight rows whatever
-    // R is, so that a row's K is cut into the same pieces (and its partial sums are added in the same order) for both.
+    // at least one super-block each, at most 8 per workgroup; beyond 16 rows counted per 16 weight rows whatever R is
     const int64_t per_group = gated ? 2 : 1, counted = mt > 1 ? (N + 15) / 16 : groups;
     int64_t w = (256 * 12 + counted * per_group - 1) / (counted * per_group);
     if (w < 1) w = 1;
-    // Q6_K on a vocabulary-sized matrix: two wavefronts per workgroup share the staged activations, which leaves room for
-    // more wavefronts per compute unit (151936 x 4096 at M = 1: 118 against 129 us with one, 124 with four)
+    // Q6_K from about 98300 columns on (fewer have two and more by the count above): two wavefronts with half of K each
+    // (151936 x 4096, us against one wavefront: one row 132 / 148, two - each stages its half of them - 133 / 159, four
+    // 141 / 145, sixteen 165 / 167; 100003 x 2048: one row 49 / 52, sixteen 60 / 63; four wavefronts gain less)
     if (QT == SNGGUF_TYPE_Q6_K && R == 2 && mt == 1 && w < 2) w = 2;
     if (w > nsb) w = nsb;
-    // long rows beyond 16 activation rows, every compute unit with a workgroup: four wavefronts with twice the run of K
-    // each (4096 x 12288, 40 rows: Q8_0 35.9 against 38.2 us, Q6_K 37.2 against 38.9)
-    const int64_t cap = gated || (mt > 1 && nsb >= 32 && groups >= 256) ? 4 : 8;
+    // Beyond 16 rows at most four wavefronts per workgroup
+    //  - with more workgroups than compute units: two operands and more leave room for eight wavefronts on a compute unit,
+    //    so a workgroup of five to eight holds the next one back and a second round begins at 8193 columns (10240 x 4096,
+    //    17 / 48 rows, us: Q8_0 21.3 / 32.2 against 27.7 / 37.0 with up to eight, Q5_0 20.4 / 30.2 against 31.3 / 37.5);
+    //  - with exactly one workgroup each, rows of K of 8192 and more and enough activation rows: twice the run of K each
+    //    (4096 x 12288, 40 rows: Q8_0 35.9 against 38.2 us, Q6_K 37.2 against 38.9).  With fewer rows the eight hide more of
+    //    the decode (17 rows: Q4_K 20.3 against 21.6 us, Q5_0 21.3 against 24.0), longest in the formats with a fifth bit.
+    constexpr int kFourFrom = QT == SNGGUF_TYPE_Q5_0 || QT == SNGGUF_TYPE_Q5_1 || QT == SNGGUF_TYPE_Q5_K ? 26 : 22;
+    const bool four = mt > 1 && (groups > 256 || (groups == 256 && nsb >= 32 && M >= kFourFrom));
+    const int64_t cap = gated || four ? 4 : 8;
     if (w > cap) w = cap;
     const int waves = (int)(gated ? 2 * w : w);
     const size_t slab = (size_t)waves * 16 * R * Slab<QT>::stride;
@@ -783,7 +790,11 @@ int launch_r(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64
 }
 
 // Weight rows per workgroup (see launch_qt) as a function, so that the arg-max caller can size its slot array.
-inline int rows_per_workgroup(int64_t M, int64_t N) { return (M <= 16 ? N >= 32768 : N > 4096) ? 32 : 16; }
+inline int rows_per_workgroup(int qtype, int64_t M, int64_t N) {
+    if (M <= 16) return N >= 32768 ? 32 : 16;
+    if (qtype == SNGGUF_TYPE_Q5_K && M > 48 && ((N > 8192 && N <= 12288) || (N > 16384 && N < 24576))) return 16;
+    return N > 4096 ? 32 : 16;
+}
 
 template <int QT, int NUM>
 int launch_qt(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64_t N, int64_t K, const bf16_t* bias,
@@ -795,8 +806,12 @@ int launch_qt(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int6
     // holds one workgroup of eight wavefronts: as soon as 16-row groups need a second round of workgroups (more than 256
     // of them), 32 rows per workgroup halve both.  40 rows, Q8_0 / Q4_K: 6144 x 4096 28.9 -> 20.3 / 26.7 -> 19.1 us,
     // 12288 x 4096 36.2 -> 31.9 / 34.2 -> 29.0 us; at 64 rows 39.8 -> 29.7 and 50.4 -> 47.3 us (Q8_0); where 16-row
-    // groups fit one round it loses (4096 x 4096, 40 rows: 15.2 -> 18.9 us).
-    if (rows_per_workgroup(M, N) == 32) return launch_r<QT, NUM, 2>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax, gate);
+    // groups fit one round it loses (4096 x 4096, 40 rows: 15.2 -> 18.9 us).  Measured for all ten formats at 1024 .. 151936
+    // columns and 17 .. 64 rows: level to 1.9 times as fast, but for Q5_K beyond 48 rows, whose four operands and two row
+    // groups do not fit the registers (45 of them go through memory): there one group stays where two leave compute units
+    // waiting in their last round (49 rows, one / two groups, us: 10240 x 4096 40 / 45, 12288 x 4096 41 / 47, 20480 x 4096
+    // 67 / 103, but 8192 x 4096 34 / 30, 14336 x 4096 53 / 49, 24576 x 4096 96 / 83).
+    if (rows_per_workgroup(QT, M, N) == 32) return launch_r<QT, NUM, 2>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax, gate);
     return launch_r<QT, NUM, 1>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax, gate);
 }
 
@@ -1176,13 +1191,13 @@ int launch_mlp_kq_decode(const void* x, int64_t M, const void* gamma, float eps,
 
 // Workgroups of a plain decode launch = (value, column) slots per activation row that its arg-max form writes.
 int64_t gemv_argmax_slots(int qtype, int64_t M, int64_t N) {
-    const int64_t rows = qtype == SNGGUF_TYPE_Q8_0 ? 16 : rows_per_workgroup(M, N);   // (Q8_0 has kernels of its own)
+    const int64_t rows = qtype == SNGGUF_TYPE_Q8_0 ? 16 : rows_per_workgroup(qtype, M, N);   // (Q8_0 has kernels of its own)
     return (N + rows - 1) / rows;
 }
 
 // 1 <= M <= 64 (SiLU-gated pair: M <= 16), K % 256 == 0, 16-byte aligned x and q (checked by the caller).  `gamma`
-// (K bf16, 16-byte aligned) switches the fused RMSNorm on; the caller keeps M (2 K + 64) <= 36 KB then.  `gate` ([M][N], M > 16,
-// no bias or residual): y = silu(gate) * projection.
+// (K bf16, 16-byte aligned) switches the fused RMSNorm on; the caller keeps M (2 K + 64) <= 36 KB then.  `gate` ([M][N],
+// M > 16, no bias or residual): y = silu(gate) * projection.
 int launch_gemv_kq_mfma(const void* x, int64_t M, const void* qa, const void* qb, int qtype, int64_t N, int64_t K,
                         const void* bias, const void* residual, void* y, int numerics, bool gated, hipStream_t stream,
                         const void* gamma, float eps, uint64_t* amax, const void* gate) {
