@@ -613,7 +613,7 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_kq_mfma_kernel(const bf16_t* _
             if (m >= M || n >= N) continue;
             const bool whole = n + 3 < N && (N & 3) == 0;
             u32x2_t gv = {0u, 0u};
-            if (gate && whole) gv = *reinterpret_cast<const u32x2_t*>(gate + yi);   // requested ahead of the sums
+            if (gate) gv = *reinterpret_cast<const u32x2_t*>(gate + yi);   // requested ahead of the sums (N % 8 == 0: whole)
             f32x4_t sum = red[i * 64 + lane];
             for (int w = 1; w < W; w++) {
                 const f32x4_t p = red[(w * R * MT + i) * 64 + lane];
@@ -627,7 +627,7 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_kq_mfma_kernel(const bf16_t* _
                 if (gate) {
                     // the up projection of a SiLU-gated pair: `gate` holds the gate projection's outputs, and the value is
                     // the rounded silu of those times the rounded output here, as the gated pair's own launch rounds
-                    const float gt = whole ? ((v & 1) ? bf16hi_to_f32(gv[v >> 1]) : bf16lo_to_f32(gv[v >> 1])) : bf16_to_f32(gate[yi + v]);
+                    const float gt = (v & 1) ? bf16hi_to_f32(gv[v >> 1]) : bf16lo_to_f32(gv[v >> 1]);
                     o[v] = bf16_to_f32(f32_to_bf16(gt / (1.0f + expf(-gt)))) * bf16_to_f32(f32_to_bf16(o[v]));
                 }
             }
@@ -1197,11 +1197,11 @@ int64_t gemv_argmax_slots(int qtype, int64_t M, int64_t N) {
 
 // 1 <= M <= 64 (SiLU-gated pair: M <= 16), K % 256 == 0, 16-byte aligned x and q (checked by the caller).  `gamma`
 // (K bf16, 16-byte aligned) switches the fused RMSNorm on; the caller keeps M (2 K + 64) <= 36 KB then.  `gate` ([M][N],
-// M > 16, no bias or residual): y = silu(gate) * projection.
+// 8-byte aligned, M > 16, N % 4 == 0, no bias or residual): y = silu(gate) * projection.
 int launch_gemv_kq_mfma(const void* x, int64_t M, const void* qa, const void* qb, int qtype, int64_t N, int64_t K,
                         const void* bias, const void* residual, void* y, int numerics, bool gated, hipStream_t stream,
                         const void* gamma, float eps, uint64_t* amax, const void* gate) {
-    if (gate && (gated || M <= 16 || bias || residual)) return SNGGUF_E_BADSHAPE;
+    if (gate && (gated || M <= 16 || N % 4 != 0 || bias || residual)) return SNGGUF_E_BADSHAPE;
     const bf16_t* gt = static_cast<const bf16_t*>(gate);
     if (amax && (gated || M > 16)) return SNGGUF_E_BADSHAPE;
     const bf16_t* gp = static_cast<const bf16_t*>(gamma);
