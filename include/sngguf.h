@@ -272,6 +272,11 @@ int sngguf_gate_up_silu(const void* x, int64_t M, const void* q_gate, const void
 int64_t sngguf_gate_up_silu_workspace_bytes(int64_t N, int64_t K);
 int sngguf_gate_up_silu_ws_fits(int qtype, int64_t M, int64_t N, int64_t K);
 int64_t sngguf_gate_up_silu_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K);
+/* The form in which this entry point is faster than two projections, silu and the product, and which M rows of this shape
+ * take with sngguf_gate_up_silu_ws_bytes of workspace; SNGGUF_PAIR_SEPARATE where there is none (the entry point still runs
+ * every shape that sngguf_gate_up_silu_ws_fits takes). */
+enum { SNGGUF_PAIR_SEPARATE = 0, SNGGUF_PAIR_DECODE = 1, SNGGUF_PAIR_SPLIT = 2, SNGGUF_PAIR_DENSE = 3 };
+int sngguf_gate_up_silu_ws_form(int qtype, int64_t M, int64_t N, int64_t K);
 int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const void* q_up, int qtype,
                            int64_t N, int64_t K, void* h, void* workspace, int64_t workspace_bytes,
                            int numerics, void* stream);

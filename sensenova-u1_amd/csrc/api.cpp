@@ -394,11 +394,18 @@ enum PairForm {
     kPairDense,   // two weight passes, one dense launch with the gated epilogue
 };
 
+// Whether the dense launch's ceil(M / 256) x ceil(N / 128) tiles come close to whole rounds of the 256 compute units (it has no
+// K split).  12288 x 4096, gated launch / two launches and the product, us: 512 rows (0.75 of a round) 183 / 199, 768
+// (1.125 rounds) 265 / 245, 1024 (1.5) 237 / 246, 1280 (1.875) 287 / 312, 1536 (2.25) 368 / 460, 2048 354 / 446, 4096 631 / 706.
+bool pair_fills(int64_t M, int64_t N) {
+    const int64_t gated_tiles = ((M + 255) / 256) * ((N + 127) / 128);
+    return M >= 512 && 10 * gated_tiles >= 7 * 256 * ((gated_tiles + 255) / 256);
+}
+
 PairForm pair_form(int qtype, int64_t M, int64_t N, int64_t K) {
     if (M <= 64 && K % 256 == 0) return kPairDecode;
-    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), gated_tiles = ((M + 255) / 256) * ((N + 127) / 128);
-    const bool fills = M >= 512 && 10 * gated_tiles >= 7 * 256 * ((gated_tiles + 255) / 256);
-    if ((qtype == SNGGUF_TYPE_Q8_0 || qtype == SNGGUF_TYPE_Q4_K) && M >= 65 && M < 4096 && tiles <= 128 && !fills) return kPairSplit;
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    if ((qtype == SNGGUF_TYPE_Q8_0 || qtype == SNGGUF_TYPE_Q4_K) && M >= 65 && M < 4096 && tiles <= 128 && !pair_fills(M, N)) return kPairSplit;
     return kPairDense;
 }
 
@@ -409,6 +416,19 @@ int64_t pair_slices(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
     return pick_pair_slices(M, N, 2 * tiles, K / 64, workspace_bytes / (8 * M * N));
 }
 }  // namespace
+
+int sngguf_gate_up_silu_ws_form(int qtype, int64_t M, int64_t N, int64_t K) {
+    if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return SNGGUF_PAIR_SEPARATE;
+    switch (pair_form(qtype, M, N, K)) {
+    // against two projections, silu and the product (12288 x 4096, graphs of the launches alone, us): Q8_0 17 / 40 / 64 rows
+    // 49 / 65 / 94 against 54 / 80 / 109, Q4_K 38 / 57 / 87 against 45 / 74 / 104
+    case kPairDecode: return SNGGUF_PAIR_DECODE;
+    // (two fp32 copies of both outputs fit the 4 N K bytes of the dense form.)  As above: Q8_0 65 / 203 / 509 rows 76 / 84 / 146
+    // against 87 / 111 / 186, Q4_K 74 / 81 / 143 against 85 / 109 / 183; 6144 x 2048, 9728 x 2560, 4096 x 4096 1.2 - 1.9 times
+    case kPairSplit: return K >= 256 && 4 * M <= K ? SNGGUF_PAIR_SPLIT : SNGGUF_PAIR_SEPARATE;
+    default: return pair_fills(M, N) ? SNGGUF_PAIR_DENSE : SNGGUF_PAIR_SEPARATE;
+    }
+}
 
 int64_t sngguf_gate_up_silu_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
     if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return 0;

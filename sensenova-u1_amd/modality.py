@@ -260,10 +260,8 @@ def _gated_activations(x, rows, gate_proj, up_proj, norm_weight, eps) -> torch.T
     return h
 
 
-# The gated launch has ceil(rows / 256) x ceil(N / 128) output tiles and no K split, so it pays when those tiles come close
-# to whole rounds of the chip's 256 compute units.  Measured on 12288 x 4096 (gated launch / two launches and the product,
-# us): 512 rows (0.75 of a round) 183 / 199, 768 (1.125 rounds) 265 / 245, 1024 (1.5) 237 / 246, 1280 (1.875) 287 / 312,
-# 1536 (2.25) 368 / 460, 2048 354 / 446, 4096 631 / 706.
+# From how many rows on, and how full, the tiles of the gated dense launch have to be for it to pay
+# (``ops.gate_up_silu_ws_form`` decides; these say by which measure).
 GATED_TILE_MIN_ROWS = 512
 GATED_TILE_MIN_FILL = 0.7
 
@@ -287,8 +285,7 @@ def _called_as_modules(mod) -> bool:
 
 def _gated_tile_route(x, rows, same, gate_proj, up_proj) -> bool:
     """Whether ``gated_mlp`` hands gate / up / SiLU to ``sngguf_gate_up_silu_ws``: both weights of one packed type and
-    shape, no bias, default GEMM policy, and enough rows and tiles to fill the chip with the gated dense launch, or a shape
-    for which the library splits K of both matrices and ends the reduction in the gated product, or at most 64 rows."""
+    shape, no bias, default GEMM policy, and a shape for which the library has a faster form than two projections."""
     if not (rows > 16 and same and x.is_cuda and x.dtype == torch.bfloat16):
         return False
     if gate_proj.bias is not None or up_proj.bias is not None:
@@ -299,26 +296,15 @@ def _gated_tile_route(x, rows, same, gate_proj, up_proj) -> bool:
         return False
     if gate_proj.numerics != up_proj.numerics:
         return False
-    filled = rows >= GATED_TILE_MIN_ROWS and gated_tile_fill(rows, gate_proj.out_features) >= GATED_TILE_MIN_FILL
+    form = ops.gate_up_silu_ws_form(int(gate_proj.weight.quant_type), rows, gate_proj.out_features, gate_proj.in_features)
+    if form == ops.PAIR_SEPARATE:
+        return False
     # where gate_proj(x) and up_proj(x) would be the modules' own calls, whatever hangs on those calls keeps them, the refusal
     # of an input that is not in a module's compute dtype included
-    if not filled and any(_called_as_modules(m) or (m.compute_dtype or x.dtype) != torch.bfloat16 for m in (gate_proj, up_proj)):
+    if form != ops.PAIR_DENSE and any(_called_as_modules(m) or (m.compute_dtype or x.dtype) != torch.bfloat16 for m in (gate_proj, up_proj)):
         return False
-    n, k, qt = gate_proj.out_features, gate_proj.in_features, int(gate_proj.weight.quant_type)
-    if rows <= 64:
-        # the decode kernels: the gate projection, then the up projection with silu and the product in its epilogue.
-        # 40 rows, whole layers of the 8B model in
-        # Q8_0: 130 us per layer against 142 with two projections, silu and the product
-        # (not while something traces or intercepts: the modules' own calls are registered ops at these sizes)
-        if k % 256 != 0 or not ops._eager(x):
-            return False
-    elif not filled:
-        # room for two fp32 copies of both outputs in the 4 n k bytes of workspace.  Against two projections, two
-        # reductions, silu and the product (12288 x 4096 pair, whole layers of the 8B model, us): 203 rows Q4_K / Q6_K
-        # 231 / 253 per layer, 509 rows Q8_0 333 / 374
-        if not (qt in (ops.Q8_0, ops.Q4_K) and 256 <= k and 4 * rows <= k and -(-rows // 256) * -(-n // 256) <= 128):
-            return False
-    return ops.gate_up_silu_ws_fits(qt, rows, n, k)
+    # (not while something traces or intercepts: the modules' own calls are registered ops at these sizes)
+    return form != ops.PAIR_DECODE or ops._eager(x)
 
 
 def _is_silu(fn) -> bool:

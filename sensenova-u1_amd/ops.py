@@ -35,7 +35,7 @@ _OUT_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 EXPORTED_SYMBOLS = (
     "sngguf_version", "sngguf_strerror", "sngguf_type_size", "sngguf_block_size", "sngguf_dequantize",
-    "sngguf_linear", "sngguf_linear_residual", "sngguf_linear_workspace_bytes", "sngguf_linear_ws_bytes", "sngguf_linear_ws", "sngguf_linear_static_max_outputs", "sngguf_linear_static", "sngguf_gate_up_silu", "sngguf_gate_up_silu_workspace_bytes", "sngguf_gate_up_silu_ws_fits", "sngguf_gate_up_silu_ws_bytes", "sngguf_gate_up_silu_ws", "sngguf_lm_head_argmax_workspace_bytes", "sngguf_lm_head_argmax", "sngguf_grouped_workspace_bytes", "sngguf_grouped_linear",
+    "sngguf_linear", "sngguf_linear_residual", "sngguf_linear_workspace_bytes", "sngguf_linear_ws_bytes", "sngguf_linear_ws", "sngguf_linear_static_max_outputs", "sngguf_linear_static", "sngguf_gate_up_silu", "sngguf_gate_up_silu_workspace_bytes", "sngguf_gate_up_silu_ws_fits", "sngguf_gate_up_silu_ws_form", "sngguf_gate_up_silu_ws_bytes", "sngguf_gate_up_silu_ws", "sngguf_lm_head_argmax_workspace_bytes", "sngguf_lm_head_argmax", "sngguf_grouped_workspace_bytes", "sngguf_grouped_linear",
     "sngguf_grouped_linear_ws", "sngguf_q8_0_tiled_bytes", "sngguf_q8_0_tile", "sngguf_linear_tiled", "sngguf_gate_up_silu_tiled",
     "sngguf_rmsnorm_fits", "sngguf_rmsnorm", "sngguf_rmsnorm_linear", "sngguf_rmsnorm_gate_up_silu",
     "sngguf_rmsnorm_linear_tiled", "sngguf_rmsnorm_gate_up_silu_tiled",
@@ -94,6 +94,8 @@ def load_library() -> ctypes.CDLL:
     lib.sngguf_gate_up_silu_ws_fits.restype = ci
     lib.sngguf_linear_ws_bytes.argtypes = [ci, i64, i64, i64]
     lib.sngguf_linear_ws_bytes.restype = i64
+    lib.sngguf_gate_up_silu_ws_form.argtypes = [ci, i64, i64, i64]
+    lib.sngguf_gate_up_silu_ws_form.restype = ci
     lib.sngguf_gate_up_silu_ws_bytes.argtypes = [ci, i64, i64, i64]
     lib.sngguf_gate_up_silu_ws_bytes.restype = i64
     lib.sngguf_gate_up_silu_ws.argtypes = [vp, i64, vp, vp, ci, i64, i64, vp, vp, i64, ci, vp]
@@ -418,6 +420,16 @@ def gate_up_silu_workspace_bytes(n: int, k: int) -> int:
 def gate_up_silu_ws_fits(quant_type: int, m: int, n: int, k: int) -> bool:
     """Whether ``gate_up_silu_ws_into`` takes ``m`` rows of this pair (shape rule of the library)."""
     return bool(load_library().sngguf_gate_up_silu_ws_fits(quant_type, m, n, k))
+
+
+PAIR_SEPARATE, PAIR_DECODE, PAIR_SPLIT, PAIR_DENSE = range(4)
+
+
+def gate_up_silu_ws_form(quant_type: int, m: int, n: int, k: int) -> int:
+    """The form in which ``gate_up_silu_ws_into`` is faster than two projections, silu and the product on ``m`` rows of this
+    pair: the decode kernels, K split over workgroups, or the dense launch where its tiles fill the chip; else
+    ``PAIR_SEPARATE``."""
+    return int(load_library().sngguf_gate_up_silu_ws_form(quant_type, m, n, k))
 
 
 def gate_up_silu_ws_bytes(quant_type: int, m: int, n: int, k: int) -> int:

@@ -69,6 +69,25 @@ def test_the_filled_dense_launch_stays_what_it_was():
     assert _route(rows, _linear(qt, n, k), _linear(qt, n, k, cls=Adapted))
 
 
+def test_the_route_follows_the_form():
+    """Everything the library has a faster form for, and nothing else; the dense launch where its tiles fill the chip."""
+    for qt in (ops.Q8_0, ops.Q4_K, ops.Q6_K, ops.BF16):
+        for n, k in ((12288, 4096), (9728, 2560), (6144, 2048), (4096, 4096), (512, 16384), (1536, 1024), (14336, 8192), (516, 1024)):
+            gate, up = _linear(qt, n, k), _linear(qt, n, k)
+            for rows in (1, 16, 65, 203, 511, 512, 768, 1000, 1024, 2048, 4095, 4096, 5000):
+                form = ops.gate_up_silu_ws_form(qt, rows, n, k)
+                assert _route(rows, gate, up) == (form != ops.PAIR_SEPARATE)
+                fits = ops.gate_up_silu_ws_fits(qt, rows, n, k)
+                filled = rows >= modality.GATED_TILE_MIN_ROWS and modality.gated_tile_fill(rows, n) >= modality.GATED_TILE_MIN_FILL
+                assert (form == ops.PAIR_DENSE) == (fits and filled)
+                few = -(-rows // 256) * -(-n // 256) <= 128 and 65 <= rows < 4096 and 4 * rows <= k
+                assert (form == ops.PAIR_SPLIT) == (fits and not filled and few and qt in (ops.Q8_0, ops.Q4_K))
+    # thousands of rows on a narrow pair with very long rows: no form but the dense launch, and that one badly filled
+    assert ops.gate_up_silu_ws_form(ops.Q8_0, 4096, 512, 16384) == ops.PAIR_SEPARATE
+    assert ops.gate_up_silu_ws_form(ops.Q6_K, 40, 512, 1024) == ops.PAIR_DECODE
+    assert ops.gate_up_silu_ws_form(ops.Q8_0, 40, 512, 1152) == ops.PAIR_SEPARATE   # K in whole 128, not 256, elements
+
+
 def test_workspace_is_what_the_form_needs():
     """2 M N bytes for the gate outputs up to 64 rows; whole fp32 copies of both outputs for a K split, within what the dense
     form would take; the interleaved weights for the dense form; never more than the size that is enough at any M."""
