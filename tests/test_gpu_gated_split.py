@@ -1,7 +1,8 @@
 """GPU: the SiLU-gated pair over a few hundred rows - both matrices in one launch with K split over workgroups, the
 reduction ending in the gated product - against the oracle (rel-L2 <= 1e-3: bf16 outputs, decoded weights the same bits)
 and against the two projections and the product as bf16 tensors.  Sizes around the 256 x 256 tile, one and several K
-slices, and a workspace too small for any (the dense gated launch)."""
+slices, and a workspace with room for exactly one copy of the sums and for none (the dense gated launch); the form of
+17 .. 64 rows, scratch sizes, and what hangs on the projections' calls."""
 import threading
 
 import pytest
@@ -30,6 +31,25 @@ def _run(dev, qt, m, n, k, num=1, x=None, gate=None, ws_bytes=None):
 def test_pair_with_split_k(dev, c_oracle, qt, num, m, n, k):
     print(f"case gated split qt={qt} num={num} {m}x{n}x{k}", flush=True)
     h, g, u = _run(dev, qt, m, n, k, num, ws_bytes=16 * 8 * m * n + ops.gate_up_silu_workspace_bytes(n, k))
+    assert go.rel_l2(h, c_oracle.silu_mul(g, u)) <= 1e-3
+
+
+@pytest.mark.parametrize("qt", [go.Q8_0, go.Q4_K])
+@pytest.mark.parametrize("num", [0, 1])
+@pytest.mark.parametrize("room", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(300, 1032, 256), (511, 520, 512), (65, 2056, 128)])
+def test_room_for_one_copy_and_for_none(dev, c_oracle, qt, num, room, m, n, k):
+    """Ragged rows and several column tiles per matrix.  One copy: K in one slice, fp32 sums and the gated reduction.  None: 16
+    bytes less, or what the dense launch needs if that is more, which must hold less than one copy then."""
+    if qt == go.Q4_K and k % 256:
+        k = 256
+    print(f"case pair room={room} qt={qt} num={num} {m}x{n}x{k}", flush=True)
+    copy, dense = 8 * m * n, ops.gate_up_silu_workspace_bytes(n, k)
+    if room == 0:
+        m += -(-max(dense - copy + 16, 0) // (8 * n))     # rows enough for a copy that the dense launch's workspace cannot hold
+        copy = 8 * m * n
+        assert dense <= copy - 16 and 65 <= m < 1024
+    h, g, u = _run(dev, qt, m, n, k, num, ws_bytes=copy if room else copy - 16)
     assert go.rel_l2(h, c_oracle.silu_mul(g, u)) <= 1e-3
 
 

@@ -36,7 +36,21 @@ def _fused(x, gate, up, qt, n, k, num=ops.NUM_UPSTREAM_FP16, extra=0):
                                       (go.Q5_1, 1000, 1000, 128), (go.Q4_K, 513, 72, 1024), (go.Q6_K, 17, 384, 256),
                                       (go.Q2_K, 700, 128, 512), (go.Q8_0, 2049, 640, 4096)])
 @pytest.mark.parametrize("num", [ops.NUM_GGML_FP32, ops.NUM_UPSTREAM_FP16])
+def test_gated_pair_against_two_projections(dev, c_oracle, qt, m, n, k, num):
+    """The form that the shape takes with the workspace that is enough for any (K split, decode kernels and dense launch)."""
+    _against_two_projections(dev, c_oracle, qt, m, n, k, num)
+
+
+@pytest.mark.parametrize("qt,m,n,k", [(go.Q4_K, 4097, 72, 256), (go.Q8_0, 4096, 136, 128), (go.Q6_K, 65, 384, 256), (go.Q6_K, 513, 72, 1024),
+                                      (go.Q3_K, 256, 130 * 8, 512), (go.Q4_0, 33, 520, 384)])
+@pytest.mark.parametrize("num", [ops.NUM_GGML_FP32, ops.NUM_UPSTREAM_FP16])
 def test_gated_pair_on_the_dense_tile_kernel(dev, c_oracle, qt, m, n, k, num):
+    """Types without a K split, 4096 rows and more, K that is not whole super-blocks: the dense launch."""
+    assert ops.gate_up_silu_ws_bytes(qt, m, n, k) == ops.gate_up_silu_workspace_bytes(n, k)
+    _against_two_projections(dev, c_oracle, qt, m, n, k, num)
+
+
+def _against_two_projections(dev, c_oracle, qt, m, n, k, num):
     print(f"case gated tiles qt={qt} {m}x{n}x{k} num={num}", flush=True)
     gate, up, x = _pair(dev, qt, m, n, k, seed=11 * n + k)
     h = _fused(x, gate, up, qt, n, k, num)
