@@ -264,10 +264,10 @@ int sngguf_gate_up_silu(const void* x, int64_t M, const void* q_gate, const void
  *  gate projection on the decode kernel, then the up projection with silu and the product in its epilogue; and Q8_0 /
  *  Q4_K from 65 rows on with at most 128 tiles of 256 x 256 (below 512 rows, or where the dense launch's tiles fill less
  *  than 0.7 of their rounds) both matrices in one launch with K split over workgroups, fp32 partial sums in the
- *  workspace, and a reduction that ends in the gated product.  The dense form
- *  pays from about 512 rows on when the launch's ceil(M / 256) x ceil(N / 128) tiles come close to whole rounds of
- *  the 256 compute units (there is no K split; 12288 x 4096 at
- *  4096 rows: 628 us against 695 us for two sngguf_linear_ws launches and the product, at 2048 rows 354 against 451).
+ *  workspace, and a reduction that ends in the gated product.  The dense form pays from about 512 rows on when the
+ *  launch's ceil(M / 256) x ceil(N / 128) tiles come close to whole rounds of the 256 compute units (there is no K split;
+ *  12288 x 4096 at 4096 rows: 628 us against 695 us for two sngguf_linear_ws launches and the product, at 2048 rows 354
+ *  against 451).
  */
 int64_t sngguf_gate_up_silu_workspace_bytes(int64_t N, int64_t K);
 int sngguf_gate_up_silu_ws_fits(int qtype, int64_t M, int64_t N, int64_t K);

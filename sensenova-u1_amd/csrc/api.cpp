@@ -148,8 +148,8 @@ namespace {
 
 // Between the decode kernels' 64 rows and a few hundred, a matrix with few 256 x 256 output tiles keeps only a few
 // compute units busy in the tile kernels, each for K / 64 steps of about 1.6 us, while the decode kernel streams the
-// whole matrix in 10 us + N K / 1.25e12 s per 64 rows (measured: 12288 x 4096 50 us, 4096 x 4096 20 us, 1024 x 4096 19 us) and less for a
-// short last chunk.  Row chunks through the decode kernel win where the sum of those stays below the tile kernel's time:
+// whole matrix in 10 us + N K / 1.25e12 s per 64 rows (64 rows, Q8_0 / Q4_K / Q6_K: 12288 x 4096 44 / 42 / 45 us, which the
+// line puts at 50, 4096 x 4096 19 / 18 / 19, 1024 x 4096 19 / 18 / 19, 4096 x 12288 49 / 47 / 50) and less for a short last chunk.  Row chunks through the decode kernel win where the sum of those stays below the tile kernel's time:
 // 4096 x 12288 at 128 rows 102 against 292 us, 4096 x 4096 41 against 102 us; 12288 x 4096 only up to 65 rows or so.
 // (Chunks start at multiples of 64 rows, so x, y and the residual keep their 16-byte alignment.)
 bool row_chunks_win(int64_t M, int64_t N, int64_t K, int qtype) {
@@ -245,8 +245,11 @@ int64_t pick_k_slices(int64_t M, int64_t N, int64_t tiles, int64_t ksteps, int64
 }
 
 // The same for a gate / up pair in one launch (`tiles` of both): any number of rounds, since a pair's tiles come closer to
-// whole ones.  A round takes its K steps and about 5 us for the first loads and the partial sums' stores.  0 if there is
-// no room for one fp32 copy of each output.
+// whole ones.  A round takes its K steps of 1.9 us and 5 us for the first loads and the partial sums' stores, which is within
+// a tenth of what was measured wherever two and more slices run (Q8_0 / Q4_K, model in brackets, us): 12288 x 4096 at 203 rows
+// one slice 137 / 125 (135), two 88 / 81 (82), at 509 rows one 151 / 142 (147); 9728 x 2560 at 203 rows one 81 / 84 (87), two
+// 66 / 57 (56), three 60 / 52 (51); 4096 x 4096 at 509 rows two 75 / 78 (79), three 63 / 66 (67), four 63 / 65 (62).  0 if there
+// is no room for one fp32 copy of each output.
 int64_t pick_pair_slices(int64_t M, int64_t N, int64_t tiles, int64_t ksteps, int64_t room) {
     int64_t smax = room < ksteps / 2 ? room : ksteps / 2;   // at least two K steps per workgroup
     if (smax > 64) smax = 64;

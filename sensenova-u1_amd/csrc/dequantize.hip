@@ -1,7 +1,8 @@
 // Standalone block dequantize: packed GGUF rows -> fp32 / fp16 / bf16 rows.
-// One thread decodes eight consecutive elements (Q4_K and Q6_K to 16-bit outputs: see HalfChain), so a wavefront reads one contiguous run of
+// One thread decodes eight consecutive elements, so a wavefront reads one contiguous run of
 // packed bytes and writes one contiguous run of 512 outputs; the kernel is bound by the
-// output stream (4 bytes out per ~1 byte in for fp32).
+// output stream (4 bytes out per ~1 byte in for fp32).  Q4_K and Q6_K to 16-bit outputs in the
+// fp16 rounding chain go by whole quant bytes instead (HalfChain).
 #include "sngguf_common.hpp"
 
 namespace sngguf {
@@ -33,8 +34,8 @@ __device__ __forceinline__ void store8(void* __restrict__ out, int64_t idx, cons
 // 4 x 8 for Q6_K (both nibbles of two byte runs that share their upper bits), each run of eight one 16-byte store.  Every
 // quant byte is then requested once and a super-block's header once per 16 or 32 outputs, where one thread per eight
 // consecutive elements asked for every byte twice (upper bits: four times) and for the header with each.  Four lanes fill
-// 64 consecutive output bytes per store.  Bound by the output stream: 12288 x 4096 Q4_K to fp16 32.3 -> 26.1 us, 4.9 TB/s of
-// the 5.4 that a large copy reaches.
+// 64 consecutive output bytes per store.  Bound by the output stream: three 12288 x 4096 Q4_K matrices to fp16 97.5 -> 78.8 us,
+// 4.9 TB/s of the 5.4 that a large copy reaches; Q6_K 1.10 times as fast at that size, level below 1024 rows.
 template <int QT>
 struct HalfChain {
     static_assert(QT == SNGGUF_TYPE_Q4_K || QT == SNGGUF_TYPE_Q6_K, "packed decode exists for Q4_K and Q6_K");

@@ -280,8 +280,9 @@ def _whole_call(dev: torch.device):
 def pooled_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
     """A device scratch tensor of at least ``nbytes`` bytes for the workspace entry points, kept per (device, stream)
     and grown on demand, so that a forward pass over many modules allocates once.  Calls on one stream are ordered (whole
-    calls, also of several host threads: ``_whole_call``), and nothing in a workspace outlives the call that filled it.  While a HIP graph is being captured a fresh tensor is
-    handed out instead (it then belongs to the graph's own memory pool)."""
+    calls, also of several host threads: ``_whole_call``), and nothing in a workspace outlives the call that filled it.
+    While a HIP graph is being captured a fresh tensor is handed out instead (it then belongs to the graph's own memory
+    pool)."""
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
     key = (dev.index if dev.index is not None else torch.cuda.current_device(), _stream(dev))
