@@ -269,8 +269,8 @@ _enqueue_locks: dict = {}
 
 
 def _whole_call(dev: torch.device):
-    """The lock under which a call with a caller's workspace is enqueued on the current stream of ``dev``.  Host threads that
-    share a stream get one pooled workspace, a call fills it with one launch and reads it with the next, and the foreign call
+    """The lock under which a call with a caller's workspace (or the library's static one) is enqueued on the current stream
+    of ``dev``.  Host threads that share a stream get one pooled workspace, a call fills it with one launch and reads it with the next, and the foreign call
     lets go of the interpreter lock: without this another thread's launches could come between them."""
     key = (dev.index, _stream(dev))
     lock = _enqueue_locks.get(key)
@@ -386,7 +386,7 @@ def linear_static_into(x2d: torch.Tensor, packed: torch.Tensor, quant_type: int,
     allocates nothing.  ``M * N`` beyond ``linear_static_max_outputs()`` is refused."""
     dev = x2d.device
     n, k = y2d.shape[1], x2d.shape[1]
-    with _on(dev):
+    with _on(dev), _whole_call(dev):
         rc = load_library().sngguf_linear_static(_ptr(x2d), x2d.shape[0], _ptr(packed), quant_type, n, k, _ptr(bias),
                                                  _ptr(y2d), numerics, _stream(dev))
     _check(rc, "sngguf_linear_static")

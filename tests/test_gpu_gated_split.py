@@ -201,6 +201,33 @@ def test_forty_rows_leave_no_weight_sized_workspace(dev):
     assert sum(ws.numel() for ws in ops._workspaces.values()) <= 2 * m * n
 
 
+@pytest.mark.parametrize("qt_down", [go.Q8_0, go.Q6_K])
+@pytest.mark.parametrize("m", [40, 203, 600])
+def test_captured_passes_replay_the_eager_ones(dev, qt_down, m):
+    """Scratch of the call's own and workspaces handed out during a capture: replays on new rows, eager passes between them."""
+    print(f"case captured gated pair m={m} down={qt_down}", flush=True)
+    n, k = 1024, 2560
+    mods = []
+    for j, (o, i, qt) in enumerate(((n, k, go.Q8_0), (n, k, go.Q8_0), (k, n, qt_down))):
+        lin = GGUFLinear(i, o, bias=False, compute_dtype=torch.bfloat16, device="meta")
+        lin.weight = GGUFParameter(synthetic.make_packed(qt, o, i, seed=60 + j, device=dev), quant_type=qt)
+        mods.append(lin)
+    x = synthetic.make_activations(m, k, seed=m, device=dev)
+    gated_mlp(x, *mods)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = gated_mlp(x, *mods)
+    for seed in (1, 2, 3):
+        rows = synthetic.make_activations(m, k, seed=seed, device=dev)
+        want = gated_mlp(rows, *mods)
+        torch.cuda.synchronize()
+        x.copy_(rows)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+
+
 @pytest.mark.parametrize("m", [17, 40, 64, 203])
 def test_threads_on_one_stream(dev, m):
     """Four host threads, each with rows of its own, through one MLP on the default stream: scratch of the call (up to 64

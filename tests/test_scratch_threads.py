@@ -61,7 +61,7 @@ def test_a_short_prompt_s_gate_outputs_are_the_call_s_own(host_scratch, monkeypa
     _in_threads(4, one)
 
 
-@pytest.mark.parametrize("entry", ["linear_ws", "gate_up_silu_ws", "grouped_linear_ws"])
+@pytest.mark.parametrize("entry", ["linear_ws", "linear_static", "gate_up_silu_ws", "grouped_linear_ws"])
 def test_calls_that_share_a_pooled_workspace_do_not_interleave(host_scratch, monkeypatch, entry):
     """The pool hands the threads of one stream the same memory; one call's launches are then enqueued as one run."""
     import contextlib
@@ -84,6 +84,8 @@ def test_calls_that_share_a_pooled_workspace_do_not_interleave(host_scratch, mon
             ws = ops.pooled_workspace(x.device, 4096 * (i + 1))
             if entry == "linear_ws":
                 ops.linear_ws_into(x, w, ops.Q8_0, None, y, ws, 1)
+            elif entry == "linear_static":
+                ops.linear_static_into(x, w, ops.Q8_0, None, y, 1)
             elif entry == "gate_up_silu_ws":
                 ops.gate_up_silu_ws_into(x, w, w, ops.Q8_0, y, ws, 1)
             else:
