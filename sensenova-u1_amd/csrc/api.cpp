@@ -231,14 +231,20 @@ namespace {
 int64_t pick_k_slices(int64_t M, int64_t N, int64_t tiles, int64_t ksteps, int64_t room, bool fused_decode) {
     int64_t smax = 256 / tiles;
     if (smax > room) smax = room;
-    if (smax > ksteps / 2) smax = ksteps / 2;   // at least two K steps per workgroup
+    // at least four K steps per workgroup: with fewer its first loads are not paid back (777 x 1024 at 512 rows, two / four steps:
+    // Q8_0 43.0 / 39.5 us, 4096 x 1024 at 100 rows, BF16 23.3 / 20.4); two where K has no more
+    if (smax > ksteps / 4) smax = ksteps >= 8 ? ksteps / 4 : ksteps / 2;
     if (smax > 64) smax = 64;
     if (smax < 2) return 1;
     const double t_step = fused_decode ? 1.9 : 1.65, t_slice = 8.0 * (double)M * (double)N / 5e6;   // us
+    // copies that lie a power of two apart, 48 MiB of them and more: about 6 us extra with the decode in the loop (512 x 2048 <- 6144,
+    // Q8_0: 11 / 12 slices 41.5 / 48.2 us, 1024 x 1024 <- 12288 11 / 12 / 16 55.4 / 60.3 / 66.7; 400 rows, 12 .. 32 slices: none)
+    const int64_t copy = 4 * M * N;
+    const bool collide = fused_decode && (copy & (copy - 1)) == 0;
     int64_t best = 2;
     double best_t = 1e30;
     for (int64_t sl = 2; sl <= smax; sl++) {
-        const double t = (double)((ksteps + sl - 1) / sl) * t_step + (double)sl * t_slice;
+        const double t = (double)((ksteps + sl - 1) / sl) * t_step + (double)sl * t_slice + (collide && sl * copy >= ((int64_t)48 << 20) ? 6.0 : 0.0);
         if (t < best_t) { best_t = t; best = sl; }
     }
     return best;
