@@ -185,9 +185,9 @@ def gated_mlp(x: torch.Tensor, gate_proj: GGUFLinear, up_proj: GGUFLinear, down_
     ``RMSNorm(x)`` (``post_attention_layernorm``, modeling_qwen3.py:938); where ``ops.rmsnorm_fits`` allows, the norm
     is part of that same launch.  With ``residual`` the result is ``residual + mlp`` (modeling_qwen3.py:940-941), added
     in the down projection's epilogue.  One or two rows of the 8B model's shape in Q8_0, or in Q4_K with a Q6_K or Q4_K
-    down projection, run as ONE launch (``sngguf_mlp_decode``; see ``ONE_LAUNCH_MLP``): same values as the separate launches up to the order in which the
-    down projection's partial sums are added.  Beyond 16 rows, where ``_gated_tile_route`` says so, gate / up / SiLU run as
-    ``sngguf_gate_up_silu_ws``."""
+    down projection, run as ONE launch (``sngguf_mlp_decode``; see ``ONE_LAUNCH_MLP``): same values as the separate
+    launches up to the order in which the down projection's partial sums are added.  Beyond 16 rows, where
+    ``_gated_tile_route`` says so, gate / up / SiLU run as ``sngguf_gate_up_silu_ws``."""
     rows = x.numel() // x.shape[-1] if x.numel() else 0
     one = _one_launch_mlp(x, rows, gate_proj, up_proj, down_proj, norm_weight, residual)
     if one is not None:

@@ -21,6 +21,10 @@ def test_what_a_shape_can_use():
             else:
                 assert nbytes == (0 if qt == ops.BF16 else 2 * n * k)
         assert ops.linear_ws_bytes(qt, 64, 4096, 4096) == 0 and ops.linear_ws_bytes(qt, 0, 4096, 4096) == 0
+    # four K steps of 64 a slice, two where K has fewer than eight; fewer copies where they lie a power of two apart
+    for qt in (ops.Q8_0, ops.BF16):
+        assert ops.linear_ws_bytes(qt, 100, 512, 1024) == 4 * 4 * 100 * 512 and ops.linear_ws_bytes(qt, 100, 512, 256) == 2 * 4 * 100 * 512
+    assert ops.linear_ws_bytes(ops.Q8_0, 512, 2048, 6144) < 48 << 20 and ops.linear_ws_bytes(ops.Q8_0, 512, 2048, 128) == 2 * 2048 * 128
     assert ops.linear_ws_bytes(ops.Q8_0, 300, 512, 96) == 0 and ops.linear_ws_bytes(16, 300, 512, 256) == 0
     assert ops.linear_ws_bytes(ops.Q8_0, 4096, 1024, 4096) == 2 * 1024 * 4096 + 4 * 4 * 4096 * 1024   # weight pass from 4096 rows on
 
