@@ -132,6 +132,18 @@ int sngguf_linear_residual(const void* x, int64_t M, const void* q, int qtype, i
                            const void* bias, const void* residual, void* y, int numerics, void* stream);
 
 /*
+ * sngguf_linear (residual NULL) or sngguf_linear_residual with device scratch for the fp32 partial sums of a K split at 17 .. 64
+ * rows (and in the 64-row chunks that a few hundred rows of a narrow matrix run as): K is cut over workgroups where the columns
+ * alone would leave much of the device idle.  scratch (16-byte aligned) of
+ * sngguf_linear_scratch_bytes(qtype, M, N, K) bytes gives a shape its fastest form, more changes nothing; 0 where none is used
+ * (every other row count among them), and without scratch the call is sngguf_linear / sngguf_linear_residual.  Nothing in it
+ * outlives the call, and no other call may use it between this call's launches (threads that share a stream take one each).
+ */
+int64_t sngguf_linear_scratch_bytes(int qtype, int64_t M, int64_t N, int64_t K);
+int sngguf_linear_scratch(const void* x, int64_t M, const void* q, int qtype, int64_t N, int64_t K, const void* bias,
+                          const void* residual, void* y, void* scratch, int64_t scratch_bytes, int numerics, void* stream);
+
+/*
  * sngguf_linear with a caller-provided workspace.  No counterpart in the reference, whose forward_native
  * materialises the dequantized weight on every call (diffusers GGUFLinear.forward_native, reached from
  * src/sensenova_u1/utils/gguf_loader.py:64-81): this is that route for callers of the bare ABI.  With

@@ -15,7 +15,8 @@ from concurrent.futures import ThreadPoolExecutor
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libsngguf.so")
-SOURCES = ["api.cpp", "gguf_reader.cpp", "dequantize.hip", "plain_bf16.hip", "rmsnorm.hip", "gemv.hip", "gemv_q8_mfma.hip", "gemv_kq_mfma.hip", "gemv_q8_tiled.hip", "gemm.hip", "gemm_tiles.hip", "gemm_dense4.hip", "static_scratch.hip", "stream_probe.hip"]
+SOURCES = ["api.cpp", "gguf_reader.cpp", "dequantize.hip", "plain_bf16.hip", "rmsnorm.hip", "gemv.hip", "gemv_q8_mfma.hip", "gemv_kq_mfma.hip", "gemv_q8_tiled.hip", "gemm.hip", "gemm_tiles.hip", "gemm_dense4.hip", "gemm_mid_plan.hip", "gemm_mid.hip", "static_scratch.hip", "stream_probe.hip"]
+HEADERS = ["sngguf_common.hpp", "gemm_args.hpp", "gemm_mid.hpp", "kq_decode.hpp"]
 
 # packed-fp32 VALU forms are switched off for every device compile of this library
 HIP_FLAGS = [
@@ -38,7 +39,9 @@ def _hipcc() -> str:
 # per-source additions.  gemv_kq_mfma.hip widens fp16 to fp32 with matrix instructions whose
 # results the vector ALU consumes at once: they must land in ordinary VGPRs, not in accumulation
 # registers that need one v_accvgpr_read per value.
-SOURCE_FLAGS = {"gemv_kq_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+SOURCE_FLAGS = {"gemv_kq_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "gemm_mid.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# sources compiled once per variant: gemm_mid.hip holds the kernels of one block format (ggml type ids)
+SOURCE_VARIANTS = {"gemm_mid.hip": [(f"_t{t}", [f"-DSNGGUF_MID_TYPE={t}"]) for t in (8, 14, 13, 12, 11, 10, 7, 6, 3, 2)]}
 
 
 def _compile(src: str, obj: str, extra: list[str]) -> None:
@@ -52,17 +55,24 @@ def _compile(src: str, obj: str, extra: list[str]) -> None:
         sys.stderr.write(warn + "\n")
 
 
-def build_library(force: bool = True, extra_flags: list[str] | None = None, jobs: int = 4) -> str:
+def _units() -> list[tuple[str, str, list[str]]]:
+    """(source, object name, flags of its own) of every compile."""
+    return [(src, os.path.splitext(src)[0] + suffix + ".o", flags) for src in SOURCES
+            for suffix, flags in SOURCE_VARIANTS.get(src, [("", [])])]
+
+
+def build_library(force: bool = True, extra_flags: list[str] | None = None, jobs: int | None = None) -> str:
     """Compile and link libsngguf.so; returns its path.  ``force=False`` skips an up-to-date library."""
-    srcs = [os.path.join(CSRC, s) for s in SOURCES] + [os.path.join(CSRC, "sngguf_common.hpp"), os.path.join(CSRC, "gemm_args.hpp"),
-                                                        os.path.join(PKG_DIR, "..", "include", "sngguf.h")]
+    srcs = [os.path.join(CSRC, s) for s in SOURCES] + [os.path.join(CSRC, h) for h in HEADERS] + [os.path.join(PKG_DIR, "..", "include", "sngguf.h")]
     if not force and os.path.exists(LIB_PATH) and all(os.path.getmtime(LIB_PATH) >= os.path.getmtime(s) for s in srcs):
         return LIB_PATH
     objdir = os.path.join(PKG_DIR, "build")
     os.makedirs(objdir, exist_ok=True)
-    objs = [os.path.join(objdir, os.path.splitext(s)[0] + ".o") for s in SOURCES]
-    with ThreadPoolExecutor(max_workers=jobs) as pool:
-        list(pool.map(lambda so: _compile(so[0], so[1], extra_flags or []), zip(SOURCES, objs)))
+    # (the variants of one source are the longest compiles: first)
+    units = sorted(_units(), key=lambda u: not u[2])
+    with ThreadPoolExecutor(max_workers=jobs or min(8, os.cpu_count() or 1)) as pool:
+        list(pool.map(lambda u: _compile(u[0], os.path.join(objdir, u[1]), [*u[2], *(extra_flags or [])]), units))
+    objs = [os.path.join(objdir, obj) for _, obj, _ in _units()]
     tmp = LIB_PATH + ".tmp"
     res = subprocess.run([_hipcc(), "-shared", "-fPIC", "--offload-arch=gfx950", "-pthread", "-o", tmp, *objs],
                          capture_output=True, text=True)

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "../../include/sngguf.h"
+#include "gemm_mid.hpp"
 
 namespace sngguf {
 int launch_dequantize(const void* q, int qtype, int64_t rows, int64_t cols, void* out, int out_dtype, int numerics,
@@ -15,7 +16,7 @@ int launch_gemv_q8_mfma(const void* x, int64_t M, const void* qa, const void* qb
                         float eps, uint64_t* amax = nullptr);
 int launch_gemv_kq_mfma(const void* x, int64_t M, const void* qa, const void* qb, int qtype, int64_t N, int64_t K,
                         const void* bias, const void* residual, void* y, int numerics, bool gated, hipStream_t stream,
-                        const void* gamma, float eps, uint64_t* amax = nullptr, const void* gate = nullptr);
+                        const void* gamma, float eps, uint64_t* amax = nullptr);
 int64_t gemv_argmax_slots(int qtype, int64_t M, int64_t N);
 int launch_argmax_reduce(const uint64_t* keys, int64_t M, int64_t slots, int64_t* out_index, hipStream_t stream);
 int launch_dequantize_bf16(const void* q, int64_t rows, int64_t cols, void* out, int out_dtype, hipStream_t stream);
@@ -146,6 +147,18 @@ int sngguf_dequantize(const void* q, int qtype, int64_t rows, int64_t cols, void
 
 namespace {
 
+// us of the decode kernel for every format (gemv_kq_mfma.hip) on 17 .. 64 rows: rounds of workgroups, each as many super-blocks
+// one after the other as a wavefront gets of K.  Fitted with the plans of gemm_mid_plan.hip (nine shapes, 20 / 40 / 60 rows, three
+// types); choosing by the two is 0.7 % slower than the faster of the two in the mean.
+double decode_kernel_us(int64_t M, int64_t N, int64_t K) {
+    const int64_t mt = (M + 15) / 16, rg = N > 4096 ? 2 : 1, groups = (N + 16 * rg - 1) / (16 * rg), nsb = K / 256, counted = (N + 15) / 16;
+    int64_t w = (256 * 12 + counted - 1) / counted;
+    const bool four = groups > 256 || (groups == 256 && nsb >= 32 && M >= 22);
+    if (w > (four ? 4 : 8)) w = four ? 4 : 8;
+    if (w > nsb) w = nsb;
+    return 6.1 + (double)((groups + 255) / 256) * (double)((nsb + w - 1) / w) * (1.33 + 0.63 * (double)(mt * rg));
+}
+
 // Between the decode kernels' 64 rows and a few hundred, a matrix with few 256 x 256 output tiles keeps only a few
 // compute units busy in the tile kernels, each for K / 64 steps of about 1.6 us, while the decode kernel streams the
 // whole matrix in 10 us + N K / 1.25e12 s per 64 rows (64 rows, Q8_0 / Q4_K / Q6_K: 12288 x 4096 44 / 42 / 45 us, which the
@@ -165,8 +178,31 @@ bool row_chunks_win(int64_t M, int64_t N, int64_t K, int qtype) {
     return (double)full * t64 + last < 0.9 * t_tile;
 }
 
+constexpr int64_t kSplitBytes = (int64_t)64 << 20;   // the most fp32 partial sums a K split of a projection writes
+
+// 17 .. 64 rows: the mid-size kernel, with its K split as far as the scratch goes, or the decode kernel; 0 bytes where that one is
+// faster or no split pays.
+sngguf::MidPlan rows_plan(int qtype, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes) {
+    sngguf::MidPlan plan{-1, 0, 0, 0, 1, 1e30};
+    if (M > 64 || !sngguf::mid_fits(qtype, M, N, K)) return plan;
+    plan = sngguf::mid_plan(M, N, K, false, (scratch_bytes < kSplitBytes ? scratch_bytes : kSplitBytes) / (4 * M * N));
+    if (plan.us > decode_kernel_us(M, N, K)) plan.form = -1;
+    return plan;
+}
+int64_t rows_scratch_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
+    const sngguf::MidPlan plan = rows_plan(qtype, M, N, K, kSplitBytes);
+    return plan.form >= 0 && plan.slices > 1 ? plan.slices * 4 * M * N : 0;
+}
+int rows_impl(const void* x, int64_t M, const void* q, int qtype, int64_t N, int64_t K, const void* bias, const void* residual, void* y,
+              void* scratch, int64_t scratch_bytes, int numerics, hipStream_t s) {
+    const sngguf::MidPlan plan = rows_plan(qtype, M, N, K, scratch ? scratch_bytes : 0);
+    if (plan.form >= 0)
+        return sngguf::launch_mid(plan, x, M, q, nullptr, qtype, N, K, bias, residual, y, static_cast<float*>(scratch), numerics, s);
+    return sngguf::launch_gemv(x, M, q, nullptr, qtype, N, K, bias, residual, y, numerics, false, s);
+}
+
 int linear_impl(const void* x, int64_t M, const void* q, int qtype, int64_t N, int64_t K, const void* bias,
-                const void* residual, void* y, int numerics, void* stream) {
+                const void* residual, void* y, int numerics, void* stream, void* scratch = nullptr, int64_t scratch_bytes = 0) {
     const int rc = check_matmul(x, M, q, qtype, N, K, y, numerics);
     if (rc != SNGGUF_OK || M == 0 || N == 0) return rc;
     if (residual && !aligned(residual, 16)) return SNGGUF_E_ALIGN;
@@ -191,7 +227,7 @@ int linear_impl(const void* x, int64_t M, const void* q, int qtype, int64_t N, i
     // decode-shaped work (weights streamed and decoded once): up to 16 rows always, up to 64 rows when the
     // rows are whole 256-element runs
     if (M <= 16 || (M <= 64 && K % 256 == 0))
-        return sngguf::launch_gemv(x, M, q, nullptr, qtype, N, K, bias, residual, y, numerics, false, s);
+        return rows_impl(x, M, q, qtype, N, K, bias, residual, y, scratch, scratch_bytes, numerics, s);
     if (row_chunks_win(M, N, K, qtype)) {
         // a few hundred rows on a matrix with few output tiles: the decode kernel on 64 rows at a time
         const char* xp = static_cast<const char*>(x);
@@ -199,8 +235,8 @@ int linear_impl(const void* x, int64_t M, const void* q, int qtype, int64_t N, i
         char* yp = static_cast<char*>(y);
         for (int64_t r0 = 0; r0 < M; r0 += 64) {
             const int64_t rows = M - r0 < 64 ? M - r0 : 64;
-            const int rc = sngguf::launch_gemv(xp + 2 * r0 * K, rows, q, nullptr, qtype, N, K, bias,
-                                               rp ? rp + 2 * r0 * N : nullptr, yp + 2 * r0 * N, numerics, false, s);
+            const int rc = rows_impl(xp + 2 * r0 * K, rows, q, qtype, N, K, bias, rp ? rp + 2 * r0 * N : nullptr, yp + 2 * r0 * N,
+                                     scratch, scratch_bytes, numerics, s);
             if (rc != SNGGUF_OK) return rc;
         }
         return SNGGUF_OK;
@@ -219,6 +255,20 @@ int sngguf_linear_residual(const void* x, int64_t M, const void* q, int qtype, i
                            const void* residual, void* y, int numerics, void* stream) {
     if (!residual && M > 0 && N > 0) return SNGGUF_E_NULLPTR;
     return linear_impl(x, M, q, qtype, N, K, bias, residual, y, numerics, stream);
+}
+
+int64_t sngguf_linear_scratch_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
+    if (M <= 16 || M >= kMaxDim || N <= 0 || N >= kMaxDim || K <= 0 || K >= kMaxDim || !sngguf::mid_fits(qtype, M, N, K)) return 0;
+    if (M <= 64) return rows_scratch_bytes(qtype, M, N, K);
+    if (!row_chunks_win(M, N, K, qtype)) return 0;
+    const int64_t whole = rows_scratch_bytes(qtype, 64, N, K), last = rows_scratch_bytes(qtype, M % 64, N, K);
+    return whole > last ? whole : last;
+}
+
+int sngguf_linear_scratch(const void* x, int64_t M, const void* q, int qtype, int64_t N, int64_t K, const void* bias,
+                          const void* residual, void* y, void* scratch, int64_t scratch_bytes, int numerics, void* stream) {
+    if (scratch && !aligned(scratch, 16)) return SNGGUF_E_ALIGN;
+    return linear_impl(x, M, q, qtype, N, K, bias, residual, y, numerics, stream, scratch, scratch_bytes);
 }
 
 namespace {
@@ -308,12 +358,39 @@ LinearSplit linear_split(int qtype, int64_t M, int64_t N, int64_t K, int64_t wor
 }
 }  // namespace
 
+namespace {
+// us of that route: workgroups of 256 x 256 tiles, 1.9 us a K step with the decode in the loop and 1.2 without, the weight pass,
+// the partial sums.  Fitted (rms 6.5 %) to twelve shapes at 65 .. 4096 rows, three types; choosing between it and the plans of
+// gemm_mid_plan.hip by the two models is 1 % slower than the fastest in the mean.
+double workspace_route_us(const LinearSplit& f, int qtype, int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), wgs = tiles * f.slices;
+    const bool pass = !(f.tile_type && f.slices >= 2);
+    const double ksteps = (double)((K / 64 + f.slices - 1) / f.slices);
+    double us = (double)((wgs + 255) / 256) * (6.3 + ksteps * (pass ? 1.21 : 1.89));
+    if (pass) us += 3.2 + (double)N * (double)K * ((double)sngguf_type_size(qtype) / (double)sngguf_block_size(qtype) + 2.0) / 4.7e6;
+    if (f.slices >= 2) us += 7.1 + (double)(f.slices * M * N) * 8.0 / 7.8e6;
+    return us;
+}
+
+// The plan for a projection from 65 rows on with `workspace_bytes` for partial sums; form -1 where the route above is faster.
+// From 2048 rows on one weight pass pays for eight row tiles and more (this route / plans, Q8_0, us: 4096 x 4096 1280 rows 71 / 54,
+// 2048 92 / 84, 3000 93 / 105; 12288 x 4096 1280 rows 141 / 124, 2048 196 / 212, 3000 280 / 317).
+sngguf::MidPlan workspace_plan(const LinearSplit& f, int qtype, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
+    sngguf::MidPlan none{-1, 0, 0, 0, 1, 1e30};
+    if (M >= 2048 || !sngguf::mid_fits(qtype, M, N, K)) return none;
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), most = tiles <= 128 ? kSplitBytes : 2 * N * K;
+    const sngguf::MidPlan plan = sngguf::mid_plan(M, N, K, false, (workspace_bytes < most ? workspace_bytes : most) / (4 * M * N));
+    return plan.us <= workspace_route_us(f, qtype, M, N, K) ? plan : none;
+}
+}  // namespace
+
 int64_t sngguf_linear_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
     if (!known_type(qtype) || M <= 0 || N <= 0 || K <= 0 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim || K % sngguf_block_size(qtype) != 0
         || !dense_route_fits(M, N, K))
         return 0;
     const LinearSplit f = linear_split(qtype, M, N, K, INT64_MAX);
-    if (f.slices >= 2) return f.dense_bytes + f.slices * 4 * M * N;
+    const sngguf::MidPlan plan = workspace_plan(f, qtype, M, N, K, INT64_MAX);
+    if (f.slices >= 2) return f.dense_bytes + (plan.form >= 0 && plan.slices > f.slices ? plan.slices : f.slices) * 4 * M * N;
     return qtype == SNGGUF_TYPE_BF16 || row_chunks_win(M, N, K, qtype) ? 0 : 2 * N * K;
 }
 
@@ -329,6 +406,9 @@ int linear_ws_impl(const void* x, int64_t M, const void* q, int qtype, int64_t N
     const bool fits = workspace && dense_route_fits(M, N, K);
     if (!fits) return linear_impl(x, M, q, qtype, N, K, bias, nullptr, y, numerics, stream);
     const LinearSplit f = linear_split(qtype, M, N, K, workspace_bytes);
+    const sngguf::MidPlan plan = workspace_plan(f, qtype, M, N, K, workspace_bytes);
+    if (plan.form >= 0)
+        return sngguf::launch_mid(plan, x, M, q, nullptr, qtype, N, K, bias, nullptr, y, static_cast<float*>(workspace), numerics, s);
     if (f.slices >= 2) {
         float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + f.dense_bytes);
         if (f.tile_type)
@@ -392,8 +472,9 @@ int sngguf_gate_up_silu_ws_fits(int qtype, int64_t M, int64_t N, int64_t K) {
 namespace {
 // How a pair beyond 16 rows runs; the shape is one that sngguf_gate_up_silu_ws_fits takes.
 enum PairForm {
-    // 17 .. 64 rows of whole 256-element runs belong to the decode kernels: the gate projection into the workspace, then the
-    // up projection with silu and the product in its epilogue (a weight pass and the dense launch take three times as long)
+    // 17 .. 64 rows of whole 256-element runs: both matrices in one launch of the mid-size kernel, which ends in the gated
+    // product and needs no workspace (two launches of the decode kernel, the gate outputs in the workspace, took 1.2 - 2.3 times
+    // as long: 12288 x 4096, us: Q8_0 20 / 40 / 60 rows 50 / 66 / 90 against 38 / 39 / 40)
     kPairDecode,
     // Few output tiles: the gated launch has no K split and would leave much of the chip idle (below 512 rows, or tiles that
     // fill less than 0.7 of their rounds), so both matrices run as one launch with K split over workgroups, and the
@@ -423,6 +504,18 @@ PairForm pair_form(int qtype, int64_t M, int64_t N, int64_t K) {
 int64_t pair_slices(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
     return pick_pair_slices(M, N, 2 * tiles, K / 64, workspace_bytes / (8 * M * N));
+}
+
+// us of the split form with `slices` K slices, or of the dense form (0 slices): two weight passes, then rounds of 256 x 256 tiles
+// that take 3 us and 1.45 a K step.
+double pair_us(int qtype, int64_t M, int64_t N, int64_t K, int64_t slices) {
+    if (slices >= 1) {
+        const int64_t wgs = 2 * ((M + 255) / 256) * ((N + 255) / 256) * slices;
+        return 10.0 + (double)((wgs + 255) / 256) * ((double)((K / 64 + slices - 1) / slices) * 1.9 + 5.0) + (double)(slices * M * N) * 16.0 / 5e6;
+    }
+    const double pass = 3.2 + (double)N * (double)K * ((double)sngguf_type_size(qtype) / (double)sngguf_block_size(qtype) + 2.0) / 4.7e6;
+    const int64_t tiles = ((M + 255) / 256) * ((N + 127) / 128);
+    return 2.0 * pass + 6.0 + (double)((tiles + 255) / 256) * (3.0 + (double)(K / 64) * 1.45);
 }
 }  // namespace
 
@@ -458,20 +551,21 @@ int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const v
     if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return qtype == SNGGUF_TYPE_BF16 ? SNGGUF_E_BADTYPE : SNGGUF_E_BADSHAPE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const PairForm form = pair_form(qtype, M, N, K);
-    if (form == kPairDecode) {
-        if (workspace_bytes < 2 * M * N) return SNGGUF_E_BADSHAPE;
-        const int rg = sngguf::launch_gemv(x, M, q_gate, nullptr, qtype, N, K, nullptr, nullptr, workspace, numerics, false, s);
-        if (rg != SNGGUF_OK) return rg;
-        return sngguf::launch_gemv_kq_mfma(x, M, q_up, nullptr, qtype, N, K, nullptr, nullptr, h, numerics, false, s, nullptr, 0.f, nullptr,
-                                           workspace);
+    const int64_t dense_bytes = sngguf_gate_up_silu_workspace_bytes(N, K);
+    const int64_t slices = form == kPairSplit && workspace_bytes > 0 ? pair_slices(M, N, K, workspace_bytes) : 0;
+    // (the workspace a form asks for is asked for whichever launch it then takes)
+    if (form == kPairDecode ? workspace_bytes < 2 * M * N : slices < 1 && workspace_bytes < dense_bytes) return SNGGUF_E_BADSHAPE;
+    if (M < 2048 && sngguf::mid_fits(qtype, M, N, K)) {   // (thousands of rows: the dense launch, 12288 x 4096 at 4096 rows 651 against 736 us)
+        // as much room for a K split as any caller has: what the form asks for
+        const int64_t asked = form == kPairDecode ? 0 : form == kPairSplit ? pair_slices(M, N, K, dense_bytes) * 8 * M * N : dense_bytes;
+        const int64_t room = (workspace_bytes < asked ? workspace_bytes : asked) / (8 * M * N);
+        const sngguf::MidPlan plan = sngguf::mid_plan(M, N, K, true, room);
+        if (form == kPairDecode || plan.us <= pair_us(qtype, M, N, K, slices))
+            return sngguf::launch_mid(plan, x, M, q_gate, q_up, qtype, N, K, nullptr, nullptr, h, static_cast<float*>(workspace), numerics, s);
     }
-    if (form == kPairSplit) {
-        const int64_t slices = workspace_bytes > 0 ? pair_slices(M, N, K, workspace_bytes) : 0;
-        if (slices >= 1)
-            return sngguf::launch_gemm_splitk_gated(x, M, q_gate, q_up, qtype, N, K, h, static_cast<float*>(workspace), (int)slices,
-                                                    numerics, s);
-    }
-    if (workspace_bytes < sngguf_gate_up_silu_workspace_bytes(N, K)) return SNGGUF_E_BADSHAPE;
+    if (slices >= 1)
+        return sngguf::launch_gemm_splitk_gated(x, M, q_gate, q_up, qtype, N, K, h, static_cast<float*>(workspace), (int)slices,
+                                                numerics, s);
     int rd = sngguf::launch_dequantize_interleaved(q_gate, qtype, N, K, workspace, 0, numerics, s);
     if (rd != SNGGUF_OK) return rd;
     rd = sngguf::launch_dequantize_interleaved(q_up, qtype, N, K, workspace, 1, numerics, s);

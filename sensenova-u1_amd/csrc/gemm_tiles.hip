@@ -605,13 +605,13 @@ int launch_tiles(const GemmArgs& a, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? SNGGUF_OK : SNGGUF_E_LAUNCH;
 }
 
-// y[m][n] = bf16(sum over slices of partial[s][m][n] + bias_g[n]), slices added in ascending order; one thread per
-// four consecutive outputs.  Row m belongs to group 1 (bias1) when indicator[m] != 0, or without an indicator when
+// y[m][n] = bf16(sum over slices of partial[s][m][n] + bias_g[n]) (+ residual[m][n], rounded again), slices added in ascending
+// order; one thread per four consecutive outputs.  Row m belongs to group 1 (bias1) when indicator[m] != 0, or without an indicator when
 // m >= n_text.
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ partial, int slices, int64_t M, int64_t N,
                                                             const uint8_t* __restrict__ indicator, int64_t n_text,
                                                             const bf16_t* __restrict__ bias0, const bf16_t* __restrict__ bias1,
-                                                            bf16_t* __restrict__ y) {
+                                                            const bf16_t* residual, bf16_t* y) {
     const int64_t total = M * N;
     const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i0 >= total) return;
@@ -628,6 +628,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 #pragma unroll
             for (int e = 0; e < 4; e++) s[e] += bf16_to_f32(bias[n + e]);
         }
+        if (residual) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) s[e] = add_residual(s[e], residual, i0 + e);
+        }
         *reinterpret_cast<u32x2_t*>(y + i0) = u32x2_t{pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3])};
     } else {
         for (int e = 0; e < 4 && i0 + e < total; e++) {
@@ -636,7 +640,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
             const int64_t m = (i0 + e) / N;
             const bf16_t* bias = bias_of(m);
             if (bias) s += bf16_to_f32(bias[(i0 + e) - m * N]);
-            y[i0 + e] = f32_to_bf16(s);
+            y[i0 + e] = f32_to_bf16(add_residual(s, residual, i0 + e));
         }
     }
 }
@@ -693,7 +697,7 @@ int launch_gemm_tiles(const GemmArgs& a, int qtype, int numerics, hipStream_t st
 int launch_splitk_reduce(const GemmArgs& a, const uint8_t* indicator, int64_t n_text, hipStream_t stream) {
     const int64_t quads = (a.M * a.N + 3) / 4;
     splitk_reduce_kernel<<<dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream>>>(a.partial, a.ksplit, a.M, a.N, indicator, n_text,
-                                                                                          a.bias[0], a.bias[1], a.y);
+                                                                                          a.bias[0], a.bias[1], a.residual, a.y);
     return hipGetLastError() == hipSuccess ? SNGGUF_OK : SNGGUF_E_LAUNCH;
 }
 

@@ -35,7 +35,7 @@ _OUT_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 EXPORTED_SYMBOLS = (
     "sngguf_version", "sngguf_strerror", "sngguf_type_size", "sngguf_block_size", "sngguf_dequantize",
-    "sngguf_linear", "sngguf_linear_residual", "sngguf_linear_workspace_bytes", "sngguf_linear_ws_bytes", "sngguf_linear_ws", "sngguf_linear_static_max_outputs", "sngguf_linear_static", "sngguf_gate_up_silu", "sngguf_gate_up_silu_workspace_bytes", "sngguf_gate_up_silu_ws_fits", "sngguf_gate_up_silu_ws_form", "sngguf_gate_up_silu_ws_bytes", "sngguf_gate_up_silu_ws", "sngguf_lm_head_argmax_workspace_bytes", "sngguf_lm_head_argmax", "sngguf_grouped_workspace_bytes", "sngguf_grouped_linear",
+    "sngguf_linear", "sngguf_linear_residual", "sngguf_linear_scratch_bytes", "sngguf_linear_scratch", "sngguf_linear_workspace_bytes", "sngguf_linear_ws_bytes", "sngguf_linear_ws", "sngguf_linear_static_max_outputs", "sngguf_linear_static", "sngguf_gate_up_silu", "sngguf_gate_up_silu_workspace_bytes", "sngguf_gate_up_silu_ws_fits", "sngguf_gate_up_silu_ws_form", "sngguf_gate_up_silu_ws_bytes", "sngguf_gate_up_silu_ws", "sngguf_lm_head_argmax_workspace_bytes", "sngguf_lm_head_argmax", "sngguf_grouped_workspace_bytes", "sngguf_grouped_linear",
     "sngguf_grouped_linear_ws", "sngguf_q8_0_tiled_bytes", "sngguf_q8_0_tile", "sngguf_linear_tiled", "sngguf_gate_up_silu_tiled",
     "sngguf_rmsnorm_fits", "sngguf_rmsnorm", "sngguf_rmsnorm_linear", "sngguf_rmsnorm_gate_up_silu",
     "sngguf_rmsnorm_linear_tiled", "sngguf_rmsnorm_gate_up_silu_tiled",
@@ -92,6 +92,10 @@ def load_library() -> ctypes.CDLL:
     lib.sngguf_gate_up_silu_workspace_bytes.restype = i64
     lib.sngguf_gate_up_silu_ws_fits.argtypes = [ci, i64, i64, i64]
     lib.sngguf_gate_up_silu_ws_fits.restype = ci
+    lib.sngguf_linear_scratch_bytes.argtypes = [ci, i64, i64, i64]
+    lib.sngguf_linear_scratch_bytes.restype = i64
+    lib.sngguf_linear_scratch.argtypes = [vp, i64, vp, ci, i64, i64, vp, vp, vp, vp, i64, ci, vp]
+    lib.sngguf_linear_scratch.restype = ci
     lib.sngguf_linear_ws_bytes.argtypes = [ci, i64, i64, i64]
     lib.sngguf_linear_ws_bytes.restype = i64
     lib.sngguf_gate_up_silu_ws_form.argtypes = [ci, i64, i64, i64]
@@ -659,6 +663,13 @@ def _dequantize_hip(packed, quant_type, out_dtype, numerics):
     return out
 
 
+def _split_scratch(dev, quant_type, m, n, k) -> Optional[torch.Tensor]:
+    """Scratch for the partial sums of a K split at 17 .. 64 rows, or in 64 rows of a few hundred (a few megabytes): the call's
+    own, as its output is, so calls of several threads on one stream need no order."""
+    nbytes = load_library().sngguf_linear_scratch_bytes(quant_type, m, n, k)
+    return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+
+
 def _linear_hip(x, packed, quant_type, bias, numerics):
     dev = _require_device(x, packed, bias)
     p, n, k = _packed_2d(packed, quant_type)
@@ -666,9 +677,14 @@ def _linear_hip(x, packed, quant_type, bias, numerics):
     y = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=dev)
     if m and n:
         b = _bias_bf16(bias, n, "linear")   # (held until the launch is enqueued)
+        scratch = _split_scratch(dev, quant_type, m, n, k) if 16 < m <= 512 else None
         with _on(dev):
-            rc = load_library().sngguf_linear(xc.data_ptr(), m, p.data_ptr(), quant_type, n, k, _ptr(b), y.data_ptr(),
-                                              numerics, _stream(dev))
+            if scratch is None:
+                rc = load_library().sngguf_linear(xc.data_ptr(), m, p.data_ptr(), quant_type, n, k, _ptr(b), y.data_ptr(),
+                                                  numerics, _stream(dev))
+            else:
+                rc = load_library().sngguf_linear_scratch(xc.data_ptr(), m, p.data_ptr(), quant_type, n, k, _ptr(b), None, y.data_ptr(),
+                                                          scratch.data_ptr(), scratch.numel(), numerics, _stream(dev))
         _check(rc, "sngguf_linear")
     return y
 
@@ -683,7 +699,15 @@ def _linear_residual_hip(x, packed, quant_type, bias, residual, numerics):
     r2d = r2d if r2d.is_contiguous() else r2d.contiguous()
     y = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=x.device)
     if y.numel():
-        linear_residual_into(x2d, p, quant_type, _bias_bf16(bias, n, "linear_residual"), r2d, y.view(-1, n), numerics)
+        b = _bias_bf16(bias, n, "linear_residual")
+        scratch = _split_scratch(x.device, quant_type, x2d.shape[0], n, k) if 16 < x2d.shape[0] <= 512 else None
+        if scratch is None:
+            linear_residual_into(x2d, p, quant_type, b, r2d, y.view(-1, n), numerics)
+        else:
+            with _on(x.device):
+                rc = load_library().sngguf_linear_scratch(x2d.data_ptr(), x2d.shape[0], p.data_ptr(), quant_type, n, k, _ptr(b), r2d.data_ptr(),
+                                                          y.data_ptr(), scratch.data_ptr(), scratch.numel(), numerics, _stream(x.device))
+            _check(rc, "sngguf_linear_scratch")
     return y
 
 

@@ -1,0 +1,26 @@
+"""Scratch that 17 .. 64 rows ask for, without a device: whole fp32 copies of the output where a K split pays, nothing elsewhere."""
+import pytest
+
+from sensenova_u1_amd import ops
+
+TYPES = [ops.Q4_0, ops.Q4_1, ops.Q5_0, ops.Q5_1, ops.Q8_0, ops.Q2_K, ops.Q3_K, ops.Q4_K, ops.Q5_K, ops.Q6_K]
+
+
+@pytest.mark.parametrize("qt", TYPES)
+def test_scratch_of_17_to_64_rows(qt):
+    size = ops.load_library().sngguf_linear_scratch_bytes
+    for m in (17, 32, 40, 64):
+        for n, k in ((512, 12288), (1024, 4096), (4096, 4096), (6144, 4096), (4096, 12288), (515, 2048), (12288, 4096)):
+            nbytes = size(qt, m, n, k)
+            copies = nbytes // (4 * m * n)
+            # two halves of K per workgroup: at least two super-blocks of 256 in a slice
+            assert nbytes % (4 * m * n) == 0 and copies != 1 and copies <= min(16, k // 512) and nbytes <= 64 << 20
+        assert size(qt, m, 4096, 12288) > 0          # 64 workgroups of 64 columns would leave three quarters of the device idle
+        assert size(qt, m, 4096, 256) == 0 and size(qt, m, 12288, 512) == 0
+    assert size(qt, 16, 4096, 12288) == 0 and size(qt, 0, 4096, 12288) == 0 and size(qt, 513, 4096, 4096) == 0
+    assert size(qt, 40, 0, 4096) == 0 and size(qt, 40, 4096, 4096 + 128) == 0 and size(qt, 40, 4096, -256) == 0
+
+
+def test_no_scratch_for_other_types():
+    size = ops.load_library().sngguf_linear_scratch_bytes
+    assert size(ops.BF16, 40, 4096, 12288) == 0 and size(16, 40, 4096, 12288) == 0
