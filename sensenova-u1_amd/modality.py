@@ -137,7 +137,7 @@ class FusedProjections(nn.Module):
         """With ``norm_weight`` the projections read ``RMSNorm(x)`` (``GGUFLinear.forward_normed``): for the q / k / v
         stack that is ``input_layernorm`` (``modeling_qwen3.py:919``), folded into the same launch at decode."""
         y = self.fused(x) if norm_weight is None else self.fused.forward_normed(x, norm_weight, eps)
-        return torch.split(y, self.splits, dim=-1)
+        return y.split_with_sizes(self.splits, -1)
 
 
 # Whether ``gated_mlp`` may run the whole MLP as ONE launch where the library offers it (``ops.mlp_decode_fits``: Q8_0,
@@ -152,25 +152,25 @@ def _one_launch_mlp(x, rows, gate_proj, up_proj, down_proj, norm_weight, residua
     its tag once.)"""
     if not (ONE_LAUNCH_MLP and 0 < rows <= 2 and x.is_cuda and x.dtype == torch.bfloat16):
         return None
-    packed, types = [], []
+    packed, types, numerics = [], [], gate_proj.numerics
     for m in (gate_proj, up_proj, down_proj):
         w = m.weight
         plain = ops._plain(w)
-        if m.bias is not None or m.decode_layout != "native" or m.numerics != gate_proj.numerics or not plain.is_cuda \
-                or (m.compute_dtype or x.dtype) != torch.bfloat16:
+        if m.bias is not None or m.decode_layout != "native" or m.numerics != numerics or not plain.is_cuda \
+                or (m.compute_dtype or torch.bfloat16) != torch.bfloat16:
             return None
         packed.append(plain)
-        types.append(m._weight_type())
+        types.append(m._weight_type(w))
     if norm_weight is not None and (norm_weight.dtype != torch.bfloat16 or norm_weight.numel() != gate_proj.in_features):
         return None
-    if residual is not None and (residual.dtype != torch.bfloat16 or tuple(residual.shape) != (*x.shape[:-1], down_proj.out_features)):
+    if residual is not None and (residual.dtype != torch.bfloat16 or residual.shape != (*x.shape[:-1], down_proj.out_features)):
         return None
     if types[0] != types[1]:
         return None
-    if (up_proj.in_features, up_proj.out_features) != (gate_proj.in_features, gate_proj.out_features) \
-            or (down_proj.in_features, down_proj.out_features) != (gate_proj.out_features, gate_proj.in_features):
+    hidden, inter = gate_proj.in_features, gate_proj.out_features
+    if up_proj.in_features != hidden or up_proj.out_features != inter or down_proj.in_features != inter or down_proj.out_features != hidden:
         return None
-    if not ops.mlp_decode_fits(types[0], types[2], rows, gate_proj.in_features, gate_proj.out_features):
+    if not ops.mlp_decode_fits(types[0], types[2], rows, hidden, inter):
         return None
     return (*packed, types[0], types[2])
 
@@ -188,23 +188,26 @@ def gated_mlp(x: torch.Tensor, gate_proj: GGUFLinear, up_proj: GGUFLinear, down_
     down projection, run as ONE launch (``sngguf_mlp_decode``; see ``ONE_LAUNCH_MLP``): same values as the separate
     launches up to the order in which the down projection's partial sums are added.  Beyond 16 rows, where
     ``_gated_tile_route`` says so, gate / up / SiLU run as ``sngguf_gate_up_silu_ws``."""
-    rows = x.numel() // x.shape[-1] if x.numel() else 0
+    numel = x.numel()
+    rows = numel // x.shape[-1] if numel else 0
     one = _one_launch_mlp(x, rows, gate_proj, up_proj, down_proj, norm_weight, residual)
     if one is not None:
         gate, up, down, qt, qt_down = one
-        ops._require_device(x, gate, up, down, norm_weight, residual)
-        for mod, w, t in ((gate_proj, gate, qt), (up_proj, up, qt), (down_proj, down, qt_down)):
+        dev = ops._require_device(x, gate, up, down, norm_weight, residual)
+        hidden, inter = gate_proj.in_features, gate_proj.out_features
+        for w, t, rows_w, cols in ((gate, qt, inter, hidden), (up, qt, inter, hidden), (down, qt_down, hidden, inter)):
             _, n, k = ops._packed_2d(w, t)
-            if (n, k) != (mod.out_features, mod.in_features):
-                raise ops.SnGgufError(f"gated_mlp: packed weight decodes to {(n, k)}, the module is {(mod.out_features, mod.in_features)}")
+            if n != rows_w or k != cols:
+                raise ops.SnGgufError(f"gated_mlp: packed weight decodes to {(n, k)}, the module is {(rows_w, cols)}")
             if not w.is_contiguous():
                 raise ops.SnGgufError("gated_mlp: the packed weights must be contiguous")
-        x2d = ops._as_bf16_rows(x, gate_proj.in_features, "gated_mlp")
-        out = torch.empty((*x.shape[:-1], down_proj.out_features), dtype=torch.bfloat16, device=x.device)
-        res2d = residual.reshape(-1, down_proj.out_features).contiguous() if residual is not None else None
-        ws = ops.mlp_decode_workspace(x.device, rows, gate_proj.in_features, gate_proj.out_features)
-        ops.mlp_decode_into(x2d, norm_weight.contiguous() if norm_weight is not None else None, eps, gate, up, qt, down, qt_down, res2d,
-                            out.view(-1, down_proj.out_features), ws, gate_proj.numerics)
+        xc, rows = ops._bf16_rows_flat(x, hidden, "gated_mlp")
+        x2d = xc if len(xc.shape) == 2 else xc.view(rows, hidden)
+        out = torch.empty((*x.shape[:-1], hidden), dtype=torch.bfloat16, device=dev)
+        ws = ops.mlp_decode_workspace(dev, rows, hidden, inter)
+        # (the outputs and the residual go in by address: their shapes are checked above, and a view costs 0.7 us)
+        ops.mlp_decode_into(x2d, norm_weight.contiguous() if norm_weight is not None else None, eps, gate, up, qt, down, qt_down,
+                            residual.contiguous() if residual is not None else None, out, ws, gate_proj.numerics)
         return out
     if residual is not None:
         return down_proj.forward_residual(_gated_activations(x, rows, gate_proj, up_proj, norm_weight, eps), residual)
@@ -422,14 +425,15 @@ class SharedInputStack:
         base = self.stacked.data_ptr()
         device = self.stacked.device
         first = self.members[0]
-        quant_type = int(first.weight.quant_type)
+        quant_type = first.weight.quant_type
+        numerics = first.numerics
         moved = False
         # (reads of the tagged parameters' attributes go through Python unless the subclass hook is off: 3 us each)
         with torch._C.DisableTorchFunctionSubclass():
             for mod, off in zip(self.members, self.offsets):
                 w = mod.weight
                 if (w.data_ptr() != base + off * self.row_bytes or w.device != device or mod.decode_layout != "native"
-                        or mod.numerics != first.numerics or int(w.quant_type) != quant_type or mod.bias is not None):
+                        or mod.numerics != numerics or w.quant_type != quant_type or mod.bias is not None):
                     moved = True
                     break
         if moved:
@@ -459,7 +463,8 @@ class SharedInputStack:
     def member_forward(self, mod: GGUFLinear, x: torch.Tensor) -> Optional[torch.Tensor]:
         """The member's output if the stack can supply it, else None (the member then runs its own launch)."""
         i = self.index[id(mod)]
-        rows = x.numel() // mod.in_features if x.numel() else 0
+        numel = x.numel()
+        rows = numel // mod.in_features if numel else 0
         # several rows: the members' outputs are column ranges of one [rows, sum(out_features)] buffer - every row
         # contiguous, rows a fixed stride apart.  Splitting the last dimension into heads (`.view(*shape[:-1], -1, head_dim)`,
         # modeling_qwen3.py:444,450,456) works on such a tensor; merging dimensions would need `.reshape`.  One row gives
@@ -489,13 +494,13 @@ class SharedInputStack:
             # x itself is kept with the result: while it is alive no other tensor can take its address, so an equal key
             # can only come from a tensor that shares its storage, shape, strides and version - the same values
             self._pending = (key, y, x)
-            return y[..., :self.splits[0]]
+            return y.narrow(-1, 0, self.splits[0])
         pending = self._pending
         if pending is None or pending[0] != key:
             return None
         if i == len(self.members) - 1:
             self._pending = None
-        return pending[1][..., self.offsets[i]:self.offsets[i] + self.splits[i]]
+        return pending[1].narrow(-1, self.offsets[i], self.splits[i])
 
     def dissolve(self) -> None:
         """Give every member its own storage back (a copy of its rows) and detach it from the stack."""

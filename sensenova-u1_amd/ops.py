@@ -178,22 +178,24 @@ def _check(rc: int, what: str) -> None:
 
 
 def _require_device(*tensors: Optional[torch.Tensor]) -> torch.device:
-    dev = None
+    dev = index = None
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise SnGgufError(
                 f"sn_gguf ops run on a HIP device only, got a tensor on '{t.device}'; "
                 "there is no CPU implementation")
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, t.get_device()
+        elif t.get_device() != index:
             raise SnGgufError(f"tensors on different devices: {dev} and {t.device}")
     return dev
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+# (a call has a device tensor in hand, so the runtime is up and the wrapper that would start it is not needed)
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 _NO_GUARD = contextlib.nullcontext()
 
 
@@ -207,7 +209,8 @@ def _stream(dev: torch.device) -> int:
 def _on(dev: torch.device):
     """Context in which ``dev`` is the current device (a launch on one of its streams needs that); free of charge when
     it already is, which is every call of a one-GPU process."""
-    if dev.index is None or dev.index == torch.cuda.current_device():
+    index = dev.index
+    if index is None or index == _current_device():
         return _NO_GUARD
     return torch.cuda.device(dev)
 
@@ -219,14 +222,17 @@ def _ptr(t: Optional[torch.Tensor]):
 
 def _packed_2d(packed: torch.Tensor, quant_type: int):
     """View the packed weight as uint8 [N, row_bytes]; returns (tensor, N, K)."""
-    if quant_type not in GGML_QUANT_SIZES:
+    sizes = GGML_QUANT_SIZES.get(quant_type)
+    if sizes is None:
         raise SnGgufError(f"quant type {quant_type} is not implemented (have Q4_0=2, Q4_1=3, Q5_0=6, Q5_1=7, Q8_0=8, Q2_K=10, Q3_K=11, Q4_K=12, Q5_K=13, Q6_K=14, BF16=30)")
-    bs, ts = GGML_QUANT_SIZES[quant_type]
-    if type(packed) is torch.Tensor and packed.dtype == torch.uint8 and packed.dim() == 2 and packed.is_contiguous() \
-            and not packed.requires_grad:
-        if packed.shape[1] % ts != 0:
-            raise SnGgufError(f"packed row of {packed.shape[1]} bytes is not a whole number of {ts}-byte blocks")
-        return packed, packed.shape[0], packed.shape[1] // ts * bs
+    bs, ts = sizes
+    if type(packed) is torch.Tensor and packed.dtype == torch.uint8 and packed.is_contiguous() and not packed.requires_grad:
+        shape = packed.shape
+        if len(shape) == 2:
+            n, row = shape
+            if row % ts != 0:
+                raise SnGgufError(f"packed row of {row} bytes is not a whole number of {ts}-byte blocks")
+            return packed, n, row // ts * bs
     p = packed.detach()
     if p.dtype != torch.uint8:
         p = p.view(torch.uint8)
@@ -348,11 +354,11 @@ def mlp_decode_into(x2d: torch.Tensor, gamma: Optional[torch.Tensor], eps: float
     to 16 rows; ONE launch where ``mlp_decode_fits`` says so."""
     dev = x2d.device
     m, hidden = x2d.shape
-    inter = gate.shape[0]
     with _on(dev):
-        rc = load_library().sngguf_mlp_decode(_ptr(x2d), m, _ptr(gamma), float(eps), _ptr(gate), _ptr(up), int(qt_gate_up), _ptr(down),
-                                              int(qt_down), hidden, inter, _ptr(residual), _ptr(y2d), _ptr(workspace),
-                                              workspace.numel() * workspace.element_size(), numerics, int(spin_limit), _stream(dev))
+        rc = load_library().sngguf_mlp_decode(x2d.data_ptr(), m, _ptr(gamma), float(eps), _ptr(gate), _ptr(up), int(qt_gate_up), _ptr(down),
+                                              int(qt_down), hidden, gate.shape[0], _ptr(residual), _ptr(y2d), workspace.data_ptr(),
+                                              workspace.numel() * workspace.element_size(), numerics,
+                                              int(spin_limit), _stream(dev))
     _check(rc, "sngguf_mlp_decode")
 
 
@@ -511,11 +517,15 @@ def rmsnorm_linear_into(x2d: torch.Tensor, gamma: torch.Tensor, eps: float, pack
                         bias: Optional[torch.Tensor], y2d: torch.Tensor, numerics: int) -> None:
     """y2d[M, N] = RMSNorm(x2d; gamma, eps) @ W^T (+ bias), the norm of Qwen3RMSNorm
     (modeling_qwen3.py:192-197) applied inside the projection kernel; shapes as ``rmsnorm_fits`` allows."""
-    dev = x2d.device
+    m, k = x2d.shape
+    _rmsnorm_linear(x2d.device, x2d, m, y2d.shape[1], k, gamma, eps, packed, quant_type, bias, y2d, numerics)
+
+
+def _rmsnorm_linear(dev, x, m, n, k, gamma, eps, packed, quant_type, bias, y, numerics) -> None:
+    """``rmsnorm_linear_into`` on tensors whose memory is the rows, whatever their shape."""
     with _on(dev):
-        rc = load_library().sngguf_rmsnorm_linear(_ptr(x2d), x2d.shape[0], _ptr(gamma), float(eps), _ptr(packed), quant_type,
-                                                  y2d.shape[1], x2d.shape[1], _ptr(bias), _ptr(y2d), numerics,
-                                                  _stream(dev))
+        rc = load_library().sngguf_rmsnorm_linear(_ptr(x), m, _ptr(gamma), float(eps), _ptr(packed), quant_type, n, k, _ptr(bias),
+                                                  _ptr(y), numerics, _stream(dev))
     _check(rc, "sngguf_rmsnorm_linear")
 
 
@@ -690,24 +700,27 @@ def _linear_hip(x, packed, quant_type, bias, numerics):
 
 
 def _linear_residual_hip(x, packed, quant_type, bias, residual, numerics):
-    _require_device(x, packed, bias, residual)
+    dev = _require_device(x, packed, bias, residual)
     p, n, k = _packed_2d(packed, quant_type)
-    x2d = _as_bf16_rows(x, k, "linear_residual")
-    if residual.dtype != torch.bfloat16 or tuple(residual.shape) != (*x.shape[:-1], n):
-        raise SnGgufError(f"linear_residual: residual must be bf16 of shape {(*x.shape[:-1], n)}")
-    r2d = residual.reshape(-1, n)
-    r2d = r2d if r2d.is_contiguous() else r2d.contiguous()
-    y = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=x.device)
-    if y.numel():
+    if k == 0:
+        raise SnGgufError("linear_residual: the weight has no columns")
+    xc, m = _bf16_rows_flat(x, k, "linear_residual")
+    shape = (*x.shape[:-1], n)
+    if residual.dtype != torch.bfloat16 or residual.shape != shape:
+        raise SnGgufError(f"linear_residual: residual must be bf16 of shape {shape}")
+    r = residual if residual.is_contiguous() else residual.contiguous()
+    y = torch.empty(shape, dtype=torch.bfloat16, device=dev)
+    if m and n:
         b = _bias_bf16(bias, n, "linear_residual")
-        scratch = _split_scratch(x.device, quant_type, x2d.shape[0], n, k) if 16 < x2d.shape[0] <= 512 else None
-        if scratch is None:
-            linear_residual_into(x2d, p, quant_type, b, r2d, y.view(-1, n), numerics)
-        else:
-            with _on(x.device):
-                rc = load_library().sngguf_linear_scratch(x2d.data_ptr(), x2d.shape[0], p.data_ptr(), quant_type, n, k, _ptr(b), r2d.data_ptr(),
-                                                          y.data_ptr(), scratch.data_ptr(), scratch.numel(), numerics, _stream(x.device))
-            _check(rc, "sngguf_linear_scratch")
+        scratch = _split_scratch(dev, quant_type, m, n, k) if 16 < m <= 512 else None
+        with _on(dev):
+            if scratch is None:
+                rc = load_library().sngguf_linear_residual(xc.data_ptr(), m, p.data_ptr(), quant_type, n, k, _ptr(b), r.data_ptr(), y.data_ptr(),
+                                                           numerics, _stream(dev))
+            else:
+                rc = load_library().sngguf_linear_scratch(xc.data_ptr(), m, p.data_ptr(), quant_type, n, k, _ptr(b), r.data_ptr(), y.data_ptr(),
+                                                          scratch.data_ptr(), scratch.numel(), numerics, _stream(dev))
+        _check(rc, "sngguf_linear_residual")
     return y
 
 

@@ -204,8 +204,9 @@ class GGUFLinear(nn.Linear):
         super().__init__(in_features, out_features, bias, device)
         self.compute_dtype = compute_dtype
 
-    def _weight_type(self) -> int:
-        w = self.weight
+    def _weight_type(self, w: Optional[torch.Tensor] = None) -> int:
+        if w is None:     # (a caller that has the parameter in hand passes it: reading it off the module costs 0.2 us)
+            w = self.weight
         if not hasattr(w, "quant_type"):
             raise RuntimeError("GGUFLinear.weight is not a GGUFParameter (no quant_type); was the checkpoint loaded?")
         return int(w.quant_type)
@@ -215,14 +216,21 @@ class GGUFLinear(nn.Linear):
         ops make: every tensor (inputs, weight, bias, ``others``) on one HIP device, the packed weight a whole
         number of blocks of shape ``[out_features, in_features]``, the input's last dim ``in_features``.  Raises
         ``SnGgufError`` before anything is launched - a host pointer handed to a kernel is a GPU memory fault."""
-        weight = ops._plain(self.weight)   # every attribute read of the tagged parameter itself goes through Python
-        ops._require_device(inputs, weight, self.bias, *others)
-        _, n, k = ops._packed_2d(weight, self._weight_type())
-        if (n, k) != (self.out_features, self.in_features):
+        self._checked_weight(inputs, self.bias, *others)
+        return ops._as_bf16_rows(inputs, self.in_features, "GGUFLinear")
+
+    def _checked_weight(self, inputs: torch.Tensor, *others: Optional[torch.Tensor]):
+        """The checks of ``_checked_rows`` on everything but the input's own type and width; returns the packed weight as a
+        plain tensor and its quant type."""
+        tagged = self.weight
+        weight, qtype = ops._plain(tagged), self._weight_type(tagged)   # attribute reads of the tagged parameter go through Python
+        ops._require_device(inputs, weight, *others)
+        _, n, k = ops._packed_2d(weight, qtype)
+        if n != self.out_features or k != self.in_features:
             raise ops.SnGgufError(f"GGUFLinear: packed weight decodes to {(n, k)}, the module is {(self.out_features, self.in_features)}")
         if not weight.is_contiguous():
             raise ops.SnGgufError("GGUFLinear: the packed weight must be contiguous")
-        return ops._as_bf16_rows(inputs, self.in_features, "GGUFLinear")
+        return weight, qtype
 
     def tiled_weight(self) -> Optional[torch.Tensor]:
         """The operand-order copy of the weight when ``decode_layout == "tiled"`` applies to this module (Q8_0,
@@ -255,12 +263,15 @@ class GGUFLinear(nn.Linear):
         return out
 
     def forward(self, inputs: torch.Tensor) -> torch.Tensor:
-        qtype = self._weight_type()
-        compute_dtype = self.compute_dtype or inputs.dtype
-        if inputs.dtype != compute_dtype:
+        weight = self.weight
+        qtype = self._weight_type(weight)
+        dtype = inputs.dtype
+        compute_dtype = self.compute_dtype or dtype
+        if dtype != compute_dtype:
             raise RuntimeError(f"GGUFLinear: input dtype {inputs.dtype} does not match compute dtype {compute_dtype}")
         if compute_dtype == torch.bfloat16:
-            rows = inputs.numel() // self.in_features if inputs.numel() else 0
+            numel = inputs.numel()
+            rows = numel // self.in_features if numel else 0
             stack = self.__dict__.get("_shared_stack")   # modality.SharedInputStack: q / k / v in one decode launch
             if stack is not None:
                 out = stack.member_forward(self, inputs)
@@ -271,7 +282,7 @@ class GGUFLinear(nn.Linear):
                 if out is not None:
                     return out
             if rows <= 16 or (rows <= 64 and self.in_features % 256 == 0) or self.gemm_policy == "fused" or qtype == ops.BF16:
-                return ops.linear(inputs, self.weight, qtype, self.bias, self.numerics)
+                return ops.linear(inputs, weight, qtype, self.bias, self.numerics)
             if self.gemm_policy not in ("auto", "two_pass", "resident"):
                 raise ValueError(f"GGUFLinear.gemm_policy is {self.gemm_policy!r}; expected 'auto', 'two_pass', 'fused' or 'resident'")
             x2d = self._checked_rows(inputs)
@@ -281,11 +292,11 @@ class GGUFLinear(nn.Linear):
                 # pooled workspace + the dense tile kernel (sngguf_linear_ws picks)
                 workspace = ops.pooled_workspace(inputs.device, self._workspace_bytes(rows))
                 bias = self.bias.detach().to(torch.bfloat16).contiguous() if self.bias is not None else None
-                ops.linear_ws_into(x2d, ops._plain(self.weight), qtype, bias, out.view(-1, self.out_features), workspace, self.numerics)
+                ops.linear_ws_into(x2d, ops._plain(weight), qtype, bias, out.view(-1, self.out_features), workspace, self.numerics)
             else:
                 self.two_pass_into(x2d, out.view(-1, self.out_features))
             return out
-        weight = ops.dequantize(self.weight, qtype, torch.float16 if self.numerics == ops.NUM_UPSTREAM_FP16 and qtype != ops.BF16
+        weight = ops.dequantize(weight, qtype, torch.float16 if self.numerics == ops.NUM_UPSTREAM_FP16 and qtype != ops.BF16
                                 else torch.float32, self.numerics).to(compute_dtype)
         bias = self.bias.to(compute_dtype) if self.bias is not None else None
         return torch.nn.functional.linear(inputs, weight, bias)
@@ -295,24 +306,26 @@ class GGUFLinear(nn.Linear):
         ``modeling_qwen3.py:192-197``; it feeds q / k / v at ``:919`` and the MLP at ``:938``).  Where the library
         offers it (Q8_0, a decode-sized input: ``ops.rmsnorm_fits``) the norm runs inside the projection kernel on
         the activations staged in LDS; otherwise as torch operations in front of ``forward``."""
-        rows = inputs.numel() // self.in_features if inputs.numel() else 0
+        numel = inputs.numel()
+        rows = numel // self.in_features if numel else 0
         fused = (inputs.is_cuda and rows > 0 and inputs.dtype == torch.bfloat16 and norm_weight.dtype == torch.bfloat16
-                 and (self.compute_dtype or inputs.dtype) == torch.bfloat16
+                 and (self.compute_dtype or torch.bfloat16) == torch.bfloat16
                  and ops.rmsnorm_fits(int(self.weight.quant_type), rows, self.in_features))
         if not fused:
             return self.forward(rms_norm(inputs, norm_weight, eps))
-        x2d = self._checked_rows(inputs, norm_weight)
-        if norm_weight.numel() != self.in_features:
-            raise ops.SnGgufError(f"GGUFLinear: norm weight has {norm_weight.numel()} elements, in_features is {self.in_features}")
-        out = torch.empty((*inputs.shape[:-1], self.out_features), dtype=torch.bfloat16, device=inputs.device)
-        bias = self.bias.detach().to(torch.bfloat16).contiguous() if self.bias is not None else None
+        bias, n, k = self.bias, self.out_features, self.in_features
+        weight, qtype = self._checked_weight(inputs, bias, norm_weight)
+        x, rows = ops._bf16_rows_flat(inputs, k, "GGUFLinear")
+        if norm_weight.numel() != k:
+            raise ops.SnGgufError(f"GGUFLinear: norm weight has {norm_weight.numel()} elements, in_features is {k}")
+        dev = inputs.device
+        out = torch.empty((*inputs.shape[:-1], n), dtype=torch.bfloat16, device=dev)
+        bias = bias.detach().to(torch.bfloat16).contiguous() if bias is not None else None
         tiled = self.tiled_weight() if self.decode_layout != "native" else None
         if tiled is not None:
-            ops.rmsnorm_linear_tiled_into(x2d, norm_weight.contiguous(), eps, tiled, bias, out.view(-1, self.out_features),
-                                          self.numerics)
+            ops.rmsnorm_linear_tiled_into(x.view(-1, k), norm_weight.contiguous(), eps, tiled, bias, out.view(-1, n), self.numerics)
         else:
-            ops.rmsnorm_linear_into(x2d, norm_weight.contiguous(), eps, ops._plain(self.weight), self._weight_type(), bias,
-                                    out.view(-1, self.out_features), self.numerics)
+            ops._rmsnorm_linear(dev, x, rows, n, k, norm_weight.contiguous(), eps, weight, qtype, bias, out, self.numerics)
         return out
 
     def forward_argmax(self, inputs: torch.Tensor) -> torch.Tensor:
@@ -327,7 +340,8 @@ class GGUFLinear(nn.Linear):
         """``residual + self(inputs)`` (the decoder layer's ``hidden_states = residual + o_proj(...)`` /
         ``residual + mlp(...)``, modeling_qwen3.py:934,940).  For bf16 inputs within the fused kernels' row
         range the add happens in the projection's epilogue; otherwise it is the plain sum."""
-        rows = inputs.numel() // self.in_features if inputs.numel() else 0
+        numel = inputs.numel()
+        rows = numel // self.in_features if numel else 0
         fused_rows = rows <= 16 or (rows <= 64 and self.in_features % 256 == 0) or self.gemm_policy == "fused"
         if inputs.dtype == torch.bfloat16 and (self.compute_dtype or inputs.dtype) == torch.bfloat16 and fused_rows \
                 and residual.dtype == torch.bfloat16:
@@ -335,7 +349,8 @@ class GGUFLinear(nn.Linear):
                 out = self._decode_tiled(inputs, residual)
                 if out is not None:
                     return out
-            return ops.linear_residual(inputs, self.weight, self._weight_type(), residual, self.bias, self.numerics)
+            weight = self.weight
+            return ops.linear_residual(inputs, weight, self._weight_type(weight), residual, self.bias, self.numerics)
         return residual + self(inputs)
 
     def _workspace_bytes(self, rows: int) -> int:
