@@ -25,6 +25,8 @@
 #include "kq_decode.hpp"
 #include "sngguf_common.hpp"
 
+#include <type_traits>
+
 namespace sngguf {
 
 namespace {
@@ -433,10 +435,14 @@ int launch_qt(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int6
 // Q8_0 kernel (MlpCtl).  Without `gamma` the gated activations are bit-identical to the gated pair's own launch (same
 // fragments, same order of accumulation), and so is the output (the down projection's own launch splits K over eight
 // wavefronts, not twelve: equal up to the order of twelve fp32 additions, which the tests allow for).
-// The decode arithmetic, not memory, bounds these formats: the launch is 0 - 5 % ahead of the two separate ones by device
-// and down type (32.3 against 33.9 us with a Q6_K down projection once the down projection's first requests are made
-// behind phase A's epilogue instead of in front of it; 31.9 - 32.8 against 32.7 - 33.0 with Q4_K), where the Q8_0 kernel
-// gains 10 %.
+// The decode arithmetic, not memory, bounds these formats (phase A takes 15 us with its requests and 15 without them; 56.6
+// MB are 10.5 us of memory): the launch is 0 - 5 % ahead of the two separate ones by device and down type (32.3 against 33.9
+// us with a Q6_K down projection once the down projection's first requests are made behind phase A's epilogue instead of in
+// front of it; 31.9 - 32.8 against 32.7 - 33.0 with Q4_K), where the Q8_0 kernel gains 10 %.  Since then, with the norm and
+// Q6_K, one row: 34.2 -> 32.4 us, of which the staging without LDS round trips is 2 us less ahead of the first decoded
+// super-block, and the falling priorities 1.5 less at the ends of both phases.  Two or four super-blocks requested ahead
+// instead of one, both halves of a super-block decoded as one block, and Q4_K's quants taken as pairs with two instructions
+// in eight fewer change nothing.
 template <int QT>
 struct SlabIo {
     typedef Slab<QT> S;
@@ -463,10 +469,10 @@ struct SlabIo {
         const uint8_t* p = base + (int64_t)s * S::ts;
 #pragma unroll
         for (int i = 0; i < kLoads - 1; i++) pre[i] = ld_piece<S::align>(p + off[i]);
-        if (tail_lane) pre[kLoads - 1] = ld_piece<S::align>(p + off[kLoads - 1]);
-        if constexpr (kQ6) {
-            if (lane < 16) pre_d = ld_u16(p + doff);
-        }
+        // (lanes past the last piece request row 0's first again: a request that some lanes skip is one that the compiler
+        // cannot count, and every wait behind it becomes a wait for all)
+        pre[kLoads - 1] = ld_piece<S::align>(p + off[kLoads - 1]);
+        if constexpr (kQ6) pre_d = ld_u16(p + doff);
     }
     __device__ __forceinline__ void store(uint8_t* slab, int lane, const u32x4_t (&pre)[kLoads], uint16_t pre_d) const {
 #pragma unroll
@@ -537,47 +543,48 @@ __global__ __launch_bounds__(64 * kMlpKqWaves) void mlp_kq_decode_kernel(const b
     uint8_t* const slab_a = lds + wave * IA::kSlab;
     u32x4_t pre_a[IA::kLoads];
     uint16_t pre_ad = 0;
-    ia.fetch(abase, sa0, lane, pre_a, pre_ad);
     if (tid < 16) cnt[tid] = 0;
-    // the activations, staged once for the workgroup (normalized in place if gamma is given)
+    // the activations, staged once for the workgroup (normalized if gamma is given): a thread keeps its 16 bytes of each row
+    // in registers across the sum of squares, and gamma's are on their way with them (hidden <= 8 x 768, M <= 2: the fits rule)
     {
-        const int pieces_per_row = (int)(hidden >> 3);
-        if (gamma == nullptr) {
-            for (int f = tid; f < M * pieces_per_row; f += 64 * kWaves) {
-                const int m = f / pieces_per_row, c = f - m * pieces_per_row;
-                *reinterpret_cast<u32x4_t*>(xs + m * xs_stride + 16 * c) = *reinterpret_cast<const u32x4_t*>(x + (int64_t)m * hidden + 8 * c);
-            }
-        } else {
+        const bool mine = tid < (int)(hidden >> 3);
+        u32x4_t xv0 = {}, xv1 = {}, gv = {};
+        if (mine) {
+            xv0 = *reinterpret_cast<const u32x4_t*>(x + 8 * tid);
+            if (M > 1) xv1 = *reinterpret_cast<const u32x4_t*>(x + hidden + 8 * tid);
+            if (gamma != nullptr) gv = *reinterpret_cast<const u32x4_t*>(gamma + 8 * tid);
+        }
+        ia.fetch(abase, sa0, lane, pre_a, pre_ad);
+        u32x4_t* const cell = reinterpret_cast<u32x4_t*>(xs + 16 * tid);
+        u32x4_t* const cell1 = reinterpret_cast<u32x4_t*>(xs + xs_stride + 16 * tid);
+        if (gamma != nullptr) {
             float* ssum = reinterpret_cast<float*>(xs + M * xs_stride);   // [M][waves]
-            for (int m = 0; m < M; m++) {
-                float ss = 0.f;
-                for (int c = tid; c < pieces_per_row; c += 64 * kWaves) {
-                    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(x + (int64_t)m * hidden + 8 * c);
-                    *reinterpret_cast<u32x4_t*>(xs + m * xs_stride + 16 * c) = v;
-                    ss += sumsq_piece(v);
-                }
-                ss = wave_sum(ss);
-                if (lane == 0) ssum[m * kWaves + wave] = ss;
+            const float ss0 = wave_sum(mine ? sumsq_piece(xv0) : 0.f);
+            if (lane == 0) ssum[wave] = ss0;
+            if (M > 1) {
+                const float ss1 = wave_sum(mine ? sumsq_piece(xv1) : 0.f);
+                if (lane == 0) ssum[kWaves + wave] = ss1;
             }
             __syncthreads();
-            for (int m = 0; m < M; m++) {
-                float tot = 0.f;
-                for (int w = 0; w < kWaves; w++) tot += ssum[m * kWaves + w];
-                const float rstd = rms_rstd(tot, hidden, eps);
-                for (int c = tid; c < pieces_per_row; c += 64 * kWaves) {
-                    u32x4_t* cell = reinterpret_cast<u32x4_t*>(xs + m * xs_stride + 16 * c);
-                    *cell = rmsnorm_piece(*cell, *reinterpret_cast<const u32x4_t*>(gamma + 8 * c), rstd);
-                }
-            }
+            float t0 = 0.f, t1 = 0.f;
+            for (int w = 0; w < kWaves; w++) t0 += ssum[w];
+            if (M > 1)
+                for (int w = 0; w < kWaves; w++) t1 += ssum[kWaves + w];
+            xv0 = rmsnorm_piece(xv0, gv, rms_rstd(t0, hidden, eps));
+            if (M > 1) xv1 = rmsnorm_piece(xv1, gv, rms_rstd(t1, hidden, eps));
+        }
+        if (mine) {
+            *cell = xv0;
+            if (M > 1) *cell1 = xv1;
         }
         __syncthreads();
     }
     const bool has_x = r < M;
     const uint8_t* xsrow = xs + (has_x ? r : M - 1) * xs_stride + 16 * g;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s = sa0; s < sa1; s++) {
+    auto step_a = [&](int s, auto more) {
         ia.store(slab_a, lane, pre_a, pre_ad);
-        if (s + 1 < sa1) ia.fetch(abase, s + 1, lane, pre_a, pre_ad);
+        if constexpr (decltype(more)::value) ia.fetch(abase, s + 1, lane, pre_a, pre_ad);
         const uint8_t* row = slab_a + r * IA::S::stride;
         auto emit0 = [&](int jj, const u32x4_t& a) {
             const u32x4_t xf = *reinterpret_cast<const u32x4_t*>(xsrow + (s * 8 + jj) * 64);
@@ -589,7 +596,21 @@ __global__ __launch_bounds__(64 * kMlpKqWaves) void mlp_kq_decode_kernel(const b
             acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, xf), acc, 0, 0, 0);
         };
         decode_half<QA, NUM, 1>(ident, row, g, emit1);
+    };
+    // A wavefront's priority falls as it gets on, a quarter of the loop at a time: the three wavefronts of a SIMD would
+    // otherwise be served oldest first, and the last would run its second half alone, where its chains of dependent
+    // instructions leave the SIMD idle (the wavefronts' ends lay 11 .. 19 us behind the start, now 13.5 .. 18).
+    for (int s = sa0; s < sa1 - 1; s++) {
+        switch ((s - sa0) * 4 / (sa1 - sa0)) {
+            case 0: __builtin_amdgcn_s_setprio(3); break;
+            case 1: __builtin_amdgcn_s_setprio(2); break;
+            case 2: __builtin_amdgcn_s_setprio(1); break;
+            default: __builtin_amdgcn_s_setprio(0); break;
+        }
+        step_a(s, std::true_type{});
     }
+    step_a(sa1 - 1, std::false_type{});
+    __builtin_amdgcn_s_setprio(3);
 
     // ---- phase B geometry: rows [16 bid, +16) of down, super-blocks [4 wave, +4) ----
     const int sb0 = wave * kSteps;
@@ -709,8 +730,11 @@ __global__ __launch_bounds__(64 * kMlpKqWaves) void mlp_kq_decode_kernel(const b
     };
     if constexpr (kAhead <= 0) decode_contract(0);
     if constexpr (kAhead <= 1) decode_contract(1);
+    __builtin_amdgcn_s_setprio(2);   // (as in phase A's loop)
     if constexpr (kAhead <= 2) decode_contract(2);
+    __builtin_amdgcn_s_setprio(1);
     if constexpr (kAhead <= 3) decode_contract(3);
+    __builtin_amdgcn_s_setprio(3);
     __syncthreads();   // every wavefront is past phase A's epilogue: its partial-sum area is free
     red_a[wave * 64 + lane] = yacc;
     __syncthreads();
