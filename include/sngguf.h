@@ -153,8 +153,10 @@ int sngguf_linear_scratch(const void* x, int64_t M, const void* q, int qtype, in
  * runs at the rate of that GEMM.  A problem with at most 128 output tiles of 256 x 256 (a few hundred rows, or a
  * narrow matrix) is split along K over floor(256 / tiles) workgroups per tile, with fp32 partial sums in the
  * workspace and a second pass that adds them: Q8_0 and Q4_K then skip the weight pass and use the 2 N K bytes
- * for the sums, the other types need 4 S M N bytes more than 2 N K for it.  Otherwise (workspace NULL or too
- * small included) it behaves exactly as sngguf_linear.  The workspace holds nothing the caller needs afterwards; calls sharing one workspace must
+ * for the sums, the other types need 4 S M N bytes more than 2 N K for it.  65 to 2047 rows with K % 256 == 0 run, in all ten
+ * types and without a weight pass, on the kernel that decodes packed rows straight into matrix operands wherever it is
+ * estimated to be the faster one in the room given (partial sums of its K slices in the workspace, 64 MiB at most unless
+ * 2 N K is more).  Otherwise (workspace NULL or too small included) it behaves exactly as sngguf_linear.  The workspace holds nothing the caller needs afterwards; calls sharing one workspace must
  * be ordered on one stream.  Never allocates.
  */
 int64_t sngguf_linear_workspace_bytes(int64_t N, int64_t K);
@@ -271,10 +273,10 @@ int sngguf_gate_up_silu(const void* x, int64_t M, const void* q_gate, const void
  *              that this shape takes needs (0 for shapes that do not fit and for M <= 16)
  *  M <= 16 runs sngguf_gate_up_silu (the workspace is not touched).  Otherwise the shape must satisfy
  *  sngguf_gate_up_silu_ws_fits(qtype, M, N, K) (M >= 17, K % 128 == 0, N % 8 == 0, M K < 2^31, a packed block
- *  format), else SNGGUF_E_BADSHAPE / SNGGUF_E_BADTYPE and the caller runs the two projections separately.  Two other
- *  forms with the same roundings take over where the dense launch does not pay: up to 64 rows with K % 256 == 0 the
- *  gate projection on the decode kernel, then the up projection with silu and the product in its epilogue; and Q8_0 /
- *  Q4_K from 65 rows on with at most 128 tiles of 256 x 256 (below 512 rows, or where the dense launch's tiles fill less
+ *  format), else SNGGUF_E_BADSHAPE / SNGGUF_E_BADTYPE and the caller runs the two projections separately.  Other
+ *  forms with the same roundings take over where the dense launch does not pay: up to 64 rows with K % 256 == 0, and up to
+ *  2047 where it is estimated to be faster, both matrices in one launch that decodes packed rows straight into matrix
+ *  operands (with K split over workgroups where there is room for the sums); and Q8_0 / Q4_K from 65 rows on with at most 128 tiles of 256 x 256 (below 512 rows, or where the dense launch's tiles fill less
  *  than 0.7 of their rounds) both matrices in one launch with K split over workgroups, fp32 partial sums in the
  *  workspace, and a reduction that ends in the gated product.  The dense form pays from about 512 rows on when the
  *  launch's ceil(M / 256) x ceil(N / 128) tiles come close to whole rounds of the 256 compute units (there is no K split;

@@ -1,7 +1,8 @@
 // Decode GEMV on the matrix cores (K % 256 == 0): the K-quants Q2_K .. Q6_K, one 256-element
 // super-block per step, and the 32-element formats Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, eight blocks per
-// step.  Up to 16 activation rows are one matrix operand; 17 .. 64 rows use MT = 2 .. 4 operands per
-// decoded weight fragment, so the weights are still fetched and decoded once.  (Q8_0 with at most
+// step.  Up to 16 activation rows are one matrix operand; 17 .. 64 rows, where gemm_mid.hip's kernel is estimated to be
+// slower (decode_kernel_us), use MT = 2 .. 4 operands per decoded weight fragment, so the weights are still fetched and
+// decoded once.  (Q8_0 with at most
 // 16 rows has faster kernels of its own.)
 //
 // Same shape as the Q8_0 kernel: a workgroup owns R * 16 weight rows (for the SiLU-gated pair the

@@ -384,7 +384,7 @@ class SharedInputStack:
     launch.  At decode that is one launch instead of three (the 4096 -> 1024 k / v launches cost more in launch overhead
     than in bytes); over thousands of image rows one launch of 384 large tiles instead of 256 + 64 + 64 (k / v alone have
     too few tiles to fill the chip).  Every output is the same dot product of the same rounded operands as the member's
-    own launch computes; beyond 64 rows the order in which the K steps' fp32 sums are added can differ (the narrow
+    own launch computes; beyond 16 rows the order in which the K steps' fp32 sums are added can differ (the narrow
     members' own launches split K over workgroups), i.e. the last place of a bf16 output now and then.
     Outputs of one step are ranges of one buffer: disjoint, every row contiguous, but not separately allocated - with
     several rows they are strided views (see ``member_forward``).  The pending result is recognised by the input's

@@ -163,15 +163,16 @@ class GGUFLinear(nn.Linear):
     """``nn.Linear`` whose weight is a :class:`GGUFParameter`.
 
     ``forward`` computes ``F.linear(x, dequantize(weight).to(compute_dtype), bias)`` with the
-    reference's rounding chain.  With bf16 activations and at most 16 rows (decode) - at most 64 rows
-    when ``in_features`` is a multiple of 256 - it is one fused dequant-GEMV launch that streams and
-    decodes the weights once.  With more rows ``gemm_policy`` decides:
+    reference's rounding chain.  With bf16 activations and at most 16 rows (decode) it is one fused
+    dequant-GEMV launch that streams and decodes the weights once; at most 64 rows, when ``in_features`` is a
+    multiple of 256, decode the weights once on the matrix cores (a second launch adds the partial sums where K
+    is split over workgroups, in scratch of the call's own).  With more rows ``gemm_policy`` decides:
 
     * ``"auto"`` (default): the library's own kernels through ``sngguf_linear_ws`` with a pooled workspace
       (``ops.pooled_workspace``, one per device and stream, reused by every module; each call asks for what its shape
-      can use, so the sums do not depend on how large the pool has grown): problems with few
-      output tiles run the large-tile kernel with K split over workgroups, the rest one weight pass into the
-      workspace (bf16, the same rounding chain) followed by the library's dense bf16 tile kernel.
+      can use, so the sums do not depend on how large the pool has grown): below 2048 rows packed rows are decoded
+      straight into matrix operands where that is faster, problems with few output tiles run the large-tile kernel
+      with K split over workgroups, the rest one weight pass into the workspace (bf16, the same rounding chain) followed by the library's dense bf16 tile kernel.
     * ``"two_pass"`` (opt-in): one HIP dequantize launch writes a transient bf16 weight and the device library's
       dense GEMM (``torch.matmul``) consumes it: no kernel of this library does the contraction then.  At 4096 rows it
       is about 10 % faster than ``"auto"`` on MI355X.
