@@ -274,11 +274,13 @@ int sngguf_gate_up_silu(const void* x, int64_t M, const void* q_gate, const void
  *  M <= 16 runs sngguf_gate_up_silu (the workspace is not touched).  Otherwise the shape must satisfy
  *  sngguf_gate_up_silu_ws_fits(qtype, M, N, K) (M >= 17, K % 128 == 0, N % 8 == 0, M K < 2^31, a packed block
  *  format), else SNGGUF_E_BADSHAPE / SNGGUF_E_BADTYPE and the caller runs the two projections separately.  Other
- *  forms with the same roundings take over where the dense launch does not pay: up to 64 rows with K % 256 == 0, and up to
- *  2047 where it is estimated to be faster, both matrices in one launch that decodes packed rows straight into matrix
- *  operands (with K split over workgroups where there is room for the sums); and Q8_0 / Q4_K from 65 rows on with at most 128 tiles of 256 x 256 (below 512 rows, or where the dense launch's tiles fill less
- *  than 0.7 of their rounds) both matrices in one launch with K split over workgroups, fp32 partial sums in the
- *  workspace, and a reduction that ends in the gated product.  The dense form pays from about 512 rows on when the
+ *  forms with the same roundings take over where the dense launch does not pay.  Up to 2047 rows with K % 256 == 0: both matrices
+ *  in one launch that decodes packed rows straight into matrix operands, with K split over workgroups (fp32 partial sums in the
+ *  workspace) where that pays, wherever it is estimated to be faster in the room given.  Otherwise, up to 64 rows, two launches of
+ *  the decode kernel with the gate outputs in the workspace (2 M N bytes are the least at these rows), and for Q8_0 / Q4_K from 65 rows
+ *  on with at most 128 tiles of 256 x 256 (below 512 rows, or where the dense launch's tiles fill less than 0.7 of their rounds)
+ *  both matrices in one launch with K split over workgroups, fp32 partial sums in the workspace, and a reduction that ends in
+ *  the gated product.  The dense form pays from about 512 rows on when the
  *  launch's ceil(M / 256) x ceil(N / 128) tiles come close to whole rounds of the 256 compute units (there is no K split;
  *  12288 x 4096 at 4096 rows: 628 us against 695 us for two sngguf_linear_ws launches and the product, at 2048 rows 354
  *  against 451).
@@ -294,6 +296,14 @@ int sngguf_gate_up_silu_ws_form(int qtype, int64_t M, int64_t N, int64_t K);
 int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const void* q_up, int qtype,
                            int64_t N, int64_t K, void* h, void* workspace, int64_t workspace_bytes,
                            int numerics, void* stream);
+
+/*
+ * Whether, given `workspace_bytes`, M rows run on the kernel that decodes packed rows straight into matrix operands - in
+ * sngguf_linear_scratch up to 64 rows, in sngguf_linear_ws beyond, in sngguf_gate_up_silu_ws if `pair` - and how (plan may be
+ * NULL): output columns of a workgroup, 16-row tiles of its kernel instance, row tiles, K slices.  Returns 1, or 0 where another kernel runs (plan
+ * untouched).  No device needed; for tests and profiles.
+ */
+int sngguf_mid_plan(int qtype, int64_t M, int64_t N, int64_t K, int pair, int64_t workspace_bytes, int64_t* plan);
 
 /*
  * RMSNorm fused in front of a decode projection.  In the decoder layer the q / k / v projections read

@@ -16,7 +16,7 @@ int launch_gemv_q8_mfma(const void* x, int64_t M, const void* qa, const void* qb
                         float eps, uint64_t* amax = nullptr);
 int launch_gemv_kq_mfma(const void* x, int64_t M, const void* qa, const void* qb, int qtype, int64_t N, int64_t K,
                         const void* bias, const void* residual, void* y, int numerics, bool gated, hipStream_t stream,
-                        const void* gamma, float eps, uint64_t* amax = nullptr);
+                        const void* gamma, float eps, uint64_t* amax = nullptr, const void* gate = nullptr);
 int64_t gemv_argmax_slots(int qtype, int64_t M, int64_t N);
 int launch_argmax_reduce(const uint64_t* keys, int64_t M, int64_t slots, int64_t* out_index, hipStream_t stream);
 int launch_dequantize_bf16(const void* q, int64_t rows, int64_t cols, void* out, int out_dtype, hipStream_t stream);
@@ -472,9 +472,9 @@ int sngguf_gate_up_silu_ws_fits(int qtype, int64_t M, int64_t N, int64_t K) {
 namespace {
 // How a pair beyond 16 rows runs; the shape is one that sngguf_gate_up_silu_ws_fits takes.
 enum PairForm {
-    // 17 .. 64 rows of whole 256-element runs: both matrices in one launch of the mid-size kernel, which ends in the gated
-    // product and needs no workspace (two launches of the decode kernel, the gate outputs in the workspace, took 1.2 - 2.3 times
-    // as long: 12288 x 4096, us: Q8_0 20 / 40 / 60 rows 50 / 66 / 90 against 38 / 39 / 40)
+    // 17 .. 64 rows of whole 256-element runs: both matrices in one launch of the mid-size kernel, K split over workgroups where the
+    // columns alone leave much of the device idle, or two launches of the decode kernel (the gate outputs into the workspace, then
+    // the up projection with silu and the product in its epilogue), whichever is estimated to be faster in the workspace given
     kPairDecode,
     // Few output tiles: the gated launch has no K split and would leave much of the chip idle (below 512 rows, or tiles that
     // fill less than 0.7 of their rounds), so both matrices run as one launch with K split over workgroups, and the
@@ -532,13 +532,43 @@ int sngguf_gate_up_silu_ws_form(int qtype, int64_t M, int64_t N, int64_t K) {
     }
 }
 
-int64_t sngguf_gate_up_silu_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
-    if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return 0;
-    const PairForm form = pair_form(qtype, M, N, K);
-    if (form == kPairDecode) return 2 * M * N;
-    const int64_t dense = sngguf_gate_up_silu_workspace_bytes(N, K);
+namespace {
+// Bytes of workspace that a pair's form can use: whole fp32 copies of both outputs for a K split (within what the dense form takes),
+// the gate outputs at 17 .. 64 rows, the interleaved weights for the dense form.
+int64_t pair_bytes(PairForm form, int qtype, int64_t M, int64_t N, int64_t K) {
+    const int64_t dense = sngguf_gate_up_silu_workspace_bytes(N, K), copy = 8 * M * N;
+    if (form == kPairDecode) {
+        const sngguf::MidPlan plan = sngguf::mid_plan(M, N, K, true, (dense < kSplitBytes ? dense : kSplitBytes) / copy);
+        const bool split = plan.slices > 1 && plan.us <= 2.0 * decode_kernel_us(M, N, K);
+        return split ? plan.slices * copy : 2 * M * N;
+    }
     const int64_t slices = form == kPairSplit ? pair_slices(M, N, K, dense) : 0;
-    return slices >= 1 ? slices * 8 * M * N : dense;
+    return slices >= 1 ? slices * copy : dense;
+}
+
+// How a pair runs with `workspace_bytes` (more than pair_bytes changes nothing): `mid` (form >= 0) on the mid-size kernel, else the
+// form's own launches, the split form with `slices` of K.
+struct PairRun {
+    PairForm form;
+    int64_t slices;
+    sngguf::MidPlan mid;
+};
+
+PairRun pair_run(int qtype, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
+    PairRun run{pair_form(qtype, M, N, K), 0, {-1, 0, 0, 0, 1, 1e30}};
+    if (run.form == kPairSplit && workspace_bytes > 0) run.slices = pair_slices(M, N, K, workspace_bytes);
+    if (M >= 2048 || !sngguf::mid_fits(qtype, M, N, K)) return run;   // (thousands of rows: the dense launch, 12288 x 4096 at 4096 rows 651 against 736 us)
+    const int64_t asked = pair_bytes(run.form, qtype, M, N, K);
+    const sngguf::MidPlan plan = sngguf::mid_plan(M, N, K, true, (workspace_bytes < asked ? workspace_bytes : asked) / (8 * M * N));
+    // (17 .. 64 rows, the decode kernel's two launches / here without a K split / with one, Q6_K, us: 1024 x 12288 at 17 rows 44 / 65 /
+    // 16.5, at 64 99 / 65 / 18; 4096 x 12288 at 17 rows 51 / 70 / 38; 1024 x 4096 19.4 / 21.9 / 11.3; 12288 x 4096, no split, 50 / 43)
+    if (plan.us <= (run.form == kPairDecode ? 2.0 * decode_kernel_us(M, N, K) : pair_us(qtype, M, N, K, run.slices))) run.mid = plan;
+    return run;
+}
+}  // namespace
+
+int64_t sngguf_gate_up_silu_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
+    return sngguf_gate_up_silu_ws_fits(qtype, M, N, K) ? pair_bytes(pair_form(qtype, M, N, K), qtype, M, N, K) : 0;
 }
 
 int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const void* q_up, int qtype, int64_t N, int64_t K,
@@ -550,27 +580,38 @@ int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const v
     if (!aligned(q_up, 16) || !aligned(workspace, 16)) return SNGGUF_E_ALIGN;
     if (!sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return qtype == SNGGUF_TYPE_BF16 ? SNGGUF_E_BADTYPE : SNGGUF_E_BADSHAPE;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const PairForm form = pair_form(qtype, M, N, K);
-    const int64_t dense_bytes = sngguf_gate_up_silu_workspace_bytes(N, K);
-    const int64_t slices = form == kPairSplit && workspace_bytes > 0 ? pair_slices(M, N, K, workspace_bytes) : 0;
-    // (the workspace a form asks for is asked for whichever launch it then takes)
-    if (form == kPairDecode ? workspace_bytes < 2 * M * N : slices < 1 && workspace_bytes < dense_bytes) return SNGGUF_E_BADSHAPE;
-    if (M < 2048 && sngguf::mid_fits(qtype, M, N, K)) {   // (thousands of rows: the dense launch, 12288 x 4096 at 4096 rows 651 against 736 us)
-        // as much room for a K split as any caller has: what the form asks for
-        const int64_t asked = form == kPairDecode ? 0 : form == kPairSplit ? pair_slices(M, N, K, dense_bytes) * 8 * M * N : dense_bytes;
-        const int64_t room = (workspace_bytes < asked ? workspace_bytes : asked) / (8 * M * N);
-        const sngguf::MidPlan plan = sngguf::mid_plan(M, N, K, true, room);
-        if (form == kPairDecode || plan.us <= pair_us(qtype, M, N, K, slices))
-            return sngguf::launch_mid(plan, x, M, q_gate, q_up, qtype, N, K, nullptr, nullptr, h, static_cast<float*>(workspace), numerics, s);
+    const PairRun run = pair_run(qtype, M, N, K, workspace_bytes);
+    // (the least workspace of a form is asked for whichever launch it then takes)
+    if (run.form == kPairDecode ? workspace_bytes < 2 * M * N : run.slices < 1 && workspace_bytes < sngguf_gate_up_silu_workspace_bytes(N, K))
+        return SNGGUF_E_BADSHAPE;
+    if (run.mid.form >= 0)
+        return sngguf::launch_mid(run.mid, x, M, q_gate, q_up, qtype, N, K, nullptr, nullptr, h, static_cast<float*>(workspace), numerics, s);
+    if (run.form == kPairDecode) {
+        const int rg = sngguf::launch_gemv(x, M, q_gate, nullptr, qtype, N, K, nullptr, nullptr, workspace, numerics, false, s);
+        if (rg != SNGGUF_OK) return rg;
+        return sngguf::launch_gemv_kq_mfma(x, M, q_up, nullptr, qtype, N, K, nullptr, nullptr, h, numerics, false, s, nullptr, 0.f, nullptr,
+                                           workspace);
     }
-    if (slices >= 1)
-        return sngguf::launch_gemm_splitk_gated(x, M, q_gate, q_up, qtype, N, K, h, static_cast<float*>(workspace), (int)slices,
+    if (run.slices >= 1)
+        return sngguf::launch_gemm_splitk_gated(x, M, q_gate, q_up, qtype, N, K, h, static_cast<float*>(workspace), (int)run.slices,
                                                 numerics, s);
     int rd = sngguf::launch_dequantize_interleaved(q_gate, qtype, N, K, workspace, 0, numerics, s);
     if (rd != SNGGUF_OK) return rd;
     rd = sngguf::launch_dequantize_interleaved(q_up, qtype, N, K, workspace, 1, numerics, s);
     if (rd != SNGGUF_OK) return rd;
     return sngguf::launch_gemm_dense_gated(x, M, workspace, N, K, h, s);
+}
+
+int sngguf_mid_plan(int qtype, int64_t M, int64_t N, int64_t K, int pair, int64_t workspace_bytes, int64_t* plan) {
+    if (M < 17 || M >= kMaxDim || N <= 0 || N >= kMaxDim || K <= 0 || K >= kMaxDim || !sngguf::mid_fits(qtype, M, N, K)) return 0;
+    if (pair && !sngguf_gate_up_silu_ws_fits(qtype, M, N, K)) return 0;
+    const sngguf::MidPlan p = pair ? pair_run(qtype, M, N, K, workspace_bytes).mid
+                            : M <= 64 ? rows_plan(qtype, M, N, K, workspace_bytes)
+                                      : workspace_plan(linear_split(qtype, M, N, K, workspace_bytes), qtype, M, N, K, workspace_bytes);
+    if (p.form < 0) return 0;
+    const int64_t out[4] = {sngguf::mid_columns(p.form), p.mt, p.row_tiles, p.slices};
+    for (int i = 0; plan && i < 4; i++) plan[i] = out[i];
+    return 1;
 }
 
 int64_t sngguf_lm_head_argmax_workspace_bytes(int64_t M, int64_t N) {

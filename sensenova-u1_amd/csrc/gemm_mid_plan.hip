@@ -42,6 +42,8 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 }  // namespace
 
+int mid_columns(int form) { return kForms[form].cols; }
+
 MidPlan mid_plan(int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices) {
     MidPlan best{-1, 0, 0, 0, 1, 1e30};
     const int64_t nsb = K >> 8, cols = pair ? 2 * N : N;

@@ -251,7 +251,7 @@ int launch_gemv_q8_mfma(const void* x, int64_t M, const void* qa, const void* qb
 
 int launch_gemv_kq_mfma(const void* x, int64_t M, const void* qa, const void* qb, int qtype, int64_t N, int64_t K,
                         const void* bias, const void* residual, void* y, int numerics, bool gated, hipStream_t stream,
-                        const void* gamma = nullptr, float eps = 0.f, uint64_t* amax = nullptr);
+                        const void* gamma = nullptr, float eps = 0.f, uint64_t* amax = nullptr, const void* gate = nullptr);
 
 // Second pass of the arg-max form of the decode kernels: keys[m][slots] -> out_index[m], one workgroup per activation
 // row.  (A key orders by value first and by lower column second, see argmax_key.)

@@ -42,7 +42,8 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_kq_mfma_kernel(const bf16_t* _
                                                                  const uint8_t* __restrict__ qa,
                                                                  const uint8_t* __restrict__ qb, int64_t N, int64_t K,
                                                                  const bf16_t* __restrict__ bias, const bf16_t* residual, bf16_t* __restrict__ y,
-                                                                 const bf16_t* __restrict__ gamma, float eps, uint64_t* __restrict__ amax) {
+                                                                 const bf16_t* __restrict__ gamma, float eps, uint64_t* __restrict__ amax,
+                                                                 const bf16_t* __restrict__ gate) {
     static_assert(!XN || MT == 1, "the fused norm is for at most 16 rows");
     typedef Slab<QT> S;
     constexpr int kRows = 16 * R;
@@ -218,12 +219,15 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_kq_mfma_kernel(const bf16_t* _
     __syncthreads();
     if constexpr (MT > 1) {
         // R * MT groups of sums: one wavefront each (one wavefront alone would walk through all of them, 8 R MT reads, while
-        // the rest of the workgroup has left).  Layout of a group as below, sums added in the same order.
+        // the rest of the workgroup has left: with the gated epilogue below, 40 rows of an 8B layer in Q8_0 130 against
+        // 142 us).  Layout of a group as below, sums added in the same order.
         for (int i = wave; i < R * MT; i += waves) {
             const int rg = i / MT, t = i - rg * MT, m = 16 * t + r;
             const int64_t n = n0 + 16 * rg + 4 * g, yi = (int64_t)m * N + n;
             if (m >= M || n >= N) continue;
             const bool whole = n + 3 < N && (N & 3) == 0;
+            u32x2_t gv = {0u, 0u};
+            if (gate) gv = *reinterpret_cast<const u32x2_t*>(gate + yi);   // requested ahead of the sums (N % 8 == 0: whole)
             f32x4_t sum = red[i * 64 + lane];
             for (int w = 1; w < W; w++) {
                 const f32x4_t p = red[(w * R * MT + i) * 64 + lane];
@@ -234,6 +238,12 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_kq_mfma_kernel(const bf16_t* _
             for (int v = 0; v < 4; v++) {
                 if (n + v >= N) continue;
                 o[v] = add_residual(sum[v] + (bias ? bf16_to_f32(bias[n + v]) : 0.f), residual, yi + v);
+                if (gate) {
+                    // the up projection of a SiLU-gated pair: `gate` holds the gate projection's outputs, and the value is
+                    // the rounded silu of those times the rounded output here, as the gated pair's own launch rounds
+                    const float gt = (v & 1) ? bf16hi_to_f32(gv[v >> 1]) : bf16lo_to_f32(gv[v >> 1]);
+                    o[v] = bf16_to_f32(f32_to_bf16(gt / (1.0f + expf(-gt)))) * bf16_to_f32(f32_to_bf16(o[v]));
+                }
             }
             if (whole) {
                 *reinterpret_cast<u32x2_t*>(y + yi) = u32x2_t{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
@@ -301,7 +311,7 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_kq_mfma_kernel(const bf16_t* _
 
 template <int QT, int NUM, int R>
 int launch_r(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64_t N, int64_t K, const bf16_t* bias,
-             const bf16_t* residual, bf16_t* y, bool gated, const bf16_t* gamma, float eps, hipStream_t stream, uint64_t* amax) {
+             const bf16_t* residual, bf16_t* y, bool gated, const bf16_t* gamma, float eps, hipStream_t stream, uint64_t* amax, const bf16_t* gate) {
     const int64_t groups = (N + 16 * R - 1) / (16 * R);
     const int nsb = (int)(K >> 8);
     const int mt = (M + 15) / 16;
@@ -351,7 +361,7 @@ int launch_r(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64
             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                                                    \
         if (attr != hipSuccess) return SNGGUF_E_LAUNCH;                                                                 \
         gemv_kq_mfma_kernel<QT, NUM, R, G, WM, 1, true><<<grid, block, lds_norm, stream>>>(x, M, qa, qb, N, K, bias,    \
-                                                                                           residual, y, gamma, eps, amax); \
+                                                                                           residual, y, gamma, eps, amax, nullptr); \
     } while (0)
         if (gated) {
             if (waves <= 4) SNGGUF_LAUNCH_XN(true, 4);
@@ -365,7 +375,7 @@ int launch_r(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64
     }
     const size_t lds_bytes = slab > red ? slab : red;
 #define SNGGUF_LAUNCH(G, WM, MT_) \
-    gemv_kq_mfma_kernel<QT, NUM, R, G, WM, MT_><<<grid, block, lds_bytes, stream>>>(x, M, qa, qb, N, K, bias, residual, y, nullptr, 0.f, amax)
+    gemv_kq_mfma_kernel<QT, NUM, R, G, WM, MT_><<<grid, block, lds_bytes, stream>>>(x, M, qa, qb, N, K, bias, residual, y, nullptr, 0.f, amax, gate)
     if (mt > 1) {
         // more than 16 activation rows: plain projections only.  The slabs of two row groups on eight wavefronts can pass
         // the default dynamic-LDS limit: raised once per kernel instance
@@ -402,7 +412,7 @@ inline int rows_per_workgroup(int qtype, int64_t M, int64_t N) {
 
 template <int QT, int NUM>
 int launch_qt(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int64_t N, int64_t K, const bf16_t* bias,
-              const bf16_t* residual, bf16_t* y, bool gated, const bf16_t* gamma, float eps, hipStream_t stream, uint64_t* amax) {
+              const bf16_t* residual, bf16_t* y, bool gated, const bf16_t* gamma, float eps, hipStream_t stream, uint64_t* amax, const bf16_t* gate) {
     // Up to 16 activation rows, two row groups per wavefront only when one per wavefront would already give far more
     // wavefronts than the chip holds (a vocabulary-sized projection): otherwise more, smaller workgroups spread more
     // evenly over the 256 compute units.  Beyond 16 rows what bounds the launch is the activation traffic - every
@@ -415,8 +425,8 @@ int launch_qt(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int6
     // groups do not fit the registers (45 of them go through memory): there one group stays where two leave compute units
     // waiting in their last round (49 rows, one / two groups, us: 10240 x 4096 40 / 45, 12288 x 4096 41 / 47, 20480 x 4096
     // 67 / 103, but 8192 x 4096 34 / 30, 14336 x 4096 53 / 49, 24576 x 4096 96 / 83).
-    if (rows_per_workgroup(QT, M, N) == 32) return launch_r<QT, NUM, 2>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax);
-    return launch_r<QT, NUM, 1>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax);
+    if (rows_per_workgroup(QT, M, N) == 32) return launch_r<QT, NUM, 2>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax, gate);
+    return launch_r<QT, NUM, 1>(x, M, qa, qb, N, K, bias, residual, y, gated, gamma, eps, stream, amax, gate);
 }
 
 // ---- the SiLU-gated MLP of a decoder layer at decode sizes in ONE launch, K-quant weights ---------------------
@@ -822,10 +832,13 @@ int64_t gemv_argmax_slots(int qtype, int64_t M, int64_t N) {
 }
 
 // 1 <= M <= 64 (SiLU-gated pair: M <= 16), K % 256 == 0, 16-byte aligned x and q (checked by the caller).  `gamma`
-// (K bf16, 16-byte aligned) switches the fused RMSNorm on; the caller keeps M (2 K + 64) <= 36 KB then.
+// (K bf16, 16-byte aligned) switches the fused RMSNorm on; the caller keeps M (2 K + 64) <= 36 KB then.  `gate` ([M][N],
+// 8-byte aligned, M > 16, N % 4 == 0, no bias or residual): y = silu(gate) * projection.
 int launch_gemv_kq_mfma(const void* x, int64_t M, const void* qa, const void* qb, int qtype, int64_t N, int64_t K,
                         const void* bias, const void* residual, void* y, int numerics, bool gated, hipStream_t stream,
-                        const void* gamma, float eps, uint64_t* amax) {
+                        const void* gamma, float eps, uint64_t* amax, const void* gate) {
+    if (gate && (gated || M <= 16 || N % 4 != 0 || bias || residual)) return SNGGUF_E_BADSHAPE;
+    const bf16_t* gt = static_cast<const bf16_t*>(gate);
     if (amax && (gated || M > 16)) return SNGGUF_E_BADSHAPE;
     const bf16_t* gp = static_cast<const bf16_t*>(gamma);
     const bf16_t* xp = static_cast<const bf16_t*>(x);
@@ -837,9 +850,9 @@ int launch_gemv_kq_mfma(const void* x, int64_t M, const void* qa, const void* qb
 #define SNGGUF_CASE(QT)                                                                                          \
     if (qtype == QT) {                                                                                           \
         if (numerics == SNGGUF_NUM_GGML_FP32)                                                                    \
-            return launch_qt<QT, SNGGUF_NUM_GGML_FP32>(xp, (int)M, a, b, N, K, bp, rp, yp, gated, gp, eps, stream, amax);          \
+            return launch_qt<QT, SNGGUF_NUM_GGML_FP32>(xp, (int)M, a, b, N, K, bp, rp, yp, gated, gp, eps, stream, amax, gt);          \
         if (numerics == SNGGUF_NUM_UPSTREAM_FP16)                                                                \
-            return launch_qt<QT, SNGGUF_NUM_UPSTREAM_FP16>(xp, (int)M, a, b, N, K, bp, rp, yp, gated, gp, eps, stream, amax);      \
+            return launch_qt<QT, SNGGUF_NUM_UPSTREAM_FP16>(xp, (int)M, a, b, N, K, bp, rp, yp, gated, gp, eps, stream, amax, gt);      \
         return SNGGUF_E_BADTYPE;                                                                                 \
     }
     SNGGUF_CASE(SNGGUF_TYPE_Q4_0)

@@ -254,7 +254,7 @@ def _gated_activations(x, rows, gate_proj, up_proj, norm_weight, eps) -> torch.T
         n, qt = gate_proj.out_features, int(gate_proj.weight.quant_type)
         h = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=x.device)
         nbytes = ops.gate_up_silu_ws_bytes(qt, rows, n, gate_proj.in_features)
-        # up to 64 rows (batched decode, a megabyte) the scratch is the call's own, as the outputs of two projections were
+        # up to 64 rows (batched decode, a few megabytes) the scratch is the call's own, as the outputs of two projections were
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if rows <= 64 else ops.pooled_workspace(x.device, nbytes)
         ops.gate_up_silu_ws_into(x2d, ops._plain(gate_proj.weight), ops._plain(up_proj.weight), qt, h.view(-1, n), ws, gate_proj.numerics,
                                  nbytes)

@@ -35,7 +35,7 @@ _OUT_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 EXPORTED_SYMBOLS = (
     "sngguf_version", "sngguf_strerror", "sngguf_type_size", "sngguf_block_size", "sngguf_dequantize",
-    "sngguf_linear", "sngguf_linear_residual", "sngguf_linear_scratch_bytes", "sngguf_linear_scratch", "sngguf_linear_workspace_bytes", "sngguf_linear_ws_bytes", "sngguf_linear_ws", "sngguf_linear_static_max_outputs", "sngguf_linear_static", "sngguf_gate_up_silu", "sngguf_gate_up_silu_workspace_bytes", "sngguf_gate_up_silu_ws_fits", "sngguf_gate_up_silu_ws_form", "sngguf_gate_up_silu_ws_bytes", "sngguf_gate_up_silu_ws", "sngguf_lm_head_argmax_workspace_bytes", "sngguf_lm_head_argmax", "sngguf_grouped_workspace_bytes", "sngguf_grouped_linear",
+    "sngguf_linear", "sngguf_linear_residual", "sngguf_linear_scratch_bytes", "sngguf_linear_scratch", "sngguf_linear_workspace_bytes", "sngguf_linear_ws_bytes", "sngguf_linear_ws", "sngguf_linear_static_max_outputs", "sngguf_linear_static", "sngguf_gate_up_silu", "sngguf_gate_up_silu_workspace_bytes", "sngguf_gate_up_silu_ws_fits", "sngguf_gate_up_silu_ws_form", "sngguf_gate_up_silu_ws_bytes", "sngguf_gate_up_silu_ws", "sngguf_mid_plan", "sngguf_lm_head_argmax_workspace_bytes", "sngguf_lm_head_argmax", "sngguf_grouped_workspace_bytes", "sngguf_grouped_linear",
     "sngguf_grouped_linear_ws", "sngguf_q8_0_tiled_bytes", "sngguf_q8_0_tile", "sngguf_linear_tiled", "sngguf_gate_up_silu_tiled",
     "sngguf_rmsnorm_fits", "sngguf_rmsnorm", "sngguf_rmsnorm_linear", "sngguf_rmsnorm_gate_up_silu",
     "sngguf_rmsnorm_linear_tiled", "sngguf_rmsnorm_gate_up_silu_tiled",
@@ -96,6 +96,8 @@ def load_library() -> ctypes.CDLL:
     lib.sngguf_linear_scratch_bytes.restype = i64
     lib.sngguf_linear_scratch.argtypes = [vp, i64, vp, ci, i64, i64, vp, vp, vp, vp, i64, ci, vp]
     lib.sngguf_linear_scratch.restype = ci
+    lib.sngguf_mid_plan.argtypes = [ci, i64, i64, i64, ci, i64, vp]
+    lib.sngguf_mid_plan.restype = ci
     lib.sngguf_linear_ws_bytes.argtypes = [ci, i64, i64, i64]
     lib.sngguf_linear_ws_bytes.restype = i64
     lib.sngguf_gate_up_silu_ws_form.argtypes = [ci, i64, i64, i64]
@@ -438,14 +440,22 @@ PAIR_SEPARATE, PAIR_DECODE, PAIR_SPLIT, PAIR_DENSE = range(4)
 
 def gate_up_silu_ws_form(quant_type: int, m: int, n: int, k: int) -> int:
     """The form in which ``gate_up_silu_ws_into`` is faster than two projections, silu and the product on ``m`` rows of this
-    pair: the decode kernels, K split over workgroups, or the dense launch where its tiles fill the chip; else
+    pair: 17 .. 64 rows, K split over workgroups, or the dense launch where its tiles fill the chip; else
     ``PAIR_SEPARATE``."""
     return int(load_library().sngguf_gate_up_silu_ws_form(quant_type, m, n, k))
 
 
 def gate_up_silu_ws_bytes(quant_type: int, m: int, n: int, k: int) -> int:
-    """Bytes of workspace the form that ``m`` rows of this pair take needs (2 m n up to 64 rows; 0 = does not fit)."""
+    """Bytes of workspace that the form which ``m`` rows of this pair take can use (up to 64 rows 2 m n are the least, and more than
+    that is partial sums; 0 = does not fit)."""
     return int(load_library().sngguf_gate_up_silu_ws_bytes(quant_type, m, n, k))
+
+
+def mid_plan(quant_type: int, m: int, n: int, k: int, pair: bool, workspace_bytes: int):
+    """How ``m`` rows run on the mid-size kernel with that much workspace: (columns of a workgroup, 16-row tiles of its kernel
+    instance, row tiles, K slices); None where another kernel runs."""
+    plan = (ctypes.c_int64 * 4)()
+    return tuple(plan) if load_library().sngguf_mid_plan(quant_type, m, n, k, int(pair), workspace_bytes, plan) else None
 
 
 def gate_up_silu_ws_into(x2d: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, quant_type: int, h2d: torch.Tensor,

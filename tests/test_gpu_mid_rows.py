@@ -66,6 +66,27 @@ def test_pair_of_every_instance(dev, c_oracle, qt, m, n, k):
     assert bool((h[m] == 7.0).all())   # nothing behind the last row
 
 
+@pytest.mark.parametrize("qt", TYPES)
+@pytest.mark.parametrize("m,n,k", [(17, 520, 12288), (48, 1032, 4096), (64, 2048, 2304)])
+def test_pair_of_few_columns_in_any_workspace(dev, c_oracle, qt, m, n, k):
+    """The K split that the shape asks for, one slice fewer, and the least workspace: the gate outputs alone, which the decode kernel's
+    two launches or the launch without a K split take.  Nothing behind the bytes handed over."""
+    num = (m + n // 8) & 1
+    gate, up = (synthetic.make_packed(qt, n, k, seed=n + j, device=dev) for j in (0, 1))
+    x = synthetic.make_activations(m, k, seed=m, device=dev)
+    cols = _columns(n, m)
+    g, u = (go.gguf_linear_forward(x.cpu(), w[cols.to(dev)].cpu(), qt, numerics=num) for w in (gate, up))
+    want, asked = c_oracle.silu_mul(g, u), ops.gate_up_silu_ws_bytes(qt, m, n, k)
+    assert asked >= 2 * 8 * m * n
+    for nbytes in (asked, asked - 16, 2 * m * n):
+        print(f"case mid few columns qt={qt} num={num} {m}x{n}x{k} workspace {nbytes}", flush=True)
+        ws = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device=dev)
+        h = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=dev)
+        ops.gate_up_silu_ws_into(x, gate, up, qt, h[:m], ws, num, nbytes)
+        _check(h[:m, cols.to(dev)].cpu(), want)
+        assert bool((ws[nbytes:] == 0xA5).all()) and bool((h[m] == 7.0).all())
+
+
 @pytest.mark.parametrize("qt", [go.Q8_0, go.Q4_K, go.Q3_K, go.Q6_K])
 @pytest.mark.parametrize("m,n,k", [(65, 1024, 2304), (203, 515, 4096), (300, 2050, 1280), (509, 4096, 2048), (1000, 1032, 768), (130, 264, 12288)])
 def test_projection_beyond_64_rows(dev, qt, m, n, k):

@@ -1,4 +1,5 @@
-"""Scratch that 17 .. 64 rows ask for, without a device: whole fp32 copies of the output where a K split pays, nothing elsewhere."""
+"""What 17 rows to two thousand ask for and how they run, without a device: whole fp32 copies of the outputs where a K split pays,
+nothing elsewhere."""
 import pytest
 
 from sensenova_u1_amd import ops
@@ -24,3 +25,20 @@ def test_scratch_of_17_to_64_rows(qt):
 def test_no_scratch_for_other_types():
     size = ops.load_library().sngguf_linear_scratch_bytes
     assert size(ops.BF16, 40, 4096, 12288) == 0 and size(16, 40, 4096, 12288) == 0
+
+
+@pytest.mark.parametrize("qt", TYPES)
+def test_pairs_of_few_columns_split_k_at_17_to_64_rows(qt):
+    """A pair of few columns leaves most of the device idle unless K is split; the least workspace (the gate outputs) still runs, and
+    more than the shape asks for changes nothing."""
+    for m in (17, 33, 64):
+        for n, k in ((512, 12288), (1024, 4096), (2048, 12288), (4096, 4096), (4096, 12288)):
+            nbytes, copy = ops.gate_up_silu_ws_bytes(qt, m, n, k), 8 * m * n
+            plan = ops.mid_plan(qt, m, n, k, True, nbytes)
+            assert plan[3] >= 2 and nbytes == plan[3] * copy <= min(64 << 20, ops.gate_up_silu_workspace_bytes(n, k))
+            assert ops.mid_plan(qt, m, n, k, True, 1 << 40) == plan
+            least = ops.mid_plan(qt, m, n, k, True, 2 * m * n)
+            assert least is None or least[3] == 1
+        # (two launches of the decode kernel instead of 48 super-blocks one after the other)
+        assert m == 64 or ops.mid_plan(qt, m, 512, 12288, True, 2 * m * 512) is None
+        assert ops.gate_up_silu_ws_bytes(qt, m, 12288, 4096) == 2 * m * 12288 and ops.gate_up_silu_ws_bytes(qt, m, 512, 256) == 2 * m * 512
