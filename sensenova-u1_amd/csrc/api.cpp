@@ -147,16 +147,17 @@ int sngguf_dequantize(const void* q, int qtype, int64_t rows, int64_t cols, void
 
 namespace {
 
-// us of the decode kernel for every format (gemv_kq_mfma.hip) on 17 .. 64 rows: rounds of workgroups, each as many super-blocks
-// one after the other as a wavefront gets of K.  Fitted with the plans of gemm_mid_plan.hip (nine shapes, 20 / 40 / 60 rows, three
-// types); choosing by the two is 0.7 % slower than the faster of the two in the mean.
-double decode_kernel_us(int64_t M, int64_t N, int64_t K) {
-    const int64_t mt = (M + 15) / 16, rg = N > 4096 ? 2 : 1, groups = (N + 16 * rg - 1) / (16 * rg), nsb = K / 256, counted = (N + 15) / 16;
-    int64_t w = (256 * 12 + counted - 1) / counted;
-    const bool four = groups > 256 || (groups == 256 && nsb >= 32 && M >= 22);
-    if (w > (four ? 4 : 8)) w = four ? 4 : 8;
-    if (w > nsb) w = nsb;
-    return 6.1 + (double)((groups + 255) / 256) * (double)((nsb + w - 1) / w) * (1.33 + 0.63 * (double)(mt * rg));
+// us of the decode kernel for every format (gemv_kq_mfma.hip) on 17 .. 64 rows: rounds of workgroups of one or two 16-row groups; for
+// each super-block a workgroup takes its activations from L2 (512 bytes a row at 50 bytes a ns, however many wavefronts share them),
+// decodes each group once and contracts it with every 16-row operand; and the weights come from memory.  Fitted (rms 4.7 %) to 600
+// timings: twelve shapes of 512 .. 24576 columns, 17 / 32 / 33 / 48 / 64 rows, ten formats.  Choosing between it and the plans of
+// gemm_mid_plan.hip by the two estimates is 0.3 % slower than the faster of the two in the mean, 14 % at worst (512 x 2048 at 48
+// rows, 9.1 against 8.0 us).
+double decode_kernel_us(int qtype, int64_t M, int64_t N, int64_t K) {
+    const int64_t mt = (M + 15) / 16, rg = N > 4096 ? 2 : 1, groups = (N + 16 * rg - 1) / (16 * rg);
+    const double element = (double)sngguf_type_size(qtype) / (double)sngguf_block_size(qtype);   // bytes
+    const double step = 0.0102 * (double)M + 0.0397 * (double)(mt * rg) + (double)rg * (0.0315 + 0.047 * element);
+    return 3.7 + (double)((groups + 255) / 256 * (K / 256)) * step + (double)N * (double)K * element * 0.08e-6;
 }
 
 // Between the decode kernels' 64 rows and a few hundred, a matrix with few 256 x 256 output tiles keeps only a few
@@ -185,8 +186,8 @@ constexpr int64_t kSplitBytes = (int64_t)64 << 20;   // the most fp32 partial su
 sngguf::MidPlan rows_plan(int qtype, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes) {
     sngguf::MidPlan plan{-1, 0, 0, 0, 1, 1e30};
     if (M > 64 || !sngguf::mid_fits(qtype, M, N, K)) return plan;
-    plan = sngguf::mid_plan(M, N, K, false, (scratch_bytes < kSplitBytes ? scratch_bytes : kSplitBytes) / (4 * M * N));
-    if (plan.us > decode_kernel_us(M, N, K)) plan.form = -1;
+    plan = sngguf::mid_plan(qtype, M, N, K, false, (scratch_bytes < kSplitBytes ? scratch_bytes : kSplitBytes) / (4 * M * N));
+    if (plan.us > decode_kernel_us(qtype, M, N, K)) plan.form = -1;
     return plan;
 }
 int64_t rows_scratch_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
@@ -359,16 +360,22 @@ LinearSplit linear_split(int qtype, int64_t M, int64_t N, int64_t K, int64_t wor
 }  // namespace
 
 namespace {
+// us of a weight pass: packed rows read, bf16 written; Q3_K and Q5_K decode behind the memory's rate (12288 x 4096 about 12 us more).
+double weight_pass_us(int qtype, int64_t N, int64_t K) {
+    const double rate = qtype == SNGGUF_TYPE_Q3_K ? 3.75e6 : qtype == SNGGUF_TYPE_Q5_K ? 4.05e6 : 4.7e6;
+    return 3.2 + (double)N * (double)K * ((double)sngguf_type_size(qtype) / (double)sngguf_block_size(qtype) + 2.0) / rate;
+}
+
 // us of that route: workgroups of 256 x 256 tiles, 1.9 us a K step with the decode in the loop and 1.2 without, the weight pass,
-// the partial sums.  Fitted (rms 6.5 %) to twelve shapes at 65 .. 4096 rows, three types; choosing between it and the plans of
-// gemm_mid_plan.hip by the two models is 1 % slower than the fastest in the mean.
+// the partial sums.  Fitted (rms 11 %) to twelve shapes at 65 .. 1024 rows, ten types; the plans of gemm_mid_plan.hip are chosen in all
+// but a few of those, and choosing by the two estimates is 0.1 % slower than the faster of the two in the mean (10 % at worst).
 double workspace_route_us(const LinearSplit& f, int qtype, int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), wgs = tiles * f.slices;
     const bool pass = !(f.tile_type && f.slices >= 2);
     const double ksteps = (double)((K / 64 + f.slices - 1) / f.slices);
     double us = (double)((wgs + 255) / 256) * (6.3 + ksteps * (pass ? 1.21 : 1.89));
-    if (pass) us += 3.2 + (double)N * (double)K * ((double)sngguf_type_size(qtype) / (double)sngguf_block_size(qtype) + 2.0) / 4.7e6;
-    if (f.slices >= 2) us += 7.1 + (double)(f.slices * M * N) * 8.0 / 7.8e6;
+    if (pass) us += weight_pass_us(qtype, N, K);
+    if (f.slices >= 2) us += 7.1 + (double)(f.slices * M * N) * 8.0 / 6.2e6;
     return us;
 }
 
@@ -379,7 +386,7 @@ sngguf::MidPlan workspace_plan(const LinearSplit& f, int qtype, int64_t M, int64
     sngguf::MidPlan none{-1, 0, 0, 0, 1, 1e30};
     if (M >= 2048 || !sngguf::mid_fits(qtype, M, N, K)) return none;
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), most = tiles <= 128 ? kSplitBytes : 2 * N * K;
-    const sngguf::MidPlan plan = sngguf::mid_plan(M, N, K, false, (workspace_bytes < most ? workspace_bytes : most) / (4 * M * N));
+    const sngguf::MidPlan plan = sngguf::mid_plan(qtype, M, N, K, false, (workspace_bytes < most ? workspace_bytes : most) / (4 * M * N));
     return plan.us <= workspace_route_us(f, qtype, M, N, K) ? plan : none;
 }
 }  // namespace
@@ -513,9 +520,8 @@ double pair_us(int qtype, int64_t M, int64_t N, int64_t K, int64_t slices) {
         const int64_t wgs = 2 * ((M + 255) / 256) * ((N + 255) / 256) * slices;
         return 10.0 + (double)((wgs + 255) / 256) * ((double)((K / 64 + slices - 1) / slices) * 1.9 + 5.0) + (double)(slices * M * N) * 16.0 / 5e6;
     }
-    const double pass = 3.2 + (double)N * (double)K * ((double)sngguf_type_size(qtype) / (double)sngguf_block_size(qtype) + 2.0) / 4.7e6;
     const int64_t tiles = ((M + 255) / 256) * ((N + 127) / 128);
-    return 2.0 * pass + 6.0 + (double)((tiles + 255) / 256) * (3.0 + (double)(K / 64) * 1.45);
+    return 2.0 * weight_pass_us(qtype, N, K) + 6.0 + (double)((tiles + 255) / 256) * (3.0 + (double)(K / 64) * 1.45);
 }
 }  // namespace
 
@@ -538,8 +544,8 @@ namespace {
 int64_t pair_bytes(PairForm form, int qtype, int64_t M, int64_t N, int64_t K) {
     const int64_t dense = sngguf_gate_up_silu_workspace_bytes(N, K), copy = 8 * M * N;
     if (form == kPairDecode) {
-        const sngguf::MidPlan plan = sngguf::mid_plan(M, N, K, true, (dense < kSplitBytes ? dense : kSplitBytes) / copy);
-        const bool split = plan.slices > 1 && plan.us <= 2.0 * decode_kernel_us(M, N, K);
+        const sngguf::MidPlan plan = sngguf::mid_plan(qtype, M, N, K, true, (dense < kSplitBytes ? dense : kSplitBytes) / copy);
+        const bool split = plan.slices > 1 && plan.us <= 2.0 * decode_kernel_us(qtype, M, N, K);
         return split ? plan.slices * copy : 2 * M * N;
     }
     const int64_t slices = form == kPairSplit ? pair_slices(M, N, K, dense) : 0;
@@ -559,10 +565,10 @@ PairRun pair_run(int qtype, int64_t M, int64_t N, int64_t K, int64_t workspace_b
     if (run.form == kPairSplit && workspace_bytes > 0) run.slices = pair_slices(M, N, K, workspace_bytes);
     if (M >= 2048 || !sngguf::mid_fits(qtype, M, N, K)) return run;   // (thousands of rows: the dense launch, 12288 x 4096 at 4096 rows 651 against 736 us)
     const int64_t asked = pair_bytes(run.form, qtype, M, N, K);
-    const sngguf::MidPlan plan = sngguf::mid_plan(M, N, K, true, (workspace_bytes < asked ? workspace_bytes : asked) / (8 * M * N));
+    const sngguf::MidPlan plan = sngguf::mid_plan(qtype, M, N, K, true, (workspace_bytes < asked ? workspace_bytes : asked) / (8 * M * N));
     // (17 .. 64 rows, the decode kernel's two launches / here without a K split / with one, Q6_K, us: 1024 x 12288 at 17 rows 44 / 65 /
     // 16.5, at 64 99 / 65 / 18; 4096 x 12288 at 17 rows 51 / 70 / 38; 1024 x 4096 19.4 / 21.9 / 11.3; 12288 x 4096, no split, 50 / 43)
-    if (plan.us <= (run.form == kPairDecode ? 2.0 * decode_kernel_us(M, N, K) : pair_us(qtype, M, N, K, run.slices))) run.mid = plan;
+    if (plan.us <= (run.form == kPairDecode ? 2.0 * decode_kernel_us(qtype, M, N, K) : pair_us(qtype, M, N, K, run.slices))) run.mid = plan;
     return run;
 }
 }  // namespace

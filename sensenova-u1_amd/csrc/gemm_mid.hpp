@@ -37,7 +37,7 @@ struct MidPlan {
 bool mid_fits(int qtype, int64_t M, int64_t N, int64_t K);
 // The fastest plan of a shape that fits by the model, with room for `max_slices` fp32 copies of the output (of both outputs of
 // a pair); 0 or 1: no K split.
-MidPlan mid_plan(int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices);
+MidPlan mid_plan(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices);
 // Output columns of a workgroup in a form.
 int mid_columns(int form);
 // Runs a plan; plan.slices > 1 needs `partial` (slices copies) and, for a pair, no bias or residual.

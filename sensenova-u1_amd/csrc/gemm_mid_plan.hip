@@ -29,14 +29,33 @@ struct FormInfo {
     int sizes[8];              // 16-row tiles an instance holds, ascending, 0-terminated
     double fixed, step, row;   // us of a workgroup: prologue and epilogue, a super-block, a super-block per 16 rows
 };
-// Fitted (log least squares, rms 4.5 %) to 3000 timings of Q8_0, Q4_K and Q6_K: twelve shapes of 512 .. 12288 columns and 2048 ..
-// 12288 elements of K, 20 .. 1024 rows, every form and tile with 1 .. 16 K slices.  Its pick is 0.6 % slower than the fastest of
-// them in the mean (17 % at worst, 4096 x 4096 at 72 rows), over the three types alike, so they share one set of constants.
+// These pick the form, the tile and the split; one set for all formats.  Fitted (log least squares) to Q8_0, Q4_K and Q6_K at twelve
+// shapes, 20 .. 1024 rows; measured over all ten formats - eleven shapes of 512 .. 24576 columns and 2048 .. 12288 elements of K, 17 ..
+// 1900 rows, every form and tile with 1 .. 16 K slices, 36090 timings - the pick is 0.6 % slower than the fastest of them in the
+// mean (17 % at worst: 100 rows of 4096 x 4096 in Q4_0 and Q4_1).
 constexpr FormInfo kForms[] = {
     {64, 2, {2, 3, 4, 0}, 1.16, 1.62, 0.16},
     {128, 2, {2, 3, 4, 6, 8, 10, 13, 0}, 3.26, 2.41, 0.35},
     {256, 1, {10, 13, 16, 0}, 3.49, 3.40, 0.19},
 };
+
+// Against other kernels it takes the time itself, which these constants miss by up to a quarter from format to format: us of a plan
+// with the super-block's share scaled by format, the split's launch and sums, and the outputs, fitted to the same timings of what
+// is picked (rms 5.8 %; one set for all 9 %, with Q6_K 19 % under).
+double format_step(int qtype) {
+    switch (qtype) {
+    case SNGGUF_TYPE_Q4_0: return 0.776;
+    case SNGGUF_TYPE_Q4_1: return 0.813;
+    case SNGGUF_TYPE_Q5_0: return 0.977;
+    case SNGGUF_TYPE_Q5_1: return 0.920;
+    case SNGGUF_TYPE_Q8_0: return 0.911;
+    case SNGGUF_TYPE_Q2_K: return 0.859;
+    case SNGGUF_TYPE_Q3_K: return 0.981;
+    case SNGGUF_TYPE_Q4_K: return 0.933;
+    case SNGGUF_TYPE_Q5_K: return 1.034;
+    default: return 1.185;   // Q6_K
+    }
+}
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
@@ -44,9 +63,11 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 int mid_columns(int form) { return kForms[form].cols; }
 
-MidPlan mid_plan(int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices) {
+MidPlan mid_plan(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices) {
     MidPlan best{-1, 0, 0, 0, 1, 1e30};
     const int64_t nsb = K >> 8, cols = pair ? 2 * N : N;
+    const double scale = format_step(qtype), outputs = (double)(2 * M * N);
+    double best_pick = 1e30;
     for (int form = 0; form < 3; form++) {
         const FormInfo& f = kForms[form];
         const int64_t col_tiles = ceil_div(cols, f.cols);
@@ -71,9 +92,12 @@ MidPlan mid_plan(int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices)
                 // two workgroups of the narrow form run on a compute unit at once and hide some of each other's latency, but the
                 // instructions of both have to be issued: two take as long as two
                 const int64_t rounds = form == kMidNarrow ? ceil_div(per_cu, 2) : per_cu;
-                double us = 3.3 + (double)rounds * f.fixed + (double)per_cu * (double)steps * step;
-                if (s > 1) us += 2.75 + (double)(s * M * cols) * 8.0 / 6.7e6;
-                if (us < best.us) best = MidPlan{form, mt, tile_rows, row_tiles, (int)s, us};
+                const double fixed = 3.3 + (double)rounds * f.fixed, sums = (double)(s * M * cols) * 8.0, loop = (double)(per_cu * steps);
+                const double pick = fixed + loop * step + (s > 1 ? 2.75 + sums / 6.7e6 : 0.0);
+                if (pick >= best_pick) continue;
+                best_pick = pick;
+                best = MidPlan{form, mt, tile_rows, row_tiles, (int)s,
+                               fixed + loop * (f.step * scale + f.row * mt) + (s > 1 ? 3.4 + sums / 5.4e6 : outputs * 0.32e-6)};
             }
         }
     }

@@ -39,6 +39,29 @@ def test_pairs_of_few_columns_split_k_at_17_to_64_rows(qt):
             assert ops.mid_plan(qt, m, n, k, True, 1 << 40) == plan
             least = ops.mid_plan(qt, m, n, k, True, 2 * m * n)
             assert least is None or least[3] == 1
-        # (two launches of the decode kernel instead of 48 super-blocks one after the other)
-        assert m == 64 or ops.mid_plan(qt, m, 512, 12288, True, 2 * m * 512) is None
+        # (17 rows: two launches of the decode kernel, 37 - 42 us, instead of 48 super-blocks one after the other, 42 - 58)
+        assert m > 17 or ops.mid_plan(qt, m, 512, 12288, True, 2 * m * 512) is None
         assert ops.gate_up_silu_ws_bytes(qt, m, 12288, 4096) == 2 * m * 12288 and ops.gate_up_silu_ws_bytes(qt, m, 512, 256) == 2 * m * 512
+
+
+@pytest.mark.parametrize("qt,m,n,k,workspace", [
+    (ops.Q6_K, 17, 24576, 2048, 1 << 30),      # decode kernel 22 us, mid-size kernel 25
+    (ops.Q4_K, 17, 1024, 4096, 1 << 30),       # 8.6, 9.4
+    (ops.Q5_K, 17, 1024, 4096, 1 << 30),       # 8.8, 9.8
+    (ops.Q6_K, 64, 4096, 12288, 0),            # no scratch, no K split: 51, 67
+    (ops.Q6_K, 1024, 12288, 4096, 1 << 40),    # weight pass and dense launch 110, mid-size kernel 123
+    (ops.Q6_K, 1024, 24576, 2048, 1 << 40)])   # 125, 134
+def test_projections_stay_on_the_faster_kernel(qt, m, n, k, workspace):
+    """Formats whose decode takes longer than the one that a shared estimate was fitted to, and 17 rows, where the decode kernel's
+    second operand is nearly empty."""
+    assert ops.mid_plan(qt, m, n, k, False, workspace) is None
+
+
+def test_projections_on_the_mid_size_kernel():
+    """(us as above, all ten formats within a few per cent): 48 rows of 4096 x 12288 37 / 21, 64 rows of 12288 x 4096 44 / 24, 203 rows of
+    6144 x 4096 37 / 31; 1024 rows of 12288 x 4096 in Q8_0 108 / 105."""
+    for qt in TYPES:
+        for m, n, k in ((48, 4096, 12288), (64, 12288, 4096), (203, 6144, 4096), (509, 4096, 12288)):
+            assert ops.mid_plan(qt, m, n, k, False, 1 << 40) is not None
+    assert ops.mid_plan(ops.Q8_0, 1024, 12288, 4096, False, 1 << 40) is not None
+    assert ops.mid_plan(ops.Q8_0, 2048, 12288, 4096, False, 1 << 40) is None and ops.mid_plan(ops.BF16, 40, 4096, 4096, False, 1 << 30) is None
