@@ -14,8 +14,8 @@ namespace {
 // integer is formed without a convert); NUM 0: exact fp32 products, one rounding in the subtraction
 // (the - 1024 - zero rides on the accumulator input of the widening instruction).  Must be called
 // by all 64 lanes; `ident` is identity_row(lane).
-// MX: fp16 -> fp32 on the matrix cores (widen_f16x4), for kernels whose vector ALU is the busier unit; without it one
-// conversion per value, for kernels whose matrix cores are (`ident` is not used then, and a decoder has no branch).
+// MX: fp16 -> fp32 on the matrix cores (widen_f16x4), for kernels whose vector ALU is the busier unit, the decoders below among
+// them; without it one conversion per value, for the kernel whose matrix cores are (gemm_mid.hip; `ident` is not used then).
 // FUSED (formats with a minimum and zero = 0): the product and the operation next to it as one fused multiply-add
 // where that gives the same bits.  NUM 0: D * q is exact in fp32 (at most 11 + 6 + 5 significant bits), so
 // fma(D, q, -DM) rounds once exactly where D * q - DM does.  NUM 1: (1024 + q) * D - 1024 * D, exact inside the
@@ -157,7 +157,7 @@ __device__ __forceinline__ uint32_t lds_u32(const uint8_t* p) {
 // row.  TS block bytes; HAS_MIN: f16 m after d, value d q + m, else d (q - 8 or 16); FIVE: 32-bit
 // fifth-bit word before the quants.  Lane group g covers elements 8 g .. 8 g + 7: bytes
 // 8 (g % 2) .. of qs, low nibbles for g < 2, high nibbles otherwise; fifth bits = byte g of qh.
-template <int NUM, int B, int TS, bool HAS_MIN, bool FIVE, bool MX>
+template <int NUM, int B, int TS, bool HAS_MIN, bool FIVE>
 __device__ __forceinline__ u32x4_t legacy_block(half4_t ident, const uint8_t* row, int g) {
     typedef Num<NUM> A;
     constexpr int kHdr = HAS_MIN ? 4 : 2;
@@ -177,16 +177,16 @@ __device__ __forceinline__ u32x4_t legacy_block(half4_t ident, const uint8_t* ro
         v1 |= ((((bits >> 4) & 0xFu) * 0x00204081u) & 0x01010101u) << 4;
     }
     uint32_t a0, a1, a2, a3;
-    kq_dword_bf16<NUM, HAS_MIN, false, MX>(ident, v0, kZero, d, DM, a0, a1);
-    kq_dword_bf16<NUM, HAS_MIN, false, MX>(ident, v1, kZero, d, DM, a2, a3);
+    kq_dword_bf16<NUM, HAS_MIN, false, true>(ident, v0, kZero, d, DM, a0, a1);
+    kq_dword_bf16<NUM, HAS_MIN, false, true>(ident, v1, kZero, d, DM, a2, a3);
     return u32x4_t{a0, a1, a2, a3};
 }
-template <int NUM, int HALF, int TS, bool HAS_MIN, bool FIVE, bool MX, typename Emit>
+template <int NUM, int HALF, int TS, bool HAS_MIN, bool FIVE, typename Emit>
 __device__ __forceinline__ void decode_legacy(half4_t ident, const uint8_t* row, int g, Emit&& emit) {
-    emit(0, legacy_block<NUM, 4 * HALF + 0, TS, HAS_MIN, FIVE, MX>(ident, row, g));
-    emit(1, legacy_block<NUM, 4 * HALF + 1, TS, HAS_MIN, FIVE, MX>(ident, row, g));
-    emit(2, legacy_block<NUM, 4 * HALF + 2, TS, HAS_MIN, FIVE, MX>(ident, row, g));
-    emit(3, legacy_block<NUM, 4 * HALF + 3, TS, HAS_MIN, FIVE, MX>(ident, row, g));
+    emit(0, legacy_block<NUM, 4 * HALF + 0, TS, HAS_MIN, FIVE>(ident, row, g));
+    emit(1, legacy_block<NUM, 4 * HALF + 1, TS, HAS_MIN, FIVE>(ident, row, g));
+    emit(2, legacy_block<NUM, 4 * HALF + 2, TS, HAS_MIN, FIVE>(ident, row, g));
+    emit(3, legacy_block<NUM, 4 * HALF + 3, TS, HAS_MIN, FIVE>(ident, row, g));
 }
 
 // Q8_0: block b at byte 34 b of the slab row: f16 d, then 32 int8 quants (2 bytes off a dword for even b)
@@ -210,7 +210,7 @@ __device__ __forceinline__ void decode_q8_0(const uint8_t* row, int g, Emit&& em
 
 // Q2_K: element 128 h + 32 j + l is bit pair j of qs[32 h + l]; its 16-element group
 // 8 h + 2 j + l / 16 has scale (low nibble) and min (high nibble) in one byte.
-template <int NUM, int HALF, bool MX, typename Emit>
+template <int NUM, int HALF, typename Emit>
 __device__ __forceinline__ void decode_q2_k(half4_t ident, const uint8_t* row, int g, Emit&& emit) {
     typedef Num<NUM> A;
     constexpr int h = HALF;
@@ -223,15 +223,15 @@ __device__ __forceinline__ void decode_q2_k(half4_t ident, const uint8_t* row, i
         const uint32_t byte = (sm[j >> 1] >> (8 * (2 * (j & 1) + (g >> 1)))) & 0xFFu;
         const typename A::T D = d * A::integer((int)(byte & 15u)), DM = dmin * A::integer((int)(byte >> 4));
         uint32_t a0, a1, a2, a3;
-        kq_dword_bf16<NUM, true, false, MX>(ident, (qs[0] >> (2 * j)) & 0x03030303u, 0.f, D, DM, a0, a1);
-        kq_dword_bf16<NUM, true, false, MX>(ident, (qs[1] >> (2 * j)) & 0x03030303u, 0.f, D, DM, a2, a3);
+        kq_dword_bf16<NUM, true, false, true>(ident, (qs[0] >> (2 * j)) & 0x03030303u, 0.f, D, DM, a0, a1);
+        kq_dword_bf16<NUM, true, false, true>(ident, (qs[1] >> (2 * j)) & 0x03030303u, 0.f, D, DM, a2, a3);
         emit(j, u32x4_t{a0, a1, a2, a3});
     }
 }
 
 // Q3_K: stored quant (0..7) = bit pair as in Q2_K | mask bit (4 h + j of hmask[l]) << 2, value
 // stored - 4; 6-bit group scales split over the 12 scale bytes, value stored - 32.
-template <int NUM, int HALF, bool MX, typename Emit>
+template <int NUM, int HALF, typename Emit>
 __device__ __forceinline__ void decode_q3_k(half4_t ident, const uint8_t* row, int g, Emit&& emit) {
     typedef Num<NUM> A;
     constexpr int h = HALF;
@@ -254,7 +254,7 @@ __device__ __forceinline__ void decode_q3_k(half4_t ident, const uint8_t* row, i
 #pragma unroll
         for (int w = 0; w < 2; w++) {
             const uint32_t v = ((qs[w] >> (2 * j)) & 0x03030303u) | (((hm[w] >> (4 * h + j)) & 0x01010101u) << 2);
-            kq_dword_bf16<NUM, false, false, MX>(ident, v, 4.f, D, D, a[2 * w], a[2 * w + 1]);
+            kq_dword_bf16<NUM, false, false, true>(ident, v, 4.f, D, D, a[2 * w], a[2 * w + 1]);
         }
         emit(j, u32x4_t{a[0], a[1], a[2], a[3]});
     }
@@ -305,7 +305,7 @@ __device__ __forceinline__ bool q4k_pairs(const u32x4_t& head, int g, typename N
 
 // The four A operands of half a super-block (sub-blocks 4 HALF .. 4 HALF + 3) of one row, fed to
 // `emit(jj, a)` with jj = 0..3.  `row` points at the row's super-block in the slab; g = lane / 16.
-template <int NUM, int HALF, bool FUSED, bool MX, typename Emit>
+template <int NUM, int HALF, bool FUSED, typename Emit>
 __device__ __forceinline__ void decode_q4_k_body(half4_t ident, const uint8_t* row, int g, const typename Num<NUM>::T (&Ds)[4],
                                                  const typename Num<NUM>::T (&DMs)[4], Emit&& emit) {
 #pragma unroll
@@ -318,25 +318,24 @@ __device__ __forceinline__ void decode_q4_k_body(half4_t ident, const uint8_t* r
             const typename Num<NUM>::T D = Ds[j - 4 * HALF], DM = DMs[j - 4 * HALF];
             const uint32_t v0 = (hi ? qs[0] >> 4 : qs[0]) & 0x0F0F0F0Fu, v1 = (hi ? qs[1] >> 4 : qs[1]) & 0x0F0F0F0Fu;
             uint32_t a0, a1, a2, a3;
-            kq_dword_bf16<NUM, true, FUSED, MX>(ident, v0, 0.f, D, DM, a0, a1);
-            kq_dword_bf16<NUM, true, FUSED, MX>(ident, v1, 0.f, D, DM, a2, a3);
+            kq_dword_bf16<NUM, true, FUSED, true>(ident, v0, 0.f, D, DM, a0, a1);
+            kq_dword_bf16<NUM, true, FUSED, true>(ident, v1, 0.f, D, DM, a2, a3);
             emit(j - 4 * HALF, u32x4_t{a0, a1, a2, a3});
         }
     }
 }
-template <int NUM, int HALF, bool MX, typename Emit>
+template <int NUM, int HALF, typename Emit>
 __device__ __forceinline__ void decode_q4_k(half4_t ident, const uint8_t* row, int g, Emit&& emit) {
     typedef Num<NUM> A;
     const u32x4_t head = *reinterpret_cast<const u32x4_t*>(row);  // d, dmin, 12 scale bytes
     typename A::T Ds[4], DMs[4];
     const bool fused = q4k_pairs<NUM, HALF>(head, g, Ds, DMs);
-    if constexpr (!MX) decode_q4_k_body<NUM, HALF, NUM == SNGGUF_NUM_GGML_FP32, false>(ident, row, g, Ds, DMs, emit);
-    else if (fused) decode_q4_k_body<NUM, HALF, true, true>(ident, row, g, Ds, DMs, emit);
-    else decode_q4_k_body<NUM, HALF, false, true>(ident, row, g, Ds, DMs, emit);
+    if (fused) decode_q4_k_body<NUM, HALF, true>(ident, row, g, Ds, DMs, emit);
+    else decode_q4_k_body<NUM, HALF, false>(ident, row, g, Ds, DMs, emit);
 }
 
 // Q5_K: as Q4_K, the fifth bit of element l of sub-block j is bit j of qh[l]
-template <int NUM, int HALF, bool FUSED, bool MX, typename Emit>
+template <int NUM, int HALF, bool FUSED, typename Emit>
 __device__ __forceinline__ void decode_q5_k_body(half4_t ident, const uint8_t* row, int g, const typename Num<NUM>::T (&Ds)[4],
                                                  const typename Num<NUM>::T (&DMs)[4], Emit&& emit) {
     const u32x2_t qh = *reinterpret_cast<const u32x2_t*>(row + 16 + 8 * g);
@@ -353,24 +352,23 @@ __device__ __forceinline__ void decode_q5_k_body(half4_t ident, const uint8_t* r
             for (int w = 0; w < 2; w++) {
                 const uint32_t lo = (hi ? qs[w] >> 4 : qs[w]) & 0x0F0F0F0Fu;
                 const uint32_t hb = ((qh[w] >> j) & 0x01010101u) << 4;
-                kq_dword_bf16<NUM, true, FUSED, MX>(ident, lo | hb, 0.f, D, DM, a[2 * w], a[2 * w + 1]);
+                kq_dword_bf16<NUM, true, FUSED, true>(ident, lo | hb, 0.f, D, DM, a[2 * w], a[2 * w + 1]);
             }
             emit(j - 4 * HALF, u32x4_t{a[0], a[1], a[2], a[3]});
         }
     }
 }
-template <int NUM, int HALF, bool MX, typename Emit>
+template <int NUM, int HALF, typename Emit>
 __device__ __forceinline__ void decode_q5_k(half4_t ident, const uint8_t* row, int g, Emit&& emit) {
     typedef Num<NUM> A;
     const u32x4_t head = *reinterpret_cast<const u32x4_t*>(row);  // d, dmin, 12 scale bytes
     typename A::T Ds[4], DMs[4];
     const bool fused = q4k_pairs<NUM, HALF>(head, g, Ds, DMs);
-    if constexpr (!MX) decode_q5_k_body<NUM, HALF, NUM == SNGGUF_NUM_GGML_FP32, false>(ident, row, g, Ds, DMs, emit);
-    else if (fused) decode_q5_k_body<NUM, HALF, true, true>(ident, row, g, Ds, DMs, emit);
-    else decode_q5_k_body<NUM, HALF, false, true>(ident, row, g, Ds, DMs, emit);
+    if (fused) decode_q5_k_body<NUM, HALF, true>(ident, row, g, Ds, DMs, emit);
+    else decode_q5_k_body<NUM, HALF, false>(ident, row, g, Ds, DMs, emit);
 }
 
-template <int NUM, int HALF, bool MX, typename Emit>
+template <int NUM, int HALF, typename Emit>
 __device__ __forceinline__ void decode_q6_k(half4_t ident, const uint8_t* row, int g, Emit&& emit) {
     typedef Num<NUM> A;
     constexpr int h = HALF;  // 128-element half of the super-block = sub-blocks 4 h .. 4 h + 3
@@ -392,7 +390,7 @@ __device__ __forceinline__ void decode_q6_k(half4_t ident, const uint8_t* row, i
             for (int w = 0; w < 2; w++) {
                 const uint32_t lo = (top ? ql[w] >> 4 : ql[w]) & 0x0F0F0F0Fu;
                 const uint32_t hb = ((qh[w] >> (2 * p)) & 0x03030303u) << 4;
-                kq_dword_bf16<NUM, false, false, MX>(ident, lo | hb, 32.f, D, D, a[2 * w], a[2 * w + 1]);
+                kq_dword_bf16<NUM, false, false, true>(ident, lo | hb, 32.f, D, D, a[2 * w], a[2 * w + 1]);
             }
             emit(p, u32x4_t{a[0], a[1], a[2], a[3]});
         }
@@ -400,20 +398,20 @@ __device__ __forceinline__ void decode_q6_k(half4_t ident, const uint8_t* row, i
 }
 
 // One half (sub-blocks 4 HALF .. 4 HALF + 3) of a slab row -> four A operands through `emit(jj, a)`.
-template <int QT, int NUM, int HALF, bool MX = true, typename Emit>
+template <int QT, int NUM, int HALF, typename Emit>
 __device__ __forceinline__ void decode_half(half4_t ident, const uint8_t* row, int g, Emit&& emit) {
-    if constexpr (QT == SNGGUF_TYPE_Q4_0) decode_legacy<NUM, HALF, 18, false, false, MX>(ident, row, g, emit);
-    else if constexpr (QT == SNGGUF_TYPE_Q4_1) decode_legacy<NUM, HALF, 20, true, false, MX>(ident, row, g, emit);
-    else if constexpr (QT == SNGGUF_TYPE_Q5_0) decode_legacy<NUM, HALF, 22, false, true, MX>(ident, row, g, emit);
-    else if constexpr (QT == SNGGUF_TYPE_Q5_1) decode_legacy<NUM, HALF, 24, true, true, MX>(ident, row, g, emit);
+    if constexpr (QT == SNGGUF_TYPE_Q4_0) decode_legacy<NUM, HALF, 18, false, false>(ident, row, g, emit);
+    else if constexpr (QT == SNGGUF_TYPE_Q4_1) decode_legacy<NUM, HALF, 20, true, false>(ident, row, g, emit);
+    else if constexpr (QT == SNGGUF_TYPE_Q5_0) decode_legacy<NUM, HALF, 22, false, true>(ident, row, g, emit);
+    else if constexpr (QT == SNGGUF_TYPE_Q5_1) decode_legacy<NUM, HALF, 24, true, true>(ident, row, g, emit);
     else if constexpr (QT == SNGGUF_TYPE_Q8_0) decode_q8_0<NUM, HALF>(row, g, emit);
-    else if constexpr (QT == SNGGUF_TYPE_Q2_K) decode_q2_k<NUM, HALF, MX>(ident, row, g, emit);
-    else if constexpr (QT == SNGGUF_TYPE_Q3_K) decode_q3_k<NUM, HALF, MX>(ident, row, g, emit);
-    else if constexpr (QT == SNGGUF_TYPE_Q4_K) decode_q4_k<NUM, HALF, MX>(ident, row, g, emit);
-    else if constexpr (QT == SNGGUF_TYPE_Q5_K) decode_q5_k<NUM, HALF, MX>(ident, row, g, emit);
+    else if constexpr (QT == SNGGUF_TYPE_Q2_K) decode_q2_k<NUM, HALF>(ident, row, g, emit);
+    else if constexpr (QT == SNGGUF_TYPE_Q3_K) decode_q3_k<NUM, HALF>(ident, row, g, emit);
+    else if constexpr (QT == SNGGUF_TYPE_Q4_K) decode_q4_k<NUM, HALF>(ident, row, g, emit);
+    else if constexpr (QT == SNGGUF_TYPE_Q5_K) decode_q5_k<NUM, HALF>(ident, row, g, emit);
     else {
         static_assert(QT == SNGGUF_TYPE_Q6_K, "no matrix-core decoder for this quant type");
-        decode_q6_k<NUM, HALF, MX>(ident, row, g, emit);
+        decode_q6_k<NUM, HALF>(ident, row, g, emit);
     }
 }
 
