@@ -160,11 +160,14 @@ double decode_kernel_us(int qtype, int64_t M, int64_t N, int64_t K) {
     return 3.7 + (double)((groups + 255) / 256 * (K / 256)) * step + (double)N * (double)K * element * 0.08e-6;
 }
 
-// Between the decode kernels' 64 rows and a few hundred, a matrix with few 256 x 256 output tiles keeps only a few
-// compute units busy in the tile kernels, each for K / 64 steps of about 1.6 us, while the decode kernel streams the
-// whole matrix in 10 us + N K / 1.25e12 s per 64 rows (64 rows, Q8_0 / Q4_K / Q6_K: 12288 x 4096 44 / 42 / 45 us, which the
-// line puts at 50, 4096 x 4096 19 / 18 / 19, 1024 x 4096 19 / 18 / 19, 4096 x 12288 49 / 47 / 50) and less for a short last chunk.  Row chunks through the decode kernel win where the sum of those stays below the tile kernel's time:
-// 4096 x 12288 at 128 rows 102 against 292 us, 4096 x 4096 41 against 102 us; 12288 x 4096 only up to 65 rows or so.
+// Between the decode kernels' 64 rows and a few hundred, without a workspace: a matrix with few 256 x 256 output tiles keeps only a
+// few compute units busy in the tile kernels, each for K / 64 steps of about 1.6 us, while the decode kernel streams the whole matrix
+// in 10 us + N K / 1.25e12 s per 64 rows (64 rows, Q8_0 / Q4_K / Q6_K: 12288 x 4096 44 / 42 / 45 us, which the line puts at 50, 4096 x
+// 4096 19 / 18 / 19, 1024 x 4096 19 / 18 / 19, 4096 x 12288 49 / 47 / 50) and less for a short last chunk.  Row chunks win where the
+// sum of those stays below the tile kernel's time: 4096 x 12288 at 128 rows 102 against 292 us, 4096 x 4096 41 against 102 us;
+// 12288 x 4096 only up to 65 rows or so.  (A chunk runs on the mid-size kernel where that is faster, 64 rows of 4096 x 12288 with
+// scratch 22 - 27 us, so a chunk takes this long at most and the line keeps to the tile kernel longer than it has to; with a
+// workspace, sngguf_linear_ws does not come here.)
 // (Chunks start at multiples of 64 rows, so x, y and the residual keep their 16-byte alignment.)
 bool row_chunks_win(int64_t M, int64_t N, int64_t K, int qtype) {
     if (K % 256 != 0 || M > 512) return false;

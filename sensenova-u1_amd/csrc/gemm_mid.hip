@@ -2,10 +2,13 @@
 // operands in registers, each decoded once per tile of up to 256 activation rows; no weight pass, and no decoded weight in LDS.
 //
 // Eight wavefronts share one tile of activations; each owns 16 or 32 weight rows and (with KW = 2) one half of the
-// workgroup's K range.  Three forms (launch_gemm_mid picks by the model in gemm_mid_plan.hip):
-//   narrow  16 rows per wavefront, two halves of K:  64 columns per workgroup, two workgroups per compute unit, up to 64 rows
+// workgroup's K range.  Three forms (mid_plan in gemm_mid_plan.hip picks):
+//   narrow  16 rows per wavefront, two halves of K:  64 columns per workgroup, up to 64 rows, two workgroups per compute unit
+//           (one with 64 rows in Q8_0 and Q6_K, whose slabs are the widest)
 //   wide    32 rows per wavefront, two halves of K: 128 columns, up to 208 rows
 //   long    32 rows per wavefront, all of K:        256 columns, up to 256 rows
+// (wide ends at 208 rows because its registers do: 224 - 256 of 256 are taken there, and Q8_0 already spills 7 of them, the only
+// instance of any format that spills.  From 209 rows on two row tiles, or the long form, take 15 - 18 % longer than 208 rows.)
 // What bounds it: up to about 64 rows the latency of a step (packed bytes -> slab -> decode -> matrix instructions, which two
 // wavefronts a SIMD hide only partly), beyond that the issue slots of the SIMD, which matrix instructions and the decode's 3.5 - 4
 // vector instructions per weight share (16x16x32 instructions alone take 3.3 us per super-block of 256 columns and 208 rows, the
@@ -260,8 +263,9 @@ template <int NUM> struct Sub<SNGGUF_TYPE_Q6_K, NUM> {
     }
 };
 
-// 64-wide tiles of the activations in a stage: two (half as many barriers) up to 64 rows.  (64 rows in the narrow form then
-// leave room for one workgroup on a compute unit; with one tile and two workgroups 4096 x 12288 takes 27.0 against 24.7 us.)
+// 64-wide tiles of the activations in a stage: two (half as many barriers) up to 64 rows.  (64 rows in the narrow form: 64 KB of
+// activations and eight slabs, 82 KB in all for Q8_0 and Q6_K, which leaves room for one workgroup on a compute unit, 74 - 78 KB and
+// two for the others; Q8_0 with one tile and two workgroups takes 27.0 against 24.7 us for 4096 x 12288.)
 constexpr int mid_tiles(int mt) { return mt <= 4 ? 2 : 1; }
 
 template <int QT, int R, int MT, int KW>

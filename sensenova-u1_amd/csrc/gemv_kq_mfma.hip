@@ -502,6 +502,8 @@ constexpr int kMlpKqWaves = 12;
 #define SNGGUF_MLPKQ_AHEAD 1
 #endif
 constexpr int kMlpKqSteps = 4;   // super-blocks of the down matrix per wavefront: inter = 12 x 4 x 256 (the launcher checks)
+constexpr int kMlpKqHidden = 4096, kMlpKqRows = 2;   // the only hidden size and the most rows (mlp_kq_decode_fits)
+static_assert(kMlpKqHidden / 8 <= 64 * kMlpKqWaves, "a thread stages at most 16 bytes of an activation row");
 
 template <int QA, int QB>
 struct MlpKqLds {
@@ -556,7 +558,8 @@ __global__ __launch_bounds__(64 * kMlpKqWaves) void mlp_kq_decode_kernel(const b
     uint16_t pre_ad = 0;
     if (tid < 16) cnt[tid] = 0;
     // the activations, staged once for the workgroup (normalized if gamma is given): a thread keeps its 16 bytes of each row
-    // in registers across the sum of squares, and gamma's are on their way with them (hidden <= 8 x 768, M <= 2: the fits rule)
+    // in registers across the sum of squares, and gamma's are on their way with them (one piece per thread and row: kMlpKqHidden,
+    // kMlpKqRows)
     {
         const bool mine = tid < (int)(hidden >> 3);
         u32x4_t xv0 = {}, xv1 = {}, gv = {};
@@ -795,7 +798,7 @@ int launch_mlp_kq(const void* x, int M, const void* gamma, float eps, const void
 // one or two rows, one resident workgroup per compute unit.
 bool mlp_kq_decode_fits(int qtype_gate_up, int qtype_down, int64_t M, int64_t hidden, int64_t inter) {
     if (qtype_gate_up != SNGGUF_TYPE_Q4_K || (qtype_down != SNGGUF_TYPE_Q6_K && qtype_down != SNGGUF_TYPE_Q4_K)) return false;
-    if (M < 1 || M > 2 || hidden != 4096 || inter != 12 * kMlpKqSteps * 256) return false;
+    if (M < 1 || M > kMlpKqRows || hidden != kMlpKqHidden || inter != kMlpKqWaves * kMlpKqSteps * 256) return false;
     static const int cus = [] {
         int dev = 0, n = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess) return 0;
