@@ -50,6 +50,25 @@ def test_both_dense_kernels_agree_and_match_the_oracle(dev, m, n, k):
         assert torch.equal(got_r, res.to(dev) + y)
 
 
+@pytest.mark.parametrize("qt,m,n,k,copies", [(go.Q8_0, 65, 264, 1088, 4), (go.Q8_0, 511, 1032, 448, 3), (go.Q4_0, 300, 520, 576, 2),
+                                             (go.Q5_1, 203, 136, 1600, 5), (go.Q4_K, 2100, 264, 512, 2), (go.Q6_K, 2100, 136, 768, 3), (go.Q2_K, 2500, 515, 1024, 4)])
+def test_k_split_of_the_tile_kernels(dev, qt, m, n, k, copies):
+    """The tile kernels' own K split, where the mid-size kernel does not take a projection (K not whole super-blocks, 2048 rows and
+    more): with the decode in the loop (Q8_0, Q4_K) and behind a weight pass."""
+    print(f"case split tiles qt={qt} {m}x{n}x{k}", flush=True)
+    nbytes = ops.linear_ws_bytes(qt, m, n, k)
+    assert ops.mid_plan(qt, m, n, k, False, nbytes) is None
+    assert nbytes == copies * 4 * m * n + (0 if qt in (go.Q8_0, go.Q4_K) else 2 * n * k)
+    packed, x = synthetic.make_packed(qt, n, k, seed=n + k, device=dev), synthetic.make_activations(m, k, seed=m, device=dev)
+    bias = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 0.5).to(torch.bfloat16)
+    y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=dev)
+    ops.linear_ws_into(x, packed, qt, bias.to(dev), y, torch.empty(nbytes, dtype=torch.uint8, device=dev), 1)
+    rows = torch.randperm(m, generator=torch.Generator().manual_seed(1))[:48]
+    rows[0], rows[1] = 0, m - 1
+    assert bool(torch.isfinite(y.float()).all())
+    assert go.rel_l2(y[rows.to(dev)].cpu(), go.gguf_linear_forward(x[rows.to(dev)].cpu(), packed.cpu(), qt, bias)) <= TOL
+
+
 @pytest.mark.parametrize("m,n,k", [(128, 4096, 12288), (512, 1024, 4096), (96, 512, 2048)])
 def test_k_split_partial_sums_of_the_workspace_route(dev, m, n, k):
     """Few output tiles: the workspace route cuts K over workgroups, the slices go out as fp32 partial sums and a

@@ -1,7 +1,8 @@
 """GPU: the SiLU-gated pair over a few hundred rows - both matrices in one launch with K split over workgroups, the
 reduction ending in the gated product - against the oracle (rel-L2 <= 1e-3: bf16 outputs, decoded weights the same bits)
-and against the two projections and the product as bf16 tensors.  Sizes around the 256 x 256 tile, one and several K
-slices, and a workspace with room for exactly one copy of the sums and for none (the dense gated launch); the form of
+and against the two projections and the product as bf16 tensors.  K in whole super-blocks of 256 runs on the mid-size kernel
+below 2048 rows, everything else on the tile kernels.  Sizes around the 256 x 256 tile, one and several K
+slices, and a workspace with room for exactly one copy of the sums and for none; the form of
 17 .. 64 rows, scratch sizes, and what hangs on the projections' calls."""
 import threading
 
@@ -70,6 +71,38 @@ def test_infinite_and_huge_gates(dev, c_oracle):
     fin = torch.isfinite(want.float())
     assert torch.equal(torch.signbit(h[:3][fin[:3]].float()), torch.signbit(want[:3][fin[:3]].float()))
     assert go.rel_l2(torch.where(fin, h.float(), 0.0), torch.where(fin, want.float(), 0.0)) <= 1e-3
+
+
+@pytest.mark.parametrize("num", [0, 1])
+@pytest.mark.parametrize("qt,m,n,k,copies", [(go.Q8_0, 65, 8, 1152, 9), (go.Q8_0, 256, 264, 640, 1), (go.Q8_0, 257, 248, 1408, 2),
+                                             (go.Q8_0, 100, 2056, 2176, 4), (go.Q8_0, 511, 520, 1152, 2), (go.Q4_K, 2100, 264, 512, 2), (go.Q8_0, 3000, 72, 768, 3)])
+def test_pair_on_the_split_tile_launch(dev, c_oracle, qt, num, m, n, k, copies):
+    """Where the mid-size kernel does not take a pair - K in half super-blocks, 2048 rows and more - the tile kernel's own split
+    launch, one slice and several."""
+    print(f"case gated split tiles qt={qt} num={num} {m}x{n}x{k}", flush=True)
+    nbytes = copies * 8 * m * n
+    assert ops.mid_plan(qt, m, n, k, True, nbytes) is None
+    h, g, u = _run(dev, qt, m, n, k, num, ws_bytes=nbytes)
+    assert go.rel_l2(h, c_oracle.silu_mul(g, u)) <= 1e-3
+
+
+@pytest.mark.parametrize("k", [384, 640])
+def test_infinite_and_huge_gates_on_the_split_tile_launch(dev, c_oracle, k):
+    qt, m, n = go.Q8_0, 130, 256
+    assert ops.mid_plan(qt, m, n, k, True, 64 << 20) is None
+    gate = synthetic.make_packed(qt, n, k, seed=71)
+    gate[:64, 0:2] = torch.tensor([100.0], dtype=torch.float16).view(torch.uint8)
+    x = synthetic.make_activations(m, k, seed=5)
+    x[:3] = 0
+    x[0, 0], x[1, 0], x[2, 0] = 1e38, -1e38, 1e30
+    h, g, u = _run(dev, qt, m, n, k, x=x, gate=gate, ws_bytes=8 * m * n)
+    want = c_oracle.silu_mul(g, u)
+    assert bool(torch.isnan(want.float()).any()) and bool(torch.isinf(want.float()).any())
+    assert torch.equal(torch.isnan(h.float()), torch.isnan(want.float()))
+    inf = torch.isinf(want.float())
+    assert torch.equal(torch.isinf(h.float()), inf) and torch.equal(h[inf], want[inf])
+    fin = torch.isfinite(want.float())
+    assert torch.equal(torch.signbit(h[:3][fin[:3]].float()), torch.signbit(want[:3][fin[:3]].float()))
 
 
 @pytest.mark.parametrize("qt,m", [(go.Q4_K, 65), (go.Q8_0, 203), (go.Q8_0, 511)])

@@ -50,6 +50,14 @@ def test_gated_pair_on_the_dense_tile_kernel(dev, c_oracle, qt, m, n, k, num):
     _against_two_projections(dev, c_oracle, qt, m, n, k, num)
 
 
+@pytest.mark.parametrize("qt,m,n,k", [(go.Q6_K, 2049, 72, 512), (go.Q3_K, 2050, 264, 256), (go.Q4_0, 300, 520, 384), (go.Q5_1, 1000, 136, 640)])
+@pytest.mark.parametrize("num", [ops.NUM_GGML_FP32, ops.NUM_UPSTREAM_FP16])
+def test_gated_pair_where_nothing_else_takes_it(dev, c_oracle, qt, m, n, k, num):
+    """The dense launch below 4096 rows: neither the mid-size kernel (K in half super-blocks, 2048 rows and more) nor a K split."""
+    assert ops.mid_plan(qt, m, n, k, True, ops.gate_up_silu_workspace_bytes(n, k)) is None
+    _against_two_projections(dev, c_oracle, qt, m, n, k, num)
+
+
 def _against_two_projections(dev, c_oracle, qt, m, n, k, num):
     print(f"case gated tiles qt={qt} {m}x{n}x{k} num={num}", flush=True)
     gate, up, x = _pair(dev, qt, m, n, k, seed=11 * n + k)

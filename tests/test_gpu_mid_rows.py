@@ -1,6 +1,6 @@
-"""GPU parity of the kernel for 17 rows to a few thousand (csrc/gemm_mid.hip): every block format, every instance (16-row tiles a
-workgroup holds x columns it covers), K shares that end early, K split over workgroups, ragged rows and columns, bias and
-residual in both epilogues, the gated pair.
+"""GPU parity of the kernel for 17 rows to a few thousand (csrc/gemm_mid.hip): every block format on every instance (16-row tiles a
+workgroup holds x columns it covers), with and without K split over workgroups, each in both numerics modes, as a projection with
+bias and as a gated pair; K shares that end early, ragged rows and columns, the residual.
 
 Bound: the decoded weights are the oracle's bits and the sums are fp32 in another order, so an output differs from the oracle's
 by at most one bf16 step now and then; rel-L2 1e-3 is every output half a step off (2^-9 / sqrt(3))."""
@@ -85,6 +85,66 @@ def test_pair_of_few_columns_in_any_workspace(dev, c_oracle, qt, m, n, k):
         ops.gate_up_silu_ws_into(x, gate, up, qt, h[:m], ws, num, nbytes)
         _check(h[:m, cols.to(dev)].cpu(), want)
         assert bool((ws[nbytes:] == 0xA5).all()) and bool((h[m] == 7.0).all())
+
+
+# (rows, columns, K) -> (columns of a workgroup, 16-row tiles of its instance, row tiles, K slices), the same for all formats
+PROJECTIONS = {
+    (65, 136, 256): (64, 2, 3, 1), (64, 136, 2048): (64, 2, 2, 4), (1000, 520, 256): (64, 3, 21, 1), (700, 136, 2048): (64, 3, 15, 4),
+    (150, 4104, 256): (64, 4, 3, 1), (1500, 136, 2304): (64, 4, 24, 3), (203, 4104, 1280): (128, 2, 7, 1), (1000, 1032, 1280): (128, 3, 21, 1),
+    (1500, 1032, 1280): (128, 4, 24, 1), (65, 16392, 256): (128, 6, 1, 1), (65, 8200, 2304): (128, 6, 1, 3), (100, 16392, 256): (128, 8, 1, 1),
+    (1000, 1032, 2304): (128, 8, 8, 3), (130, 16392, 512): (128, 10, 1, 1), (1000, 1032, 2048): (128, 10, 7, 4), (203, 16392, 512): (128, 13, 1, 1),
+    (130, 16392, 256): (256, 10, 1, 1), (100, 16392, 2304): (256, 10, 1, 3), (509, 16392, 1280): (256, 13, 3, 1), (203, 16392, 2304): (256, 13, 1, 3),
+    (209, 16392, 2048): (256, 16, 1, 3)}
+PAIRS = {
+    (17, 136, 256): (64, 2, 1, 1), (17, 136, 2048): (64, 2, 1, 4), (1000, 264, 256): (64, 3, 21, 1), (400, 136, 2048): (64, 3, 9, 4),
+    (1500, 264, 256): (64, 4, 24, 1), (509, 264, 2304): (64, 4, 8, 3), (203, 2056, 1280): (128, 2, 7, 1), (1000, 520, 1280): (128, 3, 21, 1),
+    (1500, 520, 1280): (128, 4, 24, 1), (65, 8200, 256): (128, 6, 1, 1), (65, 4104, 2304): (128, 6, 1, 3), (100, 8200, 256): (128, 8, 1, 1),
+    (100, 4104, 2304): (128, 8, 1, 3), (130, 8200, 512): (128, 10, 1, 1), (150, 4104, 2304): (128, 10, 1, 3), (509, 4104, 512): (128, 13, 3, 1),
+    (130, 8200, 256): (256, 10, 1, 1), (100, 8200, 2304): (256, 10, 1, 3), (203, 16392, 256): (256, 13, 1, 1), (203, 8200, 2304): (256, 13, 1, 3),
+    (209, 16392, 256): (256, 16, 1, 1), (209, 8200, 2048): (256, 16, 1, 3)}
+
+
+def workspace_bytes(qt, m, n, k, pair):
+    if pair:
+        return ops.gate_up_silu_ws_bytes(qt, m, n, k)
+    return ops.load_library().sngguf_linear_scratch_bytes(qt, m, n, k) if m <= 64 else ops.linear_ws_bytes(qt, m, n, k)
+
+
+@pytest.mark.parametrize("qt", TYPES)
+@pytest.mark.parametrize("m,n,k", PROJECTIONS)
+def test_projection_on_each_instance(dev, qt, m, n, k):
+    num = (TYPES.index(qt) + list(PROJECTIONS).index((m, n, k))) & 1
+    print(f"case mid projection qt={qt} num={num} {m}x{n}x{k}", flush=True)
+    nbytes = workspace_bytes(qt, m, n, k, False)
+    assert ops.mid_plan(qt, m, n, k, False, nbytes) == PROJECTIONS[m, n, k]
+    packed, x = synthetic.make_packed(qt, n, k, seed=n, device=dev), synthetic.make_activations(m, k, seed=m, device=dev)
+    bias = (torch.randn(n, generator=torch.Generator().manual_seed(k)) * 0.5).to(torch.bfloat16).to(dev)
+    ws = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device=dev)
+    y = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=dev)
+    call = ops.load_library().sngguf_linear_scratch if m <= 64 else ops.load_library().sngguf_linear_ws
+    args = (x.data_ptr(), m, packed.data_ptr(), qt, n, k, bias.data_ptr())
+    assert call(*args, *((None,) if m <= 64 else ()), y.data_ptr(), ws.data_ptr(), nbytes, num, ops._stream(dev)) == 0
+    cols = _columns(n, m)
+    _check(y[:m, cols.to(dev)].cpu(), go.gguf_linear_forward(x.cpu(), packed[cols.to(dev)].cpu(), qt, bias.cpu()[cols], numerics=num))
+    assert bool((ws[nbytes:] == 0xA5).all()) and bool((y[m] == 7.0).all())
+
+
+@pytest.mark.parametrize("qt", TYPES)
+@pytest.mark.parametrize("m,n,k", PAIRS)
+def test_pair_on_each_instance(dev, c_oracle, qt, m, n, k):
+    num = (TYPES.index(qt) + list(PAIRS).index((m, n, k))) & 1
+    print(f"case mid pair instance qt={qt} num={num} {m}x{n}x{k}", flush=True)
+    nbytes = workspace_bytes(qt, m, n, k, True)
+    assert ops.mid_plan(qt, m, n, k, True, nbytes) == PAIRS[m, n, k]
+    gate, up = (synthetic.make_packed(qt, n, k, seed=n + j, device=dev) for j in (0, 1))
+    x = synthetic.make_activations(m, k, seed=m, device=dev)
+    ws = torch.full((nbytes + 64,), 0xA5, dtype=torch.uint8, device=dev)
+    h = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=dev)
+    ops.gate_up_silu_ws_into(x, gate, up, qt, h[:m], ws, num, nbytes)
+    cols = _columns(n, m)
+    g, u = (go.gguf_linear_forward(x.cpu(), w[cols.to(dev)].cpu(), qt, numerics=num) for w in (gate, up))
+    _check(h[:m, cols.to(dev)].cpu(), c_oracle.silu_mul(g, u))
+    assert bool((ws[nbytes:] == 0xA5).all()) and bool((h[m] == 7.0).all())
 
 
 @pytest.mark.parametrize("qt", [go.Q8_0, go.Q4_K, go.Q3_K, go.Q6_K])

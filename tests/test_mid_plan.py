@@ -3,6 +3,7 @@ nothing elsewhere."""
 import pytest
 
 from sensenova_u1_amd import ops
+from tests.test_gpu_mid_rows import INSTANCES, PAIRS, PROJECTIONS, workspace_bytes
 
 TYPES = [ops.Q4_0, ops.Q4_1, ops.Q5_0, ops.Q5_1, ops.Q8_0, ops.Q2_K, ops.Q3_K, ops.Q4_K, ops.Q5_K, ops.Q6_K]
 
@@ -65,3 +66,17 @@ def test_projections_on_the_mid_size_kernel():
             assert ops.mid_plan(qt, m, n, k, False, 1 << 40) is not None
     assert ops.mid_plan(ops.Q8_0, 1024, 12288, 4096, False, 1 << 40) is not None
     assert ops.mid_plan(ops.Q8_0, 2048, 12288, 4096, False, 1 << 40) is None and ops.mid_plan(ops.BF16, 40, 4096, 4096, False, 1 << 30) is None
+
+
+FORMS = {64: (2, 3, 4), 128: (2, 3, 4, 6, 8, 10, 13), 256: (10, 13, 16)}   # columns of a workgroup: 16-row tiles of its instances
+
+
+@pytest.mark.parametrize("qt", TYPES)
+@pytest.mark.parametrize("pair,shapes", [(False, PROJECTIONS), (True, PAIRS)])
+def test_the_parity_tests_run_every_instance(qt, pair, shapes):
+    """What the shapes of the parity tests are listed for: all thirteen instances, with and without a K split in each form."""
+    assert {s: ops.mid_plan(qt, *s, pair, workspace_bytes(qt, *s, pair)) for s in shapes} == shapes
+    assert {p[:2] for p in shapes.values()} == {(cols, mt) for cols in FORMS for mt in FORMS[cols]}
+    assert {(p[0], p[3] > 1) for p in shapes.values()} == {(cols, split) for cols in FORMS for split in (False, True)}
+    enough = lambda m, n, k: ops.gate_up_silu_workspace_bytes(n, k) + 2 * m * n
+    assert len({ops.mid_plan(qt, *s, True, enough(*s))[:2] for s in INSTANCES}) == 13
