@@ -184,18 +184,35 @@ bool row_chunks_win(int64_t M, int64_t N, int64_t K, int qtype) {
 
 constexpr int64_t kSplitBytes = (int64_t)64 << 20;   // the most fp32 partial sums a K split of a projection writes
 
-// 17 .. 64 rows: the mid-size kernel, with its K split as far as the scratch goes, or the decode kernel; 0 bytes where that one is
-// faster or no split pays.
+// 17 .. 64 rows of a projection, or of a pair: the mid-size kernel's plan with as much room for a K split as the shape can use
+// (`most` bytes of partial sums, `copy` bytes each), and whether that split pays against the decode kernel's `other_us`.
+struct RowsPlan {
+    sngguf::MidPlan full;
+    bool split;
+    int64_t copy;
+    double other_us;
+
+    int64_t bytes() const { return split ? full.slices * copy : 0; }
+    // The plan with `room` bytes (more than bytes() changes nothing); form -1: the decode kernel.
+    sngguf::MidPlan with(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t room) const {
+        const bool as_asked = split ? room >= bytes() : full.slices == 1;
+        sngguf::MidPlan plan = as_asked ? full : sngguf::mid_plan(qtype, M, N, K, pair, split ? room / copy : 0);
+        if (plan.us > other_us) plan.form = -1;
+        return plan;
+    }
+};
+RowsPlan plan_rows(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t most) {
+    const int64_t copy = (pair ? 8 : 4) * M * N;
+    const sngguf::MidPlan full = sngguf::mid_plan(qtype, M, N, K, pair, most / copy);
+    const double other_us = (pair ? 2.0 : 1.0) * decode_kernel_us(qtype, M, N, K);
+    return {full, full.slices > 1 && full.us <= other_us, copy, other_us};
+}
 sngguf::MidPlan rows_plan(int qtype, int64_t M, int64_t N, int64_t K, int64_t scratch_bytes) {
-    sngguf::MidPlan plan{-1, 0, 0, 0, 1, 1e30};
-    if (M > 64 || !sngguf::mid_fits(qtype, M, N, K)) return plan;
-    plan = sngguf::mid_plan(qtype, M, N, K, false, (scratch_bytes < kSplitBytes ? scratch_bytes : kSplitBytes) / (4 * M * N));
-    if (plan.us > decode_kernel_us(qtype, M, N, K)) plan.form = -1;
-    return plan;
+    if (M > 64 || !sngguf::mid_fits(qtype, M, N, K)) return {-1, 0, 0, 0, 1, 1e30};
+    return plan_rows(qtype, M, N, K, false, kSplitBytes).with(qtype, M, N, K, false, scratch_bytes);
 }
 int64_t rows_scratch_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
-    const sngguf::MidPlan plan = rows_plan(qtype, M, N, K, kSplitBytes);
-    return plan.form >= 0 && plan.slices > 1 ? plan.slices * 4 * M * N : 0;
+    return M > 64 || !sngguf::mid_fits(qtype, M, N, K) ? 0 : plan_rows(qtype, M, N, K, false, kSplitBytes).bytes();
 }
 int rows_impl(const void* x, int64_t M, const void* q, int qtype, int64_t N, int64_t K, const void* bias, const void* residual, void* y,
               void* scratch, int64_t scratch_bytes, int numerics, hipStream_t s) {
@@ -382,15 +399,16 @@ double workspace_route_us(const LinearSplit& f, int qtype, int64_t M, int64_t N,
     return us;
 }
 
-// The plan for a projection from 65 rows on with `workspace_bytes` for partial sums; form -1 where the route above is faster.
+// The plan for a projection from 65 rows on with `workspace_bytes` for partial sums; form -1 where the route above is faster.  `slices`
+// of it are those that the shape has a use for with any room, whether or not it is the faster one.
 // From 2048 rows on one weight pass pays for eight row tiles and more (this route / plans, Q8_0, us: 4096 x 4096 1280 rows 71 / 54,
 // 2048 92 / 84, 3000 93 / 105; 12288 x 4096 1280 rows 141 / 124, 2048 196 / 212, 3000 280 / 317).
 sngguf::MidPlan workspace_plan(const LinearSplit& f, int qtype, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
-    sngguf::MidPlan none{-1, 0, 0, 0, 1, 1e30};
-    if (M >= 2048 || !sngguf::mid_fits(qtype, M, N, K)) return none;
+    if (M >= 2048 || !sngguf::mid_fits(qtype, M, N, K)) return {-1, 0, 0, 0, 1, 1e30};
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), most = tiles <= 128 ? kSplitBytes : 2 * N * K;
-    const sngguf::MidPlan plan = sngguf::mid_plan(qtype, M, N, K, false, (workspace_bytes < most ? workspace_bytes : most) / (4 * M * N));
-    return plan.us <= workspace_route_us(f, qtype, M, N, K) ? plan : none;
+    sngguf::MidPlan plan = sngguf::mid_plan(qtype, M, N, K, false, (workspace_bytes < most ? workspace_bytes : most) / (4 * M * N));
+    if (plan.us > workspace_route_us(f, qtype, M, N, K)) plan.form = -1;
+    return plan;
 }
 }  // namespace
 
@@ -400,7 +418,8 @@ int64_t sngguf_linear_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
         return 0;
     const LinearSplit f = linear_split(qtype, M, N, K, INT64_MAX);
     const sngguf::MidPlan plan = workspace_plan(f, qtype, M, N, K, INT64_MAX);
-    if (f.slices >= 2) return f.dense_bytes + (plan.form >= 0 && plan.slices > f.slices ? plan.slices : f.slices) * 4 * M * N;
+    // (room for a plan's slices whether or not it is taken: this much workspace and any more decide alike)
+    if (f.slices >= 2) return f.dense_bytes + (plan.slices > f.slices ? plan.slices : f.slices) * 4 * M * N;
     return qtype == SNGGUF_TYPE_BF16 || row_chunks_win(M, N, K, qtype) ? 0 : 2 * N * K;
 }
 
@@ -542,17 +561,21 @@ int sngguf_gate_up_silu_ws_form(int qtype, int64_t M, int64_t N, int64_t K) {
 }
 
 namespace {
+// (what is asked for stays within the workspace that is enough at any row count)
+RowsPlan decode_pair(int qtype, int64_t M, int64_t N, int64_t K) {
+    const int64_t dense = sngguf_gate_up_silu_workspace_bytes(N, K);
+    return plan_rows(qtype, M, N, K, true, dense < kSplitBytes ? dense : kSplitBytes);
+}
+
 // Bytes of workspace that a pair's form can use: whole fp32 copies of both outputs for a K split (within what the dense form takes),
 // the gate outputs at 17 .. 64 rows, the interleaved weights for the dense form.
 int64_t pair_bytes(PairForm form, int qtype, int64_t M, int64_t N, int64_t K) {
-    const int64_t dense = sngguf_gate_up_silu_workspace_bytes(N, K), copy = 8 * M * N;
     if (form == kPairDecode) {
-        const sngguf::MidPlan plan = sngguf::mid_plan(qtype, M, N, K, true, (dense < kSplitBytes ? dense : kSplitBytes) / copy);
-        const bool split = plan.slices > 1 && plan.us <= 2.0 * decode_kernel_us(qtype, M, N, K);
-        return split ? plan.slices * copy : 2 * M * N;
+        const RowsPlan p = decode_pair(qtype, M, N, K);
+        return p.split ? p.bytes() : 2 * M * N;
     }
-    const int64_t slices = form == kPairSplit ? pair_slices(M, N, K, dense) : 0;
-    return slices >= 1 ? slices * copy : dense;
+    const int64_t dense = sngguf_gate_up_silu_workspace_bytes(N, K), slices = form == kPairSplit ? pair_slices(M, N, K, dense) : 0;
+    return slices >= 1 ? slices * 8 * M * N : dense;
 }
 
 // How a pair runs with `workspace_bytes` (more than pair_bytes changes nothing): `mid` (form >= 0) on the mid-size kernel, else the
@@ -567,11 +590,15 @@ PairRun pair_run(int qtype, int64_t M, int64_t N, int64_t K, int64_t workspace_b
     PairRun run{pair_form(qtype, M, N, K), 0, {-1, 0, 0, 0, 1, 1e30}};
     if (run.form == kPairSplit && workspace_bytes > 0) run.slices = pair_slices(M, N, K, workspace_bytes);
     if (M >= 2048 || !sngguf::mid_fits(qtype, M, N, K)) return run;   // (thousands of rows: the dense launch, 12288 x 4096 at 4096 rows 651 against 736 us)
+    if (run.form == kPairDecode) {
+        // (decode kernel's two launches / here without a K split / with one, Q6_K, us: 1024 x 12288 at 17 rows 44 / 65 / 16.5, at 64 99 /
+        // 65 / 18; 4096 x 12288 at 17 rows 51 / 70 / 38; 1024 x 4096 19.4 / 21.9 / 11.3; 12288 x 4096, no split, 50 / 43)
+        run.mid = decode_pair(qtype, M, N, K).with(qtype, M, N, K, true, workspace_bytes);
+        return run;
+    }
     const int64_t asked = pair_bytes(run.form, qtype, M, N, K);
     const sngguf::MidPlan plan = sngguf::mid_plan(qtype, M, N, K, true, (workspace_bytes < asked ? workspace_bytes : asked) / (8 * M * N));
-    // (17 .. 64 rows, the decode kernel's two launches / here without a K split / with one, Q6_K, us: 1024 x 12288 at 17 rows 44 / 65 /
-    // 16.5, at 64 99 / 65 / 18; 4096 x 12288 at 17 rows 51 / 70 / 38; 1024 x 4096 19.4 / 21.9 / 11.3; 12288 x 4096, no split, 50 / 43)
-    if (plan.us <= (run.form == kPairDecode ? 2.0 * decode_kernel_us(qtype, M, N, K) : pair_us(qtype, M, N, K, run.slices))) run.mid = plan;
+    if (plan.us <= pair_us(qtype, M, N, K, run.slices)) run.mid = plan;
     return run;
 }
 }  // namespace

@@ -68,6 +68,21 @@ def test_projections_on_the_mid_size_kernel():
     assert ops.mid_plan(ops.Q8_0, 2048, 12288, 4096, False, 1 << 40) is None and ops.mid_plan(ops.BF16, 40, 4096, 4096, False, 1 << 30) is None
 
 
+@pytest.mark.parametrize("qt", TYPES)
+@pytest.mark.parametrize("pair", [False, True])
+def test_more_than_what_is_asked_for_changes_nothing(qt, pair):
+    """Which kernel runs and how K is cut is the shape's own, whatever a caller's scratch or a pool has grown to."""
+    for m in (17, 33, 48, 64, 65, 130, 300, 509, 1024, 1500):
+        for n in (8, 512, 515, 1024, 2056, 4096, 6144, 9728, 24576):
+            for k in (256, 1024, 2048, 4096, 12288):
+                nbytes = workspace_bytes(qt, m, n, k, pair)
+                if (nbytes == 0 and m > 64) or (pair and n % 8):
+                    continue
+                plan = ops.mid_plan(qt, m, n, k, pair, nbytes)
+                for more in (nbytes + 16, 2 * nbytes + (32 << 20), 1 << 40):
+                    assert ops.mid_plan(qt, m, n, k, pair, more) == plan, (m, n, k, more)
+
+
 FORMS = {64: (2, 3, 4), 128: (2, 3, 4, 6, 8, 10, 13), 256: (10, 13, 16)}   # columns of a workgroup: 16-row tiles of its instances
 
 
