@@ -450,10 +450,10 @@ int launch_qt(const bf16_t* x, int M, const uint8_t* qa, const uint8_t* qb, int6
 // MB are 10.5 us of memory): the launch is 0 - 5 % ahead of the two separate ones by device and down type (32.3 against 33.9
 // us with a Q6_K down projection once the down projection's first requests are made behind phase A's epilogue instead of in
 // front of it; 31.9 - 32.8 against 32.7 - 33.0 with Q4_K), where the Q8_0 kernel gains 10 %.  Since then, with the norm and
-// Q6_K, one row: 34.2 -> 32.4 us, of which the staging without LDS round trips is 2 us less ahead of the first decoded
-// super-block, and the falling priorities 1.5 less at the ends of both phases.  Two or four super-blocks requested ahead
-// instead of one, both halves of a super-block decoded as one block, and Q4_K's quants taken as pairs with two instructions
-// in eight fewer change nothing.
+// Q6_K, one row, in a kernel trace of decode passes: 36.2 -> 33.7 us at best, 36.9 -> 35.0 in the mean; the staging without LDS round
+// trips brings the first decoded super-block 2 us forward, the falling priorities the ends of both phases 1.5 us.  Two or four
+// super-blocks requested ahead instead of one, both halves of a super-block decoded as one block, and Q4_K's quants taken as
+// pairs with two instructions in eight fewer change nothing.
 template <int QT>
 struct SlabIo {
     typedef Slab<QT> S;
