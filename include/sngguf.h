@@ -290,7 +290,9 @@ int sngguf_gate_up_silu_ws_fits(int qtype, int64_t M, int64_t N, int64_t K);
 int64_t sngguf_gate_up_silu_ws_bytes(int qtype, int64_t M, int64_t N, int64_t K);
 /* The form in which this entry point is faster than two projections, silu and the product, and which M rows of this shape
  * take with sngguf_gate_up_silu_ws_bytes of workspace; SNGGUF_PAIR_SEPARATE where there is none (the entry point still runs
- * every shape that sngguf_gate_up_silu_ws_fits takes). */
+ * every shape that sngguf_gate_up_silu_ws_fits takes).  Beyond 64 rows it weighs the split and the dense launch only: a pair in
+ * another format than Q8_0 / Q4_K can be SNGGUF_PAIR_SEPARATE although the launch that decodes packed rows straight into matrix
+ * operands would run it faster (sngguf_mid_plan with `pair` tells whether that one takes it). */
 enum { SNGGUF_PAIR_SEPARATE = 0, SNGGUF_PAIR_DECODE = 1, SNGGUF_PAIR_SPLIT = 2, SNGGUF_PAIR_DENSE = 3 };
 int sngguf_gate_up_silu_ws_form(int qtype, int64_t M, int64_t N, int64_t K);
 int sngguf_gate_up_silu_ws(const void* x, int64_t M, const void* q_gate, const void* q_up, int qtype,
