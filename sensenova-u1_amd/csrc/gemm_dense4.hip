@@ -33,24 +33,6 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const void* p) {
     return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
 }
 
-// exp(-g) for a g with at most 16 significant bits (here: bf16 values)
-__device__ __forceinline__ float exp_neg(float g) {
-    const float e = __builtin_amdgcn_exp2f(g * -1.44268798828125f);               // exact product
-    const float c = __builtin_fmaf(e, g * -4.8884952e-06f, e);                    // x exp2(-g lo), lo ln 2 = 4.8884952e-6
-    return e == 0.f ? 0.f : c;                                                    // (0 x inf at g = +inf)
-}
-
-// g / (1 + exp(-g)): hardware reciprocal, then one correction step of the quotient with the exact remainder
-__device__ __forceinline__ float silu_f32(float g) {
-    const float d = 1.0f + exp_neg(g);
-    const float r = __builtin_amdgcn_rcpf(d);
-    const float q = g * r;
-    const float c = __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q);
-    // exp(-g) overflows below g = -88.7: the quotient is -0 as it stands; at g = +inf the remainder inf - inf is a NaN
-    // and the quotient +inf is the value
-    return (d < __builtin_inff() && __builtin_fabsf(g) < __builtin_inff()) ? c : q;
-}
-
 // byte offset of an LDS address within the workgroup's LDS allocation (what M0 and the ds instructions take)
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;

@@ -7,14 +7,17 @@
 //           (one with 64 rows in Q8_0 and Q6_K, whose slabs are the widest)
 //   wide    32 rows per wavefront, two halves of K: 128 columns, up to 208 rows
 //   long    32 rows per wavefront, all of K:        256 columns, up to 256 rows
-// (wide ends at 208 rows because its registers do: 224 - 256 of 256 are taken there, and Q8_0 already spills 7 of them, the only
-// instance of any format that spills.  From 209 rows on two row tiles, or the long form, take 15 - 18 % longer than 208 rows.)
+// (wide ends at 208 rows because its registers do: 230 - 256 of 256 are taken there.  From 209 rows on two row tiles, or the long
+// form, take 15 - 18 % longer than 208 rows.)
 // What bounds it: up to about 64 rows the latency of a step (packed bytes -> slab -> decode -> matrix instructions, which two
-// wavefronts a SIMD hide only partly), beyond that the issue slots of the SIMD, which matrix instructions and the decode's 3.5 - 4
-// vector instructions per weight share (16x16x32 instructions alone take 3.3 us per super-block of 256 columns and 208 rows, the
-// kernel 4.9 - 5.8).  So the loop is written out instruction group by instruction group: two matrix instructions, the
-// activation fragment of four groups later, an eighth of the next sub-block's decode, a scheduling fence.  Left to the
-// compiler's scheduler the fragments are read one instruction ahead (gate / up of 12288 x 4096 at 203 rows 100 us against 69).
+// wavefronts a SIMD hide only partly), beyond that no one unit: a stage of 208 rows keeps the matrix cores busy for half of its
+// cycles, the vector ALU for about as many, and from 500 rows on the clock falls with the power drawn (1.9 GHz of 2.4), so that what
+// counts is work left out rather than cycles.  Leaving out (203 rows, pair of 12288 x 4096 in Q4_K, 67 us) the activations' copies
+// gives 54 us, the packed rows' requests 58, the decode 55, the matrix instructions 52.  So the loop is written out instruction group
+// by instruction group: two matrix instructions, the activation fragment of four groups later, a part of the next sub-block's decode
+// or one request, a scheduling fence.  Left to the compiler's scheduler the fragments are read one instruction ahead (100 us against 69).
+// Measured and not taken: 32x32x16 instructions on groups of 32 rows (12 - 16 % fewer cycles, but up to 5 % more time from 500 rows on:
+// twice the accumulator traffic per product, which the clock pays for), other cache hints on the copies (nontemporal + 10 %).
 //
 // Per wavefront and unit of 128 elements of K: the packed bytes are requested a unit ahead into registers (16-byte pieces,
 // consecutive lanes walking along a row) and put into a slab of the wavefront's own; the decode reads them from there.
@@ -27,6 +30,14 @@
 //   203 rows  pair 65 / 61 (split tiles 84 / 83), 4096 x 12288 41 / 39 / 44 (51 / 50 / 75), 6144 x 4096 31 / 30 / 32 (37 / 37 / 49)
 //   509 rows  pair 114 / 109 (150 / 142), 4096 x 12288 70 / 70 (79 / 79)
 //   1024 rows pair 220 / 220 (dense launch with two weight passes 247 / 232), 4096 x 4096 55 / 56 (68 / 68)
+// Since then, launches back to back (us, before -> now): the requests between the matrix instructions (8 copies and 3 - 5 pieces a stage
+// and wavefront used to be issued in one go behind the barrier), falling priorities, decode without byte permutes and an epilogue that
+// writes whole rows with the hardware's exp2 and reciprocal:
+//   203 rows  pair 68.4 -> 62.6 (Q8_0), 66.9 -> 62.7 (Q4_K), 72.7 -> 68.6 (Q6_K); 6144 x 4096 in Q4_K 30.8 -> 28.9
+//   509 rows  pair 125 -> 117, 6144 x 4096 51.5 -> 48.0, 4096 x 12288 75.4 -> 73.1 (Q8_0)
+//   1024 rows pair 227 -> 210, 6144 x 4096 72 -> 67, 4096 x 4096 57 -> 51.5 (Q4_K), 4096 x 12288 129 -> 127 (Q6_K)
+//   (96-row instances of a single projection with K split lose 3 - 5 %, 12288 x 4096 at 90 rows in Q6_K 35.1 -> 36.6; pairs of the same
+//   rows gain 4 %)
 #include "gemm_mid.hpp"
 
 #include "kq_decode.hpp"
@@ -102,16 +113,56 @@ template <> struct Unit<SNGGUF_TYPE_Q6_K> {   // low and high bits of the half, 
     static __device__ __forceinline__ int src(int h, int p) { return p < 4 ? 64 * h + 16 * p : p < 6 ? 64 + 32 * h + 16 * p : 192; }
 };
 
+// A field of MASK << P bits of every 16-bit half of v, as halves base + field with base = 2^(10 - P): under that exponent the field's
+// lowest bit is worth one, so nothing is shifted down to bit 0.  Shifts and v_bitop3 issue in 2.2 cycles with two wavefronts on a
+// SIMD; v_perm, v_and_or, the packed and the converting instructions in 4.2.
+template <int P, uint32_t MASK>
+__device__ __forceinline__ half2_t field(uint32_t v) {
+    return __builtin_bit_cast(half2_t, (uint32_t)__builtin_amdgcn_bitop3_b32(v, MASK * 0x00010001u << P, (0x6400u - (P << 10)) * 0x00010001u, 0xEA));
+}
+// The same with TOP of w, shifted left by SHIFT (or right), at bit AT above it
+template <int P, uint32_t MASK, uint32_t TOP, int AT, int SHIFT>
+__device__ __forceinline__ half2_t field2(uint32_t v, uint32_t w) {
+    const uint32_t ws = SHIFT > 0 ? w << (SHIFT > 0 ? SHIFT : 0) : w >> (SHIFT < 0 ? -SHIFT : 0);
+    const uint32_t top = __builtin_amdgcn_bitop3_b32(ws, TOP * 0x00010001u << AT, (0x6400u - (P << 10)) * 0x00010001u, 0xEA);
+    return __builtin_bit_cast(half2_t, (uint32_t)__builtin_amdgcn_bitop3_b32(v, MASK * 0x00010001u << P, top, 0xEA));
+}
+
+// Halves base + integer -> the same halves as weights in the rounding chain (fp16: three operations, or two without a minimum) ...
+template <int NUM, bool HAS_MIN>
+__device__ __forceinline__ void chain_pair(half2_t& h, float off, typename Num<NUM>::T D, typename Num<NUM>::T DM) {
+    const _Float16 o = (_Float16)off;
+    h = h - half2_t{o, o};   // whole numbers: exact
+    if constexpr (NUM == SNGGUF_NUM_UPSTREAM_FP16) {
+        h = h * half2_t{D, D};
+        if constexpr (HAS_MIN) h = h - half2_t{DM, DM};
+    }
+}
+// ... and elements 0 .. 3 of these as bf16
+template <int NUM, bool HAS_MIN>
+__device__ __forceinline__ void chain_bf16(half2_t a, half2_t b, typename Num<NUM>::T D, typename Num<NUM>::T DM, uint32_t& p01, uint32_t& p23) {
+    float w[4] = {(float)a[0], (float)b[0], (float)a[1], (float)b[1]};
+    if constexpr (NUM != SNGGUF_NUM_UPSTREAM_FP16) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            w[e] = D * w[e];
+            if constexpr (HAS_MIN) w[e] = w[e] - DM;
+        }
+    }
+    p01 = pack_bf16(w[0], w[1]);
+    p23 = pack_bf16(w[2], w[3]);
+}
+
 // One 32-element sub-block of a slab row for lane group g, in three parts that the K loop places between matrix
-// instructions: the LDS reads (`load`), the sub-block's scale and minimum (`scales`), and its eight quants as two dwords
-// of four unsigned bytes (`quads`).  J: sub-block 0 .. 7 of the 256 elements.
+// instructions: the LDS reads (`load`), the sub-block's scale and minimum (`scales`), and elements 4 W .. 4 W + 3 of the lane's eight
+// (`pairs`: the halves (0, 2) and (1, 3), each base() + the stored unsigned integer).  J: sub-block 0 .. 7 of the 256 elements.
 template <int QT, int NUM> struct Sub;
 
 template <int NUM, int TS, bool HAS_MIN, bool FIVE>
 struct SubLegacy {
     typedef typename Num<NUM>::T V;
     static constexpr bool kMin = HAS_MIN;
-    static constexpr float kZero = HAS_MIN ? 0.f : (FIVE ? 16.f : 8.f);
+    static constexpr int kZero = HAS_MIN ? 0 : (FIVE ? 16 : 8);
     uint32_t hd, fifth;
     u32x2_t qs;
     template <int J> __device__ __forceinline__ void load(const uint8_t* row, int g) {
@@ -127,10 +178,18 @@ struct SubLegacy {
         DM = D;
         if constexpr (HAS_MIN) DM = -Num<NUM>::scale((uint16_t)(hd >> 16));
     }
-    template <int J, int W> __device__ __forceinline__ uint32_t quads(int g) const {
-        uint32_t v = (qs[W] >> (4 * (g >> 1))) & 0x0F0F0F0Fu;
-        if constexpr (FIVE) v |= ((((fifth >> (8 * g + 4 * W)) & 0xFu) * 0x00204081u) & 0x01010101u) << 4;
-        return v;
+    template <int J> static constexpr int base() { return 1024; }
+    template <int J, int W> __device__ __forceinline__ void pairs(int g, half2_t& a, half2_t& b) const {
+        const uint32_t v = qs[W] >> (4 * (g >> 1));
+        if constexpr (FIVE) {
+            // bits 0 .. 3 of this quarter to bit 4 of bytes 0 .. 3
+            const uint32_t bits = (((fifth >> (8 * g + 4 * W)) & 0xFu) * 0x00204081u) & 0x01010101u;
+            a = field2<0, 0xF, 1, 4, 4>(v, bits);
+            b = field2<0, 0xF, 1, 4, -4>(v >> 8, bits);
+        } else {
+            a = field<0, 0xF>(v);
+            b = field<0, 0xF>(v >> 8);
+        }
     }
 };
 template <int NUM> struct Sub<SNGGUF_TYPE_Q4_0, NUM> : SubLegacy<NUM, 18, false, false> {};
@@ -141,7 +200,7 @@ template <int NUM> struct Sub<SNGGUF_TYPE_Q5_1, NUM> : SubLegacy<NUM, 24, true, 
 template <int NUM> struct Sub<SNGGUF_TYPE_Q8_0, NUM> {
     typedef typename Num<NUM>::T V;
     static constexpr bool kMin = false;
-    static constexpr float kZero = 128.f;
+    static constexpr int kZero = 128;
     uint32_t hd;
     u32x2_t qs;
     template <int J> __device__ __forceinline__ void load(const uint8_t* row, int g) {
@@ -151,13 +210,18 @@ template <int NUM> struct Sub<SNGGUF_TYPE_Q8_0, NUM> {
         qs = lds_u64<(jj & 1) == 1>(row + 34 * jj + 2 + 8 * g + (jj == 3 && g == 3 ? 8 : 0));
     }
     template <int J> __device__ __forceinline__ void scales(int, V& D, V& DM) const { DM = D = Num<NUM>::scale((uint16_t)hd); }
-    template <int J, int W> __device__ __forceinline__ uint32_t quads(int) const { return qs[W] ^ 0x80808080u; }
+    template <int J> static constexpr int base() { return 1024; }
+    // (the sign bit of each byte is turned with the mask: stored + 128)
+    template <int J, int W> __device__ __forceinline__ void pairs(int, half2_t& a, half2_t& b) const {
+        a = __builtin_bit_cast(half2_t, (uint32_t)__builtin_amdgcn_bitop3_b32(qs[W], 0x00FF00FFu, 0x64806480u, 0x6A));
+        b = __builtin_bit_cast(half2_t, (uint32_t)__builtin_amdgcn_bitop3_b32(qs[W] >> 8, 0x00FF00FFu, 0x64806480u, 0x6A));
+    }
 };
 
 template <int NUM> struct Sub<SNGGUF_TYPE_Q2_K, NUM> {
     typedef typename Num<NUM>::T V;
     static constexpr bool kMin = true;
-    static constexpr float kZero = 0.f;
+    static constexpr int kZero = 0;
     uint32_t sm, dd;
     u32x2_t qs;
     template <int J> __device__ __forceinline__ void load(const uint8_t* row, int g) {
@@ -170,13 +234,17 @@ template <int NUM> struct Sub<SNGGUF_TYPE_Q2_K, NUM> {
         D = Num<NUM>::scale((uint16_t)(dd & 0xFFFF)) * Num<NUM>::integer((int)(byte & 15u));
         DM = Num<NUM>::scale((uint16_t)(dd >> 16)) * Num<NUM>::integer((int)(byte >> 4));
     }
-    template <int J, int W> __device__ __forceinline__ uint32_t quads(int) const { return (qs[W] >> (2 * (J & 3))) & 0x03030303u; }
+    template <int J> static constexpr int base() { return 1024 >> (2 * (J & 3)); }
+    template <int J, int W> __device__ __forceinline__ void pairs(int, half2_t& a, half2_t& b) const {
+        a = field<2 * (J & 3), 3>(qs[W]);
+        b = field<2 * (J & 3), 3>(qs[W] >> 8);
+    }
 };
 
 template <int NUM> struct Sub<SNGGUF_TYPE_Q3_K, NUM> {
     typedef typename Num<NUM>::T V;
     static constexpr bool kMin = false;
-    static constexpr float kZero = 4.f;
+    static constexpr int kZero = 4;
     u32x4_t t;
     u32x2_t hm, qs;
     template <int J> __device__ __forceinline__ void load(const uint8_t* row, int g) {
@@ -193,16 +261,43 @@ template <int NUM> struct Sub<SNGGUF_TYPE_Q3_K, NUM> {
         const uint32_t hi = ((s2 >> (8 * t3)) >> (2 * (2 * h + (j >> 1)))) & 3u;
         DM = D = Num<NUM>::scale((uint16_t)(t[3] >> 16)) * Num<NUM>::integer((int)(lo | (hi << 4)) - 32);
     }
-    template <int J, int W> __device__ __forceinline__ uint32_t quads(int) const {
-        return ((qs[W] >> (2 * (J & 3))) & 0x03030303u) | (((hm[W] >> J) & 0x01010101u) << 2);
+    template <int J> static constexpr int base() { return 1024 >> (2 * (J & 3)); }
+    template <int J, int W> __device__ __forceinline__ void pairs(int, half2_t& a, half2_t& b) const {
+        constexpr int P = 2 * (J & 3);
+        a = field2<P, 3, 1, P + 2, P + 2 - J>(qs[W], hm[W]);
+        b = field2<P, 3, 1, P + 2, P + 2 - J - 8>(qs[W] >> 8, hm[W]);
     }
 };
+
+// Scale and minimum of sub-block J of a Q4_K or Q5_K head
+template <int J, int NUM>
+__device__ __forceinline__ void q45k_scales(const u32x4_t& head, typename Num<NUM>::T& D, typename Num<NUM>::T& DM) {
+    constexpr int i = 8 * (J & 3);
+    uint32_t sc, mn;
+    if constexpr (J < 4) {
+        sc = (head[1] >> i) & 63u;
+        mn = (head[2] >> i) & 63u;
+    } else {
+        sc = ((head[3] >> i) & 15u) | (((head[1] >> (i + 6)) & 3u) << 4);
+        mn = ((head[3] >> (i + 4)) & 15u) | (((head[2] >> (i + 6)) & 3u) << 4);
+    }
+    if constexpr (NUM == SNGGUF_NUM_UPSTREAM_FP16) {
+        // both products in one packed multiplication; 0x6400 | n is the half 1024 + n
+        const half2_t k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+        const half2_t both = (__builtin_bit_cast(half2_t, (mn << 16) | sc | 0x64006400u) - k1024) * __builtin_bit_cast(half2_t, head[0]);
+        D = both[0];
+        DM = both[1];
+    } else {
+        D = Num<NUM>::scale((uint16_t)(head[0] & 0xFFFF)) * Num<NUM>::integer((int)sc);
+        DM = Num<NUM>::scale((uint16_t)(head[0] >> 16)) * Num<NUM>::integer((int)mn);
+    }
+}
 
 template <int NUM, bool FIVE>
 struct SubQ45K {
     typedef typename Num<NUM>::T V;
     static constexpr bool kMin = true;
-    static constexpr float kZero = 0.f;
+    static constexpr int kZero = 0;
     u32x4_t head;
     u32x2_t qs, qh;
     template <int J> __device__ __forceinline__ void load(const uint8_t* row, int g) {
@@ -210,31 +305,17 @@ struct SubQ45K {
         if constexpr (FIVE) qh = *reinterpret_cast<const u32x2_t*>(row + 16 + 8 * g);
         qs = *reinterpret_cast<const u32x2_t*>(row + (FIVE ? 48 : 16) + 32 * ((J & 3) >> 1) + 8 * g);
     }
-    template <int J> __device__ __forceinline__ void scales(int, V& D, V& DM) const {
-        constexpr int i = 8 * (J & 3);
-        uint32_t sc, mn;
-        if constexpr (J < 4) {
-            sc = (head[1] >> i) & 63u;
-            mn = (head[2] >> i) & 63u;
+    template <int J> __device__ __forceinline__ void scales(int, V& D, V& DM) const { q45k_scales<J, NUM>(head, D, DM); }
+    template <int J> static constexpr int base() { return 1024 >> (4 * (J & 1)); }
+    template <int J, int W> __device__ __forceinline__ void pairs(int, half2_t& a, half2_t& b) const {
+        constexpr int P = 4 * (J & 1);
+        if constexpr (FIVE) {
+            a = field2<P, 0xF, 1, P + 4, P + 4 - J>(qs[W], qh[W]);
+            b = field2<P, 0xF, 1, P + 4, P + 4 - J - 8>(qs[W] >> 8, qh[W]);
         } else {
-            sc = ((head[3] >> i) & 15u) | (((head[1] >> (i + 6)) & 3u) << 4);
-            mn = ((head[3] >> (i + 4)) & 15u) | (((head[2] >> (i + 6)) & 3u) << 4);
+            a = field<P, 0xF>(qs[W]);
+            b = field<P, 0xF>(qs[W] >> 8);
         }
-        if constexpr (NUM == SNGGUF_NUM_UPSTREAM_FP16) {
-            // both products in one packed multiplication; 0x6400 | n is the half 1024 + n
-            const half2_t k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
-            const half2_t both = (__builtin_bit_cast(half2_t, (mn << 16) | sc | 0x64006400u) - k1024) * __builtin_bit_cast(half2_t, head[0]);
-            D = both[0];
-            DM = both[1];
-        } else {
-            D = Num<NUM>::scale((uint16_t)(head[0] & 0xFFFF)) * Num<NUM>::integer((int)sc);
-            DM = Num<NUM>::scale((uint16_t)(head[0] >> 16)) * Num<NUM>::integer((int)mn);
-        }
-    }
-    template <int J, int W> __device__ __forceinline__ uint32_t quads(int) const {
-        uint32_t v = (qs[W] >> (4 * (J & 1))) & 0x0F0F0F0Fu;
-        if constexpr (FIVE) v |= ((qh[W] >> J) & 0x01010101u) << 4;
-        return v;
     }
 };
 template <int NUM> struct Sub<SNGGUF_TYPE_Q4_K, NUM> : SubQ45K<NUM, false> {};
@@ -243,7 +324,7 @@ template <int NUM> struct Sub<SNGGUF_TYPE_Q5_K, NUM> : SubQ45K<NUM, true> {};
 template <int NUM> struct Sub<SNGGUF_TYPE_Q6_K, NUM> {
     typedef typename Num<NUM>::T V;
     static constexpr bool kMin = false;
-    static constexpr float kZero = 32.f;
+    static constexpr int kZero = 32;
     uint32_t sw, d;
     u32x2_t ql, qh;
     template <int J> __device__ __forceinline__ void load(const uint8_t* row, int g) {
@@ -257,9 +338,11 @@ template <int NUM> struct Sub<SNGGUF_TYPE_Q6_K, NUM> {
         const int sc = (int)(int8_t)((sw >> (8 * (2 * (J & 1) + (g >> 1)))) & 0xFF);
         DM = D = Num<NUM>::scale((uint16_t)d) * Num<NUM>::integer(sc);
     }
-    template <int J, int W> __device__ __forceinline__ uint32_t quads(int) const {
-        constexpr int p = J & 3;
-        return ((ql[W] >> (4 * (p >> 1))) & 0x0F0F0F0Fu) | (((qh[W] >> (2 * p)) & 0x03030303u) << 4);
+    template <int J> static constexpr int base() { return 1024 >> (4 * ((J & 3) >> 1)); }
+    template <int J, int W> __device__ __forceinline__ void pairs(int, half2_t& a, half2_t& b) const {
+        constexpr int p = J & 3, P = 4 * (p >> 1);
+        a = field2<P, 0xF, 3, P + 4, P + 4 - 2 * p>(ql[W], qh[W]);
+        b = field2<P, 0xF, 3, P + 4, P + 4 - 2 * p - 8>(ql[W] >> 8, qh[W]);
     }
 };
 
@@ -268,10 +351,14 @@ template <int NUM> struct Sub<SNGGUF_TYPE_Q6_K, NUM> {
 // two for the others; Q8_0 with one tile and two workgroups takes 27.0 against 24.7 us for 4096 x 12288.)
 constexpr int mid_tiles(int mt) { return mt <= 4 ? 2 : 1; }
 
+// Bytes of a row of 32 outputs, and of 32 sums, in LDS behind the loop: odd numbers of 16-byte groups, so that eight rows start in
+// different banks
+constexpr int kOutRow = 80, kTurnRow = 144;
+
 template <int QT, int R, int MT, int KW>
 constexpr int mid_lds_bytes() {
     constexpr int x = 2 * KW * mid_tiles(MT) * 16 * MT * 128, slab = kWaves * 16 * R * Unit<QT>::stride;
-    constexpr int red = KW == 2 ? kWaves * MT * 1024 : kWaves * R * ((MT + 1) / 2) * 1024;
+    constexpr int red = KW == 2 ? kWaves * MT * 1024 : kWaves * MT * 16 * kOutRow;
     return x + slab > red ? x + slab : red;
 }
 
@@ -292,13 +379,16 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     constexpr int kBlocks = 2 * MT;               // blocks of 8 rows (one request of a wavefront) in a tile
     constexpr int kReq = (kBlocks + kWaves - 1) / kWaves;
     constexpr bool kEarly = MT <= 8;              // a sub-block's bytes are read one sub-block ahead of its decode
+    // Copies and requests between the matrix instructions, not in one go; up to 64 rows a stage is short and waits for what it asked
+    // for late (40 rows of 4096 x 12288 in Q8_0 22.5 us in one go, 24.9 spread; 509 of 6144 x 4096 51 and 48).
+    constexpr bool kSpread = MT > 4;
+    static_assert(!kSpread || T == 1, "two stages between a unit's requests and the next unit's");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kw = wave / NW, nw = wave % NW;
     const int r = lane & 15, g = lane >> 4;
-    const half4_t ident = identity_row(lane);
 
     // ---- tile: row tiles of the same columns and K slice next to each other on one XCD (workgroup ids are dealt round-robin
     // over 8), so that they find the packed rows in its L2 ----
@@ -349,13 +439,17 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     uint8_t* slab = lds + 2 * kStage + wave * kRows * S::stride;
     u32x4_t pre[kLoads];
     uint16_t pre_d = 0;
-    // unit h of super-block s of the share (a share that ends early re-reads the slice's last super-block)
-    auto fetch = [&](int s, auto H) {
+    // request i of unit h of super-block s of the share (a share that ends early re-reads the slice's last super-block)
+    constexpr int kFetch = kLoads + (kQ6 ? 1 : 0);
+    auto fetch_req = [&](int s, auto H, int i) {
         constexpr int h = decltype(H)::value;
         const uint8_t* p = base + (int64_t)(my0 + s < sb1 ? my0 + s : sb1 - 1) * kTs;
+        if (i < kLoads) pre[i] = ld_piece<S::align>(p + off[h][i]);
+        else if constexpr (kQ6) pre_d = ld_u16(p + doff);
+    };
+    auto fetch = [&](int s, auto H) {
 #pragma unroll
-        for (int i = 0; i < kLoads; i++) pre[i] = ld_piece<S::align>(p + off[h][i]);
-        if constexpr (kQ6) pre_d = ld_u16(p + doff);
+        for (int i = 0; i < kFetch; i++) fetch_req(s, H, i);
     };
     auto put = [&]() {
 #pragma unroll
@@ -372,24 +466,28 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
         if (gr >= row_end) gr = row_end - 1;
         xoff[i] = (uint32_t)(2 * gr * a.K + 16 * ((lane & 7) ^ ((row >> 1) & 7)));
     }
-    // the tiles of stage st of super-block s of every K share (a shorter last share stays inside the row)
+    // (the last request of a tile that is no multiple of 64 rows is for some wavefronts only: the others make it with no lane
+    // enabled - a branch there would cut the stage into basic blocks, and the decode that belongs between the matrix
+    // instructions of one stage would be moved to the head of the next)
+    const int last_req = __builtin_amdgcn_readfirstlane(wave < kBlocks - kWaves * (kReq - 1) ? -1 : 0);
+    // request q of the tiles of stage st of super-block s of every K share
+    constexpr int kCopies = KW * T * kReq;
+    auto load_x_req = [&](int s, int st, int q) {
+        const int k = q / (T * kReq), t = q / kReq % T, i = q % kReq;
+        int col = (sb0 + k * steps + s) * 512 + 128 * T * st;      // byte column
+        if (KW > 1 && col > xlast) col = xlast;
+        const uint8_t* xb = wave_ptr(reinterpret_cast<const uint8_t*>(a.x) + col + 128 * t);
+        const uint32_t to = lds_addr(lds) + (uint32_t)((st & 1) * kStage + (k * T + t) * kTile + (wave + kWaves * i) * 1024);
+        // (as the dense kernels' copies: M0 holds the destination, one wait state between its write and the request)
+        if (kBlocks % kWaves != 0 && i == kReq - 1)
+            asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
+                         ::"s"(to), "v"(xoff[i]), "s"(xb), "s"(last_req) : "memory", "m0");
+        else
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(xoff[i]), "s"(xb) : "memory", "m0");
+    };
     auto load_x = [&](int s, int st) {
 #pragma unroll
-        for (int k = 0; k < KW; k++) {
-            int col = (sb0 + k * steps + s) * 512 + 128 * T * st;      // byte column
-            if (KW > 1 && col > xlast) col = xlast;
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                const uint8_t* xb = wave_ptr(reinterpret_cast<const uint8_t*>(a.x) + col + 128 * t);
-#pragma unroll
-                for (int i = 0; i < kReq; i++) {
-                    if (kBlocks % kWaves != 0 && i == kReq - 1 && wave >= kBlocks - kWaves * (kReq - 1)) break;
-                    const uint32_t to = lds_addr(lds) + (uint32_t)((st & 1) * kStage + (k * T + t) * kTile + (wave + kWaves * i) * 1024);
-                    // (as the dense kernels' copies: M0 holds the destination, one wait state between its write and the request)
-                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(xoff[i]), "s"(xb) : "memory", "m0");
-                }
-            }
-        }
+        for (int q = 0; q < kCopies; q++) load_x_req(s, st, q);
     };
     int foff[2];
 #pragma unroll
@@ -401,27 +499,33 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
 #pragma unroll
         for (int t = 0; t < MT; t++) acc[rg][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    // ---- decode of a sub-block into operands d: per row group its scales, then two dwords of quants ----
+    // ---- decode of a sub-block into operands d: per row group its LDS reads, then five parts of at most a dozen instructions: scales, and
+    // each dword of four weights in two halves ----
     Sub<QT, NUM> sub[kEarly ? 2 : 1][R];
     typename Num<NUM>::T D[R], DM[R];
+    half2_t ha, hb;
     auto read_part = [&](auto J, int rg) {
         constexpr int j = decltype(J)::value & 7;
         sub[kEarly ? j & 1 : 0][rg].template load<j>(slab + (16 * rg + r) * S::stride, g);
     };
-    auto decode_part = [&](auto J, int c, u32x4_t (&d)[R]) {
-        constexpr int j = decltype(J)::value & 7;
+    auto decode_part = [&](auto J, auto C, u32x4_t (&d)[R]) {
+        constexpr int j = decltype(J)::value & 7, rg = decltype(C)::value / 5, part = decltype(C)::value % 5, w = (part - 1) / 2;
         typedef Sub<QT, NUM> B;
-        const int rg = c / 3, part = c % 3;
         const B& b = sub[kEarly ? j & 1 : 0][rg];
-        uint32_t p01, p23;
-        if (part == 0) {
+        // (a part's results are pinned to its place: left to itself the compiler computes them where they are used)
+        if constexpr (part == 0) {
             b.template scales<j>(g, D[rg], DM[rg]);
-        } else if (part == 1) {
-            kq_dword_bf16<NUM, B::kMin, false, false>(ident, b.template quads<j, 0>(g), B::kZero, D[rg], DM[rg], p01, p23);
-            d[rg][0] = p01; d[rg][1] = p23;
+        } else if constexpr (part % 2 == 1) {
+            constexpr float off = (float)(B::template base<j>() + B::kZero);
+            b.template pairs<j, w>(g, ha, hb);
+            chain_pair<NUM, B::kMin>(ha, off, D[rg], DM[rg]);
+            chain_pair<NUM, B::kMin>(hb, off, D[rg], DM[rg]);
+            asm volatile("" : "+v"(ha), "+v"(hb));
         } else {
-            kq_dword_bf16<NUM, B::kMin, false, false>(ident, b.template quads<j, 1>(g), B::kZero, D[rg], DM[rg], p01, p23);
-            d[rg][2] = p01; d[rg][3] = p23;
+            uint32_t p01, p23;
+            chain_bf16<NUM, B::kMin>(ha, hb, D[rg], DM[rg], p01, p23);
+            asm volatile("" : "+v"(p01), "+v"(p23));
+            d[rg][2 * w] = p01; d[rg][2 * w + 1] = p23;
         }
     };
     u32x4_t af[2][R];
@@ -438,31 +542,43 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
 #pragma unroll
         for (int i = 0; i < kRing && i < n; i++) xf[i] = frag(i);
         __builtin_amdgcn_sched_barrier(0);
-        static_for<2 * T>([&](auto U) {
-            constexpr int u = decltype(U)::value, j = 2 * T * st + u;
+        static_for<n>([&](auto I) {
+            constexpr int i = decltype(I)::value, u = i / MT, t = i % MT, j = 2 * T * st + u;
             constexpr int jr = kEarly ? j + 2 : j + 1;       // sub-block whose bytes are read under this one
-            if constexpr (jr == 4) {
+            // A wavefront's priority falls as it gets through the stage: the two of a SIMD would otherwise be served oldest first, and
+            // the younger would run its last third alone (203 rows: contracting took 2070 and 3180 cycles of a stage of 3340, now 2440
+            // and 2950 of 3120).
+            if constexpr (i == 0) __builtin_amdgcn_s_setprio(3);
+            else if constexpr (i == n / 4) __builtin_amdgcn_s_setprio(2);
+            else if constexpr (i == n / 2) __builtin_amdgcn_s_setprio(1);
+            else if constexpr (i == 3 * n / 4) __builtin_amdgcn_s_setprio(0);
+            if constexpr (t == 0 && (jr == 4 || (jr == 8 && !last))) {
                 put();
-                if constexpr (!last) fetch(s + 1, int_c<0>{});
-            } else if constexpr (jr == 8 && !last) {
-                put();
-                fetch(s + 1, int_c<1>{});
+                if constexpr (!kSpread && !last) fetch(s + 1, int_c<jr / 4 - 1>{});
             }
 #pragma unroll
-            for (int t = 0; t < MT; t++) {
-                const int i = u * MT + t;
+            for (int rg = 0; rg < R; rg++)
+                acc[rg][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, af[j & 1][rg]), xf[i % kRing], acc[rg][t], 0, 0, 0);
+            if constexpr (i + kRing < n) xf[i % kRing] = frag(i + kRing);
+            if constexpr (kSpread) {
+                // the next stage's copies under the first half of this one, the packed pieces of the next unit but one under the
+                // second half of the stage in which the next unit went to the slab (the wait for the copies counts on that order)
+                if constexpr (!last || st + 1 < kStages)
 #pragma unroll
-                for (int rg = 0; rg < R; rg++)
-                    acc[rg][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, af[j & 1][rg]), xf[i % kRing], acc[rg][t], 0, 0, 0);
-                if (i + kRing < n) xf[i % kRing] = frag(i + kRing);
+                    for (int q = 0; q < kCopies; q++)
+                        if (q * (n / 2) / kCopies == i) load_x_req(s + (st + 1) / kStages, (st + 1) % kStages, q);
+                if constexpr (!last && (st & 1) == 1)
 #pragma unroll
-                for (int c = 0; c < 4 * R; c++) {
-                    if (c * MT / (4 * R) != t) continue;
-                    if (c < R) { if constexpr (!last || jr < 8) read_part(int_c<jr>{}, c); }
-                    else { if constexpr (!last || j < 7) decode_part(int_c<j + 1>{}, c - R, af[(j + 1) & 1]); }
-                }
-                __builtin_amdgcn_sched_barrier(0);
+                    for (int q = 0; q < kFetch; q++)
+                        if (n / 2 + q * (n / 2) / kFetch == i) fetch_req(s + 1, int_c<st / 2>{}, q);
             }
+            constexpr int first = (t * 6 * R + MT - 1) / MT, past = ((t + 1) * 6 * R + MT - 1) / MT;   // parts of this group
+            static_for<past - first>([&](auto C) {
+                constexpr int c = first + decltype(C)::value;
+                if constexpr (c < R) { if constexpr (!last || jr < 8) read_part(int_c<jr>{}, c); }
+                else if constexpr (!last || j < 7) decode_part(int_c<j + 1>{}, int_c<(c < R ? 0 : c - R)>{}, af[(j + 1) & 1]);
+            });
+            __builtin_amdgcn_sched_barrier(0);
         });
     };
     // One super-block.  A stage's tiles must have arrived when it begins; they were requested at the start of the stage before
@@ -477,7 +593,7 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kYoung) : "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            if constexpr (!last || st + 1 < kStages) load_x(s + (st + 1) / kStages, (st + 1) % kStages);
+            if constexpr ((!work || !kSpread) && (!last || st + 1 < kStages)) load_x(s + (st + 1) / kStages, (st + 1) % kStages);
             if constexpr (work) contract(ST, LAST, s);
         });
     };
@@ -490,8 +606,7 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
         read_part(int_c<0>{}, c);
         if (kEarly) read_part(int_c<1>{}, c);
     }
-#pragma unroll
-    for (int c = 0; c < 3 * R; c++) decode_part(int_c<0>{}, c, af[0]);
+    static_for<5 * R>([&](auto C) { decode_part(int_c<0>{}, C, af[0]); });
     int s = 0;
     for (const int whole = mine < steps ? mine : steps - 1; s < whole; s++) super_block(int_c<true>{}, int_c<false>{}, s);
     if (mine == steps) {
@@ -532,13 +647,11 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
                 if (n + e < a.N) a.y[yi + e] = f32_to_bf16(o[e]);
         }
     };
+    auto gated_bf16 = [](float gv, float uv) { return bf16_to_f32(f32_to_bf16(silu_f32(gv))) * uv; };
     auto store_gated = [&](int64_t m, int64_t n, const f32x4_t& gt, const f32x4_t& ut) {
         float o[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float gv = bf16_to_f32(f32_to_bf16(gt[e])), uv = bf16_to_f32(f32_to_bf16(ut[e]));
-            o[e] = bf16_to_f32(f32_to_bf16(gv / (1.0f + expf(-gv)))) * uv;
-        }
+        for (int e = 0; e < 4; e++) o[e] = gated_bf16(bf16_to_f32(f32_to_bf16(gt[e])), bf16_to_f32(f32_to_bf16(ut[e])));
         *reinterpret_cast<u32x2_t*>(a.y + m * a.N + n) = u32x2_t{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
     };
     if constexpr (R == 1) {
@@ -563,52 +676,73 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
         }
         return;
     }
-    // two halves of K: wavefront kw keeps row group kw (in acc[0]) and adds the other half's sums to it
-    constexpr int kOwn = KW == 2 ? 1 : R;
-    const int64_t nown = n0 + (KW == 2 ? 16 * kw : 0) + 4 * g;
     if constexpr (KW == 2) {
+        // two halves of K: wavefront kw keeps tiles kw, kw + 2, .. and adds the other half's sums to them
+        constexpr int kOdd = MT / 2, kEven = MT - kOdd;
+        f32x4_t* give = red + (kw == 0 ? nw * kOdd : NW * kOdd + nw * kEven) * (R * 64) + lane;
+        const f32x4_t* take = red + (kw == 0 ? NW * kOdd + nw * kEven : nw * kOdd) * (R * 64) + lane;
 #pragma unroll
-        for (int t = 0; t < MT; t++) red[(wave * MT + t) * 64 + lane] = kw == 0 ? acc[R - 1][t] : acc[0][t];
+        for (int t = 0; t < MT; t++) {
+            if ((t & 1) == kw) continue;
+#pragma unroll
+            for (int rg = 0; rg < R; rg++) give[(t / 2 * R + rg) * 64] = acc[rg][t];
+        }
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < MT; t++) {
-            const f32x4_t p = red[((wave ^ NW) * MT + t) * 64 + lane];
-            f32x4_t m = kw == 0 ? acc[0][t] : acc[R - 1][t];
-            m[0] += p[0]; m[1] += p[1]; m[2] += p[2]; m[3] += p[3];
-            acc[0][t] = m;
+            if ((t & 1) != kw) continue;
+#pragma unroll
+            for (int rg = 0; rg < R; rg++) {
+                const f32x4_t p = take[(t / 2 * R + rg) * 64];
+                acc[rg][t][0] += p[0]; acc[rg][t][1] += p[1]; acc[rg][t][2] += p[2]; acc[rg][t][3] += p[3];
+            }
         }
         __syncthreads();
     }
     if (a.pair && !a.partial) {
-        // gate wavefronts finish the even row tiles, up wavefronts the odd ones
-        constexpr int kHalf = (MT + 1) / 2;
+        // both projections' outputs, rounded, as rows of 32 columns in LDS; gate wavefronts finish every other tile, up wavefronts
+        // the rest, eight columns a lane
+        constexpr int kOwn = (MT + KW - 1) / KW;
+        uint8_t* out = lds + wave * (kOwn * 16 * kOutRow);
 #pragma unroll
-        for (int rg = 0; rg < kOwn; rg++)
+        for (int t = 0; t < MT; t++) {
+            if (KW == 2 && (t & 1) != kw) continue;
 #pragma unroll
-            for (int t = 0; t < MT; t++)
-                if ((t & 1) != second) red[((wave * kOwn + rg) * kHalf + t / 2) * 64 + lane] = acc[rg][t];
+            for (int rg = 0; rg < R; rg++)
+                *reinterpret_cast<u32x2_t*>(out + (t / KW * 16 + r) * kOutRow + 32 * rg + 8 * g) =
+                    u32x2_t{pack_bf16(acc[rg][t][0], acc[rg][t][1]), pack_bf16(acc[rg][t][2], acc[rg][t][3])};
+        }
         __syncthreads();
-        const int other = wave ^ (NW / 2);
+        const uint8_t* gates = lds + (second ? wave - NW / 2 : wave) * (kOwn * 16 * kOutRow);
+        const uint8_t* ups = gates + NW / 2 * (kOwn * 16 * kOutRow);
+        const int row = lane >> 2;
+        const int64_t n = n0 + 8 * (lane & 3);
+        for (int o = second; o < kOwn; o += 2) {
+            const int64_t m = row_begin + 16 * (KW == 2 ? 2 * o + kw : o) + row;
+            if (m >= row_end || n >= a.N) continue;
+            const u32x4_t gt = *reinterpret_cast<const u32x4_t*>(gates + (o * 16 + row) * kOutRow + 16 * (lane & 3));
+            const u32x4_t ut = *reinterpret_cast<const u32x4_t*>(ups + (o * 16 + row) * kOutRow + 16 * (lane & 3));
+            u32x4_t h;
 #pragma unroll
-        for (int rg = 0; rg < kOwn; rg++)
-#pragma unroll
-            for (int t = 0; t < MT; t++) {
-                if ((t & 1) != second) continue;
-                const int64_t m = row_begin + 16 * t + r, n = nown + 16 * rg;
-                if (m >= row_end || n >= a.N) continue;
-                const f32x4_t p = red[((other * kOwn + rg) * kHalf + t / 2) * 64 + lane];
-                store_gated(m, n, second ? p : acc[rg][t], second ? acc[rg][t] : p);
-            }
+            for (int e = 0; e < 4; e++)
+                h[e] = pack_bf16(gated_bf16(bf16lo_to_f32(gt[e]), bf16lo_to_f32(ut[e])), gated_bf16(bf16hi_to_f32(gt[e]), bf16hi_to_f32(ut[e])));
+            *reinterpret_cast<u32x4_t*>(a.y + m * a.N + n) = h;   // (a pair has whole groups of eight columns)
+        }
         return;
     }
+    // a tile at a time through LDS of the wavefront's own, so that a store writes whole rows of 32 columns (128 bytes of partial sums)
+    uint8_t* turn = lds + wave * (16 * kTurnRow);
 #pragma unroll
     for (int t = 0; t < MT; t++) {
-        const int64_t m = row_begin + 16 * t + r;
-        if (m >= row_end) continue;
+        if (KW == 2 && (t & 1) != kw) continue;
 #pragma unroll
-        for (int rg = 0; rg < kOwn; rg++) {
-            const int64_t n = nown + 16 * rg;
-            if (n < a.N) store(second, m, n, acc[rg][t]);
+        for (int rg = 0; rg < R; rg++) *reinterpret_cast<f32x4_t*>(turn + r * kTurnRow + 64 * rg + 16 * g) = acc[rg][t];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int row = 8 * i + (lane >> 3);
+            const f32x4_t v = *reinterpret_cast<const f32x4_t*>(turn + row * kTurnRow + 16 * (lane & 7));
+            const int64_t m = row_begin + 16 * t + row, n = n0 + 4 * (lane & 7);
+            if (m < row_end && n < a.N) store(second, m, n, v);
         }
     }
 }

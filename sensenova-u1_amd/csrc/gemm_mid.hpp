@@ -13,7 +13,7 @@ struct MidArgs {
     const bf16_t* bias;      // (one matrix, no partial sums)
     const bf16_t* residual;  // [M][N] added to the rounded output (one matrix, no partial sums)
     // K split over `ksplit` workgroups per tile: fp32 sums to partial[matrix][slice][M][N], to be added by a reduction; NULL:
-    // ksplit = 1, outputs to y - for a pair silu(gate) * up, rounded as the decode kernels' gated pair rounds (N % 4 == 0).
+    // ksplit = 1, outputs to y - for a pair silu(gate) * up, rounded as the decode kernels' gated pair rounds (N % 8 == 0).
     float* partial;
     int ksplit;
     bool pair;

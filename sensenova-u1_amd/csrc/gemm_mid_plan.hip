@@ -106,7 +106,7 @@ MidPlan mid_plan(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t 
 
 int launch_mid(const MidPlan& plan, const void* x, int64_t M, const void* q, const void* q_up, int qtype, int64_t N, int64_t K,
                const void* bias, const void* residual, void* y, float* partial, int numerics, hipStream_t stream) {
-    if (plan.form < 0 || plan.slices < 1 || (q_up && (N % 4 != 0 || bias || residual))) return SNGGUF_E_BADSHAPE;
+    if (plan.form < 0 || plan.slices < 1 || (q_up && (N % 8 != 0 || bias || residual))) return SNGGUF_E_BADSHAPE;
     if (plan.slices > 1 && !partial) return SNGGUF_E_NULLPTR;
     MidArgs a{};
     a.x = static_cast<const bf16_t*>(x);

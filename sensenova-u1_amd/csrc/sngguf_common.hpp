@@ -51,6 +51,24 @@ __device__ __forceinline__ float add_residual(float v, const bf16_t* residual, i
     return residual ? bf16_to_f32(residual[idx]) + bf16_to_f32(f32_to_bf16(v)) : v;
 }
 
+// exp(-g) for a g with at most 16 significant bits (here: bf16 values)
+__device__ __forceinline__ float exp_neg(float g) {
+    const float e = __builtin_amdgcn_exp2f(g * -1.44268798828125f);               // exact product
+    const float c = __builtin_fmaf(e, g * -4.8884952e-06f, e);                    // x exp2(-g lo), lo ln 2 = 4.8884952e-6
+    return e == 0.f ? 0.f : c;                                                    // (0 x inf at g = +inf)
+}
+
+// g / (1 + exp(-g)): hardware reciprocal, then one correction step of the quotient with the exact remainder
+__device__ __forceinline__ float silu_f32(float g) {
+    const float d = 1.0f + exp_neg(g);
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float q = g * r;
+    const float c = __builtin_fmaf(__builtin_fmaf(-d, q, g), r, q);
+    // exp(-g) overflows below g = -88.7: the quotient is -0 as it stands; at g = +inf the remainder inf - inf is a NaN
+    // and the quotient +inf is the value
+    return (d < __builtin_inff() && __builtin_fabsf(g) < __builtin_inff()) ? c : q;
+}
+
 // Arithmetic of the block decode.  Num<SNGGUF_NUM_GGML_FP32> works in fp32, where every product
 // of the three formats is exact.  Num<SNGGUF_NUM_UPSTREAM_FP16> works in native fp16
 // (v_mul_f16 / v_sub_f16, round-to-nearest-even, subnormals and signed zeros kept): each
