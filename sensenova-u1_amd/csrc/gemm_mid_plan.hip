@@ -59,11 +59,7 @@ double format_step(int qtype) {
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-}  // namespace
-
-int mid_columns(int form) { return kForms[form].cols; }
-
-MidPlan mid_plan(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices) {
+MidPlan best_plan(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices) {
     MidPlan best{-1, 0, 0, 0, 1, 1e30};
     const int64_t nsb = K >> 8, cols = pair ? 2 * N : N;
     const double scale = format_step(qtype), outputs = (double)(2 * M * N);
@@ -102,6 +98,31 @@ MidPlan mid_plan(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t 
         }
     }
     return best;
+}
+
+}  // namespace
+
+int mid_columns(int form) { return kForms[form].cols; }
+
+// A call asks for its plan two to four times (how much scratch, which kernel, the launch), 0.7 - 1.7 us each with a search over some
+// hundred plans, and a layer's shapes come round with every layer: each thread keeps its last plans, a function of these
+// numbers alone, one to a slot.
+MidPlan mid_plan(int qtype, int64_t M, int64_t N, int64_t K, bool pair, int64_t max_slices) {
+    struct Slot {
+        int64_t M, N, K, max_slices;
+        int qtype, pair;
+        MidPlan plan;
+    };
+    constexpr int kSlots = 64;
+    static thread_local Slot slots[kSlots] = {};   // (M = 0: empty)
+    if (max_slices > 16) max_slices = 16;          // the most that a plan has
+    if (M <= 0) return best_plan(qtype, M, N, K, pair, max_slices);
+    const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull ^ (uint64_t)N * 0xC2B2AE3D27D4EB4Full ^ (uint64_t)K * 0x165667B19E3779F9ull) +
+                       (uint64_t)(max_slices * 64 + qtype * 2 + pair) * 0xD6E8FEB86659FD93ull;
+    Slot& slot = slots[h >> 58];
+    if (slot.M != M || slot.N != N || slot.K != K || slot.max_slices != max_slices || slot.qtype != qtype || slot.pair != (int)pair)
+        slot = Slot{M, N, K, max_slices, qtype, pair, best_plan(qtype, M, N, K, pair, max_slices)};
+    return slot.plan;
 }
 
 int launch_mid(const MidPlan& plan, const void* x, int64_t M, const void* q, const void* q_up, int qtype, int64_t N, int64_t K,
