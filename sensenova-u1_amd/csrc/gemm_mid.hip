@@ -22,7 +22,8 @@
 // Per wavefront and unit of 128 elements of K: the packed bytes are requested a unit ahead into registers (16-byte pieces,
 // consecutive lanes walking along a row) and put into a slab of the wavefront's own; the decode reads them from there.
 // Activations: 64 (or, up to 64 rows, 128) columns of every row and half of K are copied global -> LDS directly one stage ahead,
-// in rows of 128 bytes whose 16-byte chunk c sits at c ^ ((row / 2) % 8); one barrier a stage.
+// in rows of 128 bytes whose 16-byte chunk c sits at c ^ ((row / 2) % 8); one barrier a stage.  (32-row instances: two units ahead, the
+// activations through registers.)
 //
 // Measured, one projection with its reduction / pair of 12288 x 4096 and what ran before it (us; graphs of launches on weights
 // from memory, Q8_0 / Q4_K / Q6_K):
@@ -36,7 +37,8 @@
 //   203 rows  pair 68.4 -> 62.6 (Q8_0), 66.9 -> 62.7 (Q4_K), 72.7 -> 68.6 (Q6_K); 6144 x 4096 in Q4_K 30.8 -> 28.9
 //   509 rows  pair 125 -> 117, 6144 x 4096 51.5 -> 48.0, 4096 x 12288 75.4 -> 73.1 (Q8_0)
 //   1024 rows pair 227 -> 210, 6144 x 4096 72 -> 67, 4096 x 4096 57 -> 51.5 (Q4_K), 4096 x 12288 129 -> 127 (Q6_K)
-//   (96-row instances of a single projection with K split lose 3 - 5 %, 12288 x 4096 at 90 rows in Q6_K 35.1 -> 36.6; pairs of the same
+//   20 rows   4096 x 12288 in Q8_0 21.5 -> 21.1; 40 rows pair 36.1 -> 32.7 (Q4_K), 39.3 -> 37.5 (Q8_0)
+//   (96-row instances of a single projection with K split lose 2 - 3 %, 12288 x 4096 at 90 rows in Q6_K 34.5 -> 35.3; pairs of the same
 //   rows gain 4 %)
 #include "gemm_mid.hpp"
 
@@ -377,12 +379,22 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     constexpr int kStage = KW * T * kTile;
     constexpr int kStages = 4 / T;                // per super-block
     constexpr int kBlocks = 2 * MT;               // blocks of 8 rows (one request of a wavefront) in a tile
+    // a stage's copies: per tile; where only all of its tiles together divide by the wavefronts, block wave + 8 q of these in one row
+    // (24 blocks a stage, 48 rows: three copies a wavefront, not four with a quarter of them masked)
+    constexpr bool kEven = kBlocks % kWaves != 0 && KW * T * kBlocks % kWaves == 0;
     constexpr int kReq = (kBlocks + kWaves - 1) / kWaves;
+    constexpr int kCopies = kEven ? KW * T * kBlocks / kWaves : KW * T * kReq;
+    constexpr int kOffs = kEven ? kCopies : kReq;   // addresses that differ by more than the tile
     constexpr bool kEarly = MT <= 8;              // a sub-block's bytes are read one sub-block ahead of its decode
     // Copies and requests between the matrix instructions, not in one go; up to 64 rows a stage is short and waits for what it asked
     // for late (40 rows of 4096 x 12288 in Q8_0 22.5 us in one go, 24.9 spread; 509 of 6144 x 4096 51 and 48).
     constexpr bool kSpread = MT > 4;
     static_assert(!kSpread || T == 1, "two stages between a unit's requests and the next unit's");
+    // 32 rows: packed pieces two units ahead, which takes the activations through registers (see load_x).  4096 x 12288 in Q8_0 at 20 rows
+    // 23.4 -> 20.0 us, 6144 x 4096 at 30 rows 16.7 -> 14.5; 48 rows are level, 64 lose 5 % (registers).
+    constexpr bool kRegX = MT == 2;
+    constexpr int kAhead = kRegX ? 2 : 1;
+    static_assert(!kRegX || kEven, "a wavefront's blocks lie in one row");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -437,57 +449,73 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     }
     const uint8_t* __restrict__ base = q + nbase * row_bytes;
     uint8_t* slab = lds + 2 * kStage + wave * kRows * S::stride;
-    u32x4_t pre[kLoads];
-    uint16_t pre_d = 0;
+    u32x4_t pre[kAhead][kLoads];
+    uint16_t pre_d[kAhead] = {};
     // request i of unit h of super-block s of the share (a share that ends early re-reads the slice's last super-block)
     constexpr int kFetch = kLoads + (kQ6 ? 1 : 0);
     auto fetch_req = [&](int s, auto H, int i) {
         constexpr int h = decltype(H)::value;
         const uint8_t* p = base + (int64_t)(my0 + s < sb1 ? my0 + s : sb1 - 1) * kTs;
-        if (i < kLoads) pre[i] = ld_piece<S::align>(p + off[h][i]);
-        else if constexpr (kQ6) pre_d = ld_u16(p + doff);
+        if (i < kLoads) pre[h % kAhead][i] = ld_piece<S::align>(p + off[h][i]);
+        else if constexpr (kQ6) pre_d[h % kAhead] = ld_u16(p + doff);
     };
     auto fetch = [&](int s, auto H) {
 #pragma unroll
         for (int i = 0; i < kFetch; i++) fetch_req(s, H, i);
     };
-    auto put = [&]() {
+    auto put = [&](auto H) {
+        constexpr int set = decltype(H)::value % kAhead;
 #pragma unroll
-        for (int i = 0; i < kLoads; i++) *reinterpret_cast<u32x4_t*>(slab + dst[i]) = pre[i];
-        if constexpr (kQ6) *reinterpret_cast<uint16_t*>(slab + (lane & (kRows - 1)) * S::stride + 112) = pre_d;
+        for (int i = 0; i < kLoads; i++) *reinterpret_cast<u32x4_t*>(slab + dst[i]) = pre[set][i];
+        if constexpr (kQ6) *reinterpret_cast<uint16_t*>(slab + (lane & (kRows - 1)) * S::stride + 112) = pre_d[set];
     };
 
     // ---- activations: rows past the end of the tile re-read its last row ----
-    uint32_t xoff[kReq];
+    uint32_t xoff[kOffs];
 #pragma unroll
-    for (int i = 0; i < kReq; i++) {
-        const int row = 8 * (wave + kWaves * i) + (lane >> 3);
+    for (int i = 0; i < kOffs; i++) {
+        const int row = 8 * (kEven ? (wave + kWaves * i) % kBlocks : wave + kWaves * i) + (lane >> 3);
         int64_t gr = row_begin + row;
         if (gr >= row_end) gr = row_end - 1;
         xoff[i] = (uint32_t)(2 * gr * a.K + 16 * ((lane & 7) ^ ((row >> 1) & 7)));
     }
-    // (the last request of a tile that is no multiple of 64 rows is for some wavefronts only: the others make it with no lane
-    // enabled - a branch there would cut the stage into basic blocks, and the decode that belongs between the matrix
-    // instructions of one stage would be moved to the head of the next)
+    // (where the copies do not divide, the last of a tile is made with no lane enabled by the other wavefronts - a branch there would
+    // cut the stage into basic blocks, and the decode that belongs between the matrix instructions of one stage would be moved to the
+    // head of the next)
     const int last_req = __builtin_amdgcn_readfirstlane(wave < kBlocks - kWaves * (kReq - 1) ? -1 : 0);
     // request q of the tiles of stage st of super-block s of every K share
-    constexpr int kCopies = KW * T * kReq;
     auto load_x_req = [&](int s, int st, int q) {
-        const int k = q / (T * kReq), t = q / kReq % T, i = q % kReq;
-        int col = (sb0 + k * steps + s) * 512 + 128 * T * st;      // byte column
+        const int block = wave + kWaves * (kEven ? q : q % kReq), kt = kEven ? block / kBlocks : q / kReq;
+        int col = (sb0 + kt / T * steps + s) * 512 + 128 * T * st;      // byte column
         if (KW > 1 && col > xlast) col = xlast;
-        const uint8_t* xb = wave_ptr(reinterpret_cast<const uint8_t*>(a.x) + col + 128 * t);
-        const uint32_t to = lds_addr(lds) + (uint32_t)((st & 1) * kStage + (k * T + t) * kTile + (wave + kWaves * i) * 1024);
+        const uint8_t* xb = wave_ptr(reinterpret_cast<const uint8_t*>(a.x) + col + 128 * (kt % T));
+        const uint32_t to = lds_addr(lds) + (uint32_t)((st & 1) * kStage + (kEven ? 0 : kt * kTile) + block * 1024);
         // (as the dense kernels' copies: M0 holds the destination, one wait state between its write and the request)
-        if (kBlocks % kWaves != 0 && i == kReq - 1)
+        if (!kEven && kBlocks % kWaves != 0 && q % kReq == kReq - 1)
             asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
-                         ::"s"(to), "v"(xoff[i]), "s"(xb), "s"(last_req) : "memory", "m0");
+                         ::"s"(to), "v"(xoff[q % kOffs]), "s"(xb), "s"(last_req) : "memory", "m0");
         else
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(xoff[i]), "s"(xb) : "memory", "m0");
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(xoff[q % kOffs]), "s"(xb) : "memory", "m0");
     };
+    // Through registers (kRegX), and to LDS at the stage's end (store_x): a copy straight to LDS is a request that the compiler does not
+    // know of, and its waits for the packed pieces of one unit would then not let those of the next stay out.
+    u32x4_t xreg[kRegX ? kCopies : 1];
     auto load_x = [&](int s, int st) {
 #pragma unroll
-        for (int q = 0; q < kCopies; q++) load_x_req(s, st, q);
+        for (int q = 0; q < kCopies; q++) {
+            if constexpr (kRegX) {
+                const int kt = (wave + kWaves * q) / kBlocks;
+                int col = (sb0 + kt / T * steps + s) * 512 + 128 * T * st;
+                if (col > xlast) col = xlast;
+                xreg[q] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint8_t*>(a.x) + col + 128 * (kt % T) + xoff[q]);
+            } else {
+                load_x_req(s, st, q);
+            }
+        }
+    };
+    auto store_x = [&](int st) {
+#pragma unroll
+        for (int q = 0; q < (kRegX ? kCopies : 0); q++) *reinterpret_cast<u32x4_t*>(lds + (st & 1) * kStage + (wave + kWaves * q) * 1024 + 16 * lane) = xreg[q];
     };
     int foff[2];
 #pragma unroll
@@ -512,7 +540,8 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
         constexpr int j = decltype(J)::value & 7, rg = decltype(C)::value / 5, part = decltype(C)::value % 5, w = (part - 1) / 2;
         typedef Sub<QT, NUM> B;
         const B& b = sub[kEarly ? j & 1 : 0][rg];
-        // (a part's results are pinned to its place: left to itself the compiler computes them where they are used)
+        // (a part's results are pinned to its place: left to itself the compiler computes them where they are used; with few matrix
+        // instructions between them, up to 64 rows, the parts' chains hide each other's latency better unpinned)
         if constexpr (part == 0) {
             b.template scales<j>(g, D[rg], DM[rg]);
         } else if constexpr (part % 2 == 1) {
@@ -520,11 +549,11 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
             b.template pairs<j, w>(g, ha, hb);
             chain_pair<NUM, B::kMin>(ha, off, D[rg], DM[rg]);
             chain_pair<NUM, B::kMin>(hb, off, D[rg], DM[rg]);
-            asm volatile("" : "+v"(ha), "+v"(hb));
+            if constexpr (kSpread) asm volatile("" : "+v"(ha), "+v"(hb));
         } else {
             uint32_t p01, p23;
             chain_bf16<NUM, B::kMin>(ha, hb, D[rg], DM[rg], p01, p23);
-            asm volatile("" : "+v"(p01), "+v"(p23));
+            if constexpr (kSpread) asm volatile("" : "+v"(p01), "+v"(p23));
             d[rg][2 * w] = p01; d[rg][2 * w + 1] = p23;
         }
     };
@@ -553,8 +582,9 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
             else if constexpr (i == n / 2) __builtin_amdgcn_s_setprio(1);
             else if constexpr (i == 3 * n / 4) __builtin_amdgcn_s_setprio(0);
             if constexpr (t == 0 && (jr == 4 || (jr == 8 && !last))) {
-                put();
-                if constexpr (!kSpread && !last) fetch(s + 1, int_c<jr / 4 - 1>{});
+                put(int_c<jr == 4>{});
+                if constexpr (kRegX && !last) fetch(s + jr / 4, int_c<jr == 4>{});
+                else if constexpr (!kSpread && !last) fetch(s + 1, int_c<jr / 4 - 1>{});
             }
 #pragma unroll
             for (int rg = 0; rg < R; rg++)
@@ -590,17 +620,22 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
         static_for<kStages>([&](auto ST) {
             constexpr int st = decltype(ST)::value;
             constexpr int kYoung = work && !last && (T == 2 || (st & 1) == 0) ? kLoads : 0;
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kYoung) : "memory");
+            if constexpr (kRegX) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kYoung) : "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             if constexpr ((!work || !kSpread) && (!last || st + 1 < kStages)) load_x(s + (st + 1) / kStages, (st + 1) % kStages);
             if constexpr (work) contract(ST, LAST, s);
+            if constexpr (kRegX && (!last || st + 1 < kStages)) store_x(st + 1);
         });
     };
     load_x(0, 0);
     fetch(0, int_c<0>{});
-    put();
-    fetch(0, int_c<1>{});
+    if constexpr (kRegX) fetch(0, int_c<1>{});
+    store_x(0);
+    put(int_c<0>{});
+    if constexpr (kRegX) fetch(1, int_c<0>{});
+    else fetch(0, int_c<1>{});
 #pragma unroll
     for (int c = 0; c < R; c++) {
         read_part(int_c<0>{}, c);

@@ -14,15 +14,14 @@ namespace {
 // integer is formed without a convert); NUM 0: exact fp32 products, one rounding in the subtraction
 // (the - 1024 - zero rides on the accumulator input of the widening instruction).  Must be called
 // by all 64 lanes; `ident` is identity_row(lane).
-// MX: fp16 -> fp32 on the matrix cores (widen_f16x4), for kernels whose vector ALU is the busier unit, the decoders below among
-// them; without it one conversion per value, for the kernel whose matrix cores are (gemm_mid.hip; `ident` is not used then).
+// fp16 -> fp32 on the matrix cores (widen_f16x4): the vector ALU is the busier unit of the kernels that use these decoders.
 // FUSED (formats with a minimum and zero = 0): the product and the operation next to it as one fused multiply-add
 // where that gives the same bits.  NUM 0: D * q is exact in fp32 (at most 11 + 6 + 5 significant bits), so
 // fma(D, q, -DM) rounds once exactly where D * q - DM does.  NUM 1: (1024 + q) * D - 1024 * D, exact inside the
 // fused operation, rounds once to fp16(q * D); -1024 * D is exact in fp16 unless it overflows, so the caller takes
 // this form only where every |D| of the wavefront is below 64 (a scale product that large has not been seen in a
 // file; the plain form stays for it).
-template <int NUM, bool HAS_MIN, bool FUSED, bool MX>
+template <int NUM, bool HAS_MIN, bool FUSED>
 __device__ __forceinline__ void kq_dword_bf16(half4_t ident, uint32_t v, float zero, typename Num<NUM>::T D,
                                               typename Num<NUM>::T DM, uint32_t& p01, uint32_t& p23) {
     const half2_t h01 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u));
@@ -46,25 +45,12 @@ __device__ __forceinline__ void kq_dword_bf16(half4_t ident, uint32_t v, float z
             a = a - M2;
             b = b - M2;
         }
-        if constexpr (MX) {
-            const f32x4_t w = widen_f16x4(ident, a, b, f32x4_t{0.f, 0.f, 0.f, 0.f});
-            p01 = pack_bf16(w[0], w[1]);
-            p23 = pack_bf16(w[2], w[3]);
-        } else {
-            p01 = pack_bf16((float)a[0], (float)a[1]);
-            p23 = pack_bf16((float)b[0], (float)b[1]);
-        }
+        const f32x4_t w = widen_f16x4(ident, a, b, f32x4_t{0.f, 0.f, 0.f, 0.f});
+        p01 = pack_bf16(w[0], w[1]);
+        p23 = pack_bf16(w[2], w[3]);
     } else {
         const float c = -(1024.0f + zero);
-        f32x4_t qf;
-        if constexpr (MX) {
-            qf = widen_f16x4(ident, h01, h23, f32x4_t{c, c, c, c});
-        } else {
-            const _Float16 off = (_Float16)c;
-            const half2_t off2 = {off, off};
-            const half2_t i01 = h01 + off2, i23 = h23 + off2;   // whole numbers below 256: exact
-            qf = f32x4_t{(float)i01[0], (float)i01[1], (float)i23[0], (float)i23[1]};
-        }
+        const f32x4_t qf = widen_f16x4(ident, h01, h23, f32x4_t{c, c, c, c});
         float w[4];
         if constexpr (FUSED && HAS_MIN) {
 #pragma unroll
@@ -177,8 +163,8 @@ __device__ __forceinline__ u32x4_t legacy_block(half4_t ident, const uint8_t* ro
         v1 |= ((((bits >> 4) & 0xFu) * 0x00204081u) & 0x01010101u) << 4;
     }
     uint32_t a0, a1, a2, a3;
-    kq_dword_bf16<NUM, HAS_MIN, false, true>(ident, v0, kZero, d, DM, a0, a1);
-    kq_dword_bf16<NUM, HAS_MIN, false, true>(ident, v1, kZero, d, DM, a2, a3);
+    kq_dword_bf16<NUM, HAS_MIN, false>(ident, v0, kZero, d, DM, a0, a1);
+    kq_dword_bf16<NUM, HAS_MIN, false>(ident, v1, kZero, d, DM, a2, a3);
     return u32x4_t{a0, a1, a2, a3};
 }
 template <int NUM, int HALF, int TS, bool HAS_MIN, bool FIVE, typename Emit>
@@ -223,8 +209,8 @@ __device__ __forceinline__ void decode_q2_k(half4_t ident, const uint8_t* row, i
         const uint32_t byte = (sm[j >> 1] >> (8 * (2 * (j & 1) + (g >> 1)))) & 0xFFu;
         const typename A::T D = d * A::integer((int)(byte & 15u)), DM = dmin * A::integer((int)(byte >> 4));
         uint32_t a0, a1, a2, a3;
-        kq_dword_bf16<NUM, true, false, true>(ident, (qs[0] >> (2 * j)) & 0x03030303u, 0.f, D, DM, a0, a1);
-        kq_dword_bf16<NUM, true, false, true>(ident, (qs[1] >> (2 * j)) & 0x03030303u, 0.f, D, DM, a2, a3);
+        kq_dword_bf16<NUM, true, false>(ident, (qs[0] >> (2 * j)) & 0x03030303u, 0.f, D, DM, a0, a1);
+        kq_dword_bf16<NUM, true, false>(ident, (qs[1] >> (2 * j)) & 0x03030303u, 0.f, D, DM, a2, a3);
         emit(j, u32x4_t{a0, a1, a2, a3});
     }
 }
@@ -254,7 +240,7 @@ __device__ __forceinline__ void decode_q3_k(half4_t ident, const uint8_t* row, i
 #pragma unroll
         for (int w = 0; w < 2; w++) {
             const uint32_t v = ((qs[w] >> (2 * j)) & 0x03030303u) | (((hm[w] >> (4 * h + j)) & 0x01010101u) << 2);
-            kq_dword_bf16<NUM, false, false, true>(ident, v, 4.f, D, D, a[2 * w], a[2 * w + 1]);
+            kq_dword_bf16<NUM, false, false>(ident, v, 4.f, D, D, a[2 * w], a[2 * w + 1]);
         }
         emit(j, u32x4_t{a[0], a[1], a[2], a[3]});
     }
@@ -318,8 +304,8 @@ __device__ __forceinline__ void decode_q4_k_body(half4_t ident, const uint8_t* r
             const typename Num<NUM>::T D = Ds[j - 4 * HALF], DM = DMs[j - 4 * HALF];
             const uint32_t v0 = (hi ? qs[0] >> 4 : qs[0]) & 0x0F0F0F0Fu, v1 = (hi ? qs[1] >> 4 : qs[1]) & 0x0F0F0F0Fu;
             uint32_t a0, a1, a2, a3;
-            kq_dword_bf16<NUM, true, FUSED, true>(ident, v0, 0.f, D, DM, a0, a1);
-            kq_dword_bf16<NUM, true, FUSED, true>(ident, v1, 0.f, D, DM, a2, a3);
+            kq_dword_bf16<NUM, true, FUSED>(ident, v0, 0.f, D, DM, a0, a1);
+            kq_dword_bf16<NUM, true, FUSED>(ident, v1, 0.f, D, DM, a2, a3);
             emit(j - 4 * HALF, u32x4_t{a0, a1, a2, a3});
         }
     }
@@ -352,7 +338,7 @@ __device__ __forceinline__ void decode_q5_k_body(half4_t ident, const uint8_t* r
             for (int w = 0; w < 2; w++) {
                 const uint32_t lo = (hi ? qs[w] >> 4 : qs[w]) & 0x0F0F0F0Fu;
                 const uint32_t hb = ((qh[w] >> j) & 0x01010101u) << 4;
-                kq_dword_bf16<NUM, true, FUSED, true>(ident, lo | hb, 0.f, D, DM, a[2 * w], a[2 * w + 1]);
+                kq_dword_bf16<NUM, true, FUSED>(ident, lo | hb, 0.f, D, DM, a[2 * w], a[2 * w + 1]);
             }
             emit(j - 4 * HALF, u32x4_t{a[0], a[1], a[2], a[3]});
         }
@@ -390,7 +376,7 @@ __device__ __forceinline__ void decode_q6_k(half4_t ident, const uint8_t* row, i
             for (int w = 0; w < 2; w++) {
                 const uint32_t lo = (top ? ql[w] >> 4 : ql[w]) & 0x0F0F0F0Fu;
                 const uint32_t hb = ((qh[w] >> (2 * p)) & 0x03030303u) << 4;
-                kq_dword_bf16<NUM, false, false, true>(ident, lo | hb, 32.f, D, D, a[2 * w], a[2 * w + 1]);
+                kq_dword_bf16<NUM, false, false>(ident, lo | hb, 32.f, D, D, a[2 * w], a[2 * w + 1]);
             }
             emit(p, u32x4_t{a[0], a[1], a[2], a[3]});
         }
