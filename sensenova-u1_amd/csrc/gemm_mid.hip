@@ -390,6 +390,10 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     // for late (40 rows of 4096 x 12288 in Q8_0 22.5 us in one go, 24.9 spread; 509 of 6144 x 4096 51 and 48).
     constexpr bool kSpread = MT > 4;
     static_assert(!kSpread || T == 1, "two stages between a unit's requests and the next unit's");
+    // A part of the decode is pinned to its place between the matrix instructions; left to itself the compiler computes it where it is
+    // used.  Not up to 64 rows, where the parts' chains hide each other's latency better unpinned, and not at 256 rows, whose registers do
+    // not suffice for it (Q5_K in fp32 decode 46 of them spilled, 1024 rows of 4096 x 12288 164 us, unpinned 125; without spills level).
+    constexpr bool kPinned = MT > 4 && MT < 16;
     // 32 rows: packed pieces two units ahead, which takes the activations through registers (see load_x).  4096 x 12288 in Q8_0 at 20 rows
     // 23.4 -> 20.0 us, 6144 x 4096 at 30 rows 16.7 -> 14.5; 48 rows are level, 64 lose 5 % (registers).
     constexpr bool kRegX = MT == 2;
@@ -540,8 +544,6 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
         constexpr int j = decltype(J)::value & 7, rg = decltype(C)::value / 5, part = decltype(C)::value % 5, w = (part - 1) / 2;
         typedef Sub<QT, NUM> B;
         const B& b = sub[kEarly ? j & 1 : 0][rg];
-        // (a part's results are pinned to its place: left to itself the compiler computes them where they are used; with few matrix
-        // instructions between them, up to 64 rows, the parts' chains hide each other's latency better unpinned)
         if constexpr (part == 0) {
             b.template scales<j>(g, D[rg], DM[rg]);
         } else if constexpr (part % 2 == 1) {
@@ -549,11 +551,11 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
             b.template pairs<j, w>(g, ha, hb);
             chain_pair<NUM, B::kMin>(ha, off, D[rg], DM[rg]);
             chain_pair<NUM, B::kMin>(hb, off, D[rg], DM[rg]);
-            if constexpr (kSpread) asm volatile("" : "+v"(ha), "+v"(hb));
+            if constexpr (kPinned) asm volatile("" : "+v"(ha), "+v"(hb));
         } else {
             uint32_t p01, p23;
             chain_bf16<NUM, B::kMin>(ha, hb, D[rg], DM[rg], p01, p23);
-            if constexpr (kSpread) asm volatile("" : "+v"(p01), "+v"(p23));
+            if constexpr (kPinned) asm volatile("" : "+v"(p01), "+v"(p23));
             d[rg][2 * w] = p01; d[rg][2 * w + 1] = p23;
         }
     };

@@ -1,4 +1,5 @@
-"""What the compiler made of the dense tile kernel's K loop, checked on the assembly (no GPU needed: hipcc cross-compiles).
+"""What the compiler made of the dense tile kernel's K loop, checked on the assembly (no GPU needed: hipcc cross-compiles), and the
+registers that the instances of the mid-size kernel take in the built library.
 
 The four-wavefront dense kernel runs one wavefront per SIMD, so its speed rests on properties of the generated loop that
 no numerical test sees: all 256 accumulators stay in their accumulation registers across the loop (small changes to the
@@ -12,6 +13,7 @@ allocate differently without anything being wrong with the kernel: a failure her
 import os
 import re
 import shutil
+import struct
 import subprocess
 
 import pytest
@@ -57,3 +59,45 @@ def test_dense_kernel_loop_keeps_its_accumulators_in_place(tmp_path):
     for field in ("vgpr_spill_count", "sgpr_spill_count", "private_segment_fixed_size"):
         vals = re.findall(rf"\.{field}:\s+(\d+)", text)
         assert vals and all(v == "0" for v in vals), (field, vals)
+
+
+def _kernel_resources(tmp_path):
+    """{kernel symbol: its metadata's numbers} over the device code objects that the built library holds."""
+    readelf = "/opt/rocm/llvm/bin/llvm-readelf"
+    if not os.path.exists(readelf) or not os.path.exists(build.LIB_PATH):
+        pytest.skip("llvm-readelf or the built library not found")
+    with open(build.LIB_PATH, "rb") as f:
+        lib = f.read()
+    magic, pos, found, objects = b"__CLANG_OFFLOAD_BUNDLE__", -1, {}, 0
+    while (pos := lib.find(magic, pos + 1)) >= 0:   # magic, count, then (offset, size, length of the target's name, name) each
+        count, at = struct.unpack_from("<Q", lib, pos + len(magic))[0], pos + len(magic) + 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", lib, at)
+            target = lib[at + 24:at + 24 + length]
+            at += 24 + length
+            if b"gfx950" not in target or size == 0:
+                continue
+            obj = tmp_path / f"object{objects}"
+            objects += 1
+            obj.write_bytes(lib[pos + offset:pos + offset + size])
+            notes = subprocess.run([readelf, "--notes", str(obj)], capture_output=True, text=True).stdout
+            for name, body in re.findall(r"\.name: +(\S+)\n(.*?)\.wavefront_size", notes, re.S):
+                found[name] = {f: int(v) for f, v in re.findall(r"\.(\w+): +(\d+)\n", body)}
+    return found
+
+
+def _mid_instances(tmp_path):
+    """{(format, numerics, row groups, 16-row tiles, K shares, ...): numbers} of gemm_mid_kernel."""
+    out = {}
+    for name, numbers in _kernel_resources(tmp_path).items():
+        m = re.search(r"gemm_mid_kernelI((?:L[ib]\d+E)+)E", name)
+        if m:
+            out[tuple(int(v) for v in re.findall(r"L[ib](\d+)E", m.group(1)))] = numbers
+    return out
+
+
+def test_mid_size_kernel_does_not_spill(tmp_path):
+    """Spilled registers of the K loop cost up to a quarter of the time and change no result."""
+    instances = _mid_instances(tmp_path)
+    assert len(instances) >= 260
+    assert {k: v["vgpr_spill_count"] for k, v in instances.items() if v["vgpr_spill_count"] or v["private_segment_fixed_size"]} == {}
