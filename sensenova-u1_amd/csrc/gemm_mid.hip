@@ -22,8 +22,8 @@
 // Per wavefront and unit of 128 elements of K: the packed bytes are requested a unit ahead into registers (16-byte pieces,
 // consecutive lanes walking along a row) and put into a slab of the wavefront's own; the decode reads them from there.
 // Activations: 64 (or, up to 64 rows, 128) columns of every row and half of K are copied global -> LDS directly one stage ahead,
-// in rows of 128 bytes whose 16-byte chunk c sits at c ^ ((row / 2) % 8); one barrier a stage.  (32-row instances: two units ahead, the
-// activations through registers.)
+// in rows of 128 bytes whose 16-byte chunk c sits at c ^ ((row / 2) % 8); one barrier a stage.  (FAR: two units ahead, the activations
+// through registers.)
 //
 // Measured, one projection with its reduction / pair of 12288 x 4096 and what ran before it (us; graphs of launches on weights
 // from memory, Q8_0 / Q4_K / Q6_K):
@@ -56,7 +56,6 @@ namespace sngguf {
 namespace {
 
 constexpr int kWaves = 8;
-constexpr int kRing = 4;          // activation fragments read ahead
 
 template <int V> struct int_c { static constexpr int value = V; };
 template <int N, int I = 0, typename F>
@@ -82,10 +81,12 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // Unit<QT>: how the bytes that hold 128 elements of one row (half a super-block, or four blocks) travel to the wavefront's
 // slab: `pieces` 16-byte loads, piece p from byte src(h, p) of the super-block (or of the eight blocks) to byte 16 p of the
 // row's `stride`-byte slot, an odd number of 16-byte groups, so that 16 rows start in 16 different groups of LDS banks.
-// Formats whose unit is no multiple of 16 bytes end with a piece that overlaps its predecessor in memory.
+// Formats whose unit is no multiple of 16 bytes end with a piece that overlaps its predecessor in memory.  `second`: how far every piece
+// of the second unit lies behind the same piece of the first, so that one set of addresses serves both; 0 where that differs from piece
+// to piece.
 template <int TS, int PIECES, int STRIDE>
 struct UnitBlocks {   // four blocks of TS bytes
-    static constexpr int pieces = PIECES, stride = STRIDE, align = 4, last = 4 * TS - 16;
+    static constexpr int pieces = PIECES, stride = STRIDE, align = 4, last = 4 * TS - 16, second = 4 * TS;
     static __device__ __forceinline__ int src(int h, int p) { return 4 * TS * h + (p == PIECES - 1 ? last : 16 * p); }
 };
 template <int QT> struct Unit;
@@ -95,23 +96,23 @@ template <> struct Unit<SNGGUF_TYPE_Q5_0> : UnitBlocks<22, 6, 112> {};
 template <> struct Unit<SNGGUF_TYPE_Q5_1> : UnitBlocks<24, 6, 112> {};
 template <> struct Unit<SNGGUF_TYPE_Q8_0> : UnitBlocks<34, 9, 144> {};
 template <> struct Unit<SNGGUF_TYPE_Q2_K> {   // scales, quants of the half, d and dmin in the last dword
-    static constexpr int pieces = 4, stride = 80, align = 4;
+    static constexpr int pieces = 4, stride = 80, align = 4, second = 0;
     static __device__ __forceinline__ int src(int h, int p) { return p == 0 ? 0 : p == 3 ? 68 : 32 * h + 16 * p; }
 };
 template <> struct Unit<SNGGUF_TYPE_Q3_K> {   // mask, quants of the half, scales and d
-    static constexpr int pieces = 5, stride = 80, align = 2;
+    static constexpr int pieces = 5, stride = 80, align = 2, second = 0;
     static __device__ __forceinline__ int src(int h, int p) { return p < 2 ? 16 * p : p == 4 ? 94 : 32 * h + 16 * p; }
 };
 template <> struct Unit<SNGGUF_TYPE_Q4_K> {   // head, quants of the half
-    static constexpr int pieces = 5, stride = 80, align = 16;
+    static constexpr int pieces = 5, stride = 80, align = 16, second = 0;
     static __device__ __forceinline__ int src(int h, int p) { return p == 0 ? 0 : 64 * h + 16 * p; }
 };
 template <> struct Unit<SNGGUF_TYPE_Q5_K> {   // head, fifth bits, quants of the half
-    static constexpr int pieces = 7, stride = 112, align = 16;
+    static constexpr int pieces = 7, stride = 112, align = 16, second = 0;
     static __device__ __forceinline__ int src(int h, int p) { return p < 3 ? 16 * p : 64 * h + 16 * p; }
 };
 template <> struct Unit<SNGGUF_TYPE_Q6_K> {   // low and high bits of the half, scales; d follows on its own at byte 112
-    static constexpr int pieces = 7, stride = 144, align = 2;
+    static constexpr int pieces = 7, stride = 144, align = 2, second = 0;
     static __device__ __forceinline__ int src(int h, int p) { return p < 4 ? 64 * h + 16 * p : p < 6 ? 64 + 32 * h + 16 * p : 192; }
 };
 
@@ -186,8 +187,9 @@ struct SubLegacy {
         if constexpr (FIVE) {
             // bits 0 .. 3 of this quarter to bit 4 of bytes 0 .. 3
             const uint32_t bits = (((fifth >> (8 * g + 4 * W)) & 0xFu) * 0x00204081u) & 0x01010101u;
-            a = field2<0, 0xF, 1, 4, 4>(v, bits);
-            b = field2<0, 0xF, 1, 4, -4>(v >> 8, bits);
+            const uint32_t quants = (uint32_t)__builtin_amdgcn_bitop3_b32(v, 0x0F0F0F0Fu, bits << 4, 0xEA);
+            a = field<0, 0x1F>(quants);
+            b = field<0, 0x1F>(quants >> 8);
         } else {
             a = field<0, 0xF>(v);
             b = field<0, 0xF>(v >> 8);
@@ -364,8 +366,9 @@ constexpr int mid_lds_bytes() {
     return x + slab > red ? x + slab : red;
 }
 
-// R: 16-row groups per wavefront, MT: 16-row tiles of the activations, KW: wavefronts that share a K range (1 or 2).
-template <int QT, int NUM, int R, int MT, int KW>
+// R: 16-row groups per wavefront, MT: 16-row tiles of the activations, KW: wavefronts that share a K range (1 or 2), FAR: packed pieces
+// two units ahead instead of one.
+template <int QT, int NUM, int R, int MT, int KW, bool FAR>
 __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(MidArgs a) {
     typedef Unit<QT> S;
     constexpr int T = mid_tiles(MT);
@@ -394,10 +397,18 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     // used.  Not up to 64 rows, where the parts' chains hide each other's latency better unpinned, and not at 256 rows, whose registers do
     // not suffice for it (Q5_K in fp32 decode 46 of them spilled, 1024 rows of 4096 x 12288 164 us, unpinned 125; without spills level).
     constexpr bool kPinned = MT > 4 && MT < 16;
-    // 32 rows: packed pieces two units ahead, which takes the activations through registers (see load_x).  4096 x 12288 in Q8_0 at 20 rows
-    // 23.4 -> 20.0 us, 6144 x 4096 at 30 rows 16.7 -> 14.5; 48 rows are level, 64 lose 5 % (registers).
-    constexpr bool kRegX = MT == 2;
+    // Two units ahead takes the activations through registers (see load_x), about 20 more of them than one.  Narrow form of 32 rows (launch_form): us in
+    // Q4_0 / Q8_0 / Q4_K, one and two units, 12288 x 4096 at 32 rows 18.5, 23.6, 19.7 and 16.8, 19.8, 18.4.  With 48 rows level, with 64 5 %
+    // slower, and in the wide form level up to 256 workgroups and slower beyond, where a compute unit then holds one instead of two
+    // (151936 x 4096 at 24 rows 127, 160, 133 and 136, 167, 148).
+    constexpr bool kRegX = FAR;
     constexpr int kAhead = kRegX ? 2 : 1;
+    // Activation fragments read ahead; one fewer keeps the wide form of 32 and 48 rows within the 128 registers of two workgroups on a
+    // compute unit in most formats (65536 x 4096 at 32 rows in Q8_0, 130 and 124 registers: 73.8 and 69.7 us).
+    constexpr int kRing = R == 2 && MT <= 3 ? 3 : 4;
+    // The narrow form of 32 rows with one unit ahead is for launches that fill the device several times over, where other workgroups fill
+    // the gaps: raised priorities would hold these back (24576 x 4096 pair at 24 rows in Q6_K 73 us with them, 64 without).
+    constexpr bool kPrio = !(R == 1 && MT == 2 && !FAR);
     static_assert(!kRegX || kEven, "a wavefront's blocks lie in one row");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
@@ -431,7 +442,7 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     const int xlast = 2 * (int)a.K - 128 * T;
 
     // ---- packed rows: pieces of this wavefront's rows (rows past the end: the last row, never stored) ----
-    uint32_t off[2][kLoads], dst[kLoads];
+    uint32_t off[S::second ? 1 : 2][kLoads], dst[kLoads];
     const int64_t nbase = n0 < a.N ? n0 : a.N - 1;
 #pragma unroll
     for (int i = 0; i < kLoads; i++) {
@@ -442,7 +453,7 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
         if (n >= a.N) n = a.N - 1;
         const uint32_t ro = (uint32_t)((n - nbase) * row_bytes);
         off[0][i] = ro + S::src(0, fp);
-        off[1][i] = ro + S::src(1, fp);
+        if constexpr (S::second == 0) off[1][i] = ro + S::src(1, fp);
         dst[i] = (uint32_t)(fr * S::stride + 16 * fp);
     }
     uint32_t doff = 0;
@@ -460,7 +471,7 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     auto fetch_req = [&](int s, auto H, int i) {
         constexpr int h = decltype(H)::value;
         const uint8_t* p = base + (int64_t)(my0 + s < sb1 ? my0 + s : sb1 - 1) * kTs;
-        if (i < kLoads) pre[h % kAhead][i] = ld_piece<S::align>(p + off[h][i]);
+        if (i < kLoads) pre[h % kAhead][i] = ld_piece<S::align>(p + h * S::second + off[S::second ? 0 : h][i]);
         else if constexpr (kQ6) pre_d[h % kAhead] = ld_u16(p + doff);
     };
     auto fetch = [&](int s, auto H) {
@@ -579,10 +590,10 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
             // A wavefront's priority falls as it gets through the stage: the two of a SIMD would otherwise be served oldest first, and
             // the younger would run its last third alone (203 rows: contracting took 2070 and 3180 cycles of a stage of 3340, now 2440
             // and 2950 of 3120).
-            if constexpr (i == 0) __builtin_amdgcn_s_setprio(3);
-            else if constexpr (i == n / 4) __builtin_amdgcn_s_setprio(2);
-            else if constexpr (i == n / 2) __builtin_amdgcn_s_setprio(1);
-            else if constexpr (i == 3 * n / 4) __builtin_amdgcn_s_setprio(0);
+            if constexpr (kPrio && i == 0) __builtin_amdgcn_s_setprio(3);
+            else if constexpr (kPrio && i == n / 4) __builtin_amdgcn_s_setprio(2);
+            else if constexpr (kPrio && i == n / 2) __builtin_amdgcn_s_setprio(1);
+            else if constexpr (kPrio && i == 3 * n / 4) __builtin_amdgcn_s_setprio(0);
             if constexpr (t == 0 && (jr == 4 || (jr == 8 && !last))) {
                 put(int_c<jr == 4>{});
                 if constexpr (kRegX && !last) fetch(s + jr / 4, int_c<jr == 4>{});
@@ -784,22 +795,28 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     }
 }
 
-template <int QT, int NUM, int R, int MT, int KW>
+template <int QT, int NUM, int R, int MT, int KW, bool FAR>
 int launch(const MidArgs& a, hipStream_t stream) {
     constexpr int kLds = mid_lds_bytes<QT, R, MT, KW>();
     static_assert(kLds <= 160 * 1024, "LDS of a compute unit");
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<QT, NUM, R, MT, KW>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_mid_kernel<QT, NUM, R, MT, KW, FAR>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (attr != hipSuccess) return SNGGUF_E_LAUNCH;
-    gemm_mid_kernel<QT, NUM, R, MT, KW><<<dim3((unsigned)(a.col_tiles * a.row_tiles * a.ksplit)), dim3(64 * kWaves), kLds, stream>>>(a);
+    gemm_mid_kernel<QT, NUM, R, MT, KW, FAR><<<dim3((unsigned)(a.col_tiles * a.row_tiles * a.ksplit)), dim3(64 * kWaves), kLds, stream>>>(a);
     return hipGetLastError() == hipSuccess ? SNGGUF_OK : SNGGUF_E_LAUNCH;
 }
 
 template <int NUM>
 int launch_form(const MidArgs& a, int form, int mt, hipStream_t stream) {
     constexpr int QT = SNGGUF_MID_TYPE;
-#define SNGGUF_CASE(FORM, R, MT, KW) if (form == FORM && mt == MT) return launch<QT, NUM, R, MT, KW>(a, stream)
-    SNGGUF_CASE(kMidNarrow, 1, 2, 2);
+#define SNGGUF_CASE(FORM, R, MT, KW) if (form == FORM && mt == MT) return launch<QT, NUM, R, MT, KW, false>(a, stream)
+    // Two units of packed rows ahead while every compute unit has at most the two workgroups that fit it so; beyond, one unit ahead (us in
+    // Q4_0 / Q2_K / Q8_0 / Q6_K, two and one: pair of 20480 x 4096 at 32 rows, 640 workgroups, 41, 44.4, 51.6, 62.8 and 41, 40.6, 51.7, 61.6;
+    // pair of 24576 x 4096 at 24 rows 49, 50.1, 56.4, 65.3 and 44.5, 43.7, 56.4, 64.0)
+    if (form == kMidNarrow && mt == 2) {
+        if (a.col_tiles * a.row_tiles * a.ksplit <= 512) return launch<QT, NUM, 1, 2, 2, true>(a, stream);
+        return launch<QT, NUM, 1, 2, 2, false>(a, stream);
+    }
     SNGGUF_CASE(kMidNarrow, 1, 3, 2);
     SNGGUF_CASE(kMidNarrow, 1, 4, 2);
     SNGGUF_CASE(kMidWide, 2, 2, 2);

@@ -101,7 +101,9 @@ PAIRS = {
     (1500, 520, 1280): (128, 4, 24, 1), (65, 8200, 256): (128, 6, 1, 1), (65, 4104, 2304): (128, 6, 1, 3), (100, 8200, 256): (128, 8, 1, 1),
     (100, 4104, 2304): (128, 8, 1, 3), (130, 8200, 512): (128, 10, 1, 1), (150, 4104, 2304): (128, 10, 1, 3), (509, 4104, 512): (128, 13, 3, 1),
     (130, 8200, 256): (256, 10, 1, 1), (100, 8200, 2304): (256, 10, 1, 3), (203, 16392, 256): (256, 13, 1, 1), (203, 8200, 2304): (256, 13, 1, 3),
-    (209, 16392, 256): (256, 16, 1, 1), (209, 8200, 2048): (256, 16, 1, 3)}
+    (209, 16392, 256): (256, 16, 1, 1), (209, 8200, 2048): (256, 16, 1, 3),
+    # more workgroups than run at once: narrow form of 32 rows with 512 (packed rows two units ahead) and 513 (one), wide form with 385
+    (32, 16384, 512): (64, 2, 1, 1), (31, 16392, 512): (64, 2, 1, 1), (29, 24584, 1280): (128, 2, 1, 1), (44, 24584, 1280): (128, 3, 1, 1)}
 
 
 def workspace_bytes(qt, m, n, k, pair):

@@ -101,3 +101,14 @@ def test_mid_size_kernel_does_not_spill(tmp_path):
     instances = _mid_instances(tmp_path)
     assert len(instances) >= 260
     assert {k: v["vgpr_spill_count"] for k, v in instances.items() if v["vgpr_spill_count"] or v["private_segment_fixed_size"]} == {}
+
+
+def test_mid_size_kernel_leaves_room_for_two_workgroups(tmp_path):
+    """Eight wavefronts of at most 128 registers fit a compute unit twice, which launches of more than 256 workgroups count on: the
+    narrow form, and the wide form of 32 and 48 rows in the formats whose decode is small enough."""
+    wide = {2: {2, 3, 6, 7, 8, 10, 11, 12}, 3: {2, 3, 7, 10, 12}}   # 16-row tiles: ggml types
+    too_many = {}
+    for (qt, _, groups, tiles, *_), numbers in (instances := _mid_instances(tmp_path)).items():
+        if (groups == 1 or qt in wide.get(tiles, ())) and numbers["vgpr_count"] > 128:
+            too_many[qt, groups, tiles] = numbers["vgpr_count"]
+    assert instances and too_many == {}
