@@ -393,6 +393,9 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     // for late (40 rows of 4096 x 12288 in Q8_0 22.5 us in one go, 24.9 spread; 509 of 6144 x 4096 51 and 48).
     constexpr bool kSpread = MT > 4;
     static_assert(!kSpread || T == 1, "two stages between a unit's requests and the next unit's");
+    // One request a group from the stage's start on, not one every few groups, in the shortest stages that are spread (90 rows of 12288 x
+    // 4096, every few groups / every group: Q6_K 36.0 / 35.3 us, Q8_0 30.5 / 29.9; pairs 54.5 / 53.5 and 47.4 / 45.6).
+    constexpr bool kDense = MT == 6;
     // A part of the decode is pinned to its place between the matrix instructions; left to itself the compiler computes it where it is
     // used.  Not up to 64 rows, where the parts' chains hide each other's latency better unpinned, and not at 256 rows, whose registers do
     // not suffice for it (Q5_K in fp32 decode 46 of them spilled, 1024 rows of 4096 x 12288 164 us, unpinned 125; without spills level).
@@ -605,15 +608,17 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
             if constexpr (i + kRing < n) xf[i % kRing] = frag(i + kRing);
             if constexpr (kSpread) {
                 // the next stage's copies under the first half of this one, the packed pieces of the next unit but one under the
-                // second half of the stage in which the next unit went to the slab (the wait for the copies counts on that order)
+                // second half (kDense: behind the copies) of the stage in which the next unit went to the slab (the wait for the copies
+                // counts on that order)
+                static_assert(!kDense || kCopies + kFetch <= n, "a group for every request");
                 if constexpr (!last || st + 1 < kStages)
 #pragma unroll
                     for (int q = 0; q < kCopies; q++)
-                        if (q * (n / 2) / kCopies == i) load_x_req(s + (st + 1) / kStages, (st + 1) % kStages, q);
+                        if ((kDense ? q : q * (n / 2) / kCopies) == i) load_x_req(s + (st + 1) / kStages, (st + 1) % kStages, q);
                 if constexpr (!last && (st & 1) == 1)
 #pragma unroll
                     for (int q = 0; q < kFetch; q++)
-                        if (n / 2 + q * (n / 2) / kFetch == i) fetch_req(s + 1, int_c<st / 2>{}, q);
+                        if ((kDense ? kCopies + q : n / 2 + q * (n / 2) / kFetch) == i) fetch_req(s + 1, int_c<st / 2>{}, q);
             }
             constexpr int first = (t * 6 * R + MT - 1) / MT, past = ((t + 1) * 6 * R + MT - 1) / MT;   // parts of this group
             static_for<past - first>([&](auto C) {
