@@ -151,8 +151,8 @@ namespace {
 // each super-block a workgroup takes its activations from L2 (512 bytes a row at 50 bytes a ns, however many wavefronts share them),
 // decodes each group once and contracts it with every 16-row operand; and the weights come from memory.  Fitted (rms 4.7 %) to 600
 // timings: twelve shapes of 512 .. 24576 columns, 17 / 32 / 33 / 48 / 64 rows, ten formats.  Choosing between it and the plans of
-// gemm_mid_plan.hip by the two estimates is 0.3 % slower than the faster of the two in the mean, 14 % at worst (512 x 2048 at 48
-// rows, 9.1 against 8.0 us).
+// gemm_mid_plan.hip by the two estimates was 0.3 % slower than the faster of the two in the mean, 14 % at worst (512 x 2048 at 48
+// rows, 9.1 against 8.0 us), with the mid-size kernel that its estimate is fitted to; the kernel has become faster since.
 double decode_kernel_us(int qtype, int64_t M, int64_t N, int64_t K) {
     const int64_t mt = (M + 15) / 16, rg = N > 4096 ? 2 : 1, groups = (N + 16 * rg - 1) / (16 * rg);
     const double element = (double)sngguf_type_size(qtype) / (double)sngguf_block_size(qtype);   // bytes
@@ -388,7 +388,8 @@ double weight_pass_us(int qtype, int64_t N, int64_t K) {
 
 // us of that route: workgroups of 256 x 256 tiles, 1.9 us a K step with the decode in the loop and 1.2 without, the weight pass,
 // the partial sums.  Fitted (rms 11 %) to twelve shapes at 65 .. 1024 rows, ten types; the plans of gemm_mid_plan.hip are chosen in all
-// but a few of those, and choosing by the two estimates is 0.1 % slower than the faster of the two in the mean (10 % at worst).
+// but a few of those, and choosing by the two estimates was 0.1 % slower than the faster of the two in the mean (10 % at worst) with the
+// mid-size kernel of that time.
 double workspace_route_us(const LinearSplit& f, int qtype, int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), wgs = tiles * f.slices;
     const bool pass = !(f.tile_type && f.slices >= 2);
@@ -401,7 +402,7 @@ double workspace_route_us(const LinearSplit& f, int qtype, int64_t M, int64_t N,
 
 // The plan for a projection from 65 rows on with `workspace_bytes` for partial sums; form -1 where the route above is faster.  `slices`
 // of it are those that the shape has a use for with any room, whether or not it is the faster one.
-// From 2048 rows on one weight pass pays for eight row tiles and more (this route / plans, Q8_0, us: 4096 x 4096 1280 rows 71 / 54,
+// From 2048 rows on one weight pass pays for eight row tiles and more (this route / plans of that kernel, Q8_0, us: 4096 x 4096 1280 rows 71 / 54,
 // 2048 92 / 84, 3000 93 / 105; 12288 x 4096 1280 rows 141 / 124, 2048 196 / 212, 3000 280 / 317).
 sngguf::MidPlan workspace_plan(const LinearSplit& f, int qtype, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
     if (M >= 2048 || !sngguf::mid_fits(qtype, M, N, K)) return {-1, 0, 0, 0, 1, 1e30};

@@ -4,20 +4,22 @@
 // Eight wavefronts share one tile of activations; each owns 16 or 32 weight rows and (with KW = 2) one half of the
 // workgroup's K range.  Three forms (mid_plan in gemm_mid_plan.hip picks):
 //   narrow  16 rows per wavefront, two halves of K:  64 columns per workgroup, up to 64 rows, two workgroups per compute unit
-//           (one with 64 rows in Q8_0 and Q6_K, whose slabs are the widest)
+//           (one with 64 rows in Q8_0 and Q6_K, whose slabs are the widest; up to three with 32 rows and one unit ahead)
 //   wide    32 rows per wavefront, two halves of K: 128 columns, up to 208 rows
 //   long    32 rows per wavefront, all of K:        256 columns, up to 256 rows
-// (wide ends at 208 rows because its registers do: 230 - 256 of 256 are taken there.  From 209 rows on two row tiles, or the long
-// form, take 15 - 18 % longer than 208 rows.)
+// (wide ends at 208 rows because its registers do: 206 - 252 of 256 are taken there, by format.  From 209 rows on two row tiles, or the
+// long form, take 17 - 23 % longer than 208 rows.)
 // What bounds it: up to about 64 rows the latency of a step (packed bytes -> slab -> decode -> matrix instructions, which two
 // wavefronts a SIMD hide only partly), beyond that no one unit: a stage of 208 rows keeps the matrix cores busy for half of its
-// cycles, the vector ALU for about as many, and from 500 rows on the clock falls with the power drawn (1.9 GHz of 2.4), so that what
-// counts is work left out rather than cycles.  Leaving out (203 rows, pair of 12288 x 4096 in Q4_K, 67 us) the activations' copies
-// gives 54 us, the packed rows' requests 58, the decode 55, the matrix instructions 52.  So the loop is written out instruction group
+// cycles, the vector ALU for about as many, and the clock falls with the power drawn (1.85 - 1.95 GHz of 2.4), so that what
+// counts is work left out rather than cycles.  Leaving out (203 rows, pair of 12288 x 4096 in Q4_K, 67 us in that copy) the activations'
+// copies gives 54 us, the packed rows' requests 58, the decode 55, the matrix instructions 52.  So the loop is written out instruction group
 // by instruction group: two matrix instructions, the activation fragment of four groups later, a part of the next sub-block's decode
 // or one request, a scheduling fence.  Left to the compiler's scheduler the fragments are read one instruction ahead (100 us against 69).
 // Measured and not taken: 32x32x16 instructions on groups of 32 rows (12 - 16 % fewer cycles, but up to 5 % more time from 500 rows on:
-// twice the accumulator traffic per product, which the clock pays for), other cache hints on the copies (nontemporal + 10 %).
+// twice the accumulator traffic per product, which the clock pays for), other cache hints on the copies (nontemporal + 10 %); from 160
+// rows on, waiting for a unit's pieces at the head of the stage that stores them, where its own copies are not out yet (the compiler's
+// wait in mid-stage takes these in): 54 timings 0.97 - 1.04, faster in Q4_K, slower in Q6_K.
 //
 // Per wavefront and unit of 128 elements of K: the packed bytes are requested a unit ahead into registers (16-byte pieces,
 // consecutive lanes walking along a row) and put into a slab of the wavefront's own; the decode reads them from there.
@@ -25,21 +27,20 @@
 // in rows of 128 bytes whose 16-byte chunk c sits at c ^ ((row / 2) % 8); one barrier a stage.  (FAR: two units ahead, the activations
 // through registers.)
 //
-// Measured, one projection with its reduction / pair of 12288 x 4096 and what ran before it (us; graphs of launches on weights
-// from memory, Q8_0 / Q4_K / Q6_K):
-//   40 rows   pair 40 / 35 / 45 (decode kernels, two launches 66 / 57 / 67), 4096 x 12288 23 / 21 / 26 (36 / 33 / 36)
-//   203 rows  pair 65 / 61 (split tiles 84 / 83), 4096 x 12288 41 / 39 / 44 (51 / 50 / 75), 6144 x 4096 31 / 30 / 32 (37 / 37 / 49)
-//   509 rows  pair 114 / 109 (150 / 142), 4096 x 12288 70 / 70 (79 / 79)
-//   1024 rows pair 220 / 220 (dense launch with two weight passes 247 / 232), 4096 x 4096 55 / 56 (68 / 68)
-// Since then, launches back to back (us, before -> now): the requests between the matrix instructions (8 copies and 3 - 5 pieces a stage
-// and wavefront used to be issued in one go behind the barrier), falling priorities, decode without byte permutes and an epilogue that
-// writes whole rows with the hardware's exp2 and reciprocal:
-//   203 rows  pair 68.4 -> 62.6 (Q8_0), 66.9 -> 62.7 (Q4_K), 72.7 -> 68.6 (Q6_K); 6144 x 4096 in Q4_K 30.8 -> 28.9
-//   509 rows  pair 125 -> 117, 6144 x 4096 51.5 -> 48.0, 4096 x 12288 75.4 -> 73.1 (Q8_0)
-//   1024 rows pair 227 -> 210, 6144 x 4096 72 -> 67, 4096 x 4096 57 -> 51.5 (Q4_K), 4096 x 12288 129 -> 127 (Q6_K)
-//   20 rows   4096 x 12288 in Q8_0 21.5 -> 21.1; 40 rows pair 36.1 -> 32.7 (Q4_K), 39.3 -> 37.5 (Q8_0)
-//   (96-row instances of a single projection with K split lose 2 - 3 %, 12288 x 4096 at 90 rows in Q6_K 34.5 -> 35.3; pairs of the same
-//   rows gain 4 %)
+// Measured, launches back to back on weights from memory, reductions included (us; Q8_0 / Q4_K / Q6_K; pair: of 12288 x 4096).  First
+// what ran before this kernel, then the kernel with a stage's requests in one go behind the barrier, bytes widened by permutes and
+// an epilogue of single columns, then as it is:
+//   40 rows    pair            66 / 57 / 67      38 / 36 / 44       35 / 33 / 43
+//   203 rows   pair            84 / 83           71 / 64 / 73       65 / 60 / 69
+//              4096 x 12288    51 / 50 / 75      46 / 41 / 44       42 / 38 / 42
+//              6144 x 4096     37 / 37 / 49      32 / 30 / 32       29 / 28 / 31
+//   509 rows   pair            150 / 142        122 / 121 / 129    115 / 115 / 128
+//   1024 rows  pair            247 / 232           / 224              / 210
+//              4096 x 12288                     123 / 121 / 130    118 / 119 / 129
+//   90 rows    12288 x 4096                      30 / 29 / 34       30 / 27 / 35
+//   24 rows    151936 x 4096                    163 / 143 / 202    162 / 140 / 197
+// Over 290 such lines of all formats, 20 - 1024 rows, the last is 0.96 of the one before in the mean, 0.86 - 1.07; with 90 rows Q8_0, Q5_0
+// and Q6_K are up to 4 % slower than it.
 #include "gemm_mid.hpp"
 
 #include "kq_decode.hpp"
@@ -117,8 +118,8 @@ template <> struct Unit<SNGGUF_TYPE_Q6_K> {   // low and high bits of the half, 
 };
 
 // A field of MASK << P bits of every 16-bit half of v, as halves base + field with base = 2^(10 - P): under that exponent the field's
-// lowest bit is worth one, so nothing is shifted down to bit 0.  Shifts and v_bitop3 issue in 2.2 cycles with two wavefronts on a
-// SIMD; v_perm, v_and_or, the packed and the converting instructions in 4.2.
+// lowest bit is worth one, so nothing is shifted down to bit 0.  Shifts and v_bitop3 issue in 2.3 - 2.5 cycles with two wavefronts on
+// a SIMD; v_perm, v_and_or, the packed and the converting instructions in 4.2 - 4.4.
 template <int P, uint32_t MASK>
 __device__ __forceinline__ half2_t field(uint32_t v) {
     return __builtin_bit_cast(half2_t, (uint32_t)__builtin_amdgcn_bitop3_b32(v, MASK * 0x00010001u << P, (0x6400u - (P << 10)) * 0x00010001u, 0xEA));
@@ -400,10 +401,10 @@ __global__ __launch_bounds__(64 * kWaves, R == 1 ? 4 : 2) void gemm_mid_kernel(M
     // used.  Not up to 64 rows, where the parts' chains hide each other's latency better unpinned, and not at 256 rows, whose registers do
     // not suffice for it (Q5_K in fp32 decode 46 of them spilled, 1024 rows of 4096 x 12288 164 us, unpinned 125; without spills level).
     constexpr bool kPinned = MT > 4 && MT < 16;
-    // Two units ahead takes the activations through registers (see load_x), about 20 more of them than one.  Narrow form of 32 rows (launch_form): us in
-    // Q4_0 / Q8_0 / Q4_K, one and two units, 12288 x 4096 at 32 rows 18.5, 23.6, 19.7 and 16.8, 19.8, 18.4.  With 48 rows level, with 64 5 %
-    // slower, and in the wide form level up to 256 workgroups and slower beyond, where a compute unit then holds one instead of two
-    // (151936 x 4096 at 24 rows 127, 160, 133 and 136, 167, 148).
+    // Two units ahead takes the activations through registers (see load_x), about 20 more of them than one.  Narrow form of 32 rows
+    // (launch_form): us in Q4_0 / Q8_0 / Q4_K, one and two units, 12288 x 4096 at 32 rows 18.5, 23.6, 19.7 and 16.8, 19.8, 18.4.  With 48
+    // rows level, with 64 5 % slower, and in the wide form level up to 256 workgroups and slower beyond, where a compute unit then holds
+    // one instead of two (151936 x 4096 at 24 rows 127, 160, 133 and 136, 167, 148).
     constexpr bool kRegX = FAR;
     constexpr int kAhead = kRegX ? 2 : 1;
     // Activation fragments read ahead; one fewer keeps the wide form of 32 and 48 rows within the 128 registers of two workgroups on a

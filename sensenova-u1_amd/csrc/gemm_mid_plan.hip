@@ -30,7 +30,9 @@ struct FormInfo {
     double fixed, step, row;   // us of a workgroup: prologue and epilogue, a super-block, a super-block per 16 rows
 };
 // These pick the form, the tile and the split; one set for all formats.  Fitted (log least squares) to Q8_0, Q4_K and Q6_K at twelve
-// shapes, 20 .. 1024 rows; measured over all ten formats - eleven shapes of 512 .. 24576 columns and 2048 .. 12288 elements of K, 17 ..
+// shapes, 20 .. 1024 rows, with the kernel as it was when it issued a stage's requests in one go (it has become 4 % faster in the mean,
+// unevenly, - 14 .. + 7 %; on ten shapes of 203 .. 1024 rows the pick is still the fastest of five to eight plans); measured then over all
+// ten formats - eleven shapes of 512 .. 24576 columns and 2048 .. 12288 elements of K, 17 ..
 // 1900 rows, every form and tile with 1 .. 16 K slices, 36090 timings - the pick is 0.6 % slower than the fastest of them in the
 // mean (17 % at worst: 100 rows of 4096 x 4096 in Q4_0 and Q4_1).
 constexpr FormInfo kForms[] = {
@@ -41,7 +43,8 @@ constexpr FormInfo kForms[] = {
 
 // Against other kernels it takes the time itself, which these constants miss by up to a quarter from format to format: us of a plan
 // with the super-block's share scaled by format, the split's launch and sums, and the outputs, fitted to the same timings of what
-// is picked (rms 5.8 %; one set for all 9 %, with Q6_K 19 % under).
+// is picked (rms 5.8 %; one set for all 9 %, with Q6_K 19 % under).  They have not been fitted again since the kernel became faster, so a
+// shape near the border still takes the other kernel where that was the faster one then.
 double format_step(int qtype) {
     switch (qtype) {
     case SNGGUF_TYPE_Q4_0: return 0.776;

@@ -89,7 +89,7 @@ FORMS = {64: (2, 3, 4), 128: (2, 3, 4, 6, 8, 10, 13), 256: (10, 13, 16)}   # col
 @pytest.mark.parametrize("qt", TYPES)
 @pytest.mark.parametrize("pair,shapes", [(False, PROJECTIONS), (True, PAIRS)])
 def test_the_parity_tests_run_every_instance(qt, pair, shapes):
-    """What the shapes of the parity tests are listed for: all thirteen instances, with and without a K split in each form."""
+    """What the shapes of the parity tests are listed for: all thirteen forms and sizes, with and without a K split in each form."""
     assert {s: ops.mid_plan(qt, *s, pair, workspace_bytes(qt, *s, pair)) for s in shapes} == shapes
     assert {p[:2] for p in shapes.values()} == {(cols, mt) for cols in FORMS for mt in FORMS[cols]}
     assert {(p[0], p[3] > 1) for p in shapes.values()} == {(cols, split) for cols in FORMS for split in (False, True)}
